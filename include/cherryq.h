@@ -171,8 +171,8 @@ int cherryq_pack_f16(int w_bits, const void *weight, const int16_t *cherry_indic
  * NON-cherry input channel replaced by FullSymQuantizer.transform of it
  * (llama/quantizer.py:165-170) under per-row scales of `group_size` consecutive compacted normal
  * channels (llama/cherry_linear.py:69-75, llama/quantizer.py:148-152), every operation rounded
- * to the weight's dtype as torch does: bit for bit the reference's result for fp16 and fp32
- * weights.  ste != 0 gives the straight-through form the training branch feeds to the matmul,
+ * to the weight's dtype as torch does: bit for bit the reference's result for fp16, bf16 and
+ * fp32 weights.  ste != 0 gives the straight-through form the training branch feeds to the matmul,
  * (q - w) + w evaluated in the weight dtype on every channel (:97-98); ste == 0 is what
  * prepare_weight_for_inference stores (:48-61).  w_bits 2..4.  cherry_indices (int32, as the
  * QAT module keeps them) need be neither sorted nor distinct; entries outside
@@ -182,6 +182,9 @@ int cherryq_pack_f16(int w_bits, const void *weight, const int16_t *cherry_indic
 int cherryq_fake_quant_f16(int w_bits, const void *weight, const int32_t *cherry_indices, void *out,
                            int in_features, int out_features, int num_cherries, int group_size, int ste,
                            void *stream);
+int cherryq_fake_quant_bf16(int w_bits, const void *weight, const int32_t *cherry_indices, void *out,
+                            int in_features, int out_features, int num_cherries, int group_size, int ste,
+                            void *stream);
 int cherryq_fake_quant_f32(int w_bits, const void *weight, const int32_t *cherry_indices, void *out,
                            int in_features, int out_features, int num_cherries, int group_size, int ste,
                            void *stream);

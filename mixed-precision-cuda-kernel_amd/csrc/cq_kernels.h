@@ -180,9 +180,10 @@ hipError_t launch_f32(const float *vec, const uint8_t *qweight, const float *che
                       const int32_t *cherry_indices, const float *scales, float *mul, int B, int K, int N, int C,
                       int G, int accumulate, void *workspace, void *scratch, hipStream_t stream);
 
-// cq_fakequant.hip: training-side quantise-dequantise of the non-cherry columns, fp16 or fp32.
+// cq_fakequant.hip: training-side quantise-dequantise of the non-cherry columns, fp16, bf16 or fp32.
+enum class FqDtype { f16, bf16, f32 };
 bool fake_quant_supported(int K, int C, int G);
-hipError_t launch_fake_quant(int bits, bool fp32, const void *w, const int32_t *idx, void *out, int K, int N, int C,
+hipError_t launch_fake_quant(int bits, FqDtype dtype, const void *w, const int32_t *idx, void *out, int K, int N, int C,
                              int G, int ste, hipStream_t stream);
 
 // cq_decode.hip: batch-1 decode-step glue kernels.

@@ -2,7 +2,7 @@
 
 Same surface as the reference's llama/cherry_linear.py: an `nn.Linear` whose weight is fake
 quantised group-wise on the fly, except for the `cherry_indices` input channels, which stay in
-full precision.  It is what `llama.qlinear.QuantLinear.pack()` consumes.  For fp16 and fp32
+full precision.  It is what `llama.qlinear.QuantLinear.pack()` consumes.  For fp16, bf16 and fp32
 weights on a GPU the fake quantisation is one fused kernel of the HIP library (bit-identical to
 the torch operations it replaces); other dtypes, layer-wise scales and CPU tensors go through
 the torch operations.
@@ -95,8 +95,8 @@ class QuantLinear(nn.Linear):
         return keep.nonzero().squeeze(1)
 
     def _fused_fake_quant(self, weight) -> bool:
-        """Whether the HIP kernel computes this weight's fake quantisation: GPU tensor, fp16 or
-        fp32, per-row group scales of the full-range quantiser, registered channels."""
+        """Whether the HIP kernel computes this weight's fake quantisation: GPU tensor, fp16, bf16
+        or fp32, per-row group scales of the full-range quantiser, registered channels."""
         if not weight.is_cuda or self.quantizer is not FullSymQuantizer or self.weight_layerwise:
             return False
         if not getattr(self, "cherry_indices_registered", False):

@@ -49,7 +49,9 @@ _lib.cherryq_unpack_f16.argtypes = [_int, _vp, _vp, _vp, _vp, _vp, _int, _int, _
 _lib.cherryq_unpack_f16.restype = _int
 _lib.cherryq_pack_f16.argtypes = [_int, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _vp]
 _lib.cherryq_pack_f16.restype = _int
-for _name in ("cherryq_fake_quant_f16", "cherryq_fake_quant_f32"):
+_FAKE_QUANT = {torch.float16: "cherryq_fake_quant_f16", torch.bfloat16: "cherryq_fake_quant_bf16",
+               torch.float32: "cherryq_fake_quant_f32"}
+for _name in _FAKE_QUANT.values():
     getattr(_lib, _name).argtypes = [_int, _vp, _vp, _vp, _int, _int, _int, _int, _int, _vp]
     getattr(_lib, _name).restype = _int
 _lib.cherryq_vecquant_matmul_f16_static.argtypes = [_int, _vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _int, _int, _vp]
@@ -491,11 +493,11 @@ FAKE_QUANT_MAX_GROUPS = 4096
 
 
 def fake_quant_supported(weight, w_bits, group_size) -> bool:
-    """Whether fake_quant_cherryq takes this weight (GPU, fp16 or fp32, 2-D, 2..4 bits, within
+    """Whether fake_quant_cherryq takes this weight (GPU, fp16, bf16 or fp32, 2-D, 2..4 bits, within
     the kernel's channel and group limits)."""
     if not (isinstance(weight, torch.Tensor) and weight.is_cuda and weight.dim() == 2):
         return False
-    if weight.dtype not in (torch.float16, torch.float32) or w_bits not in (2, 3, 4):
+    if weight.dtype not in _FAKE_QUANT or w_bits not in (2, 3, 4):
         return False
     k = weight.shape[1]
     g = int(group_size) if int(group_size) > 0 else k
@@ -504,13 +506,13 @@ def fake_quant_supported(weight, w_bits, group_size) -> bool:
 
 def fake_quant_cherryq(w_bits, weight, cherry_indices, group_size, ste=False, out=None):
     """The weight the training-side QuantLinear multiplies with: every non-cherry input channel of
-    `weight` (out, in; fp16 or fp32) replaced by its group-wise quantise-dequantise value, bit
+    `weight` (out, in; fp16, bf16 or fp32) replaced by its group-wise quantise-dequantise value, bit
     for bit what QuantLinear._adjust_weight computes with torch operations
     (llama/cherry_linear.py:77-99, llama/quantizer.py:148-152 and 165-170), in one pass over the
     matrix.  `ste` selects the straight-through arithmetic form (q - w) + w; the gradient is
     the caller's business.  No counterpart in the reference extension."""
-    if not isinstance(weight, torch.Tensor) or weight.dtype not in (torch.float16, torch.float32):
-        raise RuntimeError("fake_quant_cherryq: weight must be an fp16 or fp32 tensor")
+    if not isinstance(weight, torch.Tensor) or weight.dtype not in _FAKE_QUANT:
+        raise RuntimeError("fake_quant_cherryq: weight must be an fp16, bf16 or fp32 tensor")
     _check(weight, "weight", weight.dtype, 2)
     dev = weight.device
     n, k = weight.shape
@@ -525,7 +527,7 @@ def fake_quant_cherryq(w_bits, weight, cherry_indices, group_size, ste=False, ou
         if out.shape != weight.shape:
             raise RuntimeError("fake_quant_cherryq: out must have the weight's shape")
     g = int(group_size) if int(group_size) > 0 else k
-    fn = _lib.cherryq_fake_quant_f16 if weight.dtype == torch.float16 else _lib.cherryq_fake_quant_f32
+    fn = getattr(_lib, _FAKE_QUANT[weight.dtype])
     with torch.cuda.device(dev):
         rc = fn(int(w_bits), weight.data_ptr(), _ptr(idx), out.data_ptr(), k, n, idx.numel(), g, int(bool(ste)),
                 _current_stream(dev.index))

@@ -246,3 +246,49 @@ def test_every_fp16_weight_under_every_fp16_group_maximum(qc, bits):
                 np.testing.assert_array_equal(bits_of(got[m - m0:m - m0 + 1].cpu().numpy()),
                                               bits_of(orc.adjust_weight(row, np.empty(0, np.int64), bits, k)))
         del w, got, s, want, same
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,k,c,g", [(5, 8, 0, 8), (3, 2048, 8, 128), (3, 2056, 8, 128), (700, 4096, 16, 128), (3, 16384, 64, 96),
+                                     (3, 16392, 64, 128), (2100, 1032, 12, 9), (2, 32768, 128, 128), (2, 32776, 128, 64),
+                                     (2, 65536, 256, 128), (9, 1003, 7, 128), (4, 512, 512, 128)])
+def test_row_kernel_edges_against_the_torch_operations(qc, dtype, n, k, c, g):
+    """Every count of chunks a thread owns and the sizes on both sides of its steps, more rows than
+    workgroups, ragged last groups, rows of cherries only: bit for bit the training module's torch
+    operations in the weight's own dtype (the branch it takes for CPU tensors), both forms."""
+    announce("fake-quant rows", dtype, n, k, c, g)
+    from llama.cherry_linear import QuantLinear as TrainLinear
+    gen = torch.Generator(device="cuda").manual_seed(k + n)
+    w = (torch.randn(n, k, device="cuda", generator=gen) * 0.02).to(dtype)
+    w[0, ::3] = w[0].abs().max()                       # many elements on the clamp
+    w[1, : k // 2] *= 1e-3                             # ratios that round across .5
+    w[n - 1] = 0
+    idx = torch.randperm(k, device="cuda", generator=gen)[:c].int()
+    with torch.device("cuda"):
+        lin = TrainLinear(k, n, w_bits=4, group_size=g, cherryq=True, cherry_fraction=0).to(dtype)
+    lin.register_cherry_indices(idx)
+    lin._fused_fake_quant = lambda weight: False
+    view = torch.int32 if dtype == torch.float32 else torch.int16
+    for ste in (False, True):
+        got = qc.fake_quant_cherryq(4, w, idx, g, ste=ste)
+        want = lin._adjust_weight(w, ste=ste) if c < k else w
+        assert torch.equal(got.view(view), want.view(view)), (ste, (got != want).nonzero()[:3].tolist())
+
+
+def test_every_bf16_weight_under_sampled_bf16_group_maxima(qc):
+    """bf16 rounds the quotient from a product with the hardware reciprocal: every bit pattern of magnitude <= M,
+    for every mantissa of M over a few exponents, against torch's own bf16 operations."""
+    announce("fake-quant bf16 quotients")
+    from llama.quantizer import FullSymQuantizer
+    k = 65536
+    pats = torch.arange(k, dtype=torch.int32, device="cuda").to(torch.int16)
+    mags = pats.to(torch.int32) & 0x7fff
+    none = torch.empty(0, dtype=torch.int32, device="cuda")
+    for exponent in (1, 60, 110, 122, 127, 200):
+        mx_pat = (exponent << 7) + torch.arange(128, dtype=torch.int32, device="cuda")
+        mx = mx_pat.to(torch.int16).view(torch.bfloat16)
+        w = torch.where(mags[None, :] <= mx_pat[:, None], pats.view(torch.bfloat16)[None, :], mx[:, None]).contiguous()
+        for bits in (2, 3, 4):
+            got = qc.fake_quant_cherryq(bits, w, none, k)
+            want = FullSymQuantizer.transform(w, FullSymQuantizer.get_scaling_factor(w, None, bits, False), bits)
+            assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (exponent, bits)
