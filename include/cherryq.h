@@ -154,6 +154,15 @@ int cherryq_unpack_f16(int w_bits, const uint8_t *qweight, const void *cherry_we
                        void *stream);
 
 /*
+ * The channels of a pack() call in the order it wants them: `cherry_indices` (num_cherries of them, in
+ * any order, index_bytes = 2, 4 or 8 bytes each) sorted ascending into `sorted`; *bad (device memory
+ * or pinned host memory, valid once the launch has completed) becomes 1 if a channel lies outside
+ * [0, in_features) or is named twice, else 0.  in_features <= 32768.
+ */
+int cherryq_sort_channels(const void *cherry_indices, int index_bytes, int16_t *sorted, int *bad, int num_cherries,
+                          int in_features, void *stream);
+
+/*
  * pack() on the device: dense fp16 `weight` (out_features, in_features), row-major, and the
  * ASCENDING cherry channels -> qweight, scales (ceil(Kn/group_size), out_features) and
  * cherry_weight (num_cherries, out_features), bit for bit what QuantLinear.pack() computes on

@@ -64,7 +64,6 @@ size_t scratch_bytes(int B, int K, int N, int C) {
     return bytes;
 }
 
-static inline bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
 static int check_tensors(const void *vec, const void *qweight, const void *cherry_weight,
                          const void *cherry_indices, const void *scales, const void *mul, int B, int K, int N,
@@ -253,6 +252,16 @@ int cherryq_unpack_f16(int w_bits, const uint8_t *qweight, const void *cherry_we
 }
 
 // ---- device-side pack, fake quantisation ----------------------------------------------------
+
+int cherryq_sort_channels(const void *cherry_indices, int index_bytes, int16_t *sorted, int *bad, int num_cherries,
+                          int in_features, void *stream) {
+    if (index_bytes != 2 && index_bytes != 4 && index_bytes != 8) return CHERRYQ_E_SHAPE;
+    if (num_cherries <= 0 || in_features <= 0 || in_features > 32768) return CHERRYQ_E_SHAPE;
+    if (!cherry_indices || !sorted || !bad) return CHERRYQ_E_NULL;
+    if (!cq::aligned(cherry_indices, index_bytes) || !cq::aligned(sorted, 2) || !cq::aligned(bad, 4)) return CHERRYQ_E_ALIGN;
+    return (int)cq::launch_sort_channels(cherry_indices, index_bytes, sorted, bad, num_cherries, in_features,
+                                         reinterpret_cast<hipStream_t>(stream));
+}
 
 int cherryq_pack_f16(int w_bits, const void *weight, const int16_t *cherry_indices, uint8_t *qweight, void *scales,
                      void *cherry_weight, int in_features, int out_features, int num_cherries, int group_size,

@@ -8,6 +8,8 @@
 
 namespace cq {
 
+static inline bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
+
 size_t workspace_bytes(int B, int K, int N, int C);
 
 // cq_generic.hip
@@ -170,6 +172,7 @@ hipError_t launch_stream_unpack(int bits, const uint8_t *stream, uint8_t *qweigh
                                 int16_t *cherry_indices, __half *scales, int K, int N, int C, int G, hipStream_t s);
 
 // cq_pack.hip: dense fp16 weight -> packed buffers on the device.
+hipError_t launch_sort_channels(const void *idx, int index_bytes, int16_t *out, int *bad, int C, int K, hipStream_t stream);
 hipError_t launch_pack(int bits, const __half *w, const int16_t *idx, uint8_t *qweight, __half *scales,
                        __half *cherry_weight, int K, int N, int C, int G, hipStream_t stream);
 

@@ -84,42 +84,74 @@ __host__ __device__ constexpr int s3_bit(int q) {
 }
 
 // ---- prepack: reference buffers -> stream ------------------------------------------------------
-template <int BITS>
-__device__ inline uint32_t ref_code(const uint8_t *__restrict__ qweight, int k, int n, int N) {
-    if (BITS == 4) return (qweight[(size_t)(k >> 1) * N + n] >> (4 * (k & 1))) & 15u;
-    const size_t r = (size_t)(k >> 3) * 3;
-    const uint32_t w24 = qweight[r * N + n] | (qweight[(r + 1) * N + n] << 8) | (qweight[(r + 2) * N + n] << 16);
-    return (w24 >> (3 * (k & 7))) & 7u;
-}
+// A workgroup rearranges one unit (128 positions) of 8 tiles (128 columns): its packed bytes are read 128 bytes a
+// row into LDS, where each lane of a tile collects the bytes of its column and stores its dwords; a tile's
+// wavefront writes the unit as one contiguous piece.  The last 8 blockIdx.y take the tiles' scales and
+// cherry rows.  Bound by HBM: the packed bytes once in, once out.  MI355X, 5120 -> 13824 in 3 bits: 16 us (3.5 TB/s
+// read + written); one workgroup a tile gathering single bytes from 16-byte runs took 192.
+constexpr int kPackTiles = 8;
 
 template <int BITS>
 __global__ __launch_bounds__(256) void stream_pack_kernel(const uint8_t *__restrict__ qweight,
                                                           const __half *__restrict__ cherry_weight,
                                                           const __half *__restrict__ scales,
-                                                          uint8_t *__restrict__ stream, int G, StreamGeo geo) {
-    const int tile = blockIdx.x;
-    uint8_t *rec = stream + geo.hdr_bytes + (size_t)tile * geo.record_bytes;
-    const int N = geo.N, Kn = geo.Kn;
-    // sections the kernel never writes codes into start out zero (padding)
-    for (uint32_t i = threadIdx.x; i < geo.off_units / 4; i += 256) reinterpret_cast<uint32_t *>(rec)[i] = 0u;
+                                                          uint8_t *__restrict__ stream, int G, int dwords, StreamGeo geo) {
+    const int N = geo.N, Kn = geo.Kn, t = threadIdx.x;
+    if ((int)blockIdx.y >= geo.ng) {
+        const int tile = blockIdx.x * kPackTiles + (int)blockIdx.y - geo.ng;
+        if (tile >= geo.ntiles) return;
+        __half *rec = reinterpret_cast<__half *>(stream + geo.hdr_bytes + (size_t)tile * geo.record_bytes);
+        const int cherry0 = (int)(geo.off_cherry / 2);
+        for (int i = t; i < (int)(geo.off_units / 2); i += 256) {
+            __half v = __float2half(0.f);  // the padding of the sections
+            if (i < geo.ng * 16) {
+                const int g = i >> 4, n = tile * 16 + (i & 15);
+                if (n < N) v = scales[(size_t)(g * kStreamUnitK / G) * N + n];
+            } else if (i >= cherry0 && i < cherry0 + geo.C * 16) {
+                // piece (lg, nn): 8 halves = cherry rows 8 lg .. 8 lg + 7 of column nn
+                const int piece = (i - cherry0) >> 3, e = (i - cherry0) & 7, lg = piece >> 4, n = tile * 16 + (piece & 15);
+                if (n < N) v = cherry_weight[(size_t)(8 * lg + e) * N + n];
+            }
+            rec[i] = v;
+        }
+        return;
+    }
+    constexpr int ROWS = 16 * BITS, STRIDE = 132, DW = BITS;  // bytes of LDS a row: 33 dwords
+    __shared__ uint32_t s_q[ROWS * STRIDE / 4];
+    const int g = blockIdx.y, n0 = blockIdx.x * kPackTiles * 16, row0 = g * ROWS, rows = Kn / 8 * BITS;
+    for (int e = t; e < ROWS * 32; e += 256) {
+        const int r = e >> 5, n = n0 + 4 * (e & 31);
+        uint32_t v = 0;
+        if (row0 + r < rows) {
+            const uint8_t *src = qweight + (size_t)(row0 + r) * N + n;
+            if (dwords) {
+                if (n < N) v = *reinterpret_cast<const uint32_t *>(src);
+            } else {
+                for (int b = 0; b < 4; b++)
+                    if (n + b < N) v |= (uint32_t)src[b] << (8 * b);
+            }
+        }
+        s_q[r * (STRIDE / 4) + (e & 31)] = v;
+    }
     __syncthreads();
-    for (int i = threadIdx.x; i < geo.ng * 16; i += 256) {
-        const int g = i >> 4, n = tile * 16 + (i & 15);
-        reinterpret_cast<__half *>(rec)[i] = n < N ? scales[(size_t)(g * kStreamUnitK / G) * N + n] : __float2half(0.f);
-    }
-    for (int i = threadIdx.x; i < geo.C * 16; i += 256) {
-        // piece (lg, nn): 8 halves = cherry rows 8 lg .. 8 lg + 7 of column nn
-        const int piece = i >> 3, e = i & 7, lg = piece >> 4, n = tile * 16 + (piece & 15);
-        reinterpret_cast<__half *>(rec + geo.off_cherry)[i] =
-            n < N ? cherry_weight[(size_t)(8 * lg + e) * N + n] : __float2half(0.f);
-    }
-    constexpr int DW = BITS;  // dwords per lane and unit
-    for (int i = threadIdx.x; i < geo.ng * 64; i += 256) {
-        const int g = i >> 6, lane = i & 63, kq = lane >> 4, n = tile * 16 + (lane & 15);
+    const uint8_t *bytes = reinterpret_cast<const uint8_t *>(s_q);
+    const int lane = t & 63, kq = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < kPackTiles / 4; i++) {
+        const int tl = (t >> 6) + 4 * i, tile = blockIdx.x * kPackTiles + tl;
+        if (tile >= geo.ntiles) return;
+        const uint8_t *src = bytes + (size_t)kq * (ROWS / 4) * STRIDE + tl * 16 + (lane & 15);
+        uint32_t part[4];  // 8 codes each
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            part[u] = 0;
+#pragma unroll
+            for (int b = 0; b < BITS; b++) part[u] |= (uint32_t)src[(u * BITS + b) * STRIDE] << (8 * b);
+        }
         uint32_t d[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
         for (int q = 0; q < 32; q++) {
-            const int k = g * kStreamUnitK + 32 * kq + q;
-            const uint32_t code = (k < Kn && n < N) ? ref_code<BITS>(qweight, k, n, N) : 0u;
+            const uint32_t code = (part[q >> 3] >> (BITS * (q & 7))) & ((1u << BITS) - 1u);
             if (BITS == 4) {
                 d[s4_dword(q)] |= code << s4_bit(q);
             } else if (s3_dword(q) < 3) {
@@ -131,7 +163,9 @@ __global__ __launch_bounds__(256) void stream_pack_kernel(const uint8_t *__restr
                 d[2] |= ((code >> 2) & 1u) << b;
             }
         }
-        uint32_t *o = reinterpret_cast<uint32_t *>(rec + geo.off_units + (size_t)g * (64 * DW * 4)) + lane * DW;
+        uint32_t *o = reinterpret_cast<uint32_t *>(stream + geo.hdr_bytes + (size_t)tile * geo.record_bytes + geo.off_units +
+                                                   (size_t)g * (64 * DW * 4)) + lane * DW;
+#pragma unroll
         for (int j = 0; j < DW; j++) o[j] = d[j];
     }
 }
@@ -1719,10 +1753,12 @@ hipError_t launch_stream_pack(int bits, const uint8_t *qweight, const __half *ch
     const StreamGeo geo = stream_geo(bits, K, N, C);
     hipLaunchKernelGGL(stream_header_kernel, dim3(ceil_div((int)geo.hdr_bytes, 256)), dim3(256), 0, s, cherry_indices, stream,
                        geo);
+    const dim3 grid(ceil_div(geo.ntiles, kPackTiles), geo.ng + kPackTiles);
+    const int dwords = N % 4 == 0 && aligned(qweight, 4);
     if (bits == 4)
-        hipLaunchKernelGGL(stream_pack_kernel<4>, dim3(geo.ntiles), dim3(256), 0, s, qweight, cherry_weight, scales, stream, G, geo);
+        hipLaunchKernelGGL(stream_pack_kernel<4>, grid, dim3(256), 0, s, qweight, cherry_weight, scales, stream, G, dwords, geo);
     else
-        hipLaunchKernelGGL(stream_pack_kernel<3>, dim3(geo.ntiles), dim3(256), 0, s, qweight, cherry_weight, scales, stream, G, geo);
+        hipLaunchKernelGGL(stream_pack_kernel<3>, grid, dim3(256), 0, s, qweight, cherry_weight, scales, stream, G, dwords, geo);
     return hipGetLastError();
 }
 

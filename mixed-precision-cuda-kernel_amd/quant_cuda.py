@@ -23,6 +23,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import threading
 from pathlib import Path
 
 import torch
@@ -49,6 +50,8 @@ _lib.cherryq_unpack_f16.argtypes = [_int, _vp, _vp, _vp, _vp, _vp, _int, _int, _
 _lib.cherryq_unpack_f16.restype = _int
 _lib.cherryq_pack_f16.argtypes = [_int, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _vp]
 _lib.cherryq_pack_f16.restype = _int
+_lib.cherryq_sort_channels.argtypes = [_vp, _int, _vp, _vp, _int, _int, _vp]
+_lib.cherryq_sort_channels.restype = _int
 _FAKE_QUANT = {torch.float16: "cherryq_fake_quant_f16", torch.bfloat16: "cherryq_fake_quant_bf16",
                torch.float32: "cherryq_fake_quant_f32"}
 for _name in _FAKE_QUANT.values():
@@ -346,6 +349,16 @@ def unpack_cherryq(w_bits, qweight, cherry_weight, cherry_indices, scaling_facto
     return dense
 
 
+class _SortFlag(threading.local):
+    """Per thread: the pinned word in which the sorting launch reports bad channels, and an event behind it."""
+
+    def __init__(self):
+        self.word, self.event = None, None
+
+
+_sort_flag = _SortFlag()
+
+
 def pack_cherryq(w_bits, weight, cherry_indices, group_size):
     """pack() on the GPU: dense fp16 `weight` (out, in) and the cherry channels (any order, any
     integer dtype) -> (cherry_indices int16 ascending, cherry_weight, qweight, scales) in the
@@ -356,21 +369,40 @@ def pack_cherryq(w_bits, weight, cherry_indices, group_size):
     if w_bits not in (3, 4):
         raise NotImplementedError(f"{w_bits} bit is not implemented yet.")
     n, k = weight.shape
-    idx = cherry_indices.to(device=dev).sort().values
-    c = idx.numel()
-    if c and (int(idx[0]) < 0 or int(idx[-1]) >= k or bool((idx[1:] == idx[:-1]).any())):
-        raise RuntimeError("cherry_indices must be distinct channels in [0, in_features)")
-    idx = idx.to(torch.int16).contiguous()
+    c = cherry_indices.numel()
     group_size = int(group_size) if int(group_size) != -1 else k
     kn = k - c
+    if c > k or (c and k > 32768):
+        raise RuntimeError("cherry_indices must be distinct channels in [0, in_features), in_features at most 32768")
     if k % 8 or c % 8 or group_size <= 0:
         raise RuntimeError(f"pack_cherryq: in_features={k}, num_cherries={c}, group_size={group_size} not packable")
+    src = cherry_indices.to(device=dev)
+    if src.dtype not in (torch.int16, torch.int32, torch.int64):
+        src = src.to(torch.int64)
+    src = src.contiguous()
+    idx = torch.empty(c, dtype=torch.int16, device=dev)
     qweight = torch.empty((kn // 8 * w_bits, n), dtype=torch.uint8, device=dev)
     scales = torch.empty((-(-kn // group_size), n), dtype=torch.float16, device=dev)
     cherry_weight = torch.empty((c, n), dtype=torch.float16, device=dev)
+    flag = _sort_flag
     with torch.cuda.device(dev):
+        stream = _current_stream(dev.index)
+        if c:
+            if flag.word is None:
+                flag.word, flag.event = torch.zeros(1, dtype=torch.int32, pin_memory=True), {}
+            if dev.index not in flag.event:
+                flag.event[dev.index] = torch.cuda.Event()
+            rc = _lib.cherryq_sort_channels(src.data_ptr(), src.element_size(), idx.data_ptr(), flag.word.data_ptr(), c, k, stream)
+            if rc != 0:
+                _fail(rc, "pack_cherryq")
+            flag.event[dev.index].record()
         rc = _lib.cherryq_pack_f16(w_bits, weight.data_ptr(), _ptr(idx), _ptr(qweight), _ptr(scales),
-                                   _ptr(cherry_weight), k, n, c, group_size, _current_stream(dev.index))
+                                   _ptr(cherry_weight), k, n, c, group_size, stream)
+        if c:
+            # the packing launch, safe for any channels, runs while the host waits for the small one in front of it
+            flag.event[dev.index].synchronize()
+            if int(flag.word[0]):
+                raise RuntimeError("cherry_indices must be distinct channels in [0, in_features)")
     if rc != 0:
         _fail(rc, "pack_cherryq")
     return idx, cherry_weight, qweight, scales

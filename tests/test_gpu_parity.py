@@ -837,3 +837,48 @@ def test_empty_batch_is_a_no_op(qc):
     y = q(torch.zeros(2, 0, k, dtype=torch.float16, device="cuda"))
     assert y.shape == (2, 0, n)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("bits", [3, 4])
+@pytest.mark.parametrize("n,k,g,where", [(4, 1024, 128, "front"), (8, 1040, 128, "back"), (132, 2048, 64, "middle"),
+                                         (128, 1024, 8, "middle"), (260, 1032, 120, "spread"), (8, 4096, 128, "front"),
+                                         (12, 512, 128, "spread"), (6, 512, 128, "spread"), (8, 512, 256, "middle")])
+def test_device_pack_tile_edges(bits, n, k, g, where):
+    """Row counts around a workgroup's 128 rows and its dwords of four, groups of 8 to 256 (the last one ragged),
+    64 cherries in one run (a group's columns then span up to 26 chunks) or spread, unsorted: the packed
+    buffers equal the host's, byte for byte, and the stream made of them equals the oracle's."""
+    announce("device pack edges", bits, n, k, g, where)
+    import quant_cuda
+    from llama.cherry_linear import QuantLinear as TrainLinear
+    from llama.qlinear import QuantLinear
+    gen = torch.Generator().manual_seed(k + n)
+    c = 64
+    first = {"front": 0, "back": k - c, "middle": k // 2 - 5}.get(where)
+    idx = torch.randperm(k, generator=gen)[:c] if first is None else first + torch.randperm(c, generator=gen)
+    lin = TrainLinear(k, n, bias=False, w_bits=bits, group_size=g, cherryq=True, cherry_fraction=c / k).half()
+    lin.weight.data.copy_((torch.randn(n, k, generator=gen) * 0.02).half())
+    lin.weight.data[0] = 0
+    lin.register_cherry_indices(idx)
+    host = QuantLinear(bits, g, lin.quantizer, c / k, k, n, bias=False) if n % 8 == 0 else None
+    got = quant_cuda.pack_cherryq(bits, lin.weight.data.cuda(), idx.cuda(), g)
+    if host is None:  # the module wants multiples of 8: pad the rows, keep the columns asked for
+        pad = TrainLinear(k, 8, bias=False, w_bits=bits, group_size=g, cherryq=True, cherry_fraction=c / k).half()
+        pad.weight.data.zero_()
+        pad.weight.data[:n % 8] = lin.weight.data[n - n % 8:]
+        pad.register_cherry_indices(idx)
+        host = QuantLinear(bits, g, lin.quantizer, c / k, k, 8, bias=False)
+        host.pack(pad)
+        want = [host.cherry_indices] + [t[:, :n % 8] for t in (host.cherry_weight, host.qweight, host.scales)]
+        got = [got[0]] + [t[:, n - n % 8:] for t in got[1:]]
+    else:
+        host.pack(lin)
+        want = [host.cherry_indices, host.cherry_weight, host.qweight, host.scales]
+    for a, b, name in zip(got, want, ("indices", "cherry_weight", "qweight", "scales")):
+        assert torch.equal(a.cpu(), b), name
+    if g % 128 == 0 and n % 8 == 0:
+        stream = quant_cuda.prepack_cherryq(bits, got[2], got[1], got[0], got[3], k, g)
+        p = {"cherry_indices": got[0], "cherry_weight": got[1], "qweight": got[2], "scales": got[3]}
+        assert np.array_equal(stream.cpu().numpy(), orc.stream_pack({m: v.cpu().numpy() for m, v in p.items()}, bits, g, k))
+    for bad in (torch.full((c,), 3), idx + k):
+        with pytest.raises(RuntimeError):
+            quant_cuda.pack_cherryq(bits, lin.weight.data.cuda(), bad, g)
