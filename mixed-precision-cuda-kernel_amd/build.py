@@ -1,4 +1,5 @@
-"""Builds libcherryq.so (HIP kernels + C ABI) for gfx950 with hipcc, in-tree.
+"""Builds libcherryq.so (HIP kernels + C ABI) for gfx950 with hipcc and cherryq_host.so (the host side of
+the Python binding) with g++, in-tree.
 
     python build.py            # rebuild if any source is newer than the library
     python build.py --force
@@ -19,6 +20,7 @@ OBJ = HERE / "build"
 LIB = HERE / "libcherryq.so"
 PROBE_LIB = HERE / "libcherryq_probe.so"  # bench-only roofline reference kernels, not part of the product library
 SOURCES = ["cq_api.hip", "cq_generic.hip", "cq_matvec.hip", "cq_stream.hip", "cq_stream_cu.hip", "cq_batch.hip", "cq_gemm.hip", "cq_f32.hip", "cq_decode.hip", "cq_pack.hip", "cq_fakequant.hip"]
+HOST_LIB = HERE / "cherryq_host.so"  # host side of the Python binding (g++, linked against torch)
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc",
@@ -32,10 +34,26 @@ def _deps():
 
 
 def needs_build() -> bool:
-    if not LIB.exists():
+    if not LIB.exists() or not HOST_LIB.exists():
         return True
-    t = LIB.stat().st_mtime
+    t = min(LIB.stat().st_mtime, HOST_LIB.stat().st_mtime)
     return any(p.stat().st_mtime > t for p in _deps())
+
+
+def build_host():
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    lib = Path(torch.__file__).resolve().parent / "lib"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-isystem{p}" for p in (*include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"])),
+           str(CSRC / "cq_host.cpp"), "-o", str(HOST_LIB),
+           f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10", "-lc10_hip"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("host binding failed:\n" + r.stdout + r.stderr)
 
 
 def build(force: bool = False, verbose: bool = False) -> Path:
@@ -67,7 +85,9 @@ def build(force: bool = False, verbose: bool = False) -> Path:
         return out
 
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as ex:
+        host = ex.submit(build_host)
         objs = list(ex.map(compile_one, SOURCES))
+        host.result()
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc", "-o", str(LIB), *map(str, objs)]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:

@@ -1,0 +1,349 @@
+// Host side of the Python binding: the calls a decoding program makes for every layer and token, from the
+// Python arguments to the kernel launch in one native function.
+//
+// A batch-1 call costs 4 to 7 us on the GPU; checking six tensors, looking up buffers and passing sixteen
+// arguments through ctypes costs two to three times that in Python, so single calls are bound by the
+// host.  These functions do the same checks on the tensor objects directly.  They take the call only when
+// everything is as the kernels need it and return None otherwise, launching nothing: the caller's Python code then
+// takes the general route (other devices, released layers, large prompts) or words the error.
+//
+// Host-only translation unit (g++).  The library's C entry points come in as addresses (bind()), so it links
+// against torch alone.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/InferenceMode.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <algorithm>
+#include <array>
+#include <cstdint>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <utility>
+#include <vector>
+
+namespace {
+
+using at::Tensor;
+
+using VecquantFn = int (*)(const void *, const void *, const void *, const void *, const void *, void *, int, int, int, int,
+                           int, int, void *, size_t, void *, size_t, void *);
+using SizeFn = size_t (*)(int, int, int, int);
+using PrepackedScratchFn = size_t (*)(int, int, int, int, int);
+using MatvecPrepackedFn = int (*)(int, const void *, const void *, size_t, void *, int, int, int, int, int, void *);
+using MatmulPrepackedFn = int (*)(int, const void *, const void *, size_t, void *, int, int, int, int, int, void *, size_t,
+                                  void *);
+using ShapeFn = int (*)(int, int, int, int, int, int);
+
+struct Api {
+    VecquantFn vecquant4, vecquant3, vecquant3_f32;
+    SizeFn workspace, scratch, scratch_f32;
+    PrepackedScratchFn prepacked_scratch;
+    MatvecPrepackedFn matvec_prepacked;
+    MatmulPrepackedFn matmul_prepacked;
+    ShapeFn prepack_supported, rows_recommended;
+} api;
+
+// ---- buffers kept per (device, stream) -----------------------------------------------------------
+// A zero-initialised workspace (the kernels leave it all zero after every call, so it is reusable as is)
+// and an uninitialised scratch buffer for the batched paths.  Both grow on demand, at least doubling.  An
+// outgrown buffer is kept alive rather than freed: a HIP graph captured earlier on that stream may still hold
+// its address (doubling bounds what is kept to the size of the live buffer).
+struct Pool {
+    std::map<std::pair<int, uintptr_t>, Tensor> live;
+    std::vector<Tensor> outgrown;
+    std::mutex lock;
+    bool zeroed;
+    int64_t floor;
+
+    Tensor get(int device, void *stream, int64_t bytes) {
+        std::lock_guard<std::mutex> hold(lock);
+        Tensor &t = live[{device, reinterpret_cast<uintptr_t>(stream)}];
+        if (!t.defined() || t.numel() < bytes) {
+            if (t.defined()) {
+                outgrown.push_back(t);
+                bytes = std::max(bytes, 2 * t.numel());
+            }
+            c10::InferenceMode normal(false);  // plain tensors, whatever mode the first caller is in
+            const auto opts = at::TensorOptions().dtype(at::kByte).device(at::kCUDA, device);
+            t = zeroed ? at::zeros({std::max(bytes, floor)}, opts) : at::empty({std::max(bytes, floor)}, opts);
+        }
+        return t;
+    }
+};
+Pool &workspaces = *new Pool{{}, {}, {}, true, 1 << 18};  // never destroyed: the runtime may be gone by then
+Pool &scratches = *new Pool{{}, {}, {}, false, 1};
+
+inline const Tensor *tensor(PyObject *o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+inline bool is(const Tensor *t, at::ScalarType type, int64_t dims, int device) {
+    return t && t->scalar_type() == type && t->dim() == dims && t->is_cuda() && t->get_device() == device &&
+           t->is_contiguous();
+}
+
+inline const void *ptr(const Tensor &t) { return t.numel() ? t.const_data_ptr() : nullptr; }
+inline void *mut(const Tensor &t) { return t.numel() ? t.mutable_data_ptr() : nullptr; }
+
+inline void *current_stream(int device) { return c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream(); }
+
+struct Packed {  // the checkpoint buffers of one layer
+    const Tensor *qweight, *cherry_weight, *cherry_indices, *scales;
+};
+
+// Without the interpreter's lock another thread may replace a module's buffers: a call's tensors are held.
+template <typename... T>
+struct Held {
+    std::array<Tensor, sizeof...(T)> tensors;
+    explicit Held(const T &...t) : tensors{t...} {}
+};
+
+// The fused matmul over the checkpoint buffers; -1 where a buffer is not what the kernels take.
+int fused(int kind, const Tensor &vec, int64_t batch, int64_t k, const Packed &p, const Tensor &out, int64_t group,
+          bool accumulate) {
+    const bool f32 = kind == 32;
+    const int bits = kind == 4 ? 4 : 3, device = vec.get_device();
+    const auto io = f32 ? at::kFloat : at::kHalf;
+    if (!is(p.qweight, at::kByte, 2, device) || !is(p.cherry_weight, io, 2, device) ||
+        !is(p.cherry_indices, f32 ? at::kInt : at::kShort, 1, device) || !is(p.scales, io, 2, device))
+        return -1;
+    const int64_t n = p.qweight->size(1), c = p.cherry_indices->size(0), kn = k - c;
+    if (p.qweight->size(0) * 8 != kn * bits || p.cherry_weight->size(0) != c || p.cherry_weight->size(1) != n || group <= 0 ||
+        (bits == 4 && group < 128) || p.scales->size(0) != (kn + group - 1) / group || p.scales->size(1) != n ||
+        out.numel() != batch * n || batch <= 0)
+        return -1;
+    if (std::max({batch, k, n, group}) > INT32_MAX || c10::hip::current_device() != device) return -1;
+    const int B = (int)batch, K = (int)k, N = (int)n, C = (int)c;
+    void *stream = current_stream(device);
+    const size_t wsb = api.workspace(B, K, N, C);
+    const size_t scb = f32 ? api.scratch_f32(B, K, N, C) : B > 1 ? api.scratch(B, K, N, C) : 0;
+    const Tensor ws = workspaces.get(device, stream, (int64_t)wsb);
+    const Tensor sc = scb ? scratches.get(device, stream, (int64_t)scb) : Tensor();
+    const VecquantFn fn = f32 ? api.vecquant3_f32 : bits == 4 ? api.vecquant4 : api.vecquant3;
+    const Held held(*p.qweight, *p.cherry_weight, *p.cherry_indices, *p.scales, vec, out);
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = fn(ptr(held.tensors[4]), ptr(held.tensors[0]), ptr(held.tensors[1]), ptr(held.tensors[2]), ptr(held.tensors[3]),
+            mut(held.tensors[5]), B, K, N, C, (int)group, accumulate, mut(ws), ws.numel(), scb ? mut(sc) : nullptr, scb ? sc.numel() : 0, stream);
+    Py_END_ALLOW_THREADS
+    return rc < 0 ? -1 : rc;  // a refusal of the library is worded by the general route
+}
+
+// 1 to 16 rows over a weight stream; -1 as above.
+int over_stream(int bits, const Tensor &vec, int64_t batch, const Tensor &weights, const Tensor &out, int64_t k, int64_t n,
+                int64_t c, bool accumulate) {
+    const int device = vec.get_device();
+    if (batch <= 0 || std::max({batch, k, n, c}) > INT32_MAX || c10::hip::current_device() != device) return -1;
+    const int B = (int)batch, K = (int)k, N = (int)n, C = (int)c;
+    void *stream = current_stream(device);
+    Tensor sc;
+    const size_t scb = B > 1 ? api.prepacked_scratch(bits, B, K, N, C) : 0;
+    if (scb) sc = scratches.get(device, stream, (int64_t)scb);
+    const Held held(weights, vec, out);
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    if (B == 1)
+        rc = api.matvec_prepacked(bits, ptr(held.tensors[1]), ptr(held.tensors[0]), held.tensors[0].numel(), mut(held.tensors[2]), B, K, N, C,
+                                  accumulate, stream);
+    else
+        rc = api.matmul_prepacked(bits, ptr(held.tensors[1]), ptr(held.tensors[0]), held.tensors[0].numel(), mut(held.tensors[2]), B, K, N, C,
+                                  accumulate,                                   scb ? mut(sc) : nullptr, scb, stream);
+    Py_END_ALLOW_THREADS
+    return rc < 0 ? -1 : rc;
+}
+
+PyObject *answer(int rc) {
+    if (rc < 0) Py_RETURN_NONE;
+    return PyLong_FromLong(rc);
+}
+
+// vecquant(kind, vec, qweight, cherry_weight, cherry_indices, scales, mul, group_size, accumulate): kind 4 and 3 are the
+// fp16 operators of that many bits, 32 the 3-bit one over fp32 tensors.  0, a HIP error code, or None.
+PyObject *vecquant(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 9 || !PyLong_CheckExact(a[7])) Py_RETURN_NONE;
+    const int kind = (int)PyLong_AsLong(a[0]);
+    const int64_t group = PyLong_AsLongLong(a[7]);
+    if (PyErr_Occurred()) {
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+    const Tensor *vec = tensor(a[1]), *mul = tensor(a[6]);
+    const auto io = kind == 32 ? at::kFloat : at::kHalf;
+    if (!vec || !vec->is_cuda()) Py_RETURN_NONE;
+    const int device = vec->get_device();
+    if (!is(vec, io, 2, device) || !is(mul, io, 2, device) || mul->size(0) != vec->size(0)) Py_RETURN_NONE;
+    const Packed p{tensor(a[2]), tensor(a[3]), tensor(a[4]), tensor(a[5])};
+    return answer(fused(kind, *vec, vec->size(0), vec->size(1), p, *mul, group, PyObject_IsTrue(a[8])));
+    END_HANDLE_TH_ERRORS
+}
+
+// matvec_prepacked(bits, vec, stream, out, in_features, num_cherries, accumulate)
+PyObject *matvec_prepacked(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 7) Py_RETURN_NONE;
+    for (int i : {0, 4, 5})
+        if (!PyLong_CheckExact(a[i])) Py_RETURN_NONE;
+    const int bits = (int)PyLong_AsLong(a[0]);
+    const int64_t k = PyLong_AsLongLong(a[4]), c = PyLong_AsLongLong(a[5]);
+    if (PyErr_Occurred()) {
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+    const Tensor *vec = tensor(a[1]), *weights = tensor(a[2]), *out = tensor(a[3]);
+    if (!vec || !vec->is_cuda()) Py_RETURN_NONE;
+    const int device = vec->get_device();
+    if (!is(vec, at::kHalf, 2, device) || !is(weights, at::kByte, 1, device) || !is(out, at::kHalf, 2, device) ||
+        vec->size(1) != k || out->size(0) != vec->size(0))
+        Py_RETURN_NONE;
+    return answer(over_stream(bits, *vec, vec->size(0), *weights, *out, k, out->size(1), c, PyObject_IsTrue(a[6])));
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- QuantLinear.forward ----------------------------------------------------------------------------
+struct Names {
+    PyObject *dict, *buffers, *stream, *released, *dequantized, *layerwise, *prefill_rows, *w_bits, *group_size, *in_features,
+        *out_features, *num_cherries, *qweight, *cherry_weight, *cherry_indices, *scales, *bias;
+} names;
+
+// An integer entry of a module's dictionary (negative: none).
+inline int64_t number(PyObject *dict, PyObject *name) {
+    PyObject *v = PyDict_GetItemWithError(dict, name);
+    return v && PyLong_CheckExact(v) ? PyLong_AsLongLong(v) : -1;
+}
+
+struct Ref {
+    PyObject *o;
+    ~Ref() { Py_XDECREF(o); }
+};
+
+// linear(module, x): the output, or None.  Everything is read from the module at every call (its dictionaries are
+// plain lookups), so replaced buffers, a dropped stream or a changed mode need no notice.
+PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (nargs != 2) Py_RETURN_NONE;
+    const Tensor *x = tensor(a[1]);
+    if (!x || !x->is_cuda() || x->dim() < 1 || x->numel() == 0 || !x->is_floating_point()) Py_RETURN_NONE;
+    Ref dict{PyObject_GetAttr(a[0], names.dict)};
+    Ref layerwise{PyObject_GetAttr(a[0], names.layerwise)};
+    if (!dict.o || !layerwise.o || !PyDict_CheckExact(dict.o)) {
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+    PyObject *buffers = PyDict_GetItemWithError(dict.o, names.buffers);
+    const int bits = (int)number(dict.o, names.w_bits);
+    const int64_t group = number(dict.o, names.group_size), k = number(dict.o, names.in_features),
+                  n = number(dict.o, names.out_features), c = number(dict.o, names.num_cherries);
+    if (layerwise.o != Py_True || PyDict_GetItemWithError(dict.o, names.dequantized) != Py_False || (bits != 3 && bits != 4) ||
+        !buffers || !PyDict_Check(buffers) || group <= 0 || k <= 0 || n <= 0 || c < 0 || x->size(-1) != k ||
+        std::max({group, k, n, c}) > INT32_MAX)
+        Py_RETURN_NONE;
+    const int64_t rows = x->numel() / k;
+    const bool released = PyDict_GetItemWithError(dict.o, names.released) != Py_False;
+    const int device = x->get_device();
+    PyObject *so = PyDict_GetItemWithError(dict.o, names.stream);
+    const Tensor *weights = so && so != Py_None ? tensor(so) : nullptr;
+    if (so && so != Py_None && !is(weights, at::kByte, 1, device)) Py_RETURN_NONE;
+    bool streamed = false;
+    // over the weight stream: one row, and the small batches that measured faster there than on the checkpoint
+    // layout's kernels; with the checkpoint buffers released, everything its kernels take
+    if (weights)
+        streamed = rows == 1 || (rows <= 16 && (released ? api.prepack_supported : api.rows_recommended)(
+                                                   bits, (int)rows, (int)k, (int)n, (int)c, (int)group));
+    Packed p{};
+    if (!streamed) {
+        if (released) Py_RETURN_NONE;
+        Ref limit{PyObject_GetAttr(a[0], names.prefill_rows)};
+        const int64_t most = limit.o && PyLong_Check(limit.o) ? PyLong_AsLongLong(limit.o) : -1;
+        if (PyErr_Occurred()) PyErr_Clear();
+        if (rows >= most) Py_RETURN_NONE;  // dequantise once and a dense product
+        auto buffer = [&](PyObject *name) {
+            PyObject *o = PyDict_GetItemWithError(buffers, name);
+            return o ? tensor(o) : nullptr;
+        };
+        p = Packed{buffer(names.qweight), buffer(names.cherry_weight), buffer(names.cherry_indices), buffer(names.scales)};
+        if (!p.qweight || p.qweight->dim() != 2 || p.qweight->size(1) != n) Py_RETURN_NONE;
+    }
+    PyObject *bo = PyDict_GetItemWithError(buffers, names.bias);
+    if (!bo) bo = PyDict_GetItemWithError(dict.o, names.bias);  // a bias set by pack() where none was registered
+    const Tensor *bias = bo && bo != Py_None ? tensor(bo) : nullptr;
+    if (bo && bo != Py_None && !bias) Py_RETURN_NONE;
+
+    c10::InferenceMode inference(true);
+    const Tensor row = x->scalar_type() == at::kHalf ? x->contiguous() : x->to(at::kHalf).contiguous();
+    c10::SmallVector<int64_t, 6> sizes(x->sizes().begin(), x->sizes().end());
+    sizes.back() = n;
+    Tensor out = at::empty(sizes, row.options());
+    const int rc = streamed ? over_stream(bits, row, rows, *weights, out, k, n, c, false)
+                            : fused(bits, row, rows, k, p, out, group, false);
+    if (rc != 0) Py_RETURN_NONE;
+    if (x->scalar_type() != at::kHalf) out = out.to(x->scalar_type());
+    if (bias) out.add_(*bias);
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// workspace(device, stream, bytes) / scratch(device, stream, bytes): the kept buffers, for the other callers
+PyObject *kept(Pool &pool, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 3) {
+        PyErr_SetString(PyExc_TypeError, "device, stream and bytes expected");
+        return nullptr;
+    }
+    const int device = (int)PyLong_AsLong(a[0]);
+    void *stream = reinterpret_cast<void *>(PyLong_AsUnsignedLongLong(a[1]));
+    const int64_t bytes = PyLong_AsLongLong(a[2]);
+    if (PyErr_Occurred()) return nullptr;
+    return THPVariable_Wrap(pool.get(device, stream, bytes));
+    END_HANDLE_TH_ERRORS
+}
+PyObject *workspace(PyObject *, PyObject *const *a, Py_ssize_t n) { return kept(workspaces, a, n); }
+PyObject *scratch(PyObject *, PyObject *const *a, Py_ssize_t n) { return kept(scratches, a, n); }
+
+// bind(addresses): the library's entry points in the order of struct Api
+PyObject *bind(PyObject *, PyObject *seq) {
+    constexpr Py_ssize_t count = sizeof(Api) / sizeof(void *);
+    if (!PyTuple_Check(seq) || PyTuple_GET_SIZE(seq) != count) {
+        PyErr_SetString(PyExc_TypeError, "one address per entry point expected");
+        return nullptr;
+    }
+    void *at[count];
+    for (Py_ssize_t i = 0; i < count; i++) {
+        at[i] = PyLong_AsVoidPtr(PyTuple_GET_ITEM(seq, i));
+        if (!at[i]) {
+            if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "null address");
+            return nullptr;
+        }
+    }
+    memcpy(&api, at, sizeof(api));
+    Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {
+    {"bind", bind, METH_O, nullptr},
+    {"vecquant", (PyCFunction)(void (*)())vecquant, METH_FASTCALL, nullptr},
+    {"matvec_prepacked", (PyCFunction)(void (*)())matvec_prepacked, METH_FASTCALL, nullptr},
+    {"linear", (PyCFunction)(void (*)())linear, METH_FASTCALL, nullptr},
+    {"workspace", (PyCFunction)(void (*)())workspace, METH_FASTCALL, nullptr},
+    {"scratch", (PyCFunction)(void (*)())scratch, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "cherryq_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_cherryq_host(void) {
+    const std::pair<PyObject **, const char *> all[] = {{&names.dict, "__dict__"}, {&names.buffers, "_buffers"},
+        {&names.stream, "_stream"}, {&names.released, "_released"}, {&names.dequantized, "dequantized"},
+        {&names.layerwise, "_layerwise_dequantize"}, {&names.prefill_rows, "prefill_rows"}, {&names.w_bits, "w_bits"},
+        {&names.group_size, "group_size"}, {&names.in_features, "in_features"}, {&names.out_features, "out_features"},
+        {&names.num_cherries, "num_cherries"}, {&names.qweight, "qweight"}, {&names.cherry_weight, "cherry_weight"},
+        {&names.cherry_indices, "cherry_indices"}, {&names.scales, "scales"}, {&names.bias, "bias"}};
+    for (auto &n : all)
+        if (!(*n.first = PyUnicode_InternFromString(n.second))) return nullptr;
+    return PyModule_Create(&module);
+}

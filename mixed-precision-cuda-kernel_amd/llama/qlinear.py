@@ -245,8 +245,13 @@ class QuantLinear(nn.Module):
         self._stream = None
 
     # ---- forward ------------------------------------------------------------------------------
-    @torch.inference_mode()
     def forward(self, x: torch.Tensor):
+        # one native call for the fused cases (the choice of path is that of _forward); None: not one of them
+        out = quant_cuda._host.linear(self, x)
+        return self._forward(x) if out is None else out
+
+    @torch.inference_mode()
+    def _forward(self, x: torch.Tensor):
         if self._layerwise_dequantize:
             if self.w_bits not in (3, 4):
                 raise NotImplementedError(f"{self.w_bits} bit kernel is not implemented yet.")

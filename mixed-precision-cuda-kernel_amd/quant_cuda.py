@@ -8,8 +8,11 @@ Drop-in for the pybind11 module built from csrc/quant_cuda.cpp:72-77 of the refe
     Dequantize4Normal(qweight, scaling_factors, out, height, cherry_size, group_size)
 
 Same positional arguments, same in-place accumulate into `mul`, nothing returned.  The work is
-done by hand-written HIP kernels in libcherryq.so (C ABI: include/cherryq.h), reached through
-ctypes with raw device pointers; torch only supplies memory and the current stream.  There is no
+done by hand-written HIP kernels in libcherryq.so (C ABI: include/cherryq.h).  The calls a decoding
+program makes per layer and token go from the arguments to the launch in one native function
+(cherryq_host.so, csrc/cq_host.cpp); where that does not take a call, and for everything else, the
+entry points are reached through ctypes with raw device pointers.  torch only supplies memory and
+the current stream.  There is no
 CPU or eager fallback: importing this module without the built library raises, and so does any
 call with tensors that are not on a GPU.
 
@@ -91,6 +94,16 @@ _lib.cherryq_version.restype = _int
 
 LIBRARY_PATH = str(_LIB_PATH)
 
+try:
+    import cherryq_host as _host
+except ImportError as e:
+    raise ImportError(f"quant_cuda: cherryq_host.so is not built. Run `python {_HERE / 'build.py'}`; there is no fallback "
+                      "implementation.") from e
+_host.bind(tuple(ctypes.cast(getattr(_lib, f"cherryq_{n}"), _vp).value for n in (
+    "vecquant4matmul_f16", "vecquant3matmul_f16", "vecquant3matmul_f32", "workspace_bytes", "scratch_bytes",
+    "scratch_bytes_f32", "prepacked_scratch_bytes", "matvec_prepacked_f16", "matmul_prepacked_f16", "prepack_supported",
+    "prepack_rows_recommended")))
+
 
 def _fail(status: int, what: str):
     raise RuntimeError(f"{what}: {_lib.cherryq_status_string(status).decode()} (status {status})")
@@ -116,36 +129,17 @@ def _check(t: torch.Tensor, name: str, dtype, ndim: int, device=None):
         raise RuntimeError(f"{name} must be contiguous")
 
 
-# Per (device, stream): a zero-initialised workspace (the kernels leave it all zero after every
-# call, so it is reusable as is) and an uninitialised scratch buffer for the batched path.  Both
-# grow on demand, at least doubling.  An outgrown buffer is kept alive rather than freed: a HIP
-# graph captured earlier on that stream may still hold its address (doubling bounds what is kept
-# to the size of the live buffer).
-_workspaces: dict = {}
-_scratches: dict = {}
-_outgrown: list = []
 _sizes: dict = {}  # (batch, in, out, cherries, dtype) -> (workspace bytes, scratch bytes) as the library reports them
 
 
-def _grown(table: dict, key, nbytes: int, floor: int, alloc, device) -> torch.Tensor:
-    buf = table.get(key)
-    if buf is None or buf.numel() < nbytes:
-        if buf is not None:
-            _outgrown.append(buf)
-            nbytes = max(nbytes, 2 * buf.numel())
-        buf = alloc(max(nbytes, floor), dtype=torch.uint8, device=device)
-        table[key] = buf
-    return buf
-
-
+# Kept per (device, stream): a zero-initialised workspace (the kernels leave it all zero after every
+# call) and an uninitialised scratch buffer for the batched paths (csrc/cq_host.cpp).
 def _workspace(device: torch.device, stream: int, nbytes: int) -> torch.Tensor:
-    return _grown(_workspaces, (device.index, stream), nbytes, 1 << 18, torch.zeros, device)
+    return _host.workspace(device.index, stream, nbytes)
 
 
 def _scratch(device: torch.device, stream: int, nbytes: int):
-    if nbytes == 0:
-        return None
-    return _grown(_scratches, (device.index, stream), nbytes, 1, torch.empty, device)
+    return _host.scratch(device.index, stream, nbytes) if nbytes else None
 
 
 # torch's current stream as a raw handle.  The private accessor costs a tenth of building a
@@ -215,6 +209,8 @@ def _matmul(fn, what, vec, qweight, cherry_weight, cherry_indices, scales, mul, 
 
 def vecquant4matmul_cherryq(vec, qweight, cherry_weight, cherry_indices, scaling_factors, mul, group_size):
     """mul += vec @ W^T for 4-bit packed W (reference: csrc/quant_cuda.cpp:56-69)."""
+    if _host.vecquant(4, vec, qweight, cherry_weight, cherry_indices, scaling_factors, mul, group_size, True) == 0:
+        return
     if int(group_size) < 128:
         raise RuntimeError("`group_size` must be multiple of 128")  # csrc/quant_cuda_kernel.cu:684
     _matmul(_lib.cherryq_vecquant4matmul_f16, "vecquant4matmul_cherryq", vec, qweight, cherry_weight,
@@ -227,6 +223,9 @@ def vecquant3matmul_cherryq(vec, qweight, cherry_weight, cherry_indices, scaling
 
     fp16=True: fp16 tensors, int16 indices.  fp16=False: fp32 tensors, int32 indices
     (the call shape of benchmark_speed.py:20-32)."""
+    if _host.vecquant(3 if fp16 else 32, vec, qweight, cherry_weight, cherry_indices, scaling_factors, mul, group_size,
+                      True) == 0:
+        return
     if fp16:
         _matmul(_lib.cherryq_vecquant3matmul_f16, "vecquant3matmul_cherryq", vec, qweight, cherry_weight,
                 cherry_indices, scaling_factors, mul, group_size, 3, torch.float16, torch.int16)
@@ -240,6 +239,9 @@ def matmul_cherryq(w_bits, vec, qweight, cherry_weight, cherry_indices, scaling_
     """fp16 fused matmul that can overwrite `out` instead of accumulating into it, which spares
     the caller the zero-fill the reference needs before every call (llama/qlinear.py:177).
     No counterpart in the reference extension."""
+    if w_bits in (3, 4) and _host.vecquant(w_bits, vec, qweight, cherry_weight, cherry_indices, scaling_factors, out,
+                                           group_size, accumulate) == 0:
+        return
     if w_bits == 4:
         if int(group_size) < 128:
             raise RuntimeError("`group_size` must be multiple of 128")
@@ -494,6 +496,8 @@ def matvec_prepacked_cherryq(w_bits, vec, stream, out, in_features, num_cherries
     """out (B, N) = (or +=) vec (B, K) @ W^T over a stream made by prepack_cherryq, 1 <= B <= 16.
     Result and arithmetic contract are those of vecquant{3,4}matmul_cherryq; no workspace, no
     atomics (from 2 rows a scratch buffer for the compacted activations, kept by this module)."""
+    if _host.matvec_prepacked(w_bits, vec, stream, out, in_features, num_cherries, accumulate) == 0:
+        return
     _check(vec, "vec", torch.float16, 2)
     dev = vec.device
     _check(stream, "stream", torch.uint8, 1, dev)
