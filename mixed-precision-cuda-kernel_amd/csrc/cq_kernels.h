@@ -176,7 +176,7 @@ hipError_t launch_sort_channels(const void *idx, int index_bytes, int16_t *out, 
 hipError_t launch_pack(int bits, const __half *w, const int16_t *idx, uint8_t *qweight, __half *scales,
                        __half *cherry_weight, int K, int N, int C, int G, hipStream_t stream);
 
-// cq_f32.hip: the 3-bit fp32-tensor variant on the fp32 matrix-core instruction, 2 rows and more.
+// cq_f32.hip: the 3-bit fp32-tensor variant, exact products on the fp16 matrix cores.
 bool f32_supported(int B, int K, int N, int C, int G);
 size_t f32_scratch_bytes(int K, int C);
 hipError_t launch_f32(const float *vec, const uint8_t *qweight, const float *cherry_weight,

@@ -882,3 +882,39 @@ def test_device_pack_tile_edges(bits, n, k, g, where):
     for bad in (torch.full((c,), 3), idx + k):
         with pytest.raises(RuntimeError):
             quant_cuda.pack_cherryq(bits, lin.weight.data.cuda(), bad, g)
+
+
+@pytest.mark.parametrize("b,k,n,c,g", [(16, 2048, 72, 16, 32), (3, 1032, 264, 8, 64), (33, 1160, 128, 136, 96), (1, 8192, 8, 0, 128),
+                                       (5, 6144, 136, 2056, 128), (2, 28672, 512, 112, 128), (16, 1024, 16448, 8, 256)])
+def test_fp32_variant_exact_products_over_the_fp32_range(qc, b, k, n, c, g):
+    """Groups of 32 to 256, ragged units, rows beyond one pass, K split over many and over no workgroups, more cherries than
+    are staged; activations whose magnitudes span 2^-40 to 2^40 inside a row and 2^-120 to 2^100 between
+    rows.  Products are exact and each of the K terms enters a sum that fp32 rounds, so the error is
+    bounded by K * 2^-24 of the sum of magnitudes per output (measured: far below); what split-K adds is
+    2^-34 absolute per workgroup."""
+    announce("fp32 exact", b, k, n, c, g)
+    rng = np.random.default_rng(b + k + n)
+    kn = k - c
+    vec = (rng.standard_normal((b, k)) * 2.0 ** rng.integers(-20, 20, (b, k))).astype(np.float32)
+    vec *= (2.0 ** np.linspace(-100, 80, b) if b > 3 else np.ones(b))[:, None].astype(np.float32)
+    qweight = rng.integers(0, 256, size=(kn // 8 * 3, n), dtype=np.uint8)
+    cw = rng.standard_normal((c, n)).astype(np.float32)
+    idx = np.sort(rng.choice(k, c, replace=False)).astype(np.int32)
+    scales = (rng.random((-(-kn // g), n)) * 0.01 + 0.005).astype(np.float32)
+    wn = (orc.unpack_codes(qweight, 3).astype(np.float64) - 3.5) * np.repeat(scales.astype(np.float64), g, axis=0)[:kn]
+    nidx = orc.normal_indices(k, idx)
+    x64 = vec.astype(np.float64)
+    want = x64[:, nidx] @ wn + x64[:, idx] @ cw.astype(np.float64)
+    mag = np.abs(x64[:, nidx]) @ np.abs(wn) + np.abs(x64[:, idx]) @ np.abs(cw.astype(np.float64))
+    args = [torch.from_numpy(a).cuda() for a in (vec, qweight, cw, idx, scales)]
+    mul = torch.zeros(b, n, device="cuda")
+    qc.vecquant3matmul_cherryq(*args, mul, g, False)
+    torch.cuda.synchronize()
+    err = np.abs(mul.cpu().numpy().astype(np.float64) - want)
+    assert (err <= 4e-6 * mag + 64 * 2.0 ** -34).all(), float((err / (mag + 1e-30)).max())
+    vec[0, int(nidx[5])] = np.inf
+    mul.zero_()
+    qc.vecquant3matmul_cherryq(torch.from_numpy(vec).cuda(), *args[1:], mul, g, False)
+    got = mul.cpu().numpy()
+    assert np.isinf(got[0]).all() and (np.sign(got[0]) == np.sign(wn[5])).all()
+    assert np.isfinite(got[1:]).all()
