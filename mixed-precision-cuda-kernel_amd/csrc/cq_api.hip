@@ -44,9 +44,11 @@ size_t workspace_bytes(int B, int K, int N, int C) {
     if (B >= 2) {
         size_t b2 = batch_workspace(K, N, C).workspace_total;
         if (b2 > bytes) bytes = b2;
+        b2 = prompt_plan(B, K, N, C).workspace_bytes;
+        if (b2 > bytes) bytes = b2;
     }
     if (B >= kGemmMinRows) {
-        size_t b3 = gemm_plan(B, K, N, C).workspace_bytes;
+        const size_t b3 = gemm_plan(B, K, N, C).workspace_bytes;
         if (b3 > bytes) bytes = b3;
     }
     return bytes;
@@ -57,9 +59,13 @@ size_t scratch_bytes(int B, int K, int N, int C) {
     clamp_dims(B, K, N, C);
     size_t bytes = B >= 2 ? batch_workspace(K, N, C).scratch_total : 0;
     if (B >= 2 && f32_scratch_bytes(K, C) > bytes) bytes = f32_scratch_bytes(K, C);  // fp32-tensor variant
-    if (B >= kGemmMinRows) {
-        size_t b3 = gemm_plan(B, K, N, C).scratch_bytes;
+    if (B >= 2) {
+        const size_t b3 = prompt_plan(B, K, N, C).scratch_bytes;
         if (b3 > bytes) bytes = b3;
+    }
+    if (B >= kGemmMinRows) {
+        const size_t b4 = gemm_plan(B, K, N, C).scratch_bytes;
+        if (b4 > bytes) bytes = b4;
     }
     return bytes;
 }
@@ -113,10 +119,15 @@ static int matmul_f16(const void *vec, const uint8_t *qweight, const void *cherr
         e = launch_matvec(BITS, x, qweight, cw, cherry_indices, sc, y, K, N, C, G, accumulate, workspace, s);
     } else if (!force_generic() && matvec_rows_preferred(BITS, B, K, N, C, G)) {
         e = launch_matvec_rows(BITS, x, qweight, cw, cherry_indices, sc, y, B, K, N, C, G, accumulate, workspace, s);
-    } else if (!force_generic() && B >= kGemmMinRows && gemm_supported(BITS, B, K, N, C, G)) {
-        e = launch_gemm(BITS, x, qweight, cw, cherry_indices, sc, y, B, K, N, C, G, accumulate, workspace, scratch, s);
-    } else if (!force_generic() && batch_supported(BITS, B, K, N, C, G)) {
+    } else if (!force_generic() && B < kGemmMinRows && batch_supported(BITS, B, K, N, C, G)) {
+        // up to a tile's 16 rows: half of the prompt kernel's smallest tile would be padding
         e = launch_batch(BITS, x, qweight, cw, cherry_indices, sc, y, B, K, N, C, G, accumulate, workspace, scratch, s);
+    } else if (!force_generic() && B >= 2 && prompt_supported(BITS, B, K, N, C, G)) {
+        // ... unless the group is no whole number of the batch kernel's units of 128 positions
+        e = launch_prompt(BITS, x, qweight, cw, cherry_indices, sc, y, B, K, N, C, G, accumulate, workspace, scratch, s);
+    } else if (!force_generic() && B >= kGemmMinRows && gemm_supported(BITS, B, K, N, C, G)) {
+        // activations of more than 2 GiB in operand order, beyond the prompt kernel's buffer offsets
+        e = launch_gemm(BITS, x, qweight, cw, cherry_indices, sc, y, B, K, N, C, G, accumulate, workspace, scratch, s);
     } else {
         e = launch_generic<BITS, __half, int16_t>(x, qweight, cw, cherry_indices, sc, y, B, K, N, C, G,
                                                   accumulate, workspace, s);

@@ -1,4 +1,5 @@
-// Prompt-sized batches (more than 16 rows): fused dequantise + GEMM on the gfx950 matrix cores.
+// Prompt-sized batches (more than 16 rows): fused dequantise + GEMM on the gfx950 matrix cores, for calls whose
+// activations take more than 2 GiB; all others run the kernel of cq_prompt.hip, which is 1.2 to 1.35 times as fast.
 //
 //   Y[M, N] (+)= Xn[M, Kn] * Wn[Kn, N] + Xc[M, C] * Wc[C, N]
 //

@@ -101,6 +101,23 @@ hipError_t launch_gemm(int bits, const __half *vec, const uint8_t *qweight, cons
                        const int16_t *cherry_indices, const __half *scales, __half *mul, int M, int K, int N, int C,
                        int G, int accumulate, void *workspace, void *scratch, hipStream_t stream);
 
+// cq_prompt.hip: the same sizes with the wavefronts of a workgroup sharing K.
+constexpr int kPromptMaxSplits = 16;
+struct PromptPlan {
+    int mt, nc, ns;                   // 16-row and 16-column pieces of a wavefront's tile, wavefronts side by side
+    int mtiles, ntiles;               // output tiles of 16 mt rows x 16 nc ns columns
+    int units, csteps, steps;         // units of 128 positions, steps of 32 cherries, steps of 32 in all
+    int splits, units_per_split;      // K splits (grid.y)
+    size_t workspace_bytes;           // zero-kept: one ticket per output tile
+    size_t a_bytes, partial_bytes;    // scratch: activations in operand order, then the per-split partial tiles
+    size_t scratch_bytes;
+};
+PromptPlan prompt_plan(int M, int K, int N, int C);
+bool prompt_supported(int bits, int M, int K, int N, int C, int G);
+hipError_t launch_prompt(int bits, const __half *vec, const uint8_t *qweight, const __half *cherry_weight,
+                         const int16_t *cherry_indices, const __half *scales, __half *mul, int M, int K, int N, int C, int G,
+                         int accumulate, void *workspace, void *scratch, hipStream_t stream);
+
 // cq_stream.hip: batch-1 matvec over a load-time repacked weight stream (tiles of 16 columns, each
 // tile's whole K range contiguous; no split-K, no workspace).
 constexpr int kStreamTileCols = 16;

@@ -918,3 +918,43 @@ def test_fp32_variant_exact_products_over_the_fp32_range(qc, b, k, n, c, g):
     got = mul.cpu().numpy()
     assert np.isinf(got[0]).all() and (np.sign(got[0]) == np.sign(wn[5])).all()
     assert np.isfinite(got[1:]).all()
+
+
+@pytest.mark.parametrize("bits,gs,k,n,rows,frac", [
+    (3, 32, 1032, 72, 2, 1 / 64),         # 32 x 64 tiles, one K split; a group per matrix step
+    (3, 64, 4096, 72, 16, 1 / 256),       # ... four K splits
+    (4, 160, 8200, 136, 33, 1 / 256),     # ... eight; groups straddle units
+    (3, 96, 1304, 520, 128, 1 / 8),       # ... many cherry steps
+    (4, 128, 5120, 1096, 65, 1 / 256),    # 64 x 64 tiles, five K splits
+    (4, 256, 1304, 8200, 97, 1 / 16),     # 128 x 64 tiles
+    (3, 128, 2056, 16392, 100, 1 / 256),  # 128 x 128 tiles
+    (3, 64, 1304, 8200, 257, 1 / 16),     # ... one row in the last row tile
+    (4, 128, 536, 16400, 200, 1 / 16),    # 128 x 256 tiles, a last unit of 118 positions
+    (3, 160, 1304, 8200, 600, 1 / 256),   # ... a last column tile of 8
+])
+def test_prompt_kernel_tile_edges(qc, bits, gs, k, n, rows, frac):
+    """Every tile shape of the prompt kernel at ragged rows, columns, positions and groups, added to what the output holds,
+    from activations that are only 4-byte aligned.  Weights are the dense path's fp16 values and products
+    are exact, so an output differs from the float64 product by its own rounding (2^-11), that of K fp32 additions
+    (K * 2^-24 of the sum of magnitudes) and the rounding of the addition."""
+    announce("prompt edges", bits, gs, k, n, rows)
+    p = orc.synthetic_packed_fast(k, n, bits, gs, seed=rows, cherry_fraction=frac)
+    rng = np.random.default_rng(rows + n)
+    x = rng.standard_normal((rows, k)).astype(np.float16)
+    start = rng.integers(-8, 9, (rows, n)).astype(np.float16)
+    d = dev(p)
+    flat = torch.zeros(rows * k + 2, dtype=torch.float16, device="cuda")
+    flat[2:] = torch.from_numpy(x.ravel()).cuda()
+    out = torch.from_numpy(start).cuda()
+    for _ in range(2):  # the tickets are left zeroed
+        out.copy_(torch.from_numpy(start))
+        qc.matmul_cherryq(bits, flat[2:].view(rows, k), *(d[name] for name in ("qweight", "cherry_weight", "cherry_indices", "scales")),
+                          out, gs, True)
+    cols = np.unique(np.r_[np.arange(min(n, 40)), rng.choice(n, 100), np.arange(max(0, n - 40), n)])
+    sub = {name: v if name == "cherry_indices" else np.ascontiguousarray(v[:, cols]) for name, v in p.items()}
+    dense = c_oracle.unpack(sub, bits, gs, k).astype(np.float64).T
+    x64 = x.astype(np.float64)
+    want = x64 @ dense + start[:, cols]
+    bound = 2.0 ** -10 * np.abs(want) + 1e-6 + k * 2.0 ** -24 * (np.abs(x64) @ np.abs(dense) + np.abs(start[:, cols]))
+    err = np.abs(out.cpu().numpy()[:, cols] - want)
+    assert (err <= bound).all(), float((err / bound).max())
