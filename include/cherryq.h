@@ -449,6 +449,25 @@ int cherryq_decode_argmax_embed_f16(const void *logits, int vocab, const void *e
                                     int history_len, int *position, void *stream);
 int cherryq_decode_silu_mul_f16(const void *gate, const void *up, void *out, int n, void *stream);
 
+/*
+ * The operations between the linears for the whole prompt (the reference's model with a sequence length above one).
+ *
+ * cherryq_prefill_norm_f16: `rows` rows of hidden_size (a multiple of 8, at most 8192):
+ *   hidden <- hidden + delta (delta may be NULL), normed <- weight * fp16(hidden * rsqrt(mean(hidden^2) + eps))
+ *   (llama/modeling_llama_quant.py:75-89).
+ * cherryq_prefill_attention_f16: causal attention of `tokens` positions that start at 0.  q is (tokens, n_heads * 128), k and v
+ *   (tokens, n_kv_heads * 128), all before the rotary embedding; cos_table / sin_table (tokens, 64) are fp16; rotated
+ *   keys and values are written to positions 0 .. tokens - 1 of the caches ([n_kv_heads][max_len][128]), out is
+ *   (tokens, n_heads * 128) (:95-210, :671-696).  scratch: cherryq_prefill_attention_bytes() bytes,
+ *   256-byte aligned, uninitialised.  All tensors 16-byte aligned; head_dim must be 128.
+ */
+int cherryq_prefill_norm_f16(void *hidden, const void *delta /* may be NULL */, const void *weight, void *normed, int rows,
+                             int hidden_size, float eps, void *stream);
+size_t cherryq_prefill_attention_bytes(int tokens, int n_kv_heads);
+int cherryq_prefill_attention_f16(const void *q, const void *k, const void *v, const void *cos_table, const void *sin_table,
+                                  void *k_cache, void *v_cache, void *out, void *scratch, size_t scratch_bytes, int tokens,
+                                  int n_heads, int n_kv_heads, int head_dim, int max_len, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -57,6 +57,12 @@ _lib.cherryq_decode_head_supported.argtypes = [_int, _int]
 _lib.cherryq_decode_head_supported.restype = _int
 _lib.cherryq_decode_head_f16.argtypes = [_vp, _vp, _f, _vp, _vp, _int, _int, _vp]
 _lib.cherryq_decode_head_f16.restype = _int
+_lib.cherryq_prefill_norm_f16.argtypes = [_vp, _vp, _vp, _vp, _int, _int, _f, _vp]
+_lib.cherryq_prefill_norm_f16.restype = _int
+_lib.cherryq_prefill_attention_bytes.argtypes = [_int, _int]
+_lib.cherryq_prefill_attention_bytes.restype = ctypes.c_size_t
+_lib.cherryq_prefill_attention_f16.argtypes = [_vp] * 9 + [ctypes.c_size_t, _int, _int, _int, _int, _int, _vp]
+_lib.cherryq_prefill_attention_f16.restype = _int
 for _n in ("cherryq_decode_add_rmsnorm_f16", "cherryq_decode_rope_cache_f16", "cherryq_decode_attention_f16",
            "cherryq_decode_silu_mul_f16", "cherryq_decode_rope_attention_f16"):
     getattr(_lib, _n).restype = _int
@@ -635,37 +641,74 @@ class CherryLlamaDecoder(nn.Module):
     def prefill(self, prompt_ids: torch.Tensor) -> torch.Tensor:
         """The whole prompt in one batched pass, as the reference's model processes it
         (llama/modeling_llama_quant.py:1009-1100): every linear sees all T rows at once (the tiled
-        GEMM kernel from 17 rows, the small-batch kernel below), RMSNorm / rotary / causal attention
-        are torch operations with the reference's rounding points.  Fills the KV caches for
-        positions 0..T-1, leaves the decoder exactly where T token steps would (position T, the
+        kernels from 17 rows, the small-batch kernel below); residual + RMSNorm, rotary + cache write, causal
+        attention and SiLU * up are launches of their own with the reference's rounding points.  Fills the KV
+        caches for positions 0..T-1, leaves the decoder exactly where T token steps would (position T, the
         first generated token predicted and embedded) and returns the last position's logits."""
         cfg = self.cfg
         ids = prompt_ids.to(self.device_)
         T, nh, nkv, hd = ids.numel(), cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
         assert ids.dim() == 1 and 1 <= T <= cfg.max_position_embeddings
-
-        def norm(x, w):
-            xf = x.float()
-            return w * (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + cfg.rms_norm_eps)).half()
-
         pos = torch.arange(T, device=self.device_, dtype=torch.float32)
         inv = 1.0 / (cfg.rope_theta ** (torch.arange(0, hd, 2, device=self.device_, dtype=torch.float32) / hd))
         fr = torch.outer(pos, inv)
-        emb = torch.cat([fr, fr], dim=-1)
-        cos, sin = emb.cos().half()[None], emb.sin().half()[None]  # (1, T, hd)
+        cos, sin = fr.cos().half(), fr.sin().half()  # (T, hd / 2)
+
+        self.reset()
+        h = self.embed_tokens[ids]
+        x = torch.empty_like(h)
+        attend = self._prefill_attention(T, cos, sin) if hd == 128 else self._prefill_attention_torch(T, cos, sin)
+
+        def rows(t):  # what the launches take; a linear's output as it is, unless a module was replaced
+            return t.to(torch.float16).contiguous()
+
+        def add_norm(delta, weight, h=h, x=x):  # h += delta, x = RMSNorm(h)
+            _ok(_lib.cherryq_prefill_norm_f16(h.data_ptr(), None if delta is None else delta.data_ptr(), weight.data_ptr(),
+                                              x.data_ptr(), h.shape[0], cfg.hidden_size, cfg.rms_norm_eps, _stream()), "prefill_norm")
+
+        delta = None
+        for li, layer in enumerate(self.layers):
+            add_norm(delta, layer.input_layernorm)
+            a = attend(li, rows(layer.q_proj(x)), rows(layer.k_proj(x)), rows(layer.v_proj(x)))
+            delta = rows(layer.o_proj(a))
+            add_norm(delta, layer.post_attention_layernorm)
+            gate, up = rows(layer.gate_proj(x)), rows(layer.up_proj(x))
+            _ok(_lib.cherryq_decode_silu_mul_f16(gate.data_ptr(), up.data_ptr(), gate.data_ptr(), gate.numel(), _stream()), "silu_mul")
+            delta = rows(layer.down_proj(gate))
+        last = slice(T - 1, T)
+        add_norm(delta[last], self.norm, h[last], self.normed)
+        self.pos.fill_(T - 1)
+        self._head(self.normed, None)  # logits of the last prompt position; greedy tail: history[T-1], next embedding, pos = T
+        return self.logits
+
+    def _prefill_attention(self, T, cos, sin):
+        """attend(layer, q, k, v) for heads of 128: rotary embedding, cache write and causal attention in two launches."""
+        cfg = self.cfg
+        nh, nkv, ml = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.max_position_embeddings
+        scratch = torch.empty(_lib.cherryq_prefill_attention_bytes(T, nkv), dtype=torch.uint8, device=self.device_)
+        out = torch.empty(T, nh * 128, dtype=torch.float16, device=self.device_)
+
+        def attend(li, q, k, v):
+            _ok(_lib.cherryq_prefill_attention_f16(q.data_ptr(), k.data_ptr(), v.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+                                                   self.k_cache[li].data_ptr(), self.v_cache[li].data_ptr(), out.data_ptr(),
+                                                   scratch.data_ptr(), scratch.numel(), T, nh, nkv, 128, ml, _stream()),
+                "prefill_attention")
+            return out
+        return attend
+
+    def _prefill_attention_torch(self, T, cos, sin):
+        """The same for other head dimensions, as tensor operations."""
+        cfg = self.cfg
+        nh, nkv, hd = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
+        cos, sin = torch.cat([cos, cos], dim=-1)[None], torch.cat([sin, sin], dim=-1)[None]  # (1, T, hd)
+        mask = torch.full((T, T), float("-inf"), device=self.device_).triu(1)
+        rep = nh // nkv
 
         def rot(x):
             return torch.cat([-x[..., hd // 2:], x[..., :hd // 2]], dim=-1)
 
-        self.reset()
-        h = self.embed_tokens[ids]
-        mask = torch.full((T, T), float("-inf"), device=self.device_).triu(1)
-        rep = nh // nkv
-        for li, layer in enumerate(self.layers):
-            x = norm(h, layer.input_layernorm)
-            q = layer.q_proj(x).view(T, nh, hd).transpose(0, 1)
-            k = layer.k_proj(x).view(T, nkv, hd).transpose(0, 1)
-            v = layer.v_proj(x).view(T, nkv, hd).transpose(0, 1)
+        def attend(li, q, k, v):
+            q, k, v = q.view(T, nh, hd).transpose(0, 1), k.view(T, nkv, hd).transpose(0, 1), v.view(T, nkv, hd).transpose(0, 1)
             q = q * cos + rot(q) * sin
             k = k * cos + rot(k) * sin
             self.k_cache[li, :, :T].copy_(k)
@@ -673,14 +716,8 @@ class CherryLlamaDecoder(nn.Module):
             kk, vv = k.repeat_interleave(rep, 0), v.repeat_interleave(rep, 0)
             att = (q @ kk.transpose(1, 2)) / math.sqrt(hd)
             att = torch.softmax(att.float() + mask, dim=-1).half()
-            a = (att @ vv).transpose(0, 1).reshape(T, nh * hd)
-            h = h + layer.o_proj(a)
-            x = norm(h, layer.post_attention_layernorm)
-            h = h + layer.down_proj(torch.nn.functional.silu(layer.gate_proj(x)) * layer.up_proj(x))
-        self.normed.copy_(norm(h[T - 1:T], self.norm))
-        self.pos.fill_(T - 1)
-        self._head(self.normed, None)  # logits of the last prompt position; greedy tail: history[T-1], next embedding, pos = T
-        return self.logits
+            return (att @ vv).transpose(0, 1).reshape(T, nh * hd)
+        return attend
 
     @torch.inference_mode()
     def generate(self, prompt_ids: torch.Tensor, max_new_tokens: int, use_graph=True, sync_each_token=False,

@@ -812,4 +812,38 @@ int cherryq_decode_silu_mul_f16(const void *gate, const void *up, void *out, int
                                     reinterpret_cast<__half *>(out), n, reinterpret_cast<hipStream_t>(stream));
 }
 
+int cherryq_prefill_norm_f16(void *hidden, const void *delta, const void *weight, void *normed, int rows, int hidden_size,
+                             float eps, void *stream) {
+    if (!hidden || !weight || !normed) return CHERRYQ_E_NULL;
+    if (rows <= 0 || hidden_size <= 0 || hidden_size % 8) return CHERRYQ_E_SHAPE;
+    if (hidden_size > cq::kPrefillMaxHidden) return CHERRYQ_E_UNSUPPORTED;
+    if (!cq::aligned(hidden, 16) || !cq::aligned(weight, 16) || !cq::aligned(normed, 16) || (delta && !cq::aligned(delta, 16)))
+        return CHERRYQ_E_ALIGN;
+    return (int)cq::launch_prefill_norm(reinterpret_cast<__half *>(hidden), reinterpret_cast<const __half *>(delta),
+                                        reinterpret_cast<const __half *>(weight), reinterpret_cast<__half *>(normed), rows,
+                                        hidden_size, eps, reinterpret_cast<hipStream_t>(stream));
+}
+
+size_t cherryq_prefill_attention_bytes(int tokens, int n_kv_heads) {
+    return tokens > 0 && n_kv_heads > 0 ? cq::prefill_attention_bytes(tokens, n_kv_heads) : 0;
+}
+
+int cherryq_prefill_attention_f16(const void *q, const void *k, const void *v, const void *cos_table, const void *sin_table,
+                                  void *k_cache, void *v_cache, void *out, void *scratch, size_t scratch_bytes, int tokens,
+                                  int n_heads, int n_kv_heads, int head_dim, int max_len, void *stream) {
+    if (!q || !k || !v || !cos_table || !sin_table || !k_cache || !v_cache || !out) return CHERRYQ_E_NULL;
+    if (tokens <= 0 || tokens > max_len || n_kv_heads <= 0 || n_heads <= 0 || n_heads % n_kv_heads) return CHERRYQ_E_SHAPE;
+    // heads and 16-query tiles are grid y dimensions
+    if (head_dim != 128 || n_kv_heads > 65535 || tokens > 1000000) return CHERRYQ_E_UNSUPPORTED;
+    for (const void *p : {q, k, v, cos_table, sin_table, (const void *)k_cache, (const void *)v_cache, (const void *)out})
+        if (!cq::aligned(p, 16)) return CHERRYQ_E_ALIGN;
+    if (!scratch || !cq::aligned(scratch, 256) || scratch_bytes < cq::prefill_attention_bytes(tokens, n_kv_heads))
+        return CHERRYQ_E_WORKSPACE;
+    return (int)cq::launch_prefill_attention(
+        reinterpret_cast<const __half *>(q), reinterpret_cast<const __half *>(k), reinterpret_cast<const __half *>(v),
+        reinterpret_cast<const __half *>(cos_table), reinterpret_cast<const __half *>(sin_table),
+        reinterpret_cast<__half *>(k_cache), reinterpret_cast<__half *>(v_cache), reinterpret_cast<__half *>(out), scratch, tokens,
+        n_heads, n_kv_heads, max_len, reinterpret_cast<hipStream_t>(stream));
+}
+
 }  // extern "C"

@@ -665,14 +665,22 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const __half *__restr
     out[i] = __float2half_rn(o);
 }
 
-// out <- fp16(silu(gate)) * up
+// out <- fp16(silu(gate)) * up, VEC elements a thread: 16-byte accesses where the operands allow them (a prompt of 128 rows
+// of 11008: 4.3 us, most of it the launch and one round trip to memory)
+template <int VEC>
 __global__ __launch_bounds__(256) void silu_mul_kernel(const __half *__restrict__ gate, const __half *__restrict__ up,
                                                        __half *__restrict__ out, int n) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const float g = __half2float(gate[i]);
-    const float a = __half2float(__float2half_rn(g / (1.f + __expf(-g))));
-    out[i] = __float2half_rn(a * __half2float(up[i]));
+    typedef _Float16 vec_t __attribute__((ext_vector_type(VEC)));
+    const size_t i = (size_t)VEC * (blockIdx.x * 256 + threadIdx.x);
+    if (i >= (size_t)n) return;
+    const vec_t g = *reinterpret_cast<const vec_t *>(gate + i), u = *reinterpret_cast<const vec_t *>(up + i);
+    vec_t o;
+#pragma unroll
+    for (int e = 0; e < VEC; e++) {
+        const float x = (float)g[e];
+        o[e] = (_Float16)((float)(_Float16)(x / (1.f + __expf(-x))) * (float)u[e]);
+    }
+    *reinterpret_cast<vec_t *>(out + i) = o;
 }
 
 // Unquantised fp16 head: logits[v] = fp16(sum_k act[k] * W[v][k]) with W (vocab, hidden) row-major
@@ -912,7 +920,10 @@ hipError_t launch_attn_combine(const __half *part, const float *ml, __half *out,
 }
 
 hipError_t launch_silu_mul(const __half *gate, const __half *up, __half *out, int n, hipStream_t stream) {
-    hipLaunchKernelGGL(silu_mul_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, stream, gate, up, out, n);
+    if (n % 8 == 0 && aligned(gate, 16) && aligned(up, 16) && aligned(out, 16))
+        hipLaunchKernelGGL(silu_mul_kernel<8>, dim3(ceil_div(n / 8, 256)), dim3(256), 0, stream, gate, up, out, n);
+    else
+        hipLaunchKernelGGL(silu_mul_kernel<1>, dim3(ceil_div(n, 256)), dim3(256), 0, stream, gate, up, out, n);
     return hipGetLastError();
 }
 

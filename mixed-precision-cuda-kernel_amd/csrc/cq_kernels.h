@@ -234,6 +234,15 @@ bool head_supported(int vocab, int hidden);
 hipError_t launch_head(const __half *h, const __half *norm_w, float eps, const __half *W, __half *logits, int vocab,
                        int hidden, hipStream_t stream);
 hipError_t launch_silu_mul(const __half *gate, const __half *up, __half *out, int n, hipStream_t stream);
+
+// cq_prefill.hip: the operations between the linears for all rows of a prompt.
+constexpr int kPrefillMaxHidden = 8192;
+hipError_t launch_prefill_norm(__half *h, const __half *delta, const __half *weight, __half *y, int rows, int H, float eps,
+                               hipStream_t stream);
+size_t prefill_attention_bytes(int T, int n_kv_heads);
+hipError_t launch_prefill_attention(const __half *q, const __half *k, const __half *v, const __half *cos_t, const __half *sin_t,
+                                    __half *k_cache, __half *v_cache, __half *out, void *scratch, int T, int n_heads,
+                                    int n_kv_heads, int max_len, hipStream_t stream);
 int attn_max_len();
 
 }  // namespace cq
