@@ -460,7 +460,17 @@ int cherryq_decode_silu_mul_f16(const void *gate, const void *up, void *out, int
  *   keys and values are written to positions 0 .. tokens - 1 of the caches ([n_kv_heads][max_len][128]), out is
  *   (tokens, n_heads * 128) (:95-210, :671-696).  scratch: cherryq_prefill_attention_bytes() bytes,
  *   256-byte aligned, uninitialised.  All tensors 16-byte aligned; head_dim must be 128.
+ * cherryq_prefill_matmul_group_f16: layers[i].mul (+)= vec W_i^T for 1 to 3 layers that read the same activations and share bits,
+ *   in_features, num_cherries and group size, two rows and more, as one product: layers that do not fill the chip each
+ *   do so together.  workspace (all zero before and after) and scratch (uninitialised) as for the single
+ *   products above, of the sizes that the two functions answer (0: arguments that are refused).
+ *   CHERRYQ_E_UNSUPPORTED: shapes that a single product would give to another kernel.
  */
+size_t cherryq_prefill_matmul_group_workspace_bytes(int rows, int in_features, int n_layers, const int *out_features, int num_cherries);
+size_t cherryq_prefill_matmul_group_scratch_bytes(int rows, int in_features, int n_layers, const int *out_features, int num_cherries);
+int cherryq_prefill_matmul_group_f16(int w_bits, const void *vec, const cherryq_layer *layers, int n_layers, int rows, int in_features,
+                                     int num_cherries, int group_size, int accumulate, void *workspace, size_t workspace_bytes,
+                                     void *scratch, size_t scratch_bytes, void *stream);
 int cherryq_prefill_norm_f16(void *hidden, const void *delta /* may be NULL */, const void *weight, void *normed, int rows,
                              int hidden_size, float eps, void *stream);
 size_t cherryq_prefill_attention_bytes(int tokens, int n_kv_heads);

@@ -116,6 +116,62 @@ def matvec_group(mods, vec, outs, vec_gate=None, accumulate=False, norm_weight=N
                                              ws.data_ptr(), ws.numel(), stream), "matvec_group")
 
 
+for _n in ("workspace", "scratch"):
+    _f2 = getattr(_lib, "cherryq_prefill_matmul_group_%s_bytes" % _n)
+    _f2.argtypes, _f2.restype = [_int, _int, _int, ctypes.POINTER(_int), _int], ctypes.c_size_t
+_lib.cherryq_prefill_matmul_group_f16.argtypes = [_int, _vp, ctypes.POINTER(_Layer), _int, _int, _int, _int, _int, _int, _vp,
+                                                  ctypes.c_size_t, _vp, ctypes.c_size_t, _vp]
+_lib.cherryq_prefill_matmul_group_f16.restype = _int
+
+
+def matmul_group_supported(mods, rows) -> bool:
+    """Whether matmul_group gives what calling each module would: plain QuantLinear modules over their
+    checkpoint buffers, of one shape family, at a number of rows that goes to the tiled kernel."""
+    m0 = mods[0]
+    if torch.nn.modules.module._has_any_global_hook():
+        return False
+    for m in mods:
+        if (type(m) is not QuantLinear or "forward" in m.__dict__ or m._forward_hooks or m._forward_pre_hooks or m.bias is not None
+                or m._released or m.dequantized or not m._layerwise_dequantize or not 17 <= rows < m.prefill_rows):
+            return False
+        if (m.w_bits, m.group_size, m.num_cherries, m.in_features) != (m0.w_bits, m0.group_size, m0.num_cherries, m0.in_features):
+            return False
+        k, n, c = m.in_features, m.out_features, m.num_cherries
+        if (m.w_bits not in (3, 4) or m.group_size <= 0 or m.group_size % 32 or c >= k
+                or m.qweight.shape != ((k - c) // 8 * m.w_bits, n) or m.cherry_weight.shape != (c, n)
+                or m.cherry_indices.shape != (c,) or m.scales.shape != (-(-(k - c) // m.group_size), n)):
+            return False
+        for t, dt in ((m.qweight, torch.uint8), (m.scales, torch.float16), (m.cherry_weight, torch.float16),
+                      (m.cherry_indices, torch.int16)):
+            if not t.is_cuda or t.device != m0.qweight.device or t.dtype != dt or not t.is_contiguous():
+                return False
+    return True
+
+
+def matmul_group(mods, x):
+    """[x @ W_i^T] for 1..3 QuantLinear modules that matmul_group_supported takes, as one product; None where the
+    library gives the single products to another kernel."""
+    m0 = mods[0]
+    rows, count = x.shape[0], len(mods)
+    if (tuple(x.shape) != (rows, m0.in_features) or x.dtype != torch.float16 or not x.is_contiguous()
+            or x.device != m0.qweight.device):
+        raise RuntimeError("matmul_group: x must be a contiguous (rows, in_features) fp16 tensor on the layers' GPU")
+    outs = [torch.empty(rows, m.out_features, dtype=torch.float16, device=x.device) for m in mods]
+    arr = (_Layer * count)(*[_Layer(m.qweight.data_ptr(), quant_cuda._ptr(m.cherry_weight), quant_cuda._ptr(m.cherry_indices),
+                                    m.scales.data_ptr(), o.data_ptr(), m.out_features) for m, o in zip(mods, outs)])
+    ns = (_int * count)(*[m.out_features for m in mods])
+    sizes = (rows, m0.in_features, count, ns, m0.num_cherries)
+    stream = _stream()
+    ws = quant_cuda._workspace(x.device, stream, _lib.cherryq_prefill_matmul_group_workspace_bytes(*sizes))
+    sc = quant_cuda._scratch(x.device, stream, _lib.cherryq_prefill_matmul_group_scratch_bytes(*sizes))
+    rc = _lib.cherryq_prefill_matmul_group_f16(m0.w_bits, x.data_ptr(), arr, count, rows, m0.in_features, m0.num_cherries,
+                                               m0.group_size, 0, ws.data_ptr(), ws.numel(), sc.data_ptr(), sc.numel(), stream)
+    if rc == -7:
+        return None
+    _ok(rc, "matmul_group")
+    return outs
+
+
 class _StreamLayer(ctypes.Structure):
     _fields_ = [("stream", _vp), ("stream_bytes", ctypes.c_size_t), ("mul", _vp), ("out_features", _int)]
 
@@ -666,13 +722,17 @@ class CherryLlamaDecoder(nn.Module):
             _ok(_lib.cherryq_prefill_norm_f16(h.data_ptr(), None if delta is None else delta.data_ptr(), weight.data_ptr(),
                                               x.data_ptr(), h.shape[0], cfg.hidden_size, cfg.rms_norm_eps, _stream()), "prefill_norm")
 
+        def project(*mods):  # layers that read x: as one product where that is what their own calls compute
+            outs = matmul_group(mods, x) if matmul_group_supported(mods, T) else None
+            return [rows(m(x)) for m in mods] if outs is None else outs
+
         delta = None
         for li, layer in enumerate(self.layers):
             add_norm(delta, layer.input_layernorm)
-            a = attend(li, rows(layer.q_proj(x)), rows(layer.k_proj(x)), rows(layer.v_proj(x)))
+            a = attend(li, *project(layer.q_proj, layer.k_proj, layer.v_proj))
             delta = rows(layer.o_proj(a))
             add_norm(delta, layer.post_attention_layernorm)
-            gate, up = rows(layer.gate_proj(x)), rows(layer.up_proj(x))
+            gate, up = project(layer.gate_proj, layer.up_proj)
             _ok(_lib.cherryq_decode_silu_mul_f16(gate.data_ptr(), up.data_ptr(), gate.data_ptr(), gate.numel(), _stream()), "silu_mul")
             delta = rows(layer.down_proj(gate))
         last = slice(T - 1, T)

@@ -124,7 +124,8 @@ static int matmul_f16(const void *vec, const uint8_t *qweight, const void *cherr
         e = launch_batch(BITS, x, qweight, cw, cherry_indices, sc, y, B, K, N, C, G, accumulate, workspace, scratch, s);
     } else if (!force_generic() && B >= 2 && prompt_supported(BITS, B, K, N, C, G)) {
         // ... unless the group is no whole number of the batch kernel's units of 128 positions
-        e = launch_prompt(BITS, x, qweight, cw, cherry_indices, sc, y, B, K, N, C, G, accumulate, workspace, scratch, s);
+        const PromptMember layer = {qweight, cw, cherry_indices, sc, y, N};
+        e = launch_prompt(BITS, x, &layer, 1, B, K, C, G, accumulate, workspace, scratch, s);
     } else if (!force_generic() && B >= kGemmMinRows && gemm_supported(BITS, B, K, N, C, G)) {
         // activations of more than 2 GiB in operand order, beyond the prompt kernel's buffer offsets
         e = launch_gemm(BITS, x, qweight, cw, cherry_indices, sc, y, B, K, N, C, G, accumulate, workspace, scratch, s);
@@ -822,6 +823,53 @@ int cherryq_prefill_norm_f16(void *hidden, const void *delta, const void *weight
     return (int)cq::launch_prefill_norm(reinterpret_cast<__half *>(hidden), reinterpret_cast<const __half *>(delta),
                                         reinterpret_cast<const __half *>(weight), reinterpret_cast<__half *>(normed), rows,
                                         hidden_size, eps, reinterpret_cast<hipStream_t>(stream));
+}
+
+static bool prefill_group_dims(int rows, int K, int n_layers, const int *N, int C) {
+    if (rows < 2 || K <= 0 || C < 0 || C >= K || n_layers < 1 || n_layers > cq::kPromptMaxGroup || !N) return false;
+    for (int i = 0; i < n_layers; i++)
+        if (N[i] <= 0) return false;
+    return true;
+}
+
+size_t cherryq_prefill_matmul_group_workspace_bytes(int rows, int in_features, int n_layers, const int *out_features, int num_cherries) {
+    if (!prefill_group_dims(rows, in_features, n_layers, out_features, num_cherries)) return 0;
+    return cq::prompt_plan(rows, in_features, out_features, n_layers, num_cherries).workspace_bytes;
+}
+
+size_t cherryq_prefill_matmul_group_scratch_bytes(int rows, int in_features, int n_layers, const int *out_features, int num_cherries) {
+    if (!prefill_group_dims(rows, in_features, n_layers, out_features, num_cherries)) return 0;
+    return cq::prompt_plan(rows, in_features, out_features, n_layers, num_cherries).scratch_bytes;
+}
+
+int cherryq_prefill_matmul_group_f16(int w_bits, const void *vec, const cherryq_layer *layers, int n_layers, int rows, int in_features,
+                                     int num_cherries, int group_size, int accumulate, void *workspace, size_t workspace_bytes,
+                                     void *scratch, size_t scratch_bytes, void *stream) {
+    using namespace cq;
+    if (w_bits != 3 && w_bits != 4) return CHERRYQ_E_BITS;
+    if (!layers) return CHERRYQ_E_NULL;
+    if (n_layers < 1 || n_layers > kPromptMaxGroup || rows < 0) return CHERRYQ_E_SHAPE;
+    const int K = in_features, C = num_cherries, G = group_size;
+    if (C > 0 && K > 32768) return CHERRYQ_E_SHAPE;  // int16 channel indices cannot name the columns
+    if (w_bits == 4 && G < 128) return CHERRYQ_E_GROUP;
+    int N[kPromptMaxGroup];
+    PromptMember members[kPromptMaxGroup];
+    for (int i = 0; i < n_layers; i++) {
+        const cherryq_layer &l = layers[i];
+        const int rc = check_tensors(vec, l.qweight, l.cherry_weight, l.cherry_indices, l.scales, l.mul, rows, K, l.out_features, C, G);
+        if (rc) return rc;
+        if (rows > 0 && (force_generic() || !prompt_supported(w_bits, rows, K, l.out_features, C, G))) return CHERRYQ_E_UNSUPPORTED;
+        N[i] = l.out_features;
+        members[i] = {l.qweight, reinterpret_cast<const __half *>(l.cherry_weight), l.cherry_indices,
+                      reinterpret_cast<const __half *>(l.scales), reinterpret_cast<__half *>(l.mul), l.out_features};
+    }
+    if (rows == 0) return CHERRYQ_OK;
+    const PromptPlan plan = prompt_plan(rows, K, N, n_layers, C);
+    if (!workspace || !aligned(workspace, 256) || workspace_bytes < plan.workspace_bytes || !scratch || !aligned(scratch, 256) ||
+        scratch_bytes < plan.scratch_bytes)
+        return CHERRYQ_E_WORKSPACE;
+    return (int)launch_prompt(w_bits, reinterpret_cast<const __half *>(vec), members, n_layers, rows, K, C, G, accumulate, workspace,
+                              scratch, reinterpret_cast<hipStream_t>(stream));
 }
 
 size_t cherryq_prefill_attention_bytes(int tokens, int n_kv_heads) {

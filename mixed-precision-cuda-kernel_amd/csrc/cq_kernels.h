@@ -112,11 +112,20 @@ struct PromptPlan {
     size_t a_bytes, partial_bytes;    // scratch: activations in operand order, then the per-split partial tiles
     size_t scratch_bytes;
 };
+constexpr int kPromptMaxGroup = 3;
+struct PromptMember {  // a layer of a launch: all read the same activations and have the same K, C and group size
+    const uint8_t *qweight;
+    const __half *cherry_weight;
+    const int16_t *cherry_indices;
+    const __half *scales;
+    __half *out;
+    int N;
+};
 PromptPlan prompt_plan(int M, int K, int N, int C);
+PromptPlan prompt_plan(int M, int K, const int *N, int count, int C);
 bool prompt_supported(int bits, int M, int K, int N, int C, int G);
-hipError_t launch_prompt(int bits, const __half *vec, const uint8_t *qweight, const __half *cherry_weight,
-                         const int16_t *cherry_indices, const __half *scales, __half *mul, int M, int K, int N, int C, int G,
-                         int accumulate, void *workspace, void *scratch, hipStream_t stream);
+hipError_t launch_prompt(int bits, const __half *vec, const PromptMember *layers, int count, int M, int K, int C, int G, int accumulate,
+                         void *workspace, void *scratch, hipStream_t stream);
 
 // cq_stream.hip: batch-1 matvec over a load-time repacked weight stream (tiles of 16 columns, each
 // tile's whole K range contiguous; no split-K, no workspace).

@@ -92,7 +92,7 @@ constexpr PromptShape kPromptShapes[] = {
     {8, 8, 2, 10.80f, 3.50f, 2.89f, 0.f, 14.20f, 0.51f},   // 128 x 256, pairs of wavefronts side by side
 };
 
-PromptPlan prompt_plan(int M, int K, int N, int C) {
+PromptPlan prompt_plan(int M, int K, const int *N, int count, int C) {
     PromptPlan best;
     float best_cost = 3.4e38f;
     const int units = K > C ? ceil_div(K - C, kUnitK) : 1;  // sizes are asked for before the launch is refused
@@ -101,7 +101,8 @@ PromptPlan prompt_plan(int M, int K, int N, int C) {
         PromptPlan p;
         p.mt = s.mt, p.nc = s.nc, p.ns = s.ns;
         p.mtiles = ceil_div(M, 16 * s.mt);
-        p.ntiles = ceil_div(N, 16 * s.nc * s.ns);
+        p.ntiles = 0;
+        for (int i = 0; i < count; i++) p.ntiles += ceil_div(N[i], 16 * s.nc * s.ns);
         const long long tiles = (long long)p.mtiles * p.ntiles;
         const int kways = prompt_kways(s.mt, s.nc, s.ns);
         for (int splits = 1; splits <= kPromptMaxSplits; splits++) {
@@ -128,24 +129,32 @@ PromptPlan prompt_plan(int M, int K, int N, int C) {
     p.steps = p.units * 4 + p.csteps;
     p.a_bytes = ((size_t)p.steps * p.mtiles * p.mt * 1024 + 255) / 256 * 256;
     p.partial_bytes = p.splits > 1 ? p.splits * tiles * p.mt * p.nc * p.ns * 256 * sizeof(float) : 0;
-    p.scratch_bytes = p.a_bytes + p.partial_bytes;
+    p.scratch_bytes = count * p.a_bytes + p.partial_bytes;
     p.workspace_bytes = (tiles * sizeof(unsigned) + 255) / 256 * 256;
     return p;
 }
 
+PromptPlan prompt_plan(int M, int K, int N, int C) { return prompt_plan(M, K, &N, 1, C); }
+
 // ---- activation preparation ------------------------------------------------------------------------
 // a[(step * m16 + tile) * 64 + lane], lane = (q, i): x[16 tile + i][positions 32 step + 8 q + ord[0..7]].  A workgroup
 // takes one unit (4 steps) of 16 rows: the unit's dense columns are a contiguous range, loaded in whole lines
-// into LDS and gathered from there.  Rows >= M and positions past the end read as 0.
+// into LDS and gathered from there.  Rows >= M and positions past the end read as 0.  Every layer of a group has its own
+// cherry channels and so its own copy (blockIdx.z).
 constexpr int kPrepCols = 256;     // dense columns of a unit that are staged; a wider range is gathered from memory
 constexpr int kPrepIdx = 1024;     // cherry channels staged
+struct PromptIndices {
+    const int16_t *of[kPromptMaxGroup];
+};
 template <int BITS>
-__global__ __launch_bounds__(256) void prompt_prep_kernel(const __half *__restrict__ x, const int16_t *__restrict__ cherry_indices,
-                                                          uint4 *__restrict__ a, int M, int K, int C, int units, int m16, int wide) {
+__global__ __launch_bounds__(256) void prompt_prep_kernel(const __half *__restrict__ x, PromptIndices indices, uint4 *__restrict__ a,
+                                                          size_t a_bytes, int M, int K, int C, int units, int m16, int wide) {
     __shared__ __attribute__((aligned(16))) uint16_t s_x[16][kPrepCols + 8];
     __shared__ int16_t s_idx[kPrepIdx];
     const int t = threadIdx.x, lane = t & 63, q = lane >> 4, i = lane & 15, tile = blockIdx.y, Kn = K - C;
-    const int row = 16 * tile + i;
+    const int row = 16 * tile + i, layer = blockIdx.z;
+    const int16_t *__restrict__ cherry_indices = layer == 0 ? indices.of[0] : layer == 1 ? indices.of[1] : indices.of[2];
+    a += layer * (a_bytes / sizeof(uint4));
     unsigned short h[8];
 #pragma unroll
     for (int kk = 0; kk < 8; kk++) h[kk] = 0;
@@ -281,12 +290,21 @@ __device__ __forceinline__ void prompt_mfma(float4_t &acc, const u32x4 &a, const
     acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), acc, 0, 0, 0);
 }
 
+// The layers of a launch: their column tiles follow one another.  Layers that read the same rows fill the chip together
+// and with larger tiles (128 rows, 4 bits, preparation included: three of 4096 -> 4096 54 -> 33 us, two of 4096 -> 11008
+// 58 -> 41, two of 8192 -> 28672 140 -> 121; with 500 rows 99 -> 71, 130 -> 116, 452 -> 447).
+struct PromptMembers {
+    const uint8_t *qweight[kPromptMaxGroup];
+    const __half *cherry_weight[kPromptMaxGroup], *scales[kPromptMaxGroup];
+    __half *out[kPromptMaxGroup];
+    int N[kPromptMaxGroup], first[kPromptMaxGroup];  // columns, first column tile (past the end: no such layer)
+};
+
 // WHOLE: groups are whole units
 template <int BITS, int MT, int NC, int NS, bool WHOLE>
 __global__ __launch_bounds__(64 * prompt_waves(MT, NC), MT * NC == 64 ? 1 : MT * NC == 8 ? 4 : 2) void prompt_kernel(
-    const uint8_t *__restrict__ qweight, const __half *__restrict__ cherry_weight, const __half *__restrict__ scales,
-    __half *__restrict__ out, const u32x4 *__restrict__ a_frag, float *__restrict__ partial, unsigned *__restrict__ tickets,
-    int M, int K, int N, int C, int G, int accumulate, PromptPlan plan) {
+    PromptMembers members, const u32x4 *__restrict__ a_all, float *__restrict__ partial, unsigned *__restrict__ tickets, int M, int K,
+    int C, int G, int accumulate, PromptPlan plan) {
     constexpr int WAVES = prompt_waves(MT, NC), KW = WAVES / NS, COLS = 16 * NC, ND = NC / 4;  // ND: dwords of a byte row a lane
     typedef uint32_t wd_t __attribute__((ext_vector_type(ND)));
     typedef uint32_t sc_t __attribute__((ext_vector_type(NC / 2)));
@@ -296,7 +314,18 @@ __global__ __launch_bounds__(64 * prompt_waves(MT, NC), MT * NC == 64 ? 1 : MT *
     const int tiles = plan.mtiles * plan.ntiles, per_xcd = ceil_div(tiles, 8);
     const int tile = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3), split = blockIdx.y;
     if (tile >= tiles) return;
-    const int ntile = tile / plan.mtiles, mtile = tile % plan.mtiles;
+    const int mtile = tile % plan.mtiles;
+    int ntile = tile / plan.mtiles;
+    // selected, not indexed: the arguments arrive with one scalar load
+    const int layer = (ntile >= members.first[1] ? 1 : 0) + (ntile >= members.first[2] ? 1 : 0);
+    auto of = [&](auto &what) { return layer == 0 ? what[0] : layer == 1 ? what[1] : what[2]; };
+    const uint8_t *__restrict__ const qweight = of(members.qweight);
+    const __half *__restrict__ const cherry_weight = of(members.cherry_weight);
+    const __half *__restrict__ const scales = of(members.scales);
+    __half *__restrict__ const out = of(members.out);
+    const u32x4 *__restrict__ const a_frag = a_all + layer * (plan.a_bytes / sizeof(u32x4));
+    const int N = of(members.N);
+    ntile -= of(members.first);
     const int kpart = wave % KW, npart = wave / KW;
     const int n0 = (ntile * NS + npart) * COLS + NC * nl, m16 = plan.mtiles * MT, Kn = K - C;
     const bool col_ok = n0 < N;
@@ -538,30 +567,39 @@ bool prompt_supported(int bits, int M, int K, int N, int C, int G) {
 }
 
 template <int BITS, int MT, int NC, int NS>
-static hipError_t launch_prompt_mt(const __half *vec, const uint8_t *qweight, const __half *cherry_weight,
-                                   const int16_t *cherry_indices, const __half *scales, __half *mul, int M, int K, int N, int C,
-                                   int G, int accumulate, const PromptPlan &plan, void *workspace, void *scratch, hipStream_t stream) {
+static hipError_t launch_prompt_mt(const __half *vec, const PromptMember *layers, int count, int M, int K, int C, int G, int accumulate,
+                                   const PromptPlan &plan, void *workspace, void *scratch, hipStream_t stream) {
     u32x4 *a = reinterpret_cast<u32x4 *>(scratch);
-    float *partial = reinterpret_cast<float *>(reinterpret_cast<char *>(scratch) + plan.a_bytes);
+    float *partial = reinterpret_cast<float *>(reinterpret_cast<char *>(scratch) + count * plan.a_bytes);
     unsigned *tickets = reinterpret_cast<unsigned *>(workspace);
-    hipLaunchKernelGGL(prompt_prep_kernel<BITS>, dim3(plan.units + ceil_div(plan.csteps, 4), plan.mtiles * MT), dim3(256), 0, stream,
-                       vec, cherry_indices, reinterpret_cast<uint4 *>(a), M, K, C, plan.units, plan.mtiles * MT, aligned(vec, 16) ? 1 : 0);
+    PromptIndices indices;
+    PromptMembers members;
+    int first = 0;
+    for (int i = 0; i < kPromptMaxGroup; i++) {
+        const PromptMember &l = layers[i < count ? i : 0];
+        indices.of[i] = l.cherry_indices;
+        members.qweight[i] = l.qweight, members.cherry_weight[i] = l.cherry_weight, members.scales[i] = l.scales, members.out[i] = l.out;
+        members.N[i] = l.N, members.first[i] = first;
+        if (i < count) first += ceil_div(l.N, 16 * NC * NS);
+    }
+    hipLaunchKernelGGL(prompt_prep_kernel<BITS>, dim3(plan.units + ceil_div(plan.csteps, 4), plan.mtiles * MT, count), dim3(256), 0, stream,
+                       vec, indices, reinterpret_cast<uint4 *>(a), plan.a_bytes, M, K, C, plan.units, plan.mtiles * MT,
+                       aligned(vec, 16) ? 1 : 0);
     const dim3 grid(8 * ceil_div(plan.mtiles * plan.ntiles, 8), plan.splits);
     auto *const kernel = G % kUnitK == 0 ? prompt_kernel<BITS, MT, NC, NS, true> : prompt_kernel<BITS, MT, NC, NS, false>;
-    hipLaunchKernelGGL(kernel, grid, dim3(64 * prompt_waves(MT, NC)), 0, stream, qweight, cherry_weight, scales, mul, a, partial, tickets, M,
-                       K, N, C, G, accumulate, plan);
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * prompt_waves(MT, NC)), 0, stream, members, a, partial, tickets, M, K, C, G, accumulate, plan);
     return hipGetLastError();
 }
 
 template <int BITS>
-static hipError_t launch_prompt_bits(const __half *vec, const uint8_t *qweight, const __half *cherry_weight,
-                                     const int16_t *cherry_indices, const __half *scales, __half *mul, int M, int K, int N,
-                                     int C, int G, int accumulate, void *workspace, void *scratch, hipStream_t stream) {
-    const PromptPlan plan = prompt_plan(M, K, N, C);
-#define CQ_PROMPT(MT_, NC_, NS_)                                                                                            \
-    if (plan.mt == MT_ && plan.nc == NC_ && plan.ns == NS_)                                                                \
-    return launch_prompt_mt<BITS, MT_, NC_, NS_>(vec, qweight, cherry_weight, cherry_indices, scales, mul, M, K, N, C, G,  \
-                                                 accumulate, plan, workspace, scratch, stream)
+static hipError_t launch_prompt_bits(const __half *vec, const PromptMember *layers, int count, int M, int K, int C, int G, int accumulate,
+                                     void *workspace, void *scratch, hipStream_t stream) {
+    int N[kPromptMaxGroup];
+    for (int i = 0; i < count; i++) N[i] = layers[i].N;
+    const PromptPlan plan = prompt_plan(M, K, N, count, C);
+#define CQ_PROMPT(MT_, NC_, NS_)                            \
+    if (plan.mt == MT_ && plan.nc == NC_ && plan.ns == NS_) \
+    return launch_prompt_mt<BITS, MT_, NC_, NS_>(vec, layers, count, M, K, C, G, accumulate, plan, workspace, scratch, stream)
     CQ_PROMPT(2, 4, 1);
     CQ_PROMPT(4, 4, 1);
     CQ_PROMPT(8, 4, 1);
@@ -571,14 +609,11 @@ static hipError_t launch_prompt_bits(const __half *vec, const uint8_t *qweight, 
     return hipErrorInvalidConfiguration;
 }
 
-hipError_t launch_prompt(int bits, const __half *vec, const uint8_t *qweight, const __half *cherry_weight,
-                         const int16_t *cherry_indices, const __half *scales, __half *mul, int M, int K, int N, int C, int G,
-                         int accumulate, void *workspace, void *scratch, hipStream_t stream) {
-    if (bits == 4)
-        return launch_prompt_bits<4>(vec, qweight, cherry_weight, cherry_indices, scales, mul, M, K, N, C, G, accumulate, workspace,
-                                     scratch, stream);
-    return launch_prompt_bits<3>(vec, qweight, cherry_weight, cherry_indices, scales, mul, M, K, N, C, G, accumulate, workspace,
-                                 scratch, stream);
+hipError_t launch_prompt(int bits, const __half *vec, const PromptMember *layers, int count, int M, int K, int C, int G, int accumulate,
+                         void *workspace, void *scratch, hipStream_t stream) {
+    if (count < 1 || count > kPromptMaxGroup) return hipErrorInvalidValue;
+    return bits == 4 ? launch_prompt_bits<4>(vec, layers, count, M, K, C, G, accumulate, workspace, scratch, stream)
+                     : launch_prompt_bits<3>(vec, layers, count, M, K, C, G, accumulate, workspace, scratch, stream);
 }
 
 }  // namespace cq

@@ -89,3 +89,25 @@ def test_silu_mul_widths(dec, n, shift):
     torch.cuda.synchronize()
     want = torch.nn.functional.silu(g.double()).cpu() * u.double().cpu()
     assert rel(o[:n], want) < 2 * 2 ** -11 and not o[n:].any()
+
+
+# layers of different widths whose tiles share a launch: a remainder of columns, K splits, groups that are no whole unit
+@pytest.mark.parametrize("bits,k,ns,rows,group", [(4, 1024, (1024, 256, 256), 17, 128), (4, 4096, (520, 8), 99, 128),
+                                                  (3, 4096, (1000, 2056, 504), 40, 64), (4, 2048, (5504, 5504), 511, 256),
+                                                  (3, 8192, (8192, 1024, 1024), 128, 128), (4, 1032, (264,), 33, 128)])
+def test_matmul_group_matches_the_single_products(dec, bits, k, ns, rows, group):
+    print("[case] matmul_group", bits, k, ns, rows, group, flush=True)
+    cfg = dec.DecoderConfig(w_bits=bits, group_size=group, cherry_fraction=1 / 64)
+    gen = torch.Generator(device="cuda").manual_seed(k + rows)
+    mods = [dec.random_packed_linear(cfg, k, n, gen, torch.device("cuda")) for n in ns]
+    x = torch.randn(rows, k, device="cuda", generator=gen).half()
+    assert dec.matmul_group_supported(mods, rows)
+    for _ in range(2):  # the second call finds the workspace as the first one left it
+        got = dec.matmul_group(mods, x)
+        for m, o in zip(mods, got):
+            # the same operands summed in another order, then rounded: half a unit of fp16 each
+            assert rel(o, m(x).double().cpu()) < 2 ** -11
+            want = x.double().cpu() @ m.unpack().double().cpu().t()
+            assert rel(o, want) < 2 ** -11
+    mods[0].register_forward_hook(lambda *a: None)
+    assert not dec.matmul_group_supported(mods, rows) and not dec.matmul_group_supported(mods[1:] or mods, 16)
