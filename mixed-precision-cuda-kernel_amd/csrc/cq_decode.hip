@@ -251,9 +251,12 @@ __global__ __launch_bounds__(1024) void rope_attn_decode_kernel(
     const uint4 *kb = reinterpret_cast<const uint4 *>(k_cache + (size_t)kvh * max_len * 128);
     const uint4 *vb = reinterpret_cast<const uint4 *>(v_cache + (size_t)kvh * max_len * 128);
     // Order of the requests = order of use: the new token's q (threads 0..63), k and v (threads
-    // 64..127) and the position, every K row of the first pass; the V rows behind the first barrier.
-    // The cache rows are requested before the position is known (rows up to max_len exist; those
-    // at or beyond the position are ignored below): one memory round trip in front of the arithmetic.
+    // 64..127) and the position, the first 128 K rows; the others of the first pass behind the position, the V
+    // rows behind the first barrier.  The first rows are requested before the position is known (rows at or
+    // beyond it are ignored below): one memory round trip in front of the arithmetic.  Of the others only
+    // those in front of the position: one compute unit accepts about 32 KB per microsecond, and a whole
+    // 256-position cache is 128 KB (7B, 4 bits, positions 0 to 31 of 256: 1072 -> 1050 us a token; this kernel alone over
+    // 40 caches: position 31 4.0, 160 4.7 -> 4.6, 255 4.7 -> 4.8 us).
     // Every request is an unconditional buffer load (rows past the cache read zeros through the
     // descriptor; every thread requests the small values, threads from 128 on drop them): all of
     // them sit in one basic block in this order, so the wait in front of the rotation counts only
@@ -274,11 +277,12 @@ __global__ __launch_bounds__(1024) void rope_attn_decode_kernel(
     asm volatile("" ::: "memory");   // (keeps the groups of requests in this order through the compiler)
     __builtin_amdgcn_sched_barrier(0);
     uint4 k_first[4], v_first[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-        const u4_t r = __builtin_amdgcn_raw_buffer_load_b128(rkc, (row + 64 * u) * 256 + l16 * 16, 0, 0);
-        k_first[u] = make_uint4(r[0], r[1], r[2], r[3]);
-    }
+    constexpr uint32_t kOobRow = 0x80000000u;  // past the descriptor: zeros, and no request to memory
+    auto load_row = [&](const __amdgpu_buffer_rsrc_t cache, int u, bool wanted) {
+        const u4_t r = __builtin_amdgcn_raw_buffer_load_b128(cache, wanted ? (uint32_t)((row + 64 * u) * 256 + l16 * 16) : kOobRow, 0, 0);
+        return make_uint4(r[0], r[1], r[2], r[3]);
+    };
+    k_first[0] = load_row(rkc, 0, true), k_first[1] = load_row(rkc, 1, true);
     asm volatile("" ::: "memory");   // (keeps the groups of requests in this order through the compiler)
     __builtin_amdgcn_sched_barrier(0);
     const __half r1 = __ushort_as_half((t & 64) ? k1 : q1), r2 = __ushort_as_half((t & 64) ? k2 : q2);
@@ -289,6 +293,10 @@ __global__ __launch_bounds__(1024) void rope_attn_decode_kernel(
         if (t < 128) out[(size_t)head * 128 + t] = __ushort_as_half((unsigned short)0x7e00);
         return;
     }
+#pragma unroll
+    for (int u = 2; u < 4; u++) k_first[u] = load_row(rkc, u, row + 64 * u < pos);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
     if (t < 128) {
         const int i = t & 63;
         const bool is_k = t >= 64;
@@ -316,10 +324,7 @@ __global__ __launch_bounds__(1024) void rope_attn_decode_kernel(
     // of it the barrier opened when all 128 KB of a 256-position cache had been taken (3 to 4 us);
     // they are not needed before the softmax is done and travel while the scores are formed.
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-        const u4_t r = __builtin_amdgcn_raw_buffer_load_b128(rvc, (row + 64 * u) * 256 + l16 * 16, 0, 0);
-        v_first[u] = make_uint4(r[0], r[1], r[2], r[3]);
-    }
+    for (int u = 0; u < 4; u++) v_first[u] = load_row(rvc, u, row + 64 * u < pos);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     // q . k over the lane's 8 dimensions as four packed fp16 dot products (fp32 accumulation), the 16
