@@ -111,3 +111,19 @@ def test_matmul_group_matches_the_single_products(dec, bits, k, ns, rows, group)
             assert rel(o, want) < 2 ** -11
     mods[0].register_forward_hook(lambda *a: None)
     assert not dec.matmul_group_supported(mods, rows) and not dec.matmul_group_supported(mods[1:] or mods, 16)
+
+
+# the channels' share decides how a unit's columns are found: staged ahead (up to 128 channels), staged behind the
+# channels, channels too many for LDS, and rows whose address allows no wide loads
+@pytest.mark.parametrize("k,fraction,shift", [(4096, 1 / 256, 0), (4104, 1 / 32, 0), (4096, 1 / 30, 0), (8192, 1 / 16, 0),
+                                              (4096, 1 / 3, 0), (4096, 1 / 256, 2), (2048, 1 / 8, 2), (1032, 0.0, 0)])
+@pytest.mark.parametrize("bits,rows", [(4, 17), (3, 99)])
+def test_activations_gathered_around_the_channels(dec, bits, rows, k, fraction, shift):
+    print("[case] gathered activations", bits, rows, k, fraction, shift, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    m = dec.random_packed_linear(dec.DecoderConfig(w_bits=bits, cherry_fraction=fraction), k, 264, gen, torch.device("cuda"))
+    x = torch.randn(rows * k + shift, device="cuda", generator=gen).half()[shift:].view(rows, k)
+    assert x.data_ptr() % 16 == 2 * shift
+    got = m(x)
+    # one rounding of the result to fp16; weights are the dense ones
+    assert rel(got, x.double().cpu() @ m.unpack().double().cpu().t()) < 2 ** -11
