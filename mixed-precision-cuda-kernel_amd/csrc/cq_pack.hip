@@ -164,7 +164,7 @@ __global__ __launch_bounds__(256) void pack_group_kernel(const __half *__restric
     const int col0 = g == 0 ? 0 : source(k0), col1 = k1 == Kn ? K : source(k1);  // [col0, col1)
     const int c0 = col0 >> 3, nch = ((col1 - 1) >> 3) - c0 + 1;
 
-    auto place = [&](const PackChunk &m, const uint4 &q, int row) {
+    auto place = [&](const PackChunk &m, const uint4 &q, int row) {  // -> the chunk's largest magnitude in the group
         const uint32_t d[4] = {q.x, q.y, q.z, q.w};
         unsigned short *o = reinterpret_cast<unsigned short *>(s_w + row * kPackStride);
         uint32_t mx = 0;
@@ -178,7 +178,6 @@ __global__ __launch_bounds__(256) void pack_group_kernel(const __half *__restric
             o[m.off[2 * p]] = (unsigned short)d[p];
             o[m.off[2 * p + 1]] = (unsigned short)(d[p] >> 16);
         }
-        atomicMax(&s_max[row], mx);
         if (m.cherry) {
             int c = m.first;
 #pragma unroll
@@ -186,6 +185,7 @@ __global__ __launch_bounds__(256) void pack_group_kernel(const __half *__restric
                 if ((m.cherry >> e) & 1u)
                     cherry_weight[(size_t)c++ * N + n0 + row] = __ushort_as_half((unsigned short)(d[e >> 1] >> (16 * (e & 1))));
         }
+        return mx;
     };
     {
         const int ci = t & 15, r0 = t >> 4;
@@ -197,14 +197,20 @@ __global__ __launch_bounds__(256) void pack_group_kernel(const __half *__restric
             if (mine && n0 + r0 + 16 * i < N) q[i] = *reinterpret_cast<const uint4 *>(src + (size_t)16 * i * K);
         const PackChunk m = pack_chunk(s_idx, C, 8 * (c0 + ci), k0, k1);
 #pragma unroll
-        for (int i = 0; i < 8; i++)
-            if (mine && n0 + r0 + 16 * i < N) place(m, q[i], r0 + 16 * i);
+        for (int i = 0; i < 8; i++) {
+            uint32_t mx = 0;
+            if (mine && n0 + r0 + 16 * i < N) mx = place(m, q[i], r0 + 16 * i);
+            // across the row's 16 lanes first: 16 atomics on one word of LDS take turns
+            mx = (uint32_t)row_max((int)mx);
+            if (ci == 0) atomicMax(&s_max[r0 + 16 * i], mx);
+        }
     }
     // the chunk or two that cherries and alignment push the range beyond 16
     for (int e = t; e < (nch - 16) * kPackRows; e += 256) {
         const int row = e & (kPackRows - 1), c = c0 + 16 + e / kPackRows;
         if (n0 + row < N)
-            place(pack_chunk(s_idx, C, 8 * c, k0, k1), *reinterpret_cast<const uint4 *>(w + (size_t)(n0 + row) * K + 8 * c), row);
+            atomicMax(&s_max[row],
+                      place(pack_chunk(s_idx, C, 8 * c, k0, k1), *reinterpret_cast<const uint4 *>(w + (size_t)(n0 + row) * K + 8 * c), row));
     }
     __syncthreads();
     if (t < kPackRows) {
