@@ -83,15 +83,15 @@ hipError_t launch_batch(int bits, const __half *vec, const uint8_t *qweight, con
                         int C, int G, int accumulate, void *workspace, void *scratch, hipStream_t stream);
 size_t scratch_bytes(int B, int K, int N, int C);
 
-// cq_prompt.hip: more than 16 rows (prompt processing) -- dequantise into registers, fp16 MFMA tiles, the wavefronts of a
-// workgroup sharing K.
+// cq_prompt.hip: more than 16 rows (prompt processing) -- wavefronts that decode weights into LDS and wavefronts of fp16 MFMAs.
 constexpr int kPromptMinRows = 17;  // fewer rows go through the 16-row kernel
 constexpr int kPromptMaxSplits = 16;
 struct PromptPlan {
-    int mt, nc, ns;                   // 16-row and 16-column pieces of a wavefront's tile, wavefronts side by side
+    int shape;                        // the tile shape, by its place in the kernel's table
+    int mt, nc, ns;                   // 16-row and 16-column pieces of a workgroup's tile: mt x nc ns
     int mtiles, ntiles;               // output tiles of 16 mt rows x 16 nc ns columns
     int units, csteps, steps;         // units of 128 positions, steps of 32 cherries, steps of 32 in all
-    int splits, units_per_split;      // K splits (grid.y)
+    int splits, units_per_split;      // K splits
     size_t workspace_bytes;           // zero-kept: one ticket per output tile
     size_t a_bytes, partial_bytes;    // scratch: activations in operand order, then the per-split partial tiles
     size_t scratch_bytes;

@@ -3,43 +3,39 @@
 //   Y[M, N] (+)= Xn[M, Kn] * Wn[Kn, N] + Xc[M, C] * Wc[C, N]
 //
 // Wn are the packed codes, Wc the fp16 cherry rows; Xn / Xc are the activations gathered at the normal / cherry
-// input channels.  Bound by the matrix cores for many rows, by the decode (vector ALU) and the weights' bytes for few.
+// input channels.  Bound by the matrix cores (and the power they draw) for many rows, by the decode and by the bytes that a
+// compute unit takes in for few.
 //
-// A workgroup of 8 or 4 wavefronts owns an output tile of 16 MT rows x 64, 128 or 256 columns and the wavefronts share K:
-// each takes units of 128 positions in turn, so that the main loop has no LDS traffic and no barrier, and partial
-// results meet once, in LDS, at the end.  (Wavefronts that share the columns instead need the dequantised weights passed
-// through LDS in every step and, where the tiles do not fill the chip, several workgroups' fp32 tiles passed
-// through memory: at 4096 -> 11008 with 128 rows those were 28 MB each way, more than the weights.)
-//   What a tile shape is bound by: every wavefront fetches its own fragments of the activations from the L2, 32 KB a
-// unit beside 4 KB of weights, so 64 columns of 128 rows wait for those (4096 -> 11008, 99 rows, counters: a compute unit
-// takes in 28 bytes a clock, its wavefronts wait two fifths of the time, the matrix cores are busy for three tenths and the
-// decode issues for a quarter of it); 128 columns (NC = 8, the fragments feed twice the MFMAs) take 256 accumulator and
-// 200 other registers, one wavefront a SIMD.  Two such
-// wavefronts side by side (NS = 2) halve the tile's partial results in LDS and its row tiles' weight reads from the L2.
-//   Measured, 4 bits, preparation included, against the kernel of wavefronts side by side that this replaces (us):
+// A workgroup owns an output tile.  Four of its wavefronts, one a SIMD, form products; the others turn weights into operands: packed
+// bytes from memory, decoded in registers, fp16 operands into LDS, two buffers, one barrier a stage.  What that is for:
+//   * a SIMD's vector ALU decodes for one wavefront while its matrix core works for another.  Decode between a wavefront's own
+//     MFMAs hardly overlaps them, and one weight is decoded once for all of a tile's rows;
+//   * loads of a wavefront return in order.  Activations (L2) that wait behind weights (HBM) in the same wavefront take HBM's
+//     latency in every step; here neither waits for the other.
+// Measured, 4 bits, preparation included (us), against the kernel that this replaces (every wavefront decoded its own operands
+// between its MFMAs and shared K with the others):
 //     rows              17      64     128     256     512    1024    2048
-//     4096 -> 11008   18.0    21.2    29.2    39.7    64.3     118     196
-//             before  22.8    26.8    37.1    51.9    80.0     131     248
-//     4096 -> 4096    12.9    16.0    18.5    23.1    33.3    47.7    77.3
-//             before  16.7    19.8    25.8    30.2    40.7    60.4    97.8
-//     11008 -> 4096   19.5    23.5    32.9    48.3    72.5    99.8     184
-//             before  25.4    29.2    37.1    53.3    78.0     132     241
-//   At 2048 rows of 4096 -> 11008 that is 0.94 PFLOP/s; the library's product of this size reaches 1.0 (behind a
-// dequantisation of 30 us), one of 8192 cubed 1.5.  Counters of the main launch there: the matrix cores are busy 45 % of the time
-// (16 cycles an MFMA), the decode's vector instructions issue for another 28 %, wavefronts wait 16 %; one wavefront a
-// SIMD does not overlap the first two.
-//   * B operands (weights) go straight from registers to v_mfma_f32_16x16x32_f16: a lane owns 4 adjacent columns
-//     (dword loads, 64 bytes of a byte row), lane group kq the 8 positions 8 kq .. 8 kq + 7 of each 32.  v_perm_b32
-//     interleaves a column's bytes, masks cut out code pairs, OR-ing 0x6400 makes them the fp16 numbers
-//     1024 + u * 2^p, one packed fma gives u - c_b (exact: the fields are first moved up one bit, 1024 + c_b itself has
-//     no fp16 value) and one packed multiply applies the group scale with the reference's single rounding, so
-//     the operands are the dense weight's values (llama/qlinear.py:120-162).
+//     4096 -> 11008   16.9    20.3    27.1    37.0    54.8     107     174
+//             before  17.4    20.9    28.5    38.9    63.6     109     186
+//     4096 -> 4096    12.3    14.4    17.9    22.3    30.5    44.3    69.1
+//             before  11.9    14.9    17.7    22.0    31.4    44.9    73.2
+//     11008 -> 4096   17.0    21.3    28.6    43.9    65.3     102     168
+//             before  17.6    21.9    31.1    45.6    68.3    96.7     173
+// (sizes that tiles or dies divide badly gain more: 60 drawn calls together 13 %, 75 rows of 22272 -> 4592 82 -> 42 us)
+// A lone wavefront's dependent vector instructions issue every 8 clocks, beside MFMAs every 12, and an operand of 512
+// weights takes 17: with 128 rows a tile the decode is the longer half, with 256 it is hidden.  At 2048 rows the clock falls to 1.95 GHz
+// (of 2.4) under the MFMAs' power: 32 accumulators of random numbers alone reach 1.5 PFLOP/s on this card for longer than 100 us.
+//   * B operands (weights): a lane owns NC adjacent columns (64 or 128 bytes of a byte row), lane group kq the 8 positions 8 kq ..
+//     8 kq + 7 of each 32.  v_perm_b32 interleaves a column's bytes, masks cut out code pairs, OR-ing 0x6400 makes them
+//     the fp16 numbers 1024 + u * 2^p, one packed fma gives u - c_b (exact: the fields are first moved up one bit, 1024 + c_b
+//     itself has no fp16 value) and one packed multiply applies the group scale with the reference's single
+//     rounding, so the operands are the dense weight's values (llama/qlinear.py:120-162).
 //   * A operands (activations) come from a small kernel in front, gathered around the cherry channels and in operand
-//     order: one contiguous 1 KB load per 16 rows and 32 positions.
-//   * Registers are reloaded in place: a step's packed bytes for the wavefront's next unit as soon as they are
-//     decoded, a fragment for the next step as soon as its four MFMAs are issued.
-// Neighbouring column tiles share 128-byte lines of the packed bytes and a column tile's row tiles share all of them:
-// tiles run in XCD-contiguous ranges.  Calls of more rows than a launch takes (prompt_max_rows) run in ranges of rows.
+//     order: one contiguous 1 KB load per 16 rows and 32 positions, 16 of them in flight a wavefront (8: 2048 rows 187 us
+//     instead of 172).  (Rows of the input in their own order cost four times as long a load, at odd addresses sixteen times.)
+//   * Registers are reloaded in place: an operand as soon as its last MFMA is issued.
+// Neighbouring column tiles share the activations, a column tile's row tiles the packed bytes: tiles of one K split run in
+// XCD-contiguous ranges.  Calls of more rows than a launch takes (prompt_max_rows) run in ranges of rows.
 //
 // Where there are too few tiles, K is split over workgroups too: fp32 tiles in scratch and one ticket per tile; the last
 // workgroup adds them in split order, so the result does not depend on arrival order.
@@ -59,10 +55,6 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// wavefronts of a workgroup: a tile of 128 x 128 leaves registers for one a SIMD, others for two and more
-__host__ __device__ constexpr int prompt_waves(int mt, int nc) { return mt * nc == 64 ? 4 : 8; }
-// ... of which this many share K where ns of them lie side by side
-__host__ __device__ constexpr int prompt_kways(int mt, int nc, int ns) { return prompt_waves(mt, nc) / ns; }
 constexpr uint32_t kRsrcFlagsP = 0x00020000u;
 constexpr uint32_t kOobP = 0x80000000u;
 
@@ -80,50 +72,113 @@ __host__ __device__ constexpr int prompt_pos(int kk) {
 }
 static_assert(prompt_ord<4>(1) == 2 && prompt_ord<4>(2) == 1 && prompt_ord<4>(5) == 6 && prompt_ord<4>(7) == 7, "");
 
-// What a call takes with one of the tile shapes, in microseconds: a fit to about 4000 measured calls (4 bits, K 1024 to
-// 28672, N 512 to 28672, M 17 to 2048, every shape and up to 16 K splits).  `first` is a launch with one round of
-// workgroups and no unit, `round` what each further round of 256 adds, `unit` a unit of 128 positions of every wavefront
-// (`pair`: of a second workgroup on the same compute unit), `split` and `mbyte` a split call and each megabyte of its
-// partial tiles.  On those calls the shape and split chosen by it are 1.4 % slower than the best on average, 22 % at worst.
+// Tile shapes.  A workgroup's tile is 16 MT WM rows x 16 NC columns: four wavefronts of products, WM over one another and WK
+// sharing K, and NP wavefronts of weights.  They meet after every S steps of 32 positions a K share; activations are asked
+// for AS steps ahead, weights D meetings.
+//   Tiles of 64 columns have four K shares: small tiles want every one of the few workgroups to itself.  Eight wavefronts of
+// weights where registers allow three a SIMD and there are few products to hide the decode behind (32 and 48 rows: 17.5 -> 16.7
+// us at 4096 -> 11008).  128 columns are eight operands of weights to four of activations, half the bytes a
+// product from the L2; 256 rows decode a weight once for them all.
+// Two small workgroups a compute unit help where there are more tiles than compute units (23 rows of 7456 -> 8832 in 3 bits
+// 24.3 -> 20.3 us).
+//        id MT NC WM WK S AS NP D
+#define CQ_PROMPT_SHAPES(X)      \
+    X(0, 2, 4, 1, 4, 2, 4, 8, 3) \
+    X(1, 3, 4, 1, 4, 2, 4, 8, 2) \
+    X(2, 4, 4, 1, 4, 2, 4, 4, 3) \
+    X(3, 5, 4, 1, 4, 4, 4, 4, 2) \
+    X(4, 7, 4, 1, 4, 4, 4, 4, 2) \
+    X(5, 4, 4, 2, 2, 4, 4, 4, 2) \
+    X(6, 3, 8, 2, 2, 4, 4, 4, 2) \
+    X(7, 4, 8, 2, 2, 4, 4, 4, 2) \
+    X(8, 3, 8, 4, 1, 4, 4, 4, 2) \
+    X(9, 4, 8, 4, 1, 4, 4, 4, 2) \
+    X(10, 2, 4, 1, 4, 2, 4, 4, 3) \
+    X(11, 3, 4, 1, 4, 2, 4, 4, 2)
+
+// What a call takes with a tile shape, in microseconds, preparation included: a fit to 37000 measured calls (3 and 4 bits, K 1024
+// to 28672, N 512 to 28672, M 17 to 2048, 1 to 16 K splits).  `first`: a launch with one round of workgroups and no unit; `round`:
+// each further round; `unit`: 128 positions a K share, 1 + crowd times as long when all compute units are at it; `split`,
+// `mbyte`, `tile`: a split call, each megabyte of its partial tiles, and each 32 KB that its last workgroup reads; `rows`:
+// 1e6 M K.  Its choices are 0.3 % slower than the best measured ones on average, 5 % at the 99th percentile.
+// 1 << `per`: workgroups that a die of 32 compute units takes at a time; `crowd` of the pairs counts once there is a second one.
+struct PromptCost {
+    int per;
+    float first, round, unit, crowd, split, mbyte, rows, tile;
+};
+constexpr PromptCost kPromptCosts[] = {
+    {5, 6.27f, 1.87f, 1.23f, 0.002f, 0.560f, 0.738f, 1.87f, 1.10f},  // 32 x 64
+    {5, 6.37f, 2.07f, 1.41f, 0.007f, 0.600f, 0.688f, 1.88f, 0.736f},  // 48 x 64
+    {5, 6.76f, 2.19f, 1.50f, 0.024f, 0.753f, 0.631f, 1.73f, 0.720f},  // 64 x 64
+    {5, 7.31f, 2.56f, 1.66f, 0.000f, 0.894f, 0.575f, 1.52f, 0.718f},  // 80 x 64
+    {5, 7.55f, 2.76f, 2.03f, 0.000f, 1.59f, 0.501f, 1.19f, 0.648f},  // 112 x 64
+    {5, 6.91f, 1.97f, 1.18f, 0.000f, 1.31f, 0.502f, 1.23f, 0.647f},  // 128 x 64
+    {5, 8.63f, 4.92f, 1.25f, 0.148f, 2.68f, 0.350f, 1.19f, 0.564f},  // 96 x 128
+    {5, 10.04f, 6.30f, 1.35f, 0.272f, 2.76f, 0.297f, 0.960f, 0.574f},  // 128 x 128
+    {5, 9.64f, 6.38f, 0.896f, 0.288f, 2.38f, 0.366f, 0.892f, 0.565f},  // 192 x 128
+    {5, 10.76f, 7.50f, 1.12f, 0.276f, 2.16f, 0.379f, 0.839f, 0.563f},  // 256 x 128
+    {6, 6.19f, 0.538f, 1.27f, 0.835f, 1.14f, 0.324f, 1.92f, 0.942f},  // 32 x 64, two a compute unit
+    {6, 6.54f, 0.366f, 1.40f, 0.911f, 0.909f, 0.465f, 2.11f, 0.985f},  // 48 x 64, two a compute unit
+};
 struct PromptShape {
-    int mt, nc, ns;
-    float first, round, unit, pair, split, mbyte;
+    int mt, nc, wm, wk;
 };
 constexpr PromptShape kPromptShapes[] = {
-    {2, 4, 1, 5.65f, 0.91f, 2.66f, 2.15f, 2.60f, 0.74f},   // 32 x 64: two workgroups a compute unit
-    {4, 4, 1, 6.00f, 2.04f, 3.32f, 0.f, 3.58f, 0.48f},     // 64 x 64
-    {8, 4, 1, 7.11f, 3.64f, 4.71f, 0.f, 5.15f, 0.38f},     // 128 x 64
-    {8, 8, 1, 10.63f, 5.90f, 3.04f, 0.f, 8.06f, 0.58f},    // 128 x 128, one wavefront a SIMD
-    {8, 8, 2, 10.80f, 3.50f, 2.89f, 0.f, 14.20f, 0.51f},   // 128 x 256, pairs of wavefronts side by side
+#define CQ_SHAPE_ROW(ID, MT, NC, WM, WK, S, AS, NP, D) {MT, NC, WM, WK},
+    CQ_PROMPT_SHAPES(CQ_SHAPE_ROW)
+#undef CQ_SHAPE_ROW
 };
+constexpr int kPromptShapeCount = sizeof(kPromptShapes) / sizeof(kPromptShapes[0]);
+static_assert(sizeof(kPromptCosts) / sizeof(kPromptCosts[0]) == kPromptShapeCount, "");
 
+// A call asks five times: for its buffers' sizes, in the checks of both, and at the launch.  The last answer of the thread is
+// kept (a few rows over a 4096 wide layer: 0.5 us of the call's host time).
+struct PromptQuery {
+    int M, K, C, count, N[kPromptMaxGroup];
+    PromptPlan plan;
+};
+static PromptPlan find_prompt_plan(int M, int K, const int *N, int count, int C);
 PromptPlan prompt_plan(int M, int K, const int *N, int count, int C) {
-    PromptPlan best;
+    static thread_local PromptQuery last = {};
+    bool same = last.M == M && last.K == K && last.C == C && last.count == count && count > 0;
+    for (int i = 0; i < count; i++) same = same && last.N[i] == N[i];
+    if (!same) {
+        last.plan = find_prompt_plan(M, K, N, count, C);
+        last.M = M, last.K = K, last.C = C, last.count = count;
+        for (int i = 0; i < count; i++) last.N[i] = N[i];
+    }
+    return last.plan;
+}
+
+static PromptPlan find_prompt_plan(int M, int K, const int *N, int count, int C) {
+    PromptPlan best = {};
     float best_cost = 3.4e38f;
     const int units = K > C ? ceil_div(K - C, kUnitK) : 1;  // sizes are asked for before the launch is refused
-    for (const PromptShape &s : kPromptShapes) {
-        if (s.mt > 2 && M <= 8 * s.mt) break;  // half of every tile would be padding
-        PromptPlan p;
-        p.mt = s.mt, p.nc = s.nc, p.ns = s.ns;
-        p.mtiles = ceil_div(M, 16 * s.mt);
+    const long long steps = 4ll * units + ceil_div(C, 32);
+    for (int id = 0; id < kPromptShapeCount; id++) {
+        const PromptShape &s = kPromptShapes[id];
+        const PromptCost &f = kPromptCosts[id];
+        PromptPlan p = {};
+        p.shape = id, p.mt = s.mt * s.wm, p.nc = s.nc, p.ns = 1;
+        if (id > 0 && M <= 8 * p.mt) continue;  // half of every tile would be padding
+        p.mtiles = ceil_div(M, 16 * p.mt);
+        if (id > 0 && (p.mtiles * p.mt > 65535 || steps * p.mtiles * p.mt > 0x7fff0000ll / 1024)) continue;
         p.ntiles = 0;
-        for (int i = 0; i < count; i++) p.ntiles += ceil_div(N[i], 16 * s.nc * s.ns);
+        for (int i = 0; i < count; i++) p.ntiles += ceil_div(N[i], 16 * s.nc);
         const long long tiles = (long long)p.mtiles * p.ntiles;
-        const int kways = prompt_kways(s.mt, s.nc, s.ns);
+        const float kbytes = (float)(p.mt * s.nc);  // a tile's fp32 results
         for (int splits = 1; splits <= kPromptMaxSplits; splits++) {
-            // more splits than one round (two for the small tile) of workgroups or than leave a wavefront a unit never pay
-            if (splits > 1 && (tiles * splits > 512 || splits > ceil_div(units, kways))) break;
+            // more splits than two rounds of workgroups or than leave a K share a unit never pay
+            if (splits > 1 && (tiles * splits > 512 || splits > ceil_div(units, s.wk))) break;
             p.units_per_split = ceil_div(units, splits);
             p.splits = ceil_div(units, p.units_per_split);
             if (p.splits < splits) continue;  // the same plan as with fewer
-            const long long load = (tiles * splits + 255) / 256;
-            const float u = (float)ceil_div(p.units_per_split, kways);
-            float cost = s.first;
-            if (s.pair > 0.f)
-                cost += s.round * (float)((load + 1) / 2 - 1) + u * (s.unit * (float)((load + 1) / 2) + s.pair * (float)(load / 2));
-            else
-                cost += s.round * (float)(load - 1) + u * s.unit * (float)load;
-            if (splits > 1) cost += s.split + s.mbyte * (float)(tiles * splits) * (float)(s.mt * s.nc * s.ns * 1024) * 1e-6f;
+            // workgroups are dealt to eight dies of 32 compute units: the fullest die counts
+            const unsigned load = (unsigned)((tiles * splits + 7) / 8), full = load >> f.per, rest = load & ((1u << f.per) - 1u);
+            const float crowd = f.crowd * (f.per == 5 ? (float)rest / 32.f : rest > 32 ? 1.f : 0.f);
+            float cost = f.first + f.round * (float)(full + (rest > 0) - 1) + f.rows * 1e-6f * (float)M * (float)K +
+                         f.unit * (float)ceil_div(p.units_per_split, s.wk) * ((float)full * (1.f + f.crowd) + (rest > 0 ? 1.f + crowd : 0.f));
+            if (splits > 1) cost += f.split + f.mbyte * (float)(tiles * splits) * kbytes * 1.024e-3f + f.tile * splits * kbytes / 32.f;
             if (cost < best_cost) best_cost = cost, best = p;
         }
     }
@@ -133,14 +188,14 @@ PromptPlan prompt_plan(int M, int K, const int *N, int count, int C) {
     p.csteps = ceil_div(C, 32);
     p.steps = p.units * 4 + p.csteps;
     p.a_bytes = ((size_t)p.steps * p.mtiles * p.mt * 1024 + 255) / 256 * 256;
-    p.partial_bytes = p.splits > 1 ? p.splits * tiles * p.mt * p.nc * p.ns * 256 * sizeof(float) : 0;
+    p.partial_bytes = p.splits > 1 ? p.splits * tiles * p.mt * p.nc * 256 * sizeof(float) : 0;
     p.scratch_bytes = count * p.a_bytes + p.partial_bytes;
     p.workspace_bytes = (tiles * sizeof(unsigned) + 255) / 256 * 256;
     return p;
 }
 
 // A launch's activations in operand order are read through one buffer descriptor, whose offsets end at 2 GiB, and their
-// tiles of 16 rows are a grid dimension.  The bound holds for every tile shape: whole tiles of 128 rows.
+// tiles of 16 rows are a grid dimension.  The bound holds for tiles of 32 and 128 rows; the plan leaves out others that pass it.
 int prompt_max_rows(int K, int C) {
     const long long steps = 4ll * (K > C ? ceil_div(K - C, kUnitK) : 1) + ceil_div(C, 32);
     return (int)(std::min(0x7fff0000ll / (steps * 1024), 65535ll) / 8) * 128;
@@ -335,13 +390,22 @@ struct PromptColumn {
     }
 };
 
+// (written out: the accumulator stays where it is.  The compiler's own form may name another destination and then
+// spills accumulators.)  Its result is next read 16 products later at the earliest, or behind mfma_drain().
 __device__ __forceinline__ void prompt_mfma(float4_t &acc, const u32x4 &a, const u32x4 &b) {
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), acc, 0, 0, 0);
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void mfma_drain() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
+
+// The wavefront's LDS accesses are done before it arrives; loads from memory stay in flight.
+__device__ __forceinline__ void stage_barrier() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
 }
 
 // The layers of a launch: their column tiles follow one another.  Layers that read the same rows fill the chip together
-// and with larger tiles (128 rows, 4 bits, preparation included: three of 4096 -> 4096 54 -> 33 us, two of 4096 -> 11008
-// 58 -> 41, two of 8192 -> 28672 140 -> 121; with 500 rows 99 -> 71, 130 -> 116, 452 -> 447).
+// and with larger tiles.
 struct PromptMembers {
     const uint8_t *qweight[kPromptMaxGroup];
     const __half *cherry_weight[kPromptMaxGroup], *scales[kPromptMaxGroup];
@@ -349,206 +413,299 @@ struct PromptMembers {
     int N[kPromptMaxGroup], first[kPromptMaxGroup];  // columns, first column tile (past the end: no such layer)
 };
 
+// A byte row's piece of a lane (NC columns) and its scales.
+template <int NC>
+struct PromptPiece {
+    typedef uint32_t w_t __attribute__((ext_vector_type(NC == 8 ? 2 : 1)));
+    typedef uint32_t s_t __attribute__((ext_vector_type(NC / 2)));
+    static __device__ __forceinline__ w_t codes(const __amdgpu_buffer_rsrc_t r, uint32_t off) {
+        if constexpr (NC == 8) return __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 2);
+        else if constexpr (NC == 4) return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 2);
+        else return (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 2);
+    }
+    static __device__ __forceinline__ s_t halves(const __amdgpu_buffer_rsrc_t r, uint32_t off) {
+        if constexpr (NC == 8) return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+        else if constexpr (NC == 4) return __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+        else return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
+    }
+};
+
 // WHOLE: groups are whole units
-template <int BITS, int MT, int NC, int NS, bool WHOLE>
-__global__ __launch_bounds__(64 * prompt_waves(MT, NC), MT * NC == 64 ? 1 : MT * NC == 8 ? 4 : 2) void prompt_kernel(
-    PromptMembers members, const u32x4 *__restrict__ a_all, float *__restrict__ partial, unsigned *__restrict__ tickets, int M, int K,
-    int C, int G, int accumulate, PromptPlan plan) {
-    constexpr int WAVES = prompt_waves(MT, NC), KW = WAVES / NS, COLS = 16 * NC, ND = NC / 4;  // ND: dwords of a byte row a lane
-    typedef uint32_t wd_t __attribute__((ext_vector_type(ND)));
-    typedef uint32_t sc_t __attribute__((ext_vector_type(NC / 2)));
-    constexpr int ROWS = WAVES * COLS == 1024 ? 16 : 32;  // rows that meet at a time: 64 KB of LDS
-    __shared__ __attribute__((aligned(16))) float s_red[WAVES][ROWS][COLS];
+template <int BITS, int MT, int NC, int WM, int WK, int S, int AS, int NP, int D, bool WHOLE>
+__global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(PromptMembers members, const u32x4 *__restrict__ a_all,
+                                                              float *__restrict__ partial, unsigned *__restrict__ tickets, int M,
+                                                              int K, int C, int G, unsigned group_magic, int accumulate, PromptPlan plan) {
+    static_assert(WM * WK == 4 && S * WK % NP == 0 && NP % WK == 0 && (AS % S == 0 || S % AS == 0) && (AS <= S || AS / S * S == 4), "");
+    typedef typename PromptPiece<NC>::w_t w_t;
+    typedef typename PromptPiece<NC>::s_t s_t;
+    constexpr int COLS = 16 * NC, ROWS = 16 * MT * WM, PS = S * WK / NP, T = 256 + 64 * NP;
+    constexpr int STAGE = WK * S * NC * 64;                        // operands of a stage, 16 bytes each
+    constexpr int RED = MT * NC * 64 * 4;                          // four wavefronts' results
+    __shared__ u32x4 s_b[2 * STAGE > RED ? 2 * STAGE : RED];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kq = lane >> 4, nl = lane & 15;
-    const int tiles = plan.mtiles * plan.ntiles, per_xcd = ceil_div(tiles, 8);
-    const int tile = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3), split = blockIdx.y;
-    if (tile >= tiles) return;
-    const int mtile = tile % plan.mtiles;
-    int ntile = tile / plan.mtiles;
+    const int tiles = plan.mtiles * plan.ntiles, piece = ((int)blockIdx.x & 7) * ((int)gridDim.x >> 3) + ((int)blockIdx.x >> 3);
+    if (piece >= tiles * plan.splits) return;
+    const int split = piece / tiles, tile = piece % tiles;
+    // blocks of up to 8 row tiles, column tiles within: the 32 workgroups of a die at a time share rows and columns four and
+    // more ways (8192 rows of 4096 -> 11008: 877 -> 697 us)
+    const int mblock = tile / (8 * plan.ntiles), mrows = min(8, plan.mtiles - 8 * mblock), in_block = tile - mblock * 8 * plan.ntiles;
+    const int mtile = 8 * mblock + in_block % mrows;
+    int ntile = in_block / mrows;
     // selected, not indexed: the arguments arrive with one scalar load
     const int layer = (ntile >= members.first[1] ? 1 : 0) + (ntile >= members.first[2] ? 1 : 0);
     auto of = [&](auto &what) { return layer == 0 ? what[0] : layer == 1 ? what[1] : what[2]; };
-    const uint8_t *__restrict__ const qweight = of(members.qweight);
-    const __half *__restrict__ const cherry_weight = of(members.cherry_weight);
-    const __half *__restrict__ const scales = of(members.scales);
     __half *__restrict__ const out = of(members.out);
-    const u32x4 *__restrict__ const a_frag = a_all + layer * (plan.a_bytes / sizeof(u32x4));
     const int N = of(members.N);
     ntile -= of(members.first);
-    const int kpart = wave % KW, npart = wave / KW;
-    const int n0 = (ntile * NS + npart) * COLS + NC * nl, m16 = plan.mtiles * MT, Kn = K - C;
-    const bool col_ok = n0 < N;
-    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)qweight, 0, Kn / 8 * BITS * N, kRsrcFlagsP);
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)scales, 0, ceil_div(Kn, G) * N * 2, kRsrcFlagsP);
-    const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc((void *)cherry_weight, 0, C * N * 2, kRsrcFlagsP);
-    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)a_frag, 0, plan.steps * m16 * 1024, kRsrcFlagsP);
-
-    wd_t w[4][BITS];
-    sc_t sc[WHOLE ? 2 : 4];
-    u32x4 a[MT], b[2][NC];
-    // Units past the wavefront's last one are asked for as unit `plan.units`, which lies past the end of the packed bytes:
-    // the bounds of the buffer answer with zeros.
-    const uint32_t w_lane = col_ok ? (uint32_t)(kq * BITS * N + n0) : kOobP, sc_lane = col_ok ? (uint32_t)n0 * 2u : kOobP;
-    auto load_w = [&](int s, int u) {
-        const uint32_t off = w_lane + (uint32_t)((u * 4 + s) * 4 * BITS * N);
-#pragma unroll
-        for (int r = 0; r < BITS; r++) {
-            if constexpr (ND == 1) w[s][r] = __builtin_amdgcn_raw_buffer_load_b32(rw, off + (uint32_t)(r * N), 0, 2);
-            else w[s][r] = __builtin_amdgcn_raw_buffer_load_b64(rw, off + (uint32_t)(r * N), 0, 2);
-        }
-    };
-    auto load_sc = [&](int s, int u) -> sc_t {
-        const uint32_t off = sc_lane + (uint32_t)((u * kUnitK + 32 * s) / G * N) * 2u;
-        if constexpr (NC == 4) return __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0);
-        else return __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0);
-    };
-    auto load_a = [&](int m, int step) {
-        return __builtin_amdgcn_raw_buffer_load_b128(ra, lane * 16, (step * m16 + mtile * MT + m) * 1024, 0);
-    };
-    const PromptDecode<BITS> decoder;
-    PromptColumn<BITS> column;
-    auto decode = [&](int s, const sc_t &scale, int c, int g, u32x4 &o) {
-        uint32_t d[BITS];
-#pragma unroll
-        for (int r = 0; r < BITS; r++) d[r] = w[s][r][c >> 2];
-        column.group(decoder, g, d, c & 3, scale[c >> 1], o);
-    };
+    const int u0 = split * plan.units_per_split, u_end = min(u0 + plan.units_per_split, plan.units);
+    const int stages = ceil_div(u_end - u0, WK) * (4 / S);
+    // cherry steps: the last split's, a chunk of S a K share at a time
+    const int csteps = split == plan.splits - 1 ? plan.csteps : 0;
 
     float4_t acc[MT][NC];
+    if (wave < 4) {
+        // ---- products
+        const int wm = wave % WM, wk = wave / WM, m16 = plan.mtiles * MT * WM, row0 = (mtile * WM + wm) * MT;
+        const u32x4 *const a_frag = a_all + layer * (plan.a_bytes / sizeof(u32x4));
+        const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)a_frag, 0, plan.steps * m16 * 1024, kRsrcFlagsP);
+        auto load_a = [&](int m, int step, bool ok) {
+            return __builtin_amdgcn_raw_buffer_load_b128(ra, ok ? lane * 16 : (int)kOobP, (step * m16 + row0 + m) * 1024, 0);
+        };
+        auto load_step = [&](int m, int q) {  // step q of this wavefront's units; past the last one: zeros
+            const int u = u0 + (q >> 2) * WK + wk;
+            return load_a(m, u < u_end ? 4 * u + (q & 3) : 0, u < u_end);
+        };
+        const u32x4 *const frag = s_b + wk * S * NC * 64 + lane;
+        u32x4 a[AS][MT], b[NC];
 #pragma unroll
-    for (int m = 0; m < MT; m++)
+        for (int m = 0; m < MT; m++)
 #pragma unroll
-        for (int c = 0; c < NC; c++) acc[m][c] = (float4_t){0.f, 0.f, 0.f, 0.f};
-
-    const int u0 = split * plan.units_per_split + kpart, u_end = min((split + 1) * plan.units_per_split, plan.units);
-    auto unit_after = [&](int u) { return u + KW < u_end ? u + KW : plan.units; };
-    if (u0 < u_end) {
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-            load_w(s, u0);
-            if (!WHOLE || s == 0) sc[s] = load_sc(s, u0);
-        }
-        if (WHOLE) sc[1] = load_sc(0, unit_after(u0));
-    }
-    // Cherry steps (32 dense fp16 rows, 8 per lane group) while the packed bytes are on their way: behind the loop their own
-    // round trip to memory would be one more.
-    if (split == plan.splits - 1) {
-        for (int cs = KW - 1 - kpart; cs < plan.csteps; cs += KW) {
-            sc_t cw[8];
-            const uint32_t off = col_ok ? (uint32_t)((32 * cs + 8 * kq) * N + n0) * 2u : kOobP;
-#pragma unroll
-            for (int r = 0; r < 8; r++) {
-                if constexpr (NC == 4) cw[r] = __builtin_amdgcn_raw_buffer_load_b64(rc, off + (uint32_t)(r * N * 2), 0, 0);
-                else cw[r] = __builtin_amdgcn_raw_buffer_load_b128(rc, off + (uint32_t)(r * N * 2), 0, 0);
-            }
-#pragma unroll
-            for (int m = 0; m < MT; m++) a[m] = load_a(m, plan.units * 4 + cs);
-#pragma unroll
-            for (int c = 0; c < NC; c++) {
-                u32x4 bc;
-#pragma unroll
-                for (int d = 0; d < 4; d++)
-                    bc[d] = __builtin_amdgcn_perm(cw[2 * d + 1][c >> 1], cw[2 * d][c >> 1], (c & 1) ? 0x07060302u : 0x05040100u);
-#pragma unroll
-                for (int m = 0; m < MT; m++) prompt_mfma(acc[m][c], a[m], bc);
-            }
-        }
-    }
-    if (u0 < u_end) {
-#pragma unroll
-        for (int m = 0; m < MT; m++) a[m] = load_a(m, u0 * 4);
-#pragma unroll
-        for (int c = 0; c < NC; c++)
-#pragma unroll
-            for (int g = 0; g < 8; g++) decode(0, sc[0], c, g, b[0][c]);
-        load_w(0, unit_after(u0));
-        if (!WHOLE) sc[0] = load_sc(0, unit_after(u0));
-    }
-    // In every step the columns of the next step are decoded between this step's MFMAs, a few instructions behind each (the
-    // scheduling barriers keep the order): the next MFMA's operands are then ready and a block of decoding never holds up a
-    // block of MFMAs.  Vector instructions of the MFMAs' own wavefront hardly overlap them; a second wavefront's
-    // would, where registers allow one.
-    // A step's packed bytes are reloaded for the unit after as soon as they are decoded, the fragments for the next step.
-#pragma nounroll
-    for (int u = u0; u < u_end;) {
-        const int un = unit_after(u), unn = unit_after(un);
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-            const int t = (s + 1) & 3;
-            const int next = s < 3 ? u * 4 + s + 1 : un < plan.units ? un * 4 : u * 4;  // the last step's own again
-#pragma unroll
-            for (int m = 0; m < MT; m++) {
-#pragma unroll
-                for (int c = 0; c < NC; c++) {
-                    prompt_mfma(acc[m][c], a[m], b[s & 1][c]);
-                    // MT * NC MFMAs take turns with NC columns' 8 groups
-                    const int slot = m * NC + c;
-#pragma unroll
-                    for (int k = slot * 8 / MT; k < (slot + 1) * 8 / MT; k++)
-                        decode(t, WHOLE ? sc[s < 3 ? 0 : 1] : sc[t], k / 8, k % 8, b[(s + 1) & 1][k / 8]);
-                    if (c == NC - 1) a[m] = load_a(m, next);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-            load_w(t, s < 3 ? un : unn);
-            if (!WHOLE) sc[t] = load_sc(t, s < 3 ? un : unn);
-        }
-        if (WHOLE) {
-            sc[0] = sc[1];
-            sc[1] = load_sc(0, unn);
-        }
-        u = un < plan.units ? un : u_end;
-    }
-
-    // ---- across the wavefronts, ROWS rows at a time; a thread finishes QUADS x 4 columns of each
-    constexpr int ROUNDS = MT * 16 / ROWS, THREADS = 64 * WAVES, QUADS = ROWS * COLS * NS / 4 / THREADS;
-    float4 sum[ROUNDS][QUADS];
-    // 16 lanes that write every second quad of a row would meet in half the banks: the upper half of a row is stored with
-    // neighbouring quads exchanged
-    auto swizzled = [](int quad) { return ND == 2 ? quad ^ ((quad >> 4) & 1) : quad; };
-#pragma unroll
-    for (int p = 0; p < ROUNDS; p++) {
-        if (p > 0) __syncthreads();
-#pragma unroll
-        for (int h = 0; h < ROWS / 16; h++)
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-#pragma unroll
-                for (int d = 0; d < ND; d++) {
-                    const int m = p * (ROWS / 16) + h;
-                    *reinterpret_cast<float4 *>(&s_red[wave][16 * h + 4 * kq + e][4 * swizzled(ND * nl + d)]) =
-                        make_float4(acc[m][4 * d][e], acc[m][4 * d + 1][e], acc[m][4 * d + 2][e], acc[m][4 * d + 3][e]);
-                }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < QUADS; q++) {
-            const int e = tid + q * THREADS, row = e / (NS * COLS / 4), quad = e % (COLS / 4), part = e / (COLS / 4) % NS;
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-            for (int k = 0; k < KW; k++) {
-                const float4 o = *reinterpret_cast<const float4 *>(&s_red[part * KW + k][row][4 * swizzled(quad)]);
-                v.x += o.x, v.y += o.y, v.z += o.z, v.w += o.w;
-            }
-            sum[p][q] = v;
-        }
-    }
-    // ---- across workgroups: tiles in scratch in the order [round][quad][thread]
-    if (plan.splits > 1) {
-        constexpr size_t TILE = (size_t)MT * 16 * COLS * NS;
-        float *base = partial + (size_t)tile * TILE + tid * 4;
-        const size_t per_split = (size_t)tiles * TILE;
-        auto word = [&](int s, int p, int q, int h) {
-            return reinterpret_cast<unsigned long long *>(base + s * per_split + (size_t)(p * QUADS + q) * THREADS * 4) + h;
+            for (int c = 0; c < NC; c++) acc[m][c] = (float4_t){0.f, 0.f, 0.f, 0.f};
+        // the cherry step `cs`; past the last one: step AS - 1 of the units, which is next
+        auto load_cherry = [&](int m, int cs) {
+            const int u = u0 + (AS - 1) / 4 * WK + wk;
+            const bool cherry = cs < csteps + wk, ok = cherry ? cs < csteps : u < u_end;
+            return load_a(m, !ok ? 0 : cherry ? 4 * plan.units + cs : 4 * u + (AS - 1) % 4, ok);
         };
 #pragma unroll
-        for (int p = 0; p < ROUNDS; p++)
+        for (int j = 0; j < AS - 1; j++)
 #pragma unroll
-            for (int q = 0; q < QUADS; q++) {
-                const float2 lo = make_float2(sum[p][q].x, sum[p][q].y), hi = make_float2(sum[p][q].z, sum[p][q].w);
-                __hip_atomic_store(word(split, p, q, 0), __builtin_bit_cast(unsigned long long, lo), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(word(split, p, q, 1), __builtin_bit_cast(unsigned long long, hi), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int m = 0; m < MT; m++) a[j][m] = load_step(m, j);
+#pragma unroll
+        for (int m = 0; m < MT; m++) a[AS - 1][m] = load_cherry(m, wk);
+        __builtin_amdgcn_s_setprio(1);
+        for (int c0 = 0; c0 < csteps; c0 += S * WK) {
+            stage_barrier();
+#pragma nounroll
+            for (int s = 0; s < S && c0 + s * WK < csteps; s++) {
+                const int next = c0 + (s + 1) * WK;
+#pragma unroll
+                for (int c = 0; c < NC; c++) {
+                    const u32x4 bc = frag[STAGE + (s * NC + c) * 64];
+#pragma unroll
+                    for (int m = 0; m < MT; m++) prompt_mfma(acc[m][c], a[AS - 1][m], bc);
+                }
+#pragma unroll
+                for (int m = 0; m < MT; m++) a[AS - 1][m] = load_cherry(m, next + wk);
             }
-        int *s_last = reinterpret_cast<int *>(&s_red[0][0][0]);
+            stage_barrier();
+        }
+        if (csteps == 0) stage_barrier();
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            b[c] = frag[c * 64];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // Every operand is asked for again as soon as its products are issued: activations AS steps ahead, weights one.  A
+        // stage's last step meets the producers once its own weights have arrived, and goes on with the next stage's.
+        constexpr int MEET = NC > 2 ? 1 : 0, U = AS > S ? AS / S : 1;
+#pragma nounroll
+        for (int st = 0; st < stages; st += U) {
+#pragma unroll
+            for (int v = 0; v < U; v++) {
+                const u32x4 *const here = frag + ((st + v) & 1) * STAGE, *const next = frag + (~(st + v) & 1) * STAGE;
+#pragma unroll
+                for (int s = 0; s < S; s++) {
+                    constexpr int last = NC - 1;
+                    const int set = (v * S + s) % AS;
+#pragma unroll
+                    for (int c = 0; c < NC; c++) {
+#pragma unroll
+                        for (int m = 0; m < MT; m++) {
+                            prompt_mfma(acc[m][c], a[set][m], b[c]);
+                            if (c == last) a[set][m] = load_step(m, (st + v) * S + s + AS);
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                        if (s < S - 1) b[c] = here[((s + 1) * NC + c) * 64];
+                        else if (c == MEET) {
+                            if (v < U - 1 || st + U < stages) stage_barrier();
+#pragma unroll
+                            for (int e = 0; e <= MEET; e++) {
+                                b[e] = next[e * 64];
+                                __builtin_amdgcn_sched_barrier(0);
+                            }
+                        } else if (c > MEET) b[c] = next[c * 64];
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+        }
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+        mfma_drain();
+        __builtin_amdgcn_sched_barrier(0);
+    } else {
+        // ---- weights
+        const uint8_t *__restrict__ const qweight = of(members.qweight);
+        const __half *__restrict__ const cherry_weight = of(members.cherry_weight);
+        const __half *__restrict__ const scales = of(members.scales);
+        const int Kn = K - C, wk = (wave - 4) / (NP / WK), sub = (wave - 4) % (NP / WK);
+        const int n0 = ntile * COLS + NC * nl;
+        const bool col_ok = n0 < N;
+        const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)qweight, 0, Kn / 8 * BITS * N, kRsrcFlagsP);
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)scales, 0, ceil_div(Kn, G) * N * 2, kRsrcFlagsP);
+        const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc((void *)cherry_weight, 0, C * N * 2, kRsrcFlagsP);
+        const uint32_t w_lane = col_ok ? (uint32_t)(kq * BITS * N + n0) : kOobP, sc_lane = col_ok ? (uint32_t)n0 * 2u : kOobP;
+        u32x4 *const frag = s_b + wk * S * NC * 64 + lane;
+        w_t w[D][PS][BITS];
+        s_t sc[D][WHOLE ? 1 : PS];
+        const PromptDecode<BITS> decoder;
+        // The steps of a stage that are this wavefront's: sub, sub + NP / WK, ...  Units past the last one are asked for as unit
+        // `plan.units`, which lies past the end of the packed bytes: the bounds of the buffer answer with zeros.
+        auto load = [&](int d, int st) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < PS; i++) {
+                const int q = st * S + sub + NP / WK * i, u = u0 + (q >> 2) * WK + wk;
+                const int step = u < u_end ? 4 * u + (q & 3) : 4 * plan.units;
+                const uint32_t off = w_lane + (uint32_t)(step * 4 * BITS * N);
+#pragma unroll
+                for (int r = 0; r < BITS; r++) w[d][i][r] = PromptPiece<NC>::codes(rw, off + (uint32_t)(r * N));
+                if (!WHOLE || i == 0) sc[d][i] = PromptPiece<NC>::halves(rs, sc_lane + __umulhi(2u * step, group_magic) * (uint32_t)N * 2u);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto fill = [&](int d, int st) {
+#pragma unroll
+            for (int i = 0; i < PS; i++)
+#pragma unroll
+                for (int c = 0; c < NC; c++) {
+                    PromptColumn<BITS> column;
+                    uint32_t codes[BITS];
+                    u32x4 o;
+#pragma unroll
+                    for (int r = 0; r < BITS; r++) codes[r] = w[d][i][r][c >> 2];
+#pragma unroll
+                    for (int g = 0; g < 8; g++) column.group(decoder, g, codes, c & 3, sc[d][WHOLE ? 0 : i][c >> 1], o);
+                    frag[(st & 1) * STAGE + ((sub + NP / WK * i) * NC + c) * 64] = o;
+                }
+        };
+        auto fill_cherries = [&](int c0) {
+#pragma unroll
+            for (int i = 0; i < PS; i++) {
+                const int s = sub + NP / WK * i, cs = c0 + s * WK + wk;
+                if (c0 + s * WK >= csteps) break;
+                s_t cw[8];
+                const uint32_t off = col_ok ? (uint32_t)((32 * cs + 8 * kq) * N + n0) * 2u : kOobP;
+#pragma unroll
+                for (int r = 0; r < 8; r++) cw[r] = PromptPiece<NC>::halves(rc, off + (uint32_t)(r * N * 2));
+#pragma unroll
+                for (int c = 0; c < NC; c++) {
+                    u32x4 o;
+#pragma unroll
+                    for (int d = 0; d < 4; d++)
+                        o[d] = __builtin_amdgcn_perm(cw[2 * d + 1][c >> 1], cw[2 * d][c >> 1], (c & 1) ? 0x07060302u : 0x05040100u);
+                    frag[STAGE + (s * NC + c) * 64] = o;
+                }
+            }
+        };
+        for (int c0 = 0; c0 < csteps; c0 += S * WK) {
+            if (c0 > 0) stage_barrier();
+            fill_cherries(c0);
+            if (c0 == 0) {
+#pragma unroll
+                for (int d = 0; d < D; d++) load(d, d);
+            }
+            if (c0 + S * WK >= csteps) break;
+            stage_barrier();
+        }
+        if (csteps == 0) {
+#pragma unroll
+            for (int d = 0; d < D; d++) load(d, d);
+        }
+        fill(0, 0);
+        load(0, D);
+        stage_barrier();
+        if (csteps > 0) stage_barrier();
+        int st = 1;
+#pragma nounroll
+        for (; st + D <= stages; st += D) {  // (one exit: the compiler's waits count on the loads' order)
+#pragma unroll
+            for (int d = 0; d < D; d++) {
+                fill((d + 1) % D, st + d);
+                load((d + 1) % D, st + d + D);
+                stage_barrier();
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < D - 1; d++) {
+            if (st + d >= stages) break;
+            fill((d + 1) % D, st + d);
+            stage_barrier();
+        }
+    }
+    // ---- across the wavefronts; a thread finishes QUADS x 4 columns
+    constexpr int QUADS = (ROWS * COLS / 4 + T - 1) / T;
+    float *const s_red = reinterpret_cast<float *>(s_b);
+    // 16 lanes that write every second quad of a row would meet in half the banks: the upper half of a row is stored with
+    // neighbouring quads exchanged
+    auto swizzled = [](int quad) { return NC == 8 ? quad ^ ((quad >> 4) & 1) : quad; };
+    __syncthreads();
+    if (wave < 4) {
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                float *const row = s_red + ((wave * MT + m) * 16 + 4 * kq + e) * COLS;
+                if constexpr (NC == 2) {
+                    *reinterpret_cast<float2 *>(row + 2 * nl) = make_float2(acc[m][0][e], acc[m][1][e]);
+                } else {
+#pragma unroll
+                    for (int d = 0; d < NC / 4; d++)
+                        *reinterpret_cast<float4 *>(row + 4 * swizzled(NC / 4 * nl + d)) =
+                            make_float4(acc[m][4 * d][e], acc[m][4 * d + 1][e], acc[m][4 * d + 2][e], acc[m][4 * d + 3][e]);
+                }
+            }
+    }
+    __syncthreads();
+    float4 sum[QUADS];
+#pragma unroll
+    for (int q = 0; q < QUADS; q++) {
+        const int e = tid + q * T, row = e / (COLS / 4), quad = e % (COLS / 4);
+        sum[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (ROWS * COLS / 4 % T && row >= ROWS) break;
+#pragma unroll
+        for (int k = 0; k < WK; k++) {
+            const float4 o = *reinterpret_cast<const float4 *>(s_red + (k * ROWS + row) * COLS + 4 * swizzled(quad));
+            sum[q].x += o.x, sum[q].y += o.y, sum[q].z += o.z, sum[q].w += o.w;
+        }
+    }
+    // ---- across workgroups: tiles in scratch in the order [quad][thread]
+    if (plan.splits > 1) {
+        constexpr size_t TILE = (size_t)ROWS * COLS;
+        float *base = partial + (size_t)tile * TILE + tid * 4;
+        const size_t per_split = (size_t)tiles * TILE;
+        auto has = [&](int q) { return ROWS * COLS / 4 % T == 0 || tid + q * T < ROWS * COLS / 4; };
+        auto word = [&](int s, int q, int h) { return reinterpret_cast<unsigned long long *>(base + s * per_split + (size_t)q * (4 * T)) + h; };
+#pragma unroll
+        for (int q = 0; q < QUADS; q++) {
+            if (!has(q)) break;
+            const float2 lo = make_float2(sum[q].x, sum[q].y), hi = make_float2(sum[q].z, sum[q].w);
+            __hip_atomic_store(word(split, q, 0), __builtin_bit_cast(unsigned long long, lo), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(word(split, q, 1), __builtin_bit_cast(unsigned long long, hi), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();  // the sums are read
+        int *s_last = reinterpret_cast<int *>(s_b);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
@@ -560,51 +717,42 @@ __global__ __launch_bounds__(64 * prompt_waves(MT, NC), MT * NC == 64 ? 1 : MT *
         if (!*s_last) return;
         if (tid == 0) __hip_atomic_store(&tickets[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-        for (int p = 0; p < ROUNDS; p++)
-#pragma unroll
-            for (int q = 0; q < QUADS; q++) sum[p][q] = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int q = 0; q < QUADS; q++) sum[q] = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll 2
         for (int s = 0; s < plan.splits; s++) {
-            float2 v[ROUNDS][QUADS][2];
+            float2 v[QUADS][2];
 #pragma unroll
-            for (int p = 0; p < ROUNDS; p++)
+            for (int q = 0; q < QUADS; q++)
 #pragma unroll
-                for (int q = 0; q < QUADS; q++)
+                for (int h = 0; h < 2; h++)
+                    v[q][h] = has(q) ? __builtin_bit_cast(float2, __hip_atomic_load(word(s, q, h), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                                     : make_float2(0.f, 0.f);
 #pragma unroll
-                    for (int h = 0; h < 2; h++)
-                        v[p][q][h] = __builtin_bit_cast(
-                            float2, __hip_atomic_load(word(s, p, q, h), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-#pragma unroll
-            for (int p = 0; p < ROUNDS; p++)
-#pragma unroll
-                for (int q = 0; q < QUADS; q++) {
-                    sum[p][q].x += v[p][q][0].x, sum[p][q].y += v[p][q][0].y;
-                    sum[p][q].z += v[p][q][1].x, sum[p][q].w += v[p][q][1].y;
-                }
+            for (int q = 0; q < QUADS; q++) {
+                sum[q].x += v[q][0].x, sum[q].y += v[q][0].y;
+                sum[q].z += v[q][1].x, sum[q].w += v[q][1].y;
+            }
         }
     }
 #pragma unroll
-    for (int p = 0; p < ROUNDS; p++)
-#pragma unroll
-        for (int q = 0; q < QUADS; q++) {
-            const int e = (tid + q * THREADS) * 4, m = mtile * MT * 16 + p * ROWS + e / (COLS * NS),
-                      n = ntile * COLS * NS + e % (COLS * NS);
-            if (m < M && n < N) {
-                uint2 *o = reinterpret_cast<uint2 *>(out + (size_t)m * N + n);
-                float v[4] = {sum[p][q].x, sum[p][q].y, sum[p][q].z, sum[p][q].w};
-                if (accumulate) {
-                    const uint2 was = *o;
-                    v[0] += __half2float(__ushort_as_half((unsigned short)was.x));
-                    v[1] += __half2float(__ushort_as_half((unsigned short)(was.x >> 16)));
-                    v[2] += __half2float(__ushort_as_half((unsigned short)was.y));
-                    v[3] += __half2float(__ushort_as_half((unsigned short)(was.y >> 16)));
-                }
-                uint32_t h[4];
-#pragma unroll
-                for (int c = 0; c < 4; c++) h[c] = __half_as_ushort(__float2half_rn(v[c]));
-                *o = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+    for (int q = 0; q < QUADS; q++) {
+        const int e = tid + q * T, row = e / (COLS / 4), m = mtile * ROWS + row, n = ntile * COLS + e % (COLS / 4) * 4;
+        if (row < ROWS && m < M && n < N) {
+            uint2 *o = reinterpret_cast<uint2 *>(out + (size_t)m * N + n);
+            float v[4] = {sum[q].x, sum[q].y, sum[q].z, sum[q].w};
+            if (accumulate) {
+                const uint2 was = *o;
+                v[0] += __half2float(__ushort_as_half((unsigned short)was.x));
+                v[1] += __half2float(__ushort_as_half((unsigned short)(was.x >> 16)));
+                v[2] += __half2float(__ushort_as_half((unsigned short)was.y));
+                v[3] += __half2float(__ushort_as_half((unsigned short)(was.y >> 16)));
             }
+            uint32_t h[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) h[c] = __half_as_ushort(__float2half_rn(v[c]));
+            *o = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
         }
+    }
 }
 
 bool prompt_supported(int bits, int M, int K, int N, int C, int G) {
@@ -615,7 +763,7 @@ bool prompt_supported(int bits, int M, int K, int N, int C, int G) {
     return wbytes < 0x7fff0000ll && cbytes < 0x7fff0000ll && sbytes < 0x7fff0000ll && prompt_max_rows(K, C) > 0;
 }
 
-template <int BITS, int MT, int NC, int NS>
+template <int BITS, int MT, int NC, int WM, int WK, int S, int AS, int NP, int D>
 static hipError_t launch_prompt_mt(const __half *vec, const PromptMember *layers, int count, int M, int K, int C, int G, int accumulate,
                                    const PromptPlan &plan, void *workspace, void *scratch, hipStream_t stream) {
     u32x4 *a = reinterpret_cast<u32x4 *>(scratch);
@@ -629,14 +777,17 @@ static hipError_t launch_prompt_mt(const __half *vec, const PromptMember *layers
         indices.of[i] = l.cherry_indices;
         members.qweight[i] = l.qweight, members.cherry_weight[i] = l.cherry_weight, members.scales[i] = l.scales, members.out[i] = l.out;
         members.N[i] = l.N, members.first[i] = first;
-        if (i < count) first += ceil_div(l.N, 16 * NC * NS);
+        if (i < count) first += ceil_div(l.N, 16 * NC);
     }
-    hipLaunchKernelGGL(prompt_prep_kernel<BITS>, dim3(plan.units + ceil_div(plan.csteps, 4), plan.mtiles * MT, count), dim3(256), 0, stream,
-                       vec, indices, reinterpret_cast<uint4 *>(a), plan.a_bytes, M, K, C, plan.units, plan.mtiles * MT,
-                       aligned(vec, 16) ? 1 : 0);
-    const dim3 grid(8 * ceil_div(plan.mtiles * plan.ntiles, 8), plan.splits);
-    auto *const kernel = G % kUnitK == 0 ? prompt_kernel<BITS, MT, NC, NS, true> : prompt_kernel<BITS, MT, NC, NS, false>;
-    hipLaunchKernelGGL(kernel, grid, dim3(64 * prompt_waves(MT, NC)), 0, stream, members, a, partial, tickets, M, K, C, G, accumulate, plan);
+    const int m16 = plan.mtiles * plan.mt;
+    hipLaunchKernelGGL(prompt_prep_kernel<BITS>, dim3(plan.units + ceil_div(plan.csteps, 4), m16, count), dim3(256), 0, stream, vec, indices,
+                       reinterpret_cast<uint4 *>(a), plan.a_bytes, M, K, C, plan.units, m16, aligned(vec, 16) ? 1 : 0);
+    const dim3 grid(8 * ceil_div(plan.mtiles * plan.ntiles * plan.splits, 8));
+    auto *const kernel =
+        G % kUnitK == 0 ? prompt_kernel<BITS, MT, NC, WM, WK, S, AS, NP, D, true> : prompt_kernel<BITS, MT, NC, WM, WK, S, AS, NP, D, false>;
+    // ceil(2^31 / steps of a group): 2 s times it, shifted right by 32, is s / steps for every s below 2^31 / steps
+    const unsigned group_magic = (unsigned)((0x80000000u + (unsigned)(G / 32) - 1u) / (unsigned)(G / 32));
+    hipLaunchKernelGGL(kernel, grid, dim3(256 + 64 * NP), 0, stream, members, a, partial, tickets, M, K, C, G, group_magic, accumulate, plan);
     return hipGetLastError();
 }
 
@@ -646,14 +797,11 @@ static hipError_t launch_prompt_bits(const __half *vec, const PromptMember *laye
     int N[kPromptMaxGroup];
     for (int i = 0; i < count; i++) N[i] = layers[i].N;
     const PromptPlan plan = prompt_plan(M, K, N, count, C);
-#define CQ_PROMPT(MT_, NC_, NS_)                            \
-    if (plan.mt == MT_ && plan.nc == NC_ && plan.ns == NS_) \
-    return launch_prompt_mt<BITS, MT_, NC_, NS_>(vec, layers, count, M, K, C, G, accumulate, plan, workspace, scratch, stream)
-    CQ_PROMPT(2, 4, 1);
-    CQ_PROMPT(4, 4, 1);
-    CQ_PROMPT(8, 4, 1);
-    CQ_PROMPT(8, 8, 1);
-    CQ_PROMPT(8, 8, 2);
+#define CQ_PROMPT(ID, MT, NC, WM, WK, S, AS, NP, D)                                                                         \
+    case ID:                                                                                                                \
+        return launch_prompt_mt<BITS, MT, NC, WM, WK, S, AS, NP, D>(vec, layers, count, M, K, C, G, accumulate, plan, workspace, scratch, \
+                                                                    stream);
+    switch (plan.shape) { CQ_PROMPT_SHAPES(CQ_PROMPT) }
 #undef CQ_PROMPT
     return hipErrorInvalidConfiguration;
 }

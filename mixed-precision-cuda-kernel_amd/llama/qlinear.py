@@ -66,10 +66,11 @@ class QuantLinear(nn.Module):
 
     _layerwise_dequantize = True
     # Rows at and above which the fused forward dequantises once and calls the library's dense GEMM
-    # instead of the fused dequantise + MFMA kernel.  The line depends on the layer (MI355X, fused / dense in us:
-    # 4096 -> 11008 with 768 rows 116 / 96, with 2048 rows 196 / 195; 8192 -> 28672 with 512 rows 243 / 332;
-    # 1024 -> 2048 with 1024 rows 16 / 40); small layers gain from a higher one.
-    prefill_rows = 512
+    # instead of the fused dequantise + MFMA kernel.  MI355X, fused / dense in us with 2048 and 3072 rows: 4096 -> 11008
+    # 188 / 198 and 295 / 335, 4096 -> 4096 72 / 76 and 114 / 98, 8192 -> 28672 796 / 851 and 1225 / 1173, 5120 -> 13824 in
+    # 3 bits 279 / 278 and 413 / 376; below, the fused kernel is ahead by up to a third (512 rows of 8192 -> 28672: 230 / 340).
+    prefill_rows = 2304
+
     @classmethod
     @contextmanager
     def dmode(cls, layerwise_dequantize=True):
