@@ -479,6 +479,31 @@ int cherryq_prefill_attention_f16(const void *q, const void *k, const void *v, c
                                   void *k_cache, void *v_cache, void *out, void *scratch, size_t scratch_bytes, int tokens,
                                   int n_heads, int n_kv_heads, int head_dim, int max_len, void *stream);
 
+/*
+ * The decoder layers of a prompt of `tokens` (17 and more) positions from 0, in one call: residual + RMSNorm, q/k/v, attention with
+ * cache writes, o_proj, residual + RMSNorm, gate/up, SiLU * up, down_proj (llama/modeling_llama_quant.py:754-775), with
+ * the roundings of the single calls above.  RMSNorm and SiLU hand their rows to the products in the order these
+ * read.  hidden (tokens, hidden_size) is updated in place; delta (tokens, hidden_size) receives the last layer's
+ * down_proj, which is still to be added.  `mul` of the products' layers is not used.  hidden_size at most 8192, intermediate sizes
+ * at most 28672, at most 248 cherries a layer, head_dim 128; o_proj reads n_heads * 128 features.
+ * workspace (all zero before and after) and scratch (uninitialised) of the sizes that the two functions answer, 256-byte aligned.
+ * Everything is checked before the first launch; CHERRYQ_E_UNSUPPORTED: layers for the single calls.
+ */
+typedef struct {
+    cherryq_layer layers[3];
+    int n_layers, w_bits, in_features, num_cherries, group_size;
+} cherryq_prefill_product;
+typedef struct {
+    const void *input_norm, *post_attention_norm; /* hidden_size fp16 each */
+    void *k_cache, *v_cache;                      /* [n_kv_heads][max_len][128] */
+    cherryq_prefill_product qkv, o, gate_up, down;
+} cherryq_prefill_layer;
+size_t cherryq_prefill_layers_workspace_bytes(const cherryq_prefill_layer *layers, int n_layers, int tokens);
+size_t cherryq_prefill_layers_scratch_bytes(const cherryq_prefill_layer *layers, int n_layers, int tokens, int n_heads, int n_kv_heads);
+int cherryq_prefill_layers_f16(const cherryq_prefill_layer *layers, int n_layers, void *hidden, void *delta, const void *cos_table,
+                               const void *sin_table, int tokens, int hidden_size, int n_heads, int n_kv_heads, int max_len, float eps,
+                               void *workspace, size_t workspace_bytes, void *scratch, size_t scratch_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -56,7 +56,7 @@ def host_command(source, output):
     return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1",
             f'-DCHERRYQ_BUILT_FOR="{built_for()}"',
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-            *(f"-isystem{p}" for p in (*include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"])),
+            f"-I{HERE.parent / 'include'}", *(f"-isystem{p}" for p in (*include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"])),
             str(source), "-o", str(output), f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10", "-lc10_hip"]
 
 

@@ -124,6 +124,26 @@ _lib.cherryq_prefill_matmul_group_f16.argtypes = [_int, _vp, ctypes.POINTER(_Lay
 _lib.cherryq_prefill_matmul_group_f16.restype = _int
 
 
+class _PrefillProduct(ctypes.Structure):
+    """struct cherryq_prefill_product of include/cherryq.h"""
+    _fields_ = [("layers", _Layer * 3), ("n_layers", _int), ("w_bits", _int), ("in_features", _int), ("num_cherries", _int),
+                ("group_size", _int)]
+
+
+class _PrefillLayer(ctypes.Structure):
+    """struct cherryq_prefill_layer of include/cherryq.h"""
+    _fields_ = [(n, _vp) for n in ("input_norm", "post_attention_norm", "k_cache", "v_cache")] + [
+        (n, _PrefillProduct) for n in ("qkv", "o", "gate_up", "down")]
+
+
+_lib.cherryq_prefill_layers_workspace_bytes.argtypes = [ctypes.POINTER(_PrefillLayer), _int, _int]
+_lib.cherryq_prefill_layers_workspace_bytes.restype = ctypes.c_size_t
+_lib.cherryq_prefill_layers_scratch_bytes.argtypes = [ctypes.POINTER(_PrefillLayer), _int, _int, _int, _int]
+_lib.cherryq_prefill_layers_scratch_bytes.restype = ctypes.c_size_t
+_lib.cherryq_prefill_layers_f16.argtypes = [ctypes.POINTER(_PrefillLayer), _int, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _int, _f,
+                                            _vp, ctypes.c_size_t, _vp, ctypes.c_size_t, _vp]
+_lib.cherryq_prefill_layers_f16.restype = _int
+
 _FORWARD = QuantLinear.forward  # as defined: a program may put another one in its place
 
 
@@ -444,6 +464,7 @@ class CherryLlamaDecoder(nn.Module):
         self.logits16 = torch.zeros(1, cfg.vocab_size, **f16)
         self.history = torch.zeros(ml, dtype=torch.int64, device=self.device_)  # history[p]: token predicted at position p
         self._graph = None
+        self._rope = None  # _rope_tables
         self.fuse_norm = True
         self.fuse_head = True  # final RMSNorm inside the head launch (False: a launch of its own in front)
         # Attention dealt to ATTN_SLICES workgroups per head, combined by a repacked o_proj's staging: None =
@@ -716,11 +737,7 @@ class CherryLlamaDecoder(nn.Module):
         ids = prompt_ids.to(self.device_)
         T, nh, nkv, hd, hidden = ids.numel(), cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim, cfg.hidden_size
         assert ids.dim() == 1 and 1 <= T <= cfg.max_position_embeddings
-        pos = torch.arange(T, device=self.device_, dtype=torch.float32)
-        inv = 1.0 / (cfg.rope_theta ** (torch.arange(0, hd, 2, device=self.device_, dtype=torch.float32) / hd))
-        fr = torch.outer(pos, inv)
-        cos, sin = fr.cos().half(), fr.sin().half()  # (T, hd / 2)
-
+        cos, sin = self._rope_tables(T)
         self.reset()
         h = self.embed_tokens[ids]
         attend = self._prefill_attention(T, cos, sin) if hd == 128 else self._prefill_attention_torch(T, cos, sin)
@@ -760,9 +777,9 @@ class CherryLlamaDecoder(nn.Module):
             _ok(_lib.cherryq_decode_silu_mul_f16(gate.data_ptr(), up.data_ptr(), act.data_ptr(), n, quant_cuda._current_stream(dev)), "silu_mul")
             return act
 
+        delta = self._prefill_layers(h, cos, sin) if hd == 128 and T >= 17 else None
         # What a module reads or returns is written once: a hook or a replaced module may keep it.
-        delta = None
-        for li, layer in enumerate(self.layers):
+        for li, layer in enumerate(self.layers if delta is None else ()):
             h, x = add_norm(h, delta, layer.input_layernorm)
             q, k, v = project(x, layer.q_proj, layer.k_proj, layer.v_proj)
             delta = layer.o_proj(attend(li, heads(q, nh), heads(k, nkv), heads(v, nkv)))
@@ -773,6 +790,59 @@ class CherryLlamaDecoder(nn.Module):
         self.pos.fill_(T - 1)
         self._head(self.normed, None)  # logits of the last prompt position; greedy tail: history[T-1], next embedding, pos = T
         return self.logits
+
+    def _rope_tables(self, T):
+        """cos and sin of the rotary angles of positions 0..T-1, (T, head_dim / 2) fp16 each: made once for all positions
+        (llama/modeling_llama_quant.py:95-210 keeps them too)."""
+        cfg, hd = self.cfg, self.cfg.head_dim
+        made_for = self.device_, cfg.rope_theta, hd, cfg.max_position_embeddings
+        if self._rope is None or self._rope[0] != made_for:
+            pos = torch.arange(cfg.max_position_embeddings, device=self.device_, dtype=torch.float32)
+            inv = 1.0 / (cfg.rope_theta ** (torch.arange(0, hd, 2, device=self.device_, dtype=torch.float32) / hd))
+            fr = torch.outer(pos, inv)
+            self._rope = made_for, fr.cos().half(), fr.sin().half()
+        return self._rope[1][:T], self._rope[2][:T]
+
+    def _prefill_layers(self, h, cos, sin):
+        """All layers in one native call where every projection is a plain module and nothing else sees what lies between them: h is
+        updated in place, the last layer's down projection returned.  Otherwise None, and nothing has been launched."""
+        cfg, dev, T = self.cfg, self.k_cache.get_device(), h.shape[0]
+        hidden, ml, n = cfg.hidden_size, cfg.max_position_embeddings, len(self.layers)
+        caches = (self.k_cache, self.v_cache)
+        if not n or not _plain(h, dev, T, hidden) or not all(
+                c.dtype == torch.float16 and c.is_contiguous() and c.shape == (n, cfg.num_key_value_heads, ml, 128) for c in caches):
+            return None
+        if torch.nn.modules.module._has_any_global_hook() or QuantLinear.forward is not _FORWARD:
+            return None
+        layers = (_PrefillLayer * n)()
+        at, size = ctypes.addressof(layers), ctypes.sizeof(_PrefillLayer)
+        (k_at, v_at), step = (c.data_ptr() for c in caches), 2 * caches[0].stride(0)
+        held = []  # what the descriptions point to: another thread may replace a module's buffers during the call
+        describe, qkv, o, gate_up, down = quant_cuda._host.describe, *(getattr(_PrefillLayer, f).offset for f in ("qkv", "o", "gate_up", "down"))
+        for a, layer in zip(layers, self.layers):
+            norms, m = (layer.input_layernorm, layer.post_attention_layernorm), layer._modules
+            if not (_plain(norms[0], dev, hidden) and _plain(norms[1], dev, hidden)
+                    and describe(at + qkv, T, dev, QuantLinear, held, m.get("q_proj"), m.get("k_proj"), m.get("v_proj"))
+                    and describe(at + o, T, dev, QuantLinear, held, m.get("o_proj"))
+                    and describe(at + gate_up, T, dev, QuantLinear, held, m.get("gate_proj"), m.get("up_proj"))
+                    and describe(at + down, T, dev, QuantLinear, held, m.get("down_proj"))):
+                return None
+            held += norms
+            a.input_norm, a.post_attention_norm, a.k_cache, a.v_cache = norms[0].data_ptr(), norms[1].data_ptr(), k_at, v_at
+            at, k_at, v_at = at + size, k_at + step, v_at + step
+        stream = quant_cuda._current_stream(dev)
+        nbytes = _lib.cherryq_prefill_layers_scratch_bytes(layers, n, T, cfg.num_attention_heads, cfg.num_key_value_heads)
+        if not nbytes:
+            return None
+        ws = quant_cuda._workspace(h.device, stream, _lib.cherryq_prefill_layers_workspace_bytes(layers, n, T))
+        sc, delta = quant_cuda._scratch(h.device, stream, nbytes), torch.empty_like(h)
+        rc = _lib.cherryq_prefill_layers_f16(layers, n, h.data_ptr(), delta.data_ptr(), cos.data_ptr(), sin.data_ptr(), T, hidden,
+                                             cfg.num_attention_heads, cfg.num_key_value_heads, ml, cfg.rms_norm_eps, ws.data_ptr(),
+                                             ws.numel(), sc.data_ptr(), sc.numel(), stream)
+        if rc == -7:
+            return None
+        _ok(rc, "prefill_layers")
+        return delta
 
     def _prefill_attention(self, T, cos, sin):
         """attend(layer, q, k, v) for heads of 128: rotary embedding, cache write and causal attention in two launches."""

@@ -1,5 +1,8 @@
 // extern "C" entry points of libcherryq: argument validation and kernel selection.
 // Declarations and the reference interfaces they replace: include/cherryq.h.
+#include <algorithm>
+#include <initializer_list>
+
 #include "../../include/cherryq.h"
 
 #include <stdlib.h>
@@ -880,6 +883,166 @@ int cherryq_prefill_attention_f16(const void *q, const void *k, const void *v, c
         reinterpret_cast<const __half *>(cos_table), reinterpret_cast<const __half *>(sin_table),
         reinterpret_cast<__half *>(k_cache), reinterpret_cast<__half *>(v_cache), reinterpret_cast<__half *>(out), scratch, tokens,
         n_heads, n_kv_heads, max_len, reinterpret_cast<hipStream_t>(stream));
+}
+
+// ---- a prompt's layers -------------------------------------------------------------------------------------------
+static cq::PromptPlan product_plan(const cherryq_prefill_product &p, int tokens) {
+    int N[3];
+    for (int i = 0; i < p.n_layers; i++) N[i] = p.layers[i].out_features;
+    return cq::prompt_plan(tokens, p.in_features, N, p.n_layers, p.num_cherries);
+}
+
+static bool product_dims(const cherryq_prefill_product &p, int tokens) {
+    int N[3] = {0, 0, 0};
+    if (p.n_layers < 1 || p.n_layers > 3) return false;
+    for (int i = 0; i < p.n_layers; i++) N[i] = p.layers[i].out_features;
+    return prefill_group_dims(tokens, p.in_features, p.n_layers, N, p.num_cherries) &&
+           cq::prompt_rows_supported(tokens, p.in_features, p.num_cherries);
+}
+
+size_t cherryq_prefill_layers_workspace_bytes(const cherryq_prefill_layer *layers, int n_layers, int tokens) {
+    size_t bytes = 0;
+    for (int l = 0; layers && l < n_layers; l++)
+        for (const cherryq_prefill_product *p : {&layers[l].qkv, &layers[l].o, &layers[l].gate_up, &layers[l].down}) {
+            if (!product_dims(*p, tokens)) return 0;
+            bytes = std::max(bytes, product_plan(*p, tokens).workspace_bytes);
+        }
+    return bytes;
+}
+
+// products' operands and partial tiles; keys and values as the attention reads them; q, k, v, the attention's result; gate and up
+struct PrefillScratch {
+    size_t attention, q, k, v, out, gate, up, total;
+};
+static bool prefill_scratch(const cherryq_prefill_layer *layers, int n_layers, int tokens, int n_heads, int n_kv_heads, PrefillScratch &s) {
+    if (!layers || n_layers < 1 || tokens < 2 || n_heads < 1 || n_kv_heads < 1) return false;
+    size_t products = 0, inter = 0;
+    for (int l = 0; l < n_layers; l++) {
+        for (const cherryq_prefill_product *p : {&layers[l].qkv, &layers[l].o, &layers[l].gate_up, &layers[l].down}) {
+            if (!product_dims(*p, tokens)) return false;
+            products = std::max(products, product_plan(*p, tokens).scratch_bytes);
+        }
+        inter = std::max(inter, (size_t)std::max(layers[l].down.in_features, 0));
+    }
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        const size_t here = at;
+        at += (bytes + 255) / 256 * 256;
+        return here;
+    };
+    take(products);
+    s.attention = take(cq::prefill_attention_bytes(tokens, n_kv_heads));
+    s.q = take((size_t)tokens * n_heads * 256), s.k = take((size_t)tokens * n_kv_heads * 256), s.v = take((size_t)tokens * n_kv_heads * 256);
+    s.out = take((size_t)tokens * n_heads * 256);
+    s.gate = take((size_t)tokens * inter * 2), s.up = take((size_t)tokens * inter * 2);
+    s.total = at;
+    return true;
+}
+
+size_t cherryq_prefill_layers_scratch_bytes(const cherryq_prefill_layer *layers, int n_layers, int tokens, int n_heads, int n_kv_heads) {
+    PrefillScratch s;
+    return prefill_scratch(layers, n_layers, tokens, n_heads, n_kv_heads, s) ? s.total : 0;
+}
+
+int cherryq_prefill_layers_f16(const cherryq_prefill_layer *layers, int n_layers, void *hidden, void *delta, const void *cos_table,
+                               const void *sin_table, int tokens, int hidden_size, int n_heads, int n_kv_heads, int max_len, float eps,
+                               void *workspace, size_t workspace_bytes, void *scratch, size_t scratch_bytes, void *stream) {
+    using namespace cq;
+    if (!layers || !hidden || !delta || !cos_table || !sin_table) return CHERRYQ_E_NULL;
+    if (n_layers < 1 || tokens < 1 || tokens > max_len || n_heads <= 0 || n_kv_heads <= 0 || n_heads % n_kv_heads || hidden_size <= 0 ||
+        hidden_size % 8)
+        return CHERRYQ_E_SHAPE;
+    if (tokens < kPromptMinRows || hidden_size > kPrefillMaxHidden || n_kv_heads > 65535 || tokens > 1000000 || force_generic())
+        return CHERRYQ_E_UNSUPPORTED;
+    for (const void *p : {(const void *)hidden, (const void *)delta, cos_table, sin_table})
+        if (!aligned(p, 16)) return CHERRYQ_E_ALIGN;
+    for (int l = 0; l < n_layers; l++) {
+        const cherryq_prefill_layer &a = layers[l];
+        if (!a.input_norm || !a.post_attention_norm || !a.k_cache || !a.v_cache) return CHERRYQ_E_NULL;
+        for (const void *p : {a.input_norm, a.post_attention_norm, (const void *)a.k_cache, (const void *)a.v_cache})
+            if (!aligned(p, 16)) return CHERRYQ_E_ALIGN;
+        const int q = 128 * n_heads, kv = 128 * n_kv_heads, inter = a.down.in_features;
+        const struct {
+            const cherryq_prefill_product &p;
+            int n, in, out[3];
+        } products[4] = {{a.qkv, 3, hidden_size, {q, kv, kv}}, {a.o, 1, q, {hidden_size}}, {a.gate_up, 2, hidden_size, {inter, inter}},
+                         {a.down, 1, inter, {hidden_size}}};
+        for (const auto &e : products) {
+            const cherryq_prefill_product &p = e.p;
+            if (p.w_bits != 3 && p.w_bits != 4) return CHERRYQ_E_BITS;
+            if (p.n_layers != e.n || p.in_features != e.in) return CHERRYQ_E_SHAPE;
+            if (p.w_bits == 4 && p.group_size < 128) return CHERRYQ_E_GROUP;
+            for (int i = 0; i < p.n_layers; i++) {
+                const cherryq_layer &w = p.layers[i];
+                if (w.out_features != e.out[i]) return CHERRYQ_E_SHAPE;
+                const int rc = check_tensors(hidden, w.qweight, w.cherry_weight, w.cherry_indices, w.scales, hidden, tokens, p.in_features,
+                                             w.out_features, p.num_cherries, p.group_size);
+                if (rc) return rc;
+                if (!prompt_supported(p.w_bits, tokens, p.in_features, w.out_features, p.num_cherries, p.group_size))
+                    return CHERRYQ_E_UNSUPPORTED;
+            }
+            if (!product_dims(p, tokens)) return CHERRYQ_E_UNSUPPORTED;
+        }
+    }
+    PrefillScratch at;
+    if (!prefill_scratch(layers, n_layers, tokens, n_heads, n_kv_heads, at)) return CHERRYQ_E_UNSUPPORTED;
+    if (!workspace || !aligned(workspace, 256) || workspace_bytes < cherryq_prefill_layers_workspace_bytes(layers, n_layers, tokens) ||
+        !scratch || !aligned(scratch, 256) || scratch_bytes < at.total)
+        return CHERRYQ_E_WORKSPACE;
+
+    const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    auto half = [&](size_t offset) { return reinterpret_cast<__half *>(reinterpret_cast<char *>(scratch) + offset); };
+    __half *const h = reinterpret_cast<__half *>(hidden), *const d = reinterpret_cast<__half *>(delta);
+    // a product's layers with their results' places, and its plan
+    struct Product {
+        PromptMember m[3];
+        PromptPlan plan;
+    };
+    auto product = [&](const cherryq_prefill_product &p, std::initializer_list<__half *> out) {
+        Product r;
+        for (int i = 0; i < p.n_layers; i++) {
+            const cherryq_layer &w = p.layers[i];
+            r.m[i] = {w.qweight, reinterpret_cast<const __half *>(w.cherry_weight), w.cherry_indices,
+                      reinterpret_cast<const __half *>(w.scales), out.begin()[i], w.out_features};
+        }
+        r.plan = product_plan(p, tokens);
+        return r;
+    };
+    auto multiply = [&](const cherryq_prefill_product &p, const Product &r) {
+        return launch_prompt_product(p.w_bits, r.m, p.n_layers, tokens, p.in_features, p.num_cherries, p.group_size, 0, r.plan, workspace,
+                                     scratch, s);
+    };
+    auto norm = [&](const cherryq_prefill_product &p, const Product &r, const __half *add, const void *weight) {
+        return launch_prompt_norm(p.w_bits, h, add, reinterpret_cast<const __half *>(weight), eps, r.m, p.n_layers, tokens, p.in_features,
+                                  p.num_cherries, r.plan, scratch, s);
+    };
+#define CQ_TRY(call)                                \
+    do {                                            \
+        const hipError_t e = (call);                \
+        if (e != hipSuccess) return (int)e;         \
+    } while (0)
+    for (int l = 0; l < n_layers; l++) {
+        const cherryq_prefill_layer &a = layers[l];
+        const Product qkv = product(a.qkv, {half(at.q), half(at.k), half(at.v)});
+        CQ_TRY(norm(a.qkv, qkv, l > 0 ? d : nullptr, a.input_norm));
+        CQ_TRY(multiply(a.qkv, qkv));
+        CQ_TRY(launch_prefill_attention(half(at.q), half(at.k), half(at.v), reinterpret_cast<const __half *>(cos_table),
+                                        reinterpret_cast<const __half *>(sin_table), reinterpret_cast<__half *>(a.k_cache),
+                                        reinterpret_cast<__half *>(a.v_cache), half(at.out), half(at.attention), tokens, n_heads, n_kv_heads,
+                                        max_len, s));
+        const Product o = product(a.o, {d});
+        CQ_TRY(launch_prompt_prep(a.o.w_bits, half(at.out), o.m, 1, tokens, a.o.in_features, a.o.num_cherries, o.plan, scratch, s));
+        CQ_TRY(multiply(a.o, o));
+        const Product gate_up = product(a.gate_up, {half(at.gate), half(at.up)});
+        CQ_TRY(norm(a.gate_up, gate_up, d, a.post_attention_norm));
+        CQ_TRY(multiply(a.gate_up, gate_up));
+        const Product down = product(a.down, {d});
+        CQ_TRY(launch_prompt_silu(a.down.w_bits, half(at.gate), half(at.up), down.m, tokens, a.down.in_features, a.down.num_cherries,
+                                  down.plan, scratch, s));
+        CQ_TRY(multiply(a.down, down));
+    }
+#undef CQ_TRY
+    return CHERRYQ_OK;
 }
 
 }  // extern "C"

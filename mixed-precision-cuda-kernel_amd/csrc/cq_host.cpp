@@ -27,6 +27,8 @@
 #include <utility>
 #include <vector>
 
+#include "cherryq.h"
+
 namespace {
 
 using at::Tensor;
@@ -221,7 +223,8 @@ PyObject *matvec_prepacked(PyObject *, PyObject *const *a, Py_ssize_t n) {
 // ---- QuantLinear.forward ----------------------------------------------------------------------------
 struct Names {
     PyObject *dict, *buffers, *stream, *released, *dequantized, *layerwise, *prefill_rows, *w_bits, *group_size, *in_features,
-        *out_features, *num_cherries, *qweight, *cherry_weight, *cherry_indices, *scales, *bias;
+        *out_features, *num_cherries, *qweight, *cherry_weight, *cherry_indices, *scales, *bias, *forward, *forward_hooks,
+        *forward_pre_hooks;
 } names;
 
 // An integer entry of a module's dictionary (negative: none).
@@ -306,6 +309,62 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
+// describe(address, rows, device, class, held, *modules): fills the cherryq_prefill_product at the address and appends the
+// buffers it points to to the list `held`.  False where a module's own call would do anything but multiply `rows` rows
+// by its checkpoint buffers with the prompt kernel: another class, hooks, a bias, another mode or shape.
+PyObject *describe(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n < 6 || n > 8 || !PyList_CheckExact(a[4])) Py_RETURN_FALSE;
+    auto *product = static_cast<cherryq_prefill_product *>(PyLong_AsVoidPtr(a[0]));
+    const int64_t rows = PyLong_AsLongLong(a[1]);
+    const int device = (int)PyLong_AsLong(a[2]);
+    if (PyErr_Occurred()) return nullptr;
+    if (!product) Py_RETURN_FALSE;
+    product->n_layers = (int)(n - 5);
+    for (Py_ssize_t i = 5; i < n; i++) {
+        PyObject *m = a[i];
+        if ((PyObject *)Py_TYPE(m) != a[3] || _PyType_Lookup(Py_TYPE(m), names.bias)) Py_RETURN_FALSE;
+        Ref dict{PyObject_GetAttr(m, names.dict)}, layerwise{PyObject_GetAttr(m, names.layerwise)}, limit{PyObject_GetAttr(m, names.prefill_rows)};
+        if (!dict.o || !layerwise.o || !limit.o || !PyDict_CheckExact(dict.o)) {
+            PyErr_Clear();
+            Py_RETURN_FALSE;
+        }
+        auto entry = [&](PyObject *name) { return PyDict_GetItemWithError(dict.o, name); };
+        PyObject *buffers = entry(names.buffers), *hooks = entry(names.forward_hooks), *pre_hooks = entry(names.forward_pre_hooks);
+        const int64_t bits = number(dict.o, names.w_bits), group = number(dict.o, names.group_size), k = number(dict.o, names.in_features),
+                      columns = number(dict.o, names.out_features), c = number(dict.o, names.num_cherries),
+                      most = PyLong_Check(limit.o) ? PyLong_AsLongLong(limit.o) : -1;
+        if (PyErr_Occurred()) PyErr_Clear();
+        if (entry(names.forward) || !buffers || !PyDict_Check(buffers) || !hooks || !PyDict_Check(hooks) || PyDict_GET_SIZE(hooks) ||
+            !pre_hooks || !PyDict_Check(pre_hooks) || PyDict_GET_SIZE(pre_hooks) || layerwise.o != Py_True ||
+            entry(names.dequantized) != Py_False || entry(names.released) != Py_False || rows >= most || (bits != 3 && bits != 4) ||
+            group <= 0 || k <= 0 || columns <= 0 || c < 0 || c >= k || std::max({group, k, columns}) > INT32_MAX)
+            Py_RETURN_FALSE;
+        PyObject *bias = entry(names.bias);
+        if (!bias) bias = PyDict_GetItemWithError(buffers, names.bias);
+        if (bias != Py_None) Py_RETURN_FALSE;
+        PyObject *const o[4] = {PyDict_GetItemWithError(buffers, names.qweight), PyDict_GetItemWithError(buffers, names.cherry_weight),
+                                PyDict_GetItemWithError(buffers, names.cherry_indices), PyDict_GetItemWithError(buffers, names.scales)};
+        const Tensor *t[4];
+        for (int j = 0; j < 4; j++) t[j] = o[j] ? tensor(o[j]) : nullptr;
+        if (!is(t[0], at::kByte, 2, device) || !is(t[1], at::kHalf, 2, device) || !is(t[2], at::kShort, 1, device) ||
+            !is(t[3], at::kHalf, 2, device) || t[0]->size(0) * 8 != (k - c) * bits || t[0]->size(1) != columns || t[1]->size(0) != c ||
+            t[1]->size(1) != columns || t[2]->size(0) != c || t[3]->size(0) != (k - c + group - 1) / group || t[3]->size(1) != columns)
+            Py_RETURN_FALSE;
+        if (i == 5) {
+            product->w_bits = (int)bits, product->in_features = (int)k, product->num_cherries = (int)c, product->group_size = (int)group;
+        } else if (product->w_bits != bits || product->in_features != k || product->num_cherries != c || product->group_size != group) {
+            Py_RETURN_FALSE;
+        }
+        for (int j = 0; j < 4; j++)
+            if (PyList_Append(a[4], o[j])) return nullptr;
+        product->layers[i - 5] = {static_cast<const uint8_t *>(ptr(*t[0])), ptr(*t[1]), static_cast<const int16_t *>(ptr(*t[2])), ptr(*t[3]),
+                                  nullptr, (int)columns};
+    }
+    Py_RETURN_TRUE;
+    END_HANDLE_TH_ERRORS
+}
+
 // plain(tensor, device, *shape): whether a launch may read the tensor's memory as fp16 of this shape, in 16-byte pieces
 PyObject *plain(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
@@ -361,6 +420,7 @@ PyMethodDef methods[] = {
     {"vecquant", (PyCFunction)(void (*)())vecquant, METH_FASTCALL, nullptr},
     {"matvec_prepacked", (PyCFunction)(void (*)())matvec_prepacked, METH_FASTCALL, nullptr},
     {"linear", (PyCFunction)(void (*)())linear, METH_FASTCALL, nullptr},
+    {"describe", (PyCFunction)(void (*)())describe, METH_FASTCALL, nullptr},
     {"plain", (PyCFunction)(void (*)())plain, METH_FASTCALL, nullptr},
     {"workspace", (PyCFunction)(void (*)())workspace, METH_FASTCALL, nullptr},
     {"scratch", (PyCFunction)(void (*)())scratch, METH_FASTCALL, nullptr},
@@ -376,7 +436,8 @@ PyMODINIT_FUNC PyInit_cherryq_host(void) {
         {&names.layerwise, "_layerwise_dequantize"}, {&names.prefill_rows, "prefill_rows"}, {&names.w_bits, "w_bits"},
         {&names.group_size, "group_size"}, {&names.in_features, "in_features"}, {&names.out_features, "out_features"},
         {&names.num_cherries, "num_cherries"}, {&names.qweight, "qweight"}, {&names.cherry_weight, "cherry_weight"},
-        {&names.cherry_indices, "cherry_indices"}, {&names.scales, "scales"}, {&names.bias, "bias"}};
+        {&names.cherry_indices, "cherry_indices"}, {&names.scales, "scales"}, {&names.bias, "bias"},
+        {&names.forward, "forward"}, {&names.forward_hooks, "_forward_hooks"}, {&names.forward_pre_hooks, "_forward_pre_hooks"}};
     for (auto &n : all)
         if (!(*n.first = PyUnicode_InternFromString(n.second))) return nullptr;
     PyObject *m = PyModule_Create(&module);

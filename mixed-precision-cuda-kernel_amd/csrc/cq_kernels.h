@@ -112,6 +112,17 @@ struct PromptBytes {
 };
 PromptBytes prompt_bytes(int M, int K, const int *N, int count, int C);  // of a call
 bool prompt_supported(int bits, int M, int K, int N, int C, int G);
+// a call's two launches: the activations in operand order (scratch: one copy a layer), and the products.  The first may be
+// formed by the operation in front instead, row by row (prompt_rows_supported): residual + RMSNorm, SiLU * up.
+hipError_t launch_prompt_prep(int bits, const __half *x, const PromptMember *layers, int count, int M, int K, int C, const PromptPlan &plan,
+                              void *scratch, hipStream_t stream);
+bool prompt_rows_supported(int M, int K, int C);
+hipError_t launch_prompt_norm(int bits, __half *h, const __half *delta, const __half *weight, float eps, const PromptMember *layers, int count,
+                              int M, int K, int C, const PromptPlan &plan, void *scratch, hipStream_t stream);
+hipError_t launch_prompt_silu(int bits, const __half *gate, const __half *up, const PromptMember *layer, int M, int K, int C,
+                              const PromptPlan &plan, void *scratch, hipStream_t stream);
+hipError_t launch_prompt_product(int bits, const PromptMember *layers, int count, int M, int K, int C, int G, int accumulate,
+                                 const PromptPlan &plan, void *workspace, void *scratch, hipStream_t stream);
 hipError_t launch_prompt(int bits, const __half *vec, const PromptMember *layers, int count, int M, int K, int C, int G, int accumulate,
                          void *workspace, void *scratch, hipStream_t stream);
 

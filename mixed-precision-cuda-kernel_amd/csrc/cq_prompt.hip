@@ -213,6 +213,23 @@ PromptBytes prompt_bytes(int M, int K, const int *N, int count, int C) {
     return bytes;
 }
 
+// #{m : at(m) <= p} for non-decreasing at(0 .. C - 1); p is first + STEP lane (others: any answer).  A whole wavefront: it compares 64 values at a time
+// with the range of its positions, and only the few inside lane by lane (a search takes a round trip to LDS per halving: 3.6 us of
+// 10 in prompt_norm_kernel).
+template <int STEP, typename At>
+__device__ __forceinline__ int count_upto(At at, int C, int first, int p) {
+    const int lane = threadIdx.x & 63;
+    int n = 0;
+#pragma unroll 4
+    for (int k = 0; k < C; k += 64) {
+        const int v = k + lane < C ? at(k + lane) : 0x7fffffff;
+        n += __popcll(__ballot(v <= first));
+        for (unsigned long long in = __ballot(v > first && v <= first + 63 * STEP); in; in &= in - 1)
+            n += __builtin_amdgcn_readlane(v, __builtin_ctzll(in)) <= p ? 1 : 0;
+    }
+    return n;
+}
+
 // ---- activation preparation ------------------------------------------------------------------------
 // a[(step * m16 + tile) * 64 + lane], lane = (q, i): x[16 tile + i][positions 32 step + 8 q + ord[0..7]].  A workgroup
 // takes one unit (4 steps) of 16 rows: the unit's dense columns are a contiguous range, loaded in whole lines
@@ -223,7 +240,6 @@ PromptBytes prompt_bytes(int M, int K, const int *N, int count, int C) {
 // (The two staged chunks are two variables: as an array the compiler keeps them in LDS, addressed through the dispatch
 // packet in host memory, and the launch takes 18 us.)
 constexpr int kPrepCols = 256;     // dense columns of a unit that are staged; a wider range is gathered from memory
-constexpr int kPrepIdx = 1024;     // cherry channels staged
 struct PromptIndices {
     const int16_t *of[kPromptMaxGroup];
 };
@@ -231,7 +247,6 @@ template <int BITS>
 __global__ __launch_bounds__(256) void prompt_prep_kernel(const __half *__restrict__ x, PromptIndices indices, uint4 *__restrict__ a,
                                                           size_t a_bytes, int M, int K, int C, int units, int m16, int wide) {
     __shared__ __attribute__((aligned(16))) uint16_t s_x[16][kPrepCols + 8];
-    __shared__ int16_t s_idx[kPrepIdx];
     __shared__ __attribute__((aligned(16))) uint16_t s_off[kUnitK];
     const int t = threadIdx.x, lane = t & 63, q = lane >> 4, i = lane & 15, tile = blockIdx.y, Kn = K - C;
     const int row = 16 * tile + i, layer = blockIdx.z;
@@ -264,19 +279,11 @@ __global__ __launch_bounds__(256) void prompt_prep_kernel(const __half *__restri
         const bool chunk = near && sch < ceil_div(k1 - k0 + C, 8);
         if (chunk && sr < M) v0 = *reinterpret_cast<const u32x4 *>(x + (size_t)sr * K + k0 + 8 * sch);
         if (chunk && sr + 8 < M) v1 = *reinterpret_cast<const u32x4 *>(x + (size_t)(sr + 8) * K + k0 + 8 * sch);
-        if (C <= kPrepIdx) {
-#pragma unroll 1
-            for (int m = t; m < C; m += 256) s_idx[m] = cherry_indices[m];
-        }
+        // the offsets of the unit's positions, once for all rows, by two wavefronts (past Kn: not used)
+        if (t < kUnitK) s_off[t] = (uint16_t)count_upto<1>([&](int m) { return cherry_indices[m] - m; }, C, k0 + (t & ~63), k0 + t);
         if (chunk) {
             *reinterpret_cast<u32x4 *>(&s_x[t >> 5][8 * sch]) = v0;
             *reinterpret_cast<u32x4 *>(&s_x[(t >> 5) + 8][8 * sch]) = v1;
-        }
-        __syncthreads();
-        // the offsets of the unit's positions, once for all rows
-        if (t < kUnitK) {
-            const int k = min(k0 + t, Kn - 1);
-            s_off[t] = (uint16_t)(C <= kPrepIdx ? gather_offset(s_idx, C, k) : gather_offset(cherry_indices, C, k));
         }
         __syncthreads();
         int c0 = k0;
@@ -313,6 +320,134 @@ __global__ __launch_bounds__(256) void prompt_prep_kernel(const __half *__restri
     }
     a[((size_t)step * m16 + tile) * 64 + lane] =
         make_uint4(h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16);
+}
+
+// ---- preparation inside the operation in front (a prompt's layers) ---------------------------------------------
+// A workgroup owns a row: the operation leaves it in LDS, and from there every layer's operands are gathered, without the row's
+// way through memory, the launch and the wait for it (7B layer, 128 rows, us: RMSNorm and preparation for three layers
+// 4.8 + 5.0 -> 7.4, SiLU and preparation for one 4.3 + 5.0 -> 7.4, and the gap between two launches).  Bound by the chain of loads,
+// sums and 16-byte stores.  The 16 rows that share 256-byte pieces of the operands run on one die, whose L2 joins the stores.
+constexpr int kPromptRowThreads = 1024;
+constexpr int kPromptRowMax = 28672, kPromptRowCherries = 248;  // counts of adjacent channels fit a byte; a row fits 64 KB of LDS
+
+__device__ __forceinline__ int prompt_row(int m16) {  // of a grid of 128 ceil(m16 / 8); past the last one: none
+    const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3, tile = j / 16 * 8 + xcd;
+    return tile < m16 ? 16 * tile + j % 16 : -1;
+}
+
+// channels[m] - m of a layer: non-decreasing, and normal position p reads channel p + #{m: channels[m] - m <= p}
+__device__ __forceinline__ void stage_channels(const int16_t *__restrict__ channels, uint16_t *s_pos, int C) {
+    for (int m = threadIdx.x; m < C; m += kPromptRowThreads) s_pos[m] = (uint16_t)(channels[m] - m);
+}
+
+template <int BITS>
+__device__ __forceinline__ void row_operands(const uint16_t *s_row, const uint16_t *s_pos, uint4 *__restrict__ a, int Kn, int C, int units,
+                                             int csteps, int m16, int row, bool live) {
+    a += (row >> 4) * 64 + (row & 15);
+    const int total = units * 16 + csteps * 4;
+    for (int o = threadIdx.x; o - (int)(threadIdx.x & 63) < total; o += kPromptRowThreads) {  // whole wavefronts
+        const bool cherry = o >= units * 16;
+        const int p = 8 * (cherry ? o - units * 16 : o);
+        // normal position p + e reads channel p + e + m + byte e of `more`
+        int m = 0;
+        unsigned long long more = 0;
+        const int first = 8 * (o - (int)(threadIdx.x & 63));
+        for (int k = 0; live && k < C; k += 64) {
+            const int lane = threadIdx.x & 63, pos = k + lane < C ? s_pos[k + lane] : 0x7fffffff;
+            m += __popcll(__ballot(pos <= first));
+            for (unsigned long long in = __ballot(pos > first && pos <= first + 511); in; in &= in - 1) {
+                const int d = __builtin_amdgcn_readlane(pos, __builtin_ctzll(in)) - p;
+                m += d <= 0 ? 1 : 0;
+                more += (unsigned)d - 1u < 7u ? 0x0101010101010101ull << (8 * d) : 0ull;
+            }
+        }
+        unsigned short v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = 0;
+        if (live && p < (cherry ? C : Kn)) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const int f = prompt_ord<BITS>(e);
+                v[e] = s_row[cherry ? s_pos[p + e] + p + e : p + f + m + (int)(more >> (8 * f) & 255u)];
+            }
+        }
+        if (o < total)
+            a[((size_t)(o >> 2) * m16) * 64 + (o & 3) * 16] = make_uint4(v[0] | v[1] << 16, v[2] | v[3] << 16, v[4] | v[5] << 16, v[6] | v[7] << 16);
+    }
+}
+
+// h <- h + delta (none: as it is);  weight * fp16(h * rsqrt(mean(h^2) + eps)) in operand order for up to three layers.  K <= 8192.
+template <int BITS>
+__global__ __launch_bounds__(kPromptRowThreads) void prompt_norm_kernel(__half *__restrict__ h, const __half *__restrict__ delta,
+                                                                        const __half *__restrict__ weight, float eps, PromptIndices indices,
+                                                                        int count, uint4 *__restrict__ a, size_t a_bytes, int M, int K, int C,
+                                                                        int units, int csteps, int m16) {
+#pragma clang fp contract(off)
+    extern __shared__ __attribute__((aligned(16))) uint16_t s_norm[];
+    __shared__ float s_part[kPromptRowThreads / 64];
+    uint16_t *const s_row = s_norm, *const s_pos = s_norm + K;
+    const int row = prompt_row(m16), t = threadIdx.x;
+    if (row < 0) return;
+    const bool live = row < M;
+    half8_t v = {}, w = {};
+    float ss = 0.f;
+    const size_t at = (size_t)row * K + 8 * t;
+    const bool mine = live && 8 * t < K;
+    if (mine) {
+        v = *reinterpret_cast<const half8_t *>(h + at);
+        w = *reinterpret_cast<const half8_t *>(weight + 8 * t);
+        if (delta) {
+            v += *reinterpret_cast<const half8_t *>(delta + at);
+            *reinterpret_cast<half8_t *>(h + at) = v;
+        }
+    }
+    for (int l = 0; l < count; l++) stage_channels(l == 0 ? indices.of[0] : l == 1 ? indices.of[1] : indices.of[2], s_pos + l * C, C);
+#pragma unroll
+    for (int e = 0; e < 8; e++) ss += (float)v[e] * (float)v[e];
+    ss = wave_sum_all(ss);
+    if ((t & 63) == 0) s_part[t >> 6] = ss;
+    __syncthreads();
+    ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < kPromptRowThreads / 64; i++) ss += s_part[i];
+    const float rs = rsqrtf(ss / (float)K + eps);
+    if (mine) {
+        half8_t o;
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[e] = w[e] * (_Float16)((float)v[e] * rs);
+        *reinterpret_cast<half8_t *>(s_row + 8 * t) = o;
+    }
+    __syncthreads();
+    for (int l = 0; l < count; l++)
+        row_operands<BITS>(s_row, s_pos + l * C, a + l * (a_bytes / sizeof(uint4)), K - C, C, units, csteps, m16, row, live);
+}
+
+// fp16(silu(gate)) * up in operand order
+template <int BITS>
+__global__ __launch_bounds__(kPromptRowThreads) void prompt_silu_kernel(const __half *__restrict__ gate, const __half *__restrict__ up,
+                                                                        PromptIndices indices, uint4 *__restrict__ a, size_t a_bytes, int M,
+                                                                        int K, int C, int units, int csteps, int m16) {
+    extern __shared__ __attribute__((aligned(16))) uint16_t s_silu[];
+    uint16_t *const s_row = s_silu, *const s_pos = s_silu + K;
+    const int row = prompt_row(m16);
+    if (row < 0) return;
+    const bool live = row < M;
+    if (live) {
+        for (int i = 8 * threadIdx.x; i < K; i += 8 * kPromptRowThreads) {
+            const half8_t g = *reinterpret_cast<const half8_t *>(gate + (size_t)row * K + i);
+            const half8_t u = *reinterpret_cast<const half8_t *>(up + (size_t)row * K + i);
+            half8_t o;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float x = (float)g[e];
+                o[e] = (_Float16)((float)(_Float16)(x / (1.f + __expf(-x))) * (float)u[e]);
+            }
+            *reinterpret_cast<half8_t *>(s_row + i) = o;
+        }
+    }
+    stage_channels(indices.of[0], s_pos, C);
+    __syncthreads();
+    row_operands<BITS>(s_row, s_pos, a, K - C, C, units, csteps, m16, row, live);
 }
 
 // ---- main kernel -----------------------------------------------------------------------------------
@@ -764,24 +899,19 @@ bool prompt_supported(int bits, int M, int K, int N, int C, int G) {
 }
 
 template <int BITS, int MT, int NC, int WM, int WK, int S, int AS, int NP, int D>
-static hipError_t launch_prompt_mt(const __half *vec, const PromptMember *layers, int count, int M, int K, int C, int G, int accumulate,
-                                   const PromptPlan &plan, void *workspace, void *scratch, hipStream_t stream) {
-    u32x4 *a = reinterpret_cast<u32x4 *>(scratch);
+static hipError_t launch_product(const PromptMember *layers, int count, int M, int K, int C, int G, int accumulate, const PromptPlan &plan,
+                                 void *workspace, void *scratch, hipStream_t stream) {
+    const u32x4 *a = reinterpret_cast<const u32x4 *>(scratch);
     float *partial = reinterpret_cast<float *>(reinterpret_cast<char *>(scratch) + count * plan.a_bytes);
     unsigned *tickets = reinterpret_cast<unsigned *>(workspace);
-    PromptIndices indices;
     PromptMembers members;
     int first = 0;
     for (int i = 0; i < kPromptMaxGroup; i++) {
         const PromptMember &l = layers[i < count ? i : 0];
-        indices.of[i] = l.cherry_indices;
         members.qweight[i] = l.qweight, members.cherry_weight[i] = l.cherry_weight, members.scales[i] = l.scales, members.out[i] = l.out;
         members.N[i] = l.N, members.first[i] = first;
         if (i < count) first += ceil_div(l.N, 16 * NC);
     }
-    const int m16 = plan.mtiles * plan.mt;
-    hipLaunchKernelGGL(prompt_prep_kernel<BITS>, dim3(plan.units + ceil_div(plan.csteps, 4), m16, count), dim3(256), 0, stream, vec, indices,
-                       reinterpret_cast<uint4 *>(a), plan.a_bytes, M, K, C, plan.units, m16, aligned(vec, 16) ? 1 : 0);
     const dim3 grid(8 * ceil_div(plan.mtiles * plan.ntiles * plan.splits, 8));
     auto *const kernel =
         G % kUnitK == 0 ? prompt_kernel<BITS, MT, NC, WM, WK, S, AS, NP, D, true> : prompt_kernel<BITS, MT, NC, WM, WK, S, AS, NP, D, false>;
@@ -792,18 +922,56 @@ static hipError_t launch_prompt_mt(const __half *vec, const PromptMember *layers
 }
 
 template <int BITS>
-static hipError_t launch_prompt_bits(const __half *vec, const PromptMember *layers, int count, int M, int K, int C, int G, int accumulate,
-                                     void *workspace, void *scratch, hipStream_t stream) {
-    int N[kPromptMaxGroup];
-    for (int i = 0; i < count; i++) N[i] = layers[i].N;
-    const PromptPlan plan = prompt_plan(M, K, N, count, C);
-#define CQ_PROMPT(ID, MT, NC, WM, WK, S, AS, NP, D)                                                                         \
-    case ID:                                                                                                                \
-        return launch_prompt_mt<BITS, MT, NC, WM, WK, S, AS, NP, D>(vec, layers, count, M, K, C, G, accumulate, plan, workspace, scratch, \
-                                                                    stream);
+static hipError_t launch_product_bits(const PromptMember *layers, int count, int M, int K, int C, int G, int accumulate,
+                                      const PromptPlan &plan, void *workspace, void *scratch, hipStream_t stream) {
+#define CQ_PROMPT(ID, MT, NC, WM, WK, S, AS, NP, D) \
+    case ID:                                        \
+        return launch_product<BITS, MT, NC, WM, WK, S, AS, NP, D>(layers, count, M, K, C, G, accumulate, plan, workspace, scratch, stream);
     switch (plan.shape) { CQ_PROMPT_SHAPES(CQ_PROMPT) }
 #undef CQ_PROMPT
     return hipErrorInvalidConfiguration;
+}
+
+hipError_t launch_prompt_product(int bits, const PromptMember *layers, int count, int M, int K, int C, int G, int accumulate,
+                                 const PromptPlan &plan, void *workspace, void *scratch, hipStream_t stream) {
+    return bits == 4 ? launch_product_bits<4>(layers, count, M, K, C, G, accumulate, plan, workspace, scratch, stream)
+                     : launch_product_bits<3>(layers, count, M, K, C, G, accumulate, plan, workspace, scratch, stream);
+}
+
+static PromptIndices indices_of(const PromptMember *layers, int count) {
+    PromptIndices indices;
+    for (int i = 0; i < kPromptMaxGroup; i++) indices.of[i] = layers[i < count ? i : 0].cherry_indices;
+    return indices;
+}
+
+// x in operand order for every layer of a group, in front of launch_prompt_product
+hipError_t launch_prompt_prep(int bits, const __half *x, const PromptMember *layers, int count, int M, int K, int C, const PromptPlan &plan,
+                              void *scratch, hipStream_t stream) {
+    const int m16 = plan.mtiles * plan.mt;
+    hipLaunchKernelGGL(bits == 4 ? prompt_prep_kernel<4> : prompt_prep_kernel<3>, dim3(plan.units + ceil_div(plan.csteps, 4), m16, count),
+                       dim3(256), 0, stream, x, indices_of(layers, count), reinterpret_cast<uint4 *>(scratch), plan.a_bytes, M, K, C,
+                       plan.units, m16, aligned(x, 16) ? 1 : 0);
+    return hipGetLastError();
+}
+
+bool prompt_rows_supported(int M, int K, int C) { return K % 8 == 0 && K <= kPromptRowMax && C <= kPromptRowCherries && M <= prompt_max_rows(K, C); }
+
+hipError_t launch_prompt_norm(int bits, __half *h, const __half *delta, const __half *weight, float eps, const PromptMember *layers, int count,
+                              int M, int K, int C, const PromptPlan &plan, void *scratch, hipStream_t stream) {
+    const int m16 = plan.mtiles * plan.mt;
+    hipLaunchKernelGGL(bits == 4 ? prompt_norm_kernel<4> : prompt_norm_kernel<3>, dim3(128 * ceil_div(m16, 8)), dim3(kPromptRowThreads),
+                       2 * (K + count * C), stream, h, delta, weight, eps, indices_of(layers, count), count, reinterpret_cast<uint4 *>(scratch),
+                       plan.a_bytes, M, K, C, plan.units, plan.csteps, m16);
+    return hipGetLastError();
+}
+
+hipError_t launch_prompt_silu(int bits, const __half *gate, const __half *up, const PromptMember *layer, int M, int K, int C,
+                              const PromptPlan &plan, void *scratch, hipStream_t stream) {
+    const int m16 = plan.mtiles * plan.mt;
+    hipLaunchKernelGGL(bits == 4 ? prompt_silu_kernel<4> : prompt_silu_kernel<3>, dim3(128 * ceil_div(m16, 8)), dim3(kPromptRowThreads),
+                       2 * (K + C), stream, gate, up, indices_of(layer, 1), reinterpret_cast<uint4 *>(scratch), plan.a_bytes, M, K, C,
+                       plan.units, plan.csteps, m16);
+    return hipGetLastError();
 }
 
 hipError_t launch_prompt(int bits, const __half *vec, const PromptMember *layers, int count, int M, int K, int C, int G, int accumulate,
@@ -816,8 +984,11 @@ hipError_t launch_prompt(int bits, const __half *vec, const PromptMember *layers
         for (int i = 0; i < count; i++) range[i] = layers[i], range[i].out += (size_t)m0 * layers[i].N;
         const __half *const x = vec + (size_t)m0 * K;
         const int rows = min(most, M - m0);
-        const hipError_t e = bits == 4 ? launch_prompt_bits<4>(x, range, count, rows, K, C, G, accumulate, workspace, scratch, stream)
-                                       : launch_prompt_bits<3>(x, range, count, rows, K, C, G, accumulate, workspace, scratch, stream);
+        int N[kPromptMaxGroup];
+        for (int i = 0; i < count; i++) N[i] = layers[i].N;
+        const PromptPlan plan = prompt_plan(rows, K, N, count, C);
+        hipError_t e = launch_prompt_prep(bits, x, range, count, rows, K, C, plan, scratch, stream);
+        if (e == hipSuccess) e = launch_prompt_product(bits, range, count, rows, K, C, G, accumulate, plan, workspace, scratch, stream);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

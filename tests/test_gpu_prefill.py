@@ -284,3 +284,39 @@ def test_prefill_of_a_decoder_with_cast_norms(dec, dtype):
     want = models[0].prefill(ids).double().cpu()
     # normalised rows in another dtype, rounded to fp16 by the 14 products that read them
     assert rel(models[1].prefill(ids), want) < 14 * 2 ** -11
+
+
+@pytest.mark.parametrize("bits,heads,kv,inter,tokens,cherries", [(4, 2, 1, 520, 17, "adjacent"), (3, 3, 3, 1032, 33, "random"),
+                                                                 (4, 8, 2, 2824, 130, "ends"), (3, 2, 2, 264, 70, "none")])
+def test_layers_in_one_call_against_single_calls(dec, bits, heads, kv, inter, tokens, cherries):
+    """The native call over all layers against the same layers module by module (a hook sends them there): products of the same
+    kernels, a RMSNorm whose sum runs in another order."""
+    print("[case] prefill layers", bits, heads, kv, inter, tokens, cherries, flush=True)
+    cfg = dec.DecoderConfig(hidden_size=128 * heads, intermediate_size=inter, num_hidden_layers=2, num_attention_heads=heads,
+                            num_key_value_heads=kv, vocab_size=512, max_position_embeddings=160, w_bits=bits,
+                            cherry_fraction=0.0 if cherries == "none" else 1 / 16)
+    model = dec.CherryLlamaDecoder(cfg, seed=5)
+    for m in model.modules():
+        if hasattr(m, "cherry_indices") and m.num_cherries:
+            k, c = m.in_features, m.num_cherries
+            if cherries == "adjacent":
+                m.cherry_indices.copy_(torch.arange(37, 37 + c))
+            elif cherries == "ends":
+                m.cherry_indices.copy_(torch.cat([torch.arange(c // 2), torch.arange(k - c + c // 2, k)]))
+    ids = torch.randint(0, 512, (tokens,), device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    called = []
+    native = dec._lib.cherryq_prefill_layers_f16
+    try:
+        dec._lib.cherryq_prefill_layers_f16 = lambda *a: called.append(0) or native(*a)
+        got = model.prefill(ids).clone(), model.k_cache.clone(), model.v_cache.clone()
+        assert len(called) == 1
+        hook = model.layers[0].q_proj.register_forward_hook(lambda *a: None)
+        want = model.prefill(ids).clone(), model.k_cache.clone(), model.v_cache.clone()
+        hook.remove()
+        assert len(called) == 1
+    finally:
+        dec._lib.cherryq_prefill_layers_f16 = native
+    for a, b in zip(got, want):
+        # 14 products' results and two norms' rounded to fp16, any of them to the neighbouring value
+        assert rel(a, b.double().cpu()) < 16 * 2 ** -11
+    assert model.pos.item() == tokens

@@ -226,3 +226,42 @@ def test_another_torch_needs_another_host_library(monkeypatch, tmp_path):
     assert build.needs_build()
     monkeypatch.setattr(torch, "__version__", version[:-1])
     assert build.needs_build()
+
+
+def test_descriptions_of_plain_modules_only(host):
+    """What the whole-prompt call is told of a product's modules, and which modules are left to their own calls."""
+    import cherryq_decoder as dec
+    from llama.qlinear import QuantLinear
+    from llama.quantizer import FullSymQuantizer
+    module = host[0]
+
+    def describe(*mods, rows=40, cls=QuantLinear):
+        product, held = dec._PrefillProduct(), []
+        ok = module.describe(ctypes.addressof(product), rows, -1, cls, held, *mods)
+        return (product, held) if ok else None
+
+    mods = [layer(), layer(), layer()]
+    for n in (1, 2, 3):
+        product, held = describe(*mods[:n])
+        assert (product.n_layers, product.w_bits, product.in_features, product.group_size) == (n, 4, K, 128)
+        assert product.num_cherries == mods[0].num_cherries and len(held) == 4 * n
+        for w, m in zip(product.layers, mods[:n]):
+            assert (w.qweight, w.scales, w.cherry_weight, w.cherry_indices, w.out_features) == (
+                m.qweight.data_ptr(), m.scales.data_ptr(), m.cherry_weight.data_ptr(), m.cherry_indices.data_ptr(), N)
+        assert any(t is mods[0].qweight for t in held)
+    assert describe(mods[0], rows=QuantLinear.prefill_rows) is None
+    assert describe(mods[0], layer(bias=True)) is None
+    assert describe(mods[0], torch.nn.Linear(K, N)) is None and describe(mods[0], None) is None
+    assert describe(type("Own", (QuantLinear,), {})(4, 128, FullSymQuantizer, 1 / 16, K, N, bias=False)) is None
+    assert describe(QuantLinear(3, 128, FullSymQuantizer, 1 / 16, K, N, bias=False), mods[0]) is None  # not of one kind
+    for change in (lambda q: q.register_forward_hook(lambda *a: None), lambda q: q.register_forward_pre_hook(lambda *a: None),
+                   lambda q: setattr(q, "forward", lambda x: x), lambda q: setattr(q, "dequantized", True),
+                   lambda q: setattr(q, "_released", True), lambda q: setattr(q, "bias", torch.nn.Parameter(torch.zeros(N))),
+                   lambda q: setattr(q, "scales", q.scales.float()), lambda q: setattr(q, "qweight", q.qweight[:-1]),
+                   lambda q: setattr(q, "cherry_weight", q.cherry_weight.t().contiguous().t())):
+        q = layer()
+        assert describe(q) is not None
+        change(q)
+        assert describe(q) is None
+    with QuantLinear.dmode(False):
+        assert describe(mods[0]) is None
