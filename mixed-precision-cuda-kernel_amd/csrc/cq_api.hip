@@ -113,11 +113,10 @@ static int matmul_f16(const void *vec, const uint8_t *qweight, const void *cherr
         e = launch_matvec(BITS, x, qweight, cw, cherry_indices, sc, y, K, N, C, G, accumulate, workspace, s);
     } else if (!force_generic() && matvec_rows_preferred(BITS, B, K, N, C, G)) {
         e = launch_matvec_rows(BITS, x, qweight, cw, cherry_indices, sc, y, B, K, N, C, G, accumulate, workspace, s);
-    } else if (!force_generic() && B < kPromptMinRows && batch_supported(BITS, B, K, N, C, G)) {
-        // up to a tile's 16 rows: half of the prompt kernel's smallest tile would be padding
+    } else if (!force_generic() && B < kPromptMinRows && batch_supported(BITS, B, K, N, C, G) &&
+               !(prompt_supported(BITS, B, K, N, C, G) && prompt_preferred(BITS, B, K, N, C))) {
         e = launch_batch(BITS, x, qweight, cw, cherry_indices, sc, y, B, K, N, C, G, accumulate, workspace, scratch, s);
     } else if (!force_generic() && B >= 2 && prompt_supported(BITS, B, K, N, C, G)) {
-        // ... unless the group is no whole number of the batch kernel's units of 128 positions
         const PromptMember layer = {qweight, cw, cherry_indices, sc, y, N};
         e = launch_prompt(BITS, x, &layer, 1, B, K, C, G, accumulate, workspace, scratch, s);
     } else {

@@ -84,7 +84,7 @@ hipError_t launch_batch(int bits, const __half *vec, const uint8_t *qweight, con
 size_t scratch_bytes(int B, int K, int N, int C);
 
 // cq_prompt.hip: more than 16 rows (prompt processing) -- wavefronts that decode weights into LDS and wavefronts of fp16 MFMAs.
-constexpr int kPromptMinRows = 17;  // fewer rows go through the 16-row kernel
+constexpr int kPromptMinRows = 17;  // fewer rows may go through the 16-row kernel
 constexpr int kPromptMaxSplits = 16;
 struct PromptPlan {
     int shape;                        // the tile shape, by its place in the kernel's table
@@ -95,6 +95,7 @@ struct PromptPlan {
     size_t workspace_bytes;           // zero-kept: one ticket per output tile
     size_t a_bytes, partial_bytes;    // scratch: activations in operand order, then the per-split partial tiles
     size_t scratch_bytes;
+    float cost;                       // about what the call takes, us
 };
 constexpr int kPromptMaxGroup = 3;
 struct PromptMember {  // a layer of a launch: all read the same activations and have the same K, C and group size
@@ -112,6 +113,7 @@ struct PromptBytes {
 };
 PromptBytes prompt_bytes(int M, int K, const int *N, int count, int C);  // of a call
 bool prompt_supported(int bits, int M, int K, int N, int C, int G);
+bool prompt_preferred(int bits, int M, int K, int N, int C);  // to the 16-row kernel, up to 16 rows
 // a call's two launches: the activations in operand order (scratch: one copy a layer), and the products.  The first may be
 // formed by the operation in front instead, row by row (prompt_rows_supported): residual + RMSNorm, SiLU * up.
 hipError_t launch_prompt_prep(int bits, const __half *x, const PromptMember *layers, int count, int M, int K, int C, const PromptPlan &plan,

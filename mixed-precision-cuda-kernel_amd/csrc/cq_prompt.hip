@@ -94,10 +94,12 @@ static_assert(prompt_ord<4>(1) == 2 && prompt_ord<4>(2) == 1 && prompt_ord<4>(5)
     X(8, 3, 8, 4, 1, 4, 4, 4, 2) \
     X(9, 4, 8, 4, 1, 4, 4, 4, 2) \
     X(10, 2, 4, 1, 4, 2, 4, 4, 3) \
-    X(11, 3, 4, 1, 4, 2, 4, 4, 2)
+    X(11, 3, 4, 1, 4, 2, 4, 4, 2) \
+    X(12, 1, 4, 1, 4, 2, 4, 8, 3) \
+    X(13, 1, 4, 1, 4, 2, 4, 4, 3)
 
-// What a call takes with a tile shape, in microseconds, preparation included: a fit to 37000 measured calls (3 and 4 bits, K 1024
-// to 28672, N 512 to 28672, M 17 to 2048, 1 to 16 K splits).  `first`: a launch with one round of workgroups and no unit; `round`:
+// What a call takes with a tile shape, in microseconds, preparation included: a fit to 43000 measured calls (3 and 4 bits, K 1024
+// to 28672, N 512 to 28672, M 4 to 2048, 1 to 16 K splits).  `first`: a launch with one round of workgroups and no unit; `round`:
 // each further round; `unit`: 128 positions a K share, 1 + crowd times as long when all compute units are at it; `split`,
 // `mbyte`, `tile`: a split call, each megabyte of its partial tiles, and each 32 KB that its last workgroup reads; `rows`:
 // 1e6 M K.  Its choices are 0.3 % slower than the best measured ones on average, 5 % at the 99th percentile.
@@ -119,6 +121,8 @@ constexpr PromptCost kPromptCosts[] = {
     {5, 10.76f, 7.50f, 1.12f, 0.276f, 2.16f, 0.379f, 0.839f, 0.563f},  // 256 x 128
     {6, 6.19f, 0.538f, 1.27f, 0.835f, 1.14f, 0.324f, 1.92f, 0.942f},  // 32 x 64, two a compute unit
     {6, 6.54f, 0.366f, 1.40f, 0.911f, 0.909f, 0.465f, 2.11f, 0.985f},  // 48 x 64, two a compute unit
+    {5, 6.15f, 1.94f, 0.996f, 0.076f, 0.703f, 0.955f, 1.59f, 2.11f},  // 16 x 64
+    {6, 5.86f, 0.945f, 1.10f, 0.843f, 0.995f, 0.555f, 2.19f, 2.14f},  // 16 x 64, two a compute unit
 };
 struct PromptShape {
     int mt, nc, wm, wk;
@@ -160,9 +164,9 @@ static PromptPlan find_prompt_plan(int M, int K, const int *N, int count, int C)
         const PromptCost &f = kPromptCosts[id];
         PromptPlan p = {};
         p.shape = id, p.mt = s.mt * s.wm, p.nc = s.nc, p.ns = 1;
-        if (id > 0 && M <= 8 * p.mt) continue;  // half of every tile would be padding
+        if (p.mt > 1 ? M <= 8 * p.mt : M > 16) continue;  // half of every tile would be padding; 16 rows: up to one tile
         p.mtiles = ceil_div(M, 16 * p.mt);
-        if (id > 0 && (p.mtiles * p.mt > 65535 || steps * p.mtiles * p.mt > 0x7fff0000ll / 1024)) continue;
+        if (p.mt != 2 && (p.mtiles * p.mt > 65535 || steps * p.mtiles * p.mt > 0x7fff0000ll / 1024)) continue;
         p.ntiles = 0;
         for (int i = 0; i < count; i++) p.ntiles += ceil_div(N[i], 16 * s.nc);
         const long long tiles = (long long)p.mtiles * p.ntiles;
@@ -179,6 +183,7 @@ static PromptPlan find_prompt_plan(int M, int K, const int *N, int count, int C)
             float cost = f.first + f.round * (float)(full + (rest > 0) - 1) + f.rows * 1e-6f * (float)M * (float)K +
                          f.unit * (float)ceil_div(p.units_per_split, s.wk) * ((float)full * (1.f + f.crowd) + (rest > 0 ? 1.f + crowd : 0.f));
             if (splits > 1) cost += f.split + f.mbyte * (float)(tiles * splits) * kbytes * 1.024e-3f + f.tile * splits * kbytes / 32.f;
+            p.cost = cost;
             if (cost < best_cost) best_cost = cost, best = p;
         }
     }
@@ -490,10 +495,12 @@ struct PromptColumn {
             uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(half2_t, f[d]), (half2_t){(_Float16)ma, (_Float16)mb},
                                                 (half2_t){(_Float16)(-(1024.f * ma + grid)), (_Float16)(-(1024.f * mb + grid))}));
     }
-    __device__ __forceinline__ uint32_t scaled(int d) const {
-        return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, y[d]) * __builtin_bit_cast(half2_t, s2));
+    template <bool SCALED>
+    __device__ __forceinline__ uint32_t operand(int d) const {
+        return !SCALED ? y[d] : __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, y[d]) * __builtin_bit_cast(half2_t, s2));
     }
     // w: the byte rows' dwords that hold the column in byte c; scale: the dword with its scale in half c & 1
+    template <bool SCALED>
     __device__ __forceinline__ void group(const PromptDecode<BITS> &k, int g, const uint32_t (&w)[BITS], int c, uint32_t scale,
                                           u32x4 &o) {
         switch (g) {
@@ -513,14 +520,14 @@ struct PromptColumn {
                 if (BITS == 4) t[1] = p[1] << 1;
                 break;
             case 2:
-                s2 = __builtin_amdgcn_perm(scale, scale, (c & 1) ? 0x03020302u : 0x01000100u);
+                if (SCALED) s2 = __builtin_amdgcn_perm(scale, scale, (c & 1) ? 0x03020302u : 0x01000100u);
                 pair(k, 0);
                 break;
             case 3: pair(k, 1), centre(0); break;
-            case 4: pair(k, 2), centre(1), o[0] = scaled(0); break;
-            case 5: pair(k, 3), centre(2), o[1] = scaled(1); break;
-            case 6: centre(3), o[2] = scaled(2); break;
-            default: o[3] = scaled(3); break;
+            case 4: pair(k, 2), centre(1), o[0] = operand<SCALED>(0); break;
+            case 5: pair(k, 3), centre(2), o[1] = operand<SCALED>(1); break;
+            case 6: centre(3), o[2] = operand<SCALED>(2); break;
+            default: o[3] = operand<SCALED>(3); break;
         }
     }
 };
@@ -529,6 +536,9 @@ struct PromptColumn {
 // spills accumulators.)  Its result is next read 16 products later at the earliest, or behind mfma_drain().
 __device__ __forceinline__ void prompt_mfma(float4_t &acc, const u32x4 &a, const u32x4 &b) {
     asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void prompt_mfma_first(float4_t &acc, const u32x4 &a, const u32x4 &b) {
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
 }
 __device__ __forceinline__ void mfma_drain() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
 
@@ -565,7 +575,8 @@ struct PromptPiece {
     }
 };
 
-// WHOLE: groups are whole units
+// WHOLE: groups are whole units.  Then a tile of 16 rows takes codes u - c_b as operands and scales a stage's sums, in fp32: 16
+// multiplications for 64 in the decode, and no rounding of the weights.
 template <int BITS, int MT, int NC, int WM, int WK, int S, int AS, int NP, int D, bool WHOLE>
 __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(PromptMembers members, const u32x4 *__restrict__ a_all,
                                                               float *__restrict__ partial, unsigned *__restrict__ tickets, int M,
@@ -573,10 +584,13 @@ __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(Pro
     static_assert(WM * WK == 4 && S * WK % NP == 0 && NP % WK == 0 && (AS % S == 0 || S % AS == 0) && (AS <= S || AS / S * S == 4), "");
     typedef typename PromptPiece<NC>::w_t w_t;
     typedef typename PromptPiece<NC>::s_t s_t;
+    constexpr bool SUMS = WHOLE && MT == 1;
+    static_assert(!SUMS || (NC == 4 && S == 2 && AS == 4), "");
     constexpr int COLS = 16 * NC, ROWS = 16 * MT * WM, PS = S * WK / NP, T = 256 + 64 * NP;
     constexpr int STAGE = WK * S * NC * 64;                        // operands of a stage, 16 bytes each
     constexpr int RED = MT * NC * 64 * 4;                          // four wavefronts' results
     __shared__ u32x4 s_b[2 * STAGE > RED ? 2 * STAGE : RED];
+    __shared__ u32x2 s_sc[SUMS ? 2 : 1][WK][16];  // a stage's scales: SUMS
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kq = lane >> 4, nl = lane & 15;
     const int tiles = plan.mtiles * plan.ntiles, piece = ((int)blockIdx.x & 7) * ((int)gridDim.x >> 3) + ((int)blockIdx.x >> 3);
     if (piece >= tiles * plan.splits) return;
@@ -651,6 +665,18 @@ __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(Pro
             b[c] = frag[c * 64];
             __builtin_amdgcn_sched_barrier(0);
         }
+        float4_t part[SUMS ? 2 : 1][NC];
+        u32x2 sc[2];
+        auto add_scaled = [&](int v) {  // the sums of a stage that ended at least four MFMAs ago
+            asm volatile("s_nop 7" : "+v"(part[v][0]), "+v"(part[v][1]), "+v"(part[v][NC / 2]), "+v"(part[v][NC - 1]));
+#pragma unroll
+            for (int c = 0; c < NC; c++) {
+                const float f = __half2float(__ushort_as_half((unsigned short)(sc[v][(c >> 1) & 1] >> (16 * (c & 1)))));
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[0][c][e] = __builtin_fmaf(f, part[v][c][e], acc[0][c][e]);
+            }
+        };
+        if constexpr (SUMS) sc[0] = s_sc[0][wk][nl];
         // Every operand is asked for again as soon as its products are issued: activations AS steps ahead, weights one.  A
         // stage's last step meets the producers once its own weights have arrived, and goes on with the next stage's.
         constexpr int MEET = NC > 2 ? 1 : 0, U = AS > S ? AS / S : 1;
@@ -667,7 +693,9 @@ __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(Pro
                     for (int c = 0; c < NC; c++) {
 #pragma unroll
                         for (int m = 0; m < MT; m++) {
-                            prompt_mfma(acc[m][c], a[set][m], b[c]);
+                            if constexpr (!SUMS) prompt_mfma(acc[m][c], a[set][m], b[c]);
+                            else if (s == 0) prompt_mfma_first(part[v][c], a[set][m], b[c]);
+                            else prompt_mfma(part[v][c], a[set][m], b[c]);
                             if (c == last) a[set][m] = load_step(m, (st + v) * S + s + AS);
                             __builtin_amdgcn_sched_barrier(0);
                         }
@@ -679,7 +707,12 @@ __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(Pro
                                 b[e] = next[e * 64];
                                 __builtin_amdgcn_sched_barrier(0);
                             }
+                            if constexpr (SUMS) sc[v ^ 1] = s_sc[v ^ 1][wk][nl];
                         } else if (c > MEET) b[c] = next[c * 64];
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    if constexpr (SUMS) {
+                        if (s == 0 && (v > 0 || st > 0)) add_scaled(v ^ 1);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
@@ -688,6 +721,7 @@ __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(Pro
         __builtin_amdgcn_s_setprio(0);
         __builtin_amdgcn_sched_barrier(0);
         mfma_drain();
+        if constexpr (SUMS) add_scaled(U - 1);
         __builtin_amdgcn_sched_barrier(0);
     } else {
         // ---- weights
@@ -721,6 +755,8 @@ __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(Pro
             __builtin_amdgcn_sched_barrier(0);
         };
         auto fill = [&](int d, int st) {
+            if constexpr (SUMS)
+                if (sub == 0 && kq == 0) s_sc[st & 1][wk][nl] = sc[d][0];
 #pragma unroll
             for (int i = 0; i < PS; i++)
 #pragma unroll
@@ -731,7 +767,7 @@ __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(Pro
 #pragma unroll
                     for (int r = 0; r < BITS; r++) codes[r] = w[d][i][r][c >> 2];
 #pragma unroll
-                    for (int g = 0; g < 8; g++) column.group(decoder, g, codes, c & 3, sc[d][WHOLE ? 0 : i][c >> 1], o);
+                    for (int g = 0; g < 8; g++) column.template group<!SUMS>(decoder, g, codes, c & 3, sc[d][WHOLE ? 0 : i][c >> 1], o);
                     frag[(st & 1) * STAGE + ((sub + NP / WK * i) * NC + c) * 64] = o;
                 }
         };
@@ -936,6 +972,18 @@ hipError_t launch_prompt_product(int bits, const PromptMember *layers, int count
                                  const PromptPlan &plan, void *workspace, void *scratch, hipStream_t stream) {
     return bits == 4 ? launch_product_bits<4>(layers, count, M, K, C, G, accumulate, plan, workspace, scratch, stream)
                      : launch_product_bits<3>(layers, count, M, K, C, G, accumulate, plan, workspace, scratch, stream);
+}
+
+// Small batches that the 16-row kernel (cq_batch.hip) takes as well.  What that takes, in us, as fitted to 4000 measured calls of 5 to
+// 16 rows (4 % off on average): its 16-row tiles reload the rows' operands for every unit and split K in memory, which costs
+// most on small layers; it streams the weights of large ones faster than operands can be decoded into LDS.  Of 2487 calls 80 %
+// come here and all together take 17 % less (16 rows, us: 4096 -> 4096 18.7 -> 11.1, 4096 -> 11008 19.5 -> 14.4, 5120 -> 13824 in 3 bits
+// 22.0 -> 16.2; 8192 -> 28672 stays at 40.8, here 44).
+bool prompt_preferred(int bits, int M, int K, int N, int C) {
+    const float mbytes = (float)K * (float)N * (float)bits * 0.125e-6f, m = (float)M;
+    if (mbytes > 64.f) return false;
+    const float batch = 8.73f + 0.436f * m + (0.266f + 0.0018f * m) * mbytes + 0.319e-4f * (float)N - 0.952e-5f * m * (float)N + 0.678e-5f * m * (float)K;
+    return prompt_plan(M, K, &N, 1, C).cost < batch;
 }
 
 static PromptIndices indices_of(const PromptMember *layers, int count) {

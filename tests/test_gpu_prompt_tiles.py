@@ -13,7 +13,7 @@ def qc():
 
 # rows around every tile height; columns off the tiles' 64 and 128; one unit of 128 positions, fewer than K shares, a ragged last
 # one; no cherries, a partial step of 32, several chunks of steps; groups of whole units, and not
-@pytest.mark.parametrize("rows", [17, 33, 48, 64, 81, 112, 113, 129, 193, 257, 520])
+@pytest.mark.parametrize("rows", [5, 16, 17, 33, 48, 64, 81, 112, 113, 129, 193, 257, 520])
 @pytest.mark.parametrize("bits,k,n,c,group", [(4, 128, 72, 0, 128), (3, 136, 64, 8, 32), (4, 520, 1032, 40, 160), (3, 1024, 264, 24, 96),
                                               (4, 1800, 2056, 520, 192), (3, 2560, 520, 296, 256), (4, 4096, 11008, 16, 128)])
 def test_rows_around_the_tiles(qc, bits, k, n, c, group, rows):
@@ -30,6 +30,8 @@ def test_rows_around_the_tiles(qc, bits, k, n, c, group, rows):
     ref = x.double() @ w
     # products are exact in fp32, k of them are added up (in any order) and the sum is rounded to fp16
     slack = k * 2.0 ** -24 * (x.double().abs() @ w.abs()) + 2.0 ** -25
+    if rows <= 16:  # the weights may go unrounded, then they differ from the dequantised ones by half a unit of theirs
+        slack = slack + 2.0 ** -11 * (x.double().abs() @ w.abs())
     for accumulate in (False, True):
         out = before.clone()
         qc.matmul_cherryq(bits, x, q, cw, idx, scales, out, group, accumulate=accumulate)
