@@ -84,21 +84,45 @@ __host__ __device__ constexpr int s3_bit(int q) {
 }
 
 // ---- prepack: reference buffers -> stream ------------------------------------------------------
+// header: for every compacted position k the number of cherry columns in front of it, low(k) (the
+// position reads activation column k + low(k); padding positions hold C and so read beyond the last
+// column, where the kernel keeps zeros), one byte
+// each, stored per block of 512 positions so that lane l of a wavefront finds the entries of
+// positions l, l + 64, ..., l + 448 in 8 consecutive bytes; then the cherry columns (uint16,
+// padded with K, the column the kernel keeps zero)
+// Bytes 256 block .. 256 block + 255 of the header: the gather table in the order of its readers, then the cherry columns.
+__device__ inline void stream_header(const int16_t *__restrict__ cherry_indices, uint8_t *__restrict__ hdr, int block,
+                                     const StreamGeo &geo) {
+    const int Knp512 = (geo.ng * kStreamUnitK + 511) & ~511, Cp = (geo.C + 31) & ~31;
+    const int i = block * 256 + threadIdx.x;
+    if (i < Knp512) {
+        const int blk = i >> 9, l = (i >> 3) & 63, j = i & 7;
+        const int k = blk * 512 + 64 * j + l;
+        hdr[i] = (uint8_t)(k < geo.Kn ? gather_offset(cherry_indices, geo.C, k) : geo.C);
+    } else if (i < Knp512 + Cp) {
+        const int m = i - Knp512;
+        reinterpret_cast<uint16_t *>(hdr + Knp512)[m] = (uint16_t)(m < geo.C ? (int)cherry_indices[m] : geo.K);
+    }
+    if (i >= Knp512 + 2 * Cp && i < (int)geo.hdr_bytes) hdr[i] = 0;  // padding of the header
+}
+
 // A workgroup rearranges one unit (128 positions) of 8 tiles (128 columns): its packed bytes are read 128 bytes a
 // row into LDS, where each lane of a tile collects the bytes of its column and stores its dwords; a tile's
 // wavefront writes the unit as one contiguous piece.  The last 8 blockIdx.y take the tiles' scales and
-// cherry rows.  Bound by HBM: the packed bytes once in, once out.  MI355X, 5120 -> 13824 in 3 bits: 16 us (3.5 TB/s
-// read + written); one workgroup a tile gathering single bytes from 16-byte runs took 192.
+// cherry rows; the first `heads` write the header, whose binary searches are a chain of loads that the rest hides (a
+// launch of its own was 4.9 us in front).  Bound by HBM: the packed bytes once in, once out.  MI355X, 5120 -> 13824 in
+// 3 bits: HDRUS us (3.5 TB/s read + written); one workgroup a tile gathering single bytes from 16-byte runs took 192.
 constexpr int kPackTiles = 8;
 
 template <int BITS>
 __global__ __launch_bounds__(256) void stream_pack_kernel(const uint8_t *__restrict__ qweight,
                                                           const __half *__restrict__ cherry_weight,
-                                                          const __half *__restrict__ scales,
-                                                          uint8_t *__restrict__ stream, int G, int dwords, StreamGeo geo) {
-    const int N = geo.N, Kn = geo.Kn, t = threadIdx.x;
-    if ((int)blockIdx.y >= geo.ng) {
-        const int tile = blockIdx.x * kPackTiles + (int)blockIdx.y - geo.ng;
+                                                          const __half *__restrict__ scales, const int16_t *__restrict__ cherry_indices,
+                                                          uint8_t *__restrict__ stream, int G, int dwords, int heads, StreamGeo geo) {
+    const int N = geo.N, Kn = geo.Kn, t = threadIdx.x, g = (int)blockIdx.y - heads;
+    if (g < 0) return stream_header(cherry_indices, stream, blockIdx.y * gridDim.x + blockIdx.x, geo);
+    if (g >= geo.ng) {
+        const int tile = blockIdx.x * kPackTiles + g - geo.ng;
         if (tile >= geo.ntiles) return;
         __half *rec = reinterpret_cast<__half *>(stream + geo.hdr_bytes + (size_t)tile * geo.record_bytes);
         const int cherry0 = (int)(geo.off_cherry / 2);
@@ -118,7 +142,7 @@ __global__ __launch_bounds__(256) void stream_pack_kernel(const uint8_t *__restr
     }
     constexpr int ROWS = 16 * BITS, STRIDE = 132, DW = BITS;  // bytes of LDS a row: 33 dwords
     __shared__ uint32_t s_q[ROWS * STRIDE / 4];
-    const int g = blockIdx.y, n0 = blockIdx.x * kPackTiles * 16, row0 = g * ROWS, rows = Kn / 8 * BITS;
+    const int n0 = blockIdx.x * kPackTiles * 16, row0 = g * ROWS, rows = Kn / 8 * BITS;
     for (int e = t; e < ROWS * 32; e += 256) {
         const int r = e >> 5, n = n0 + 4 * (e & 31);
         uint32_t v = 0;
@@ -222,27 +246,6 @@ __global__ __launch_bounds__(256) void stream_unpack_kernel(const uint8_t *__res
             }
         }
     }
-}
-
-// header: for every compacted position k the number of cherry columns in front of it, low(k) (the
-// position reads activation column k + low(k); padding positions hold C and so read beyond the last
-// column, where the kernel keeps zeros), one byte
-// each, stored per block of 512 positions so that lane l of a wavefront finds the entries of
-// positions l, l + 64, ..., l + 448 in 8 consecutive bytes; then the cherry columns (uint16,
-// padded with K, the column the kernel keeps zero)
-__global__ __launch_bounds__(256) void stream_header_kernel(const int16_t *__restrict__ cherry_indices,
-                                                            uint8_t *__restrict__ hdr, StreamGeo geo) {
-    const int Knp512 = (geo.ng * kStreamUnitK + 511) & ~511, Cp = (geo.C + 31) & ~31;
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < Knp512) {
-        const int blk = i >> 9, l = (i >> 3) & 63, j = i & 7;
-        const int k = blk * 512 + 64 * j + l;
-        hdr[i] = (uint8_t)(k < geo.Kn ? gather_offset(cherry_indices, geo.C, k) : geo.C);
-    } else if (i < Knp512 + Cp) {
-        const int m = i - Knp512;
-        reinterpret_cast<uint16_t *>(hdr + Knp512)[m] = (uint16_t)(m < geo.C ? (int)cherry_indices[m] : geo.K);
-    }
-    if (i >= Knp512 + 2 * Cp && i < (int)geo.hdr_bytes) hdr[i] = 0;  // padding of the header
 }
 
 __global__ __launch_bounds__(256) void stream_header_unpack_kernel(const uint8_t *__restrict__ hdr,
@@ -1751,14 +1754,13 @@ hipError_t launch_stream_pack(int bits, const uint8_t *qweight, const __half *ch
                               const int16_t *cherry_indices, const __half *scales, uint8_t *stream, int K, int N,
                               int C, int G, hipStream_t s) {
     const StreamGeo geo = stream_geo(bits, K, N, C);
-    hipLaunchKernelGGL(stream_header_kernel, dim3(ceil_div((int)geo.hdr_bytes, 256)), dim3(256), 0, s, cherry_indices, stream,
-                       geo);
-    const dim3 grid(ceil_div(geo.ntiles, kPackTiles), geo.ng + kPackTiles);
+    const int tiles = ceil_div(geo.ntiles, kPackTiles), heads = ceil_div(ceil_div((int)geo.hdr_bytes, 256), tiles);
+    const dim3 grid(tiles, heads + geo.ng + kPackTiles);
     const int dwords = N % 4 == 0 && aligned(qweight, 4);
     if (bits == 4)
-        hipLaunchKernelGGL(stream_pack_kernel<4>, grid, dim3(256), 0, s, qweight, cherry_weight, scales, stream, G, dwords, geo);
+        hipLaunchKernelGGL(stream_pack_kernel<4>, grid, dim3(256), 0, s, qweight, cherry_weight, scales, cherry_indices, stream, G, dwords, heads, geo);
     else
-        hipLaunchKernelGGL(stream_pack_kernel<3>, grid, dim3(256), 0, s, qweight, cherry_weight, scales, stream, G, dwords, geo);
+        hipLaunchKernelGGL(stream_pack_kernel<3>, grid, dim3(256), 0, s, qweight, cherry_weight, scales, cherry_indices, stream, G, dwords, heads, geo);
     return hipGetLastError();
 }
 
