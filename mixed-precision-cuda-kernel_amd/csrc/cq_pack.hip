@@ -105,16 +105,17 @@ __global__ __launch_bounds__(256) void pack_cherry_kernel(const __half *__restri
 // finds it once for the 8 rows it loads (two searches of the index list per chunk and row were what the
 // general form spent its time on).  A row of 65 dwords makes both the scatter (16 chunks x 4 rows) and
 // the later reads free of bank conflicts; bytes of four neighbouring rows leave as one dword, 128 bytes a line.
-// Bound by HBM and vector ALU alike: one read of the weight and about 20 operations an element.  MI355X, 13824 x 5120
-// to 3 bits: 60 us (3.2 TB/s read + written), where the general form's three launches took 549.
+// Bound by vector ALU first (about 14 operations an element, twice as many wavefronts a CU change nothing) and by one
+// read of the weight.  MI355X, 13824 x 5120 to 3 bits: 51 us (3.4 TB/s read + written; 28672 x 8192 to 4 bits 160),
+// with an address formed for each half and row, comparisons around loads and stores, cherry columns stored half by
+// half in the scatter and quotients of six operations 59 (188); the general form's three launches took 549.
 constexpr int kPackRows = 128, kPackStride = 65;  // dwords of LDS a row; halves 128 and 129 take what belongs nowhere
 constexpr int kPackMaxCherries = 1024;
+constexpr int kPackThreads = 256, kPackLoads = kPackRows * 16 / kPackThreads;  // 16-byte chunks a thread loads
 
 struct PackChunk {
     uint32_t off[8];   // LDS half of each of the 8 columns
     uint32_t valid[4]; // per pair of columns: 0x7fff where the column belongs to the group
-    uint32_t cherry;   // the cherry columns
-    int first;         // rank of the first of them
 };
 
 __device__ __forceinline__ PackChunk pack_chunk(const int16_t *s_idx, int C, int col0, int k0, int k1) {
@@ -124,13 +125,12 @@ __device__ __forceinline__ PackChunk pack_chunk(const int16_t *s_idx, int C, int
         const int mid = (lo + hi) >> 1;
         if ((int)s_idx[mid] < col0) lo = mid + 1; else hi = mid;
     }
-    m.first = lo;
-    m.cherry = 0;
-    for (int c = lo; c < C && (int)s_idx[c] < col0 + 8; c++) m.cherry |= 1u << ((int)s_idx[c] - col0);
+    uint32_t cherry = 0;
+    for (int c = lo; c < C && (int)s_idx[c] < col0 + 8; c++) cherry |= 1u << ((int)s_idx[c] - col0);
     int pos = col0 - lo;
 #pragma unroll
     for (int e = 0; e < 8; e++) {
-        const bool normal = !((m.cherry >> e) & 1u), in = normal && pos >= k0 && pos < k1;
+        const bool normal = !((cherry >> e) & 1u), in = normal && pos >= k0 && pos < k1;
         m.off[e] = in ? pos - k0 : 128;
         if (e & 1) m.valid[e >> 1] |= in ? 0x7fff0000u : 0u;
         else m.valid[e >> 1] = in ? 0x7fffu : 0u;
@@ -139,8 +139,30 @@ __device__ __forceinline__ PackChunk pack_chunk(const int16_t *s_idx, int C, int
     return m;
 }
 
+// Two quotients x / s: the product with the reciprocal and one correction step.  The mixed-precision forms read the
+// halves where they lie and round once, to fp16: three operations a value instead of six.
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ half2_t pack_quotients(uint32_t x, float s, float rs) {
+    float q0, q1, e0, e1;
+    uint32_t r;
+    asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(q0) : "v"(x), "v"(rs));
+    asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(q1) : "v"(x), "v"(rs));
+    asm("v_fma_mix_f32 %0, -%1, %2, %3 op_sel_hi:[0,0,1]" : "=v"(e0) : "v"(q0), "v"(s), "v"(x));
+    asm("v_fma_mix_f32 %0, -%1, %2, %3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(e1) : "v"(q1), "v"(s), "v"(x));
+    asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "=v"(r) : "v"(e0), "v"(rs), "v"(q0));
+    asm("v_fma_mixhi_f16 %0, %1, %2, %3" : "+v"(r) : "v"(e1), "v"(rs), "v"(q1));
+    return __builtin_bit_cast(half2_t, r);
+}
+// Both halves clamped to +-(2^(BITS-1) - 0.01) rounded to fp16, NaN to the lower end.
 template <int BITS>
-__global__ __launch_bounds__(256) void pack_group_kernel(const __half *__restrict__ w, const int16_t *__restrict__ idx,
+__device__ __forceinline__ half2_t pack_clamp(half2_t v) {
+    constexpr uint32_t top = BITS == 4 ? 0x47fd47fdu : 0x43fb43fbu;
+    asm("v_pk_max_f16 %0, %0, %1\n\tv_pk_min_f16 %0, %0, %2" : "+v"(v) : "s"(top | 0x80008000u), "s"(top));
+    return v;
+}
+
+template <int BITS>
+__global__ __launch_bounds__(kPackThreads) void pack_group_kernel(const __half *__restrict__ w, const int16_t *__restrict__ idx,
                                                          uint8_t *__restrict__ qweight, __half *__restrict__ scales,
                                                          __half *__restrict__ cherry_weight, int K, int N, int C, int G) {
     __shared__ uint32_t s_w[kPackRows * kPackStride];
@@ -149,7 +171,7 @@ __global__ __launch_bounds__(256) void pack_group_kernel(const __half *__restric
     __shared__ int16_t s_idx[kPackMaxCherries];
     const int t = threadIdx.x, g = blockIdx.x, n0 = blockIdx.y * kPackRows;
     const int Kn = K - C, k0 = g * G, k1 = min(k0 + G, Kn);
-    for (int i = t; i < C; i += 256) s_idx[i] = idx[i];
+    for (int i = t; i < C; i += kPackThreads) s_idx[i] = idx[i];
     if (t < kPackRows) s_max[t] = 0;
     __syncthreads();
     // the group's columns, with the cherries behind its last normal column (in front of column 0's too)
@@ -164,9 +186,9 @@ __global__ __launch_bounds__(256) void pack_group_kernel(const __half *__restric
     const int col0 = g == 0 ? 0 : source(k0), col1 = k1 == Kn ? K : source(k1);  // [col0, col1)
     const int c0 = col0 >> 3, nch = ((col1 - 1) >> 3) - c0 + 1;
 
-    auto place = [&](const PackChunk &m, const uint4 &q, int row) {  // -> the chunk's largest magnitude in the group
+    // `at`: where the chunk's columns go in the row's LDS -> the chunk's largest magnitude in the group
+    auto place = [&](const PackChunk &m, unsigned short *const (&at)[8], const uint4 &q, int step) {
         const uint32_t d[4] = {q.x, q.y, q.z, q.w};
-        unsigned short *o = reinterpret_cast<unsigned short *>(s_w + row * kPackStride);
         // Two halves at a time, moved up by 0x83ff: magnitudes up to infinity (0x7c00) end at 0xffff, a NaN's wrap to below
         // 0x83ff and take no part in the maximum.
         typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
@@ -175,42 +197,46 @@ __global__ __launch_bounds__(256) void pack_group_kernel(const __half *__restric
         for (int p = 0; p < 4; p++) {
             const u16x2 a = __builtin_bit_cast(u16x2, d[p] & m.valid[p]) + (u16x2){0x83ff, 0x83ff};
             top = __builtin_elementwise_max(top, a);
-            o[m.off[2 * p]] = (unsigned short)d[p];
-            o[m.off[2 * p + 1]] = (unsigned short)(d[p] >> 16);
-        }
-        if (m.cherry) {
-            int c = m.first;
-#pragma unroll
-            for (int e = 0; e < 8; e++)
-                if ((m.cherry >> e) & 1u)
-                    cherry_weight[(size_t)c++ * N + n0 + row] = __ushort_as_half((unsigned short)(d[e >> 1] >> (16 * (e & 1))));
+            at[2 * p][step * 2 * kPackStride] = (unsigned short)d[p];
+            at[2 * p + 1][step * 2 * kPackStride] = (unsigned short)(d[p] >> 16);
         }
         return (uint32_t)max(top[0], top[1]) - 0x83ffu;
     };
+    auto columns = [&](const PackChunk &m, int row, unsigned short *(&at)[8]) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) at[e] = reinterpret_cast<unsigned short *>(s_w + row * kPackStride) + m.off[e];
+    };
     {
-        const int ci = t & 15, r0 = t >> 4;
-        const bool mine = ci < nch;
-        const __half *src = w + (size_t)(n0 + r0) * K + 8 * (c0 + ci);
-        uint4 q[8];
+        // A thread without a chunk or a row of its own repeats the last one: the same bytes to the same place (rows past N are
+        // not read again), and neither loads nor stores wait for a comparison.
+        const int ci = min(t & 15, nch - 1), r0 = t >> 4;
+        uint4 q[kPackLoads];
 #pragma unroll
-        for (int i = 0; i < 8; i++)
-            if (mine && n0 + r0 + 16 * i < N) q[i] = *reinterpret_cast<const uint4 *>(src + (size_t)16 * i * K);
+        for (int i = 0; i < kPackLoads; i++)
+            q[i] = *reinterpret_cast<const uint4 *>(w + (size_t)min(n0 + r0 + kPackThreads / 16 * i, N - 1) * K + 8 * (c0 + ci));
         const PackChunk m = pack_chunk(s_idx, C, 8 * (c0 + ci), k0, k1);
+        unsigned short *at[8];
+        columns(m, r0, at);
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            uint32_t mx = 0;
-            if (mine && n0 + r0 + 16 * i < N) mx = place(m, q[i], r0 + 16 * i);
+        for (int i = 0; i < kPackLoads; i++) {
             // across the row's 16 lanes first: 16 atomics on one word of LDS take turns
-            mx = (uint32_t)row_max((int)mx);
-            if (ci == 0) atomicMax(&s_max[r0 + 16 * i], mx);
+            const uint32_t mx = (uint32_t)row_max((int)place(m, at, q[i], kPackThreads / 16 * i));
+            if ((t & 15) == 0) atomicMax(&s_max[r0 + kPackThreads / 16 * i], mx);
         }
     }
     // the chunk or two that cherries and alignment push the range beyond 16
-    for (int e = t; e < (nch - 16) * kPackRows; e += 256) {
+    for (int e = t; e < (nch - 16) * kPackRows; e += kPackThreads) {
         const int row = e & (kPackRows - 1), c = c0 + 16 + e / kPackRows;
-        if (n0 + row < N)
-            atomicMax(&s_max[row],
-                      place(pack_chunk(s_idx, C, 8 * c, k0, k1), *reinterpret_cast<const uint4 *>(w + (size_t)(n0 + row) * K + 8 * c), row));
+        const PackChunk m = pack_chunk(s_idx, C, 8 * c, k0, k1);
+        unsigned short *at[8];
+        columns(m, row, at);
+        atomicMax(&s_max[row], place(m, at, *reinterpret_cast<const uint4 *>(w + (size_t)min(n0 + row, N - 1) * K + 8 * c), 0));
+    }
+    // the cherry columns among them, from the lines just read: 128 neighbouring halves of an output row leave together
+    const int cherry0 = col0 - k0, cherries = col1 - k1 - cherry0;
+    for (int e = t; e < cherries * kPackRows; e += kPackThreads) {
+        const int row = e & (kPackRows - 1), c = cherry0 + e / kPackRows;
+        if (n0 + row < N) cherry_weight[(size_t)c * N + n0 + row] = w[(size_t)(n0 + row) * K + s_idx[c]];
     }
     __syncthreads();
     if (t < kPackRows) {
@@ -222,10 +248,9 @@ __global__ __launch_bounds__(256) void pack_group_kernel(const __half *__restric
         s_r[t] = __builtin_amdgcn_rcpf(__half2float(sh));
     }
     __syncthreads();
-    const float qmax = (float)(1 << (BITS - 1)) - 1e-2f;
     const float magic = 12582912.f + (float)(1 << (BITS - 1));  // 1.5 * 2^23: adding it rounds to the nearest even integer
     const int units = (k1 - k0) / 8;
-    for (int it = t; it < 32 * units; it += 256) {
+    for (int it = t; it < 32 * units; it += kPackThreads) {
         const int rq = it & 31, j = it >> 5;
         if (n0 + 4 * rq >= N) continue;
         uint32_t word[4];
@@ -235,23 +260,23 @@ __global__ __launch_bounds__(256) void pack_group_kernel(const __half *__restric
             const float s = s_s[row], rs = s_r[row];
             const float sf = __builtin_isinf(s) ? 0.f : s;  // finite / inf: the correction below must not form inf * 0
             const uint32_t *src = s_w + row * kPackStride + 4 * j;
-            word[r] = 0;
+            uint32_t half[2];
 #pragma unroll
             for (int p = 0; p < 4; p++) {
-                const uint32_t d = src[p];
-#pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    // RN16(x / s) from the reciprocal and one correction step (less than one fp32 ulp off; a
-                    // quotient of two 11-bit significands stays more than 2^-23 away from every fp16 tie)
-                    const float x = __half2float(__ushort_as_half((unsigned short)(d >> (16 * h))));
-                    const float q0 = x * rs;
-                    const float qf = __builtin_fmaf(__builtin_fmaf(-q0, sf, x), rs, q0);
-                    float v = __half2float(__float2half_rn(qf));
-                    v = fminf(fmaxf(v, -qmax), qmax) - 0.5f;
-                    const uint32_t code = __float_as_uint(v + magic) & ((1u << BITS) - 1u);
-                    word[r] |= code << (BITS * (2 * p + h));
-                }
+                // RN16(x / s) from the reciprocal and one correction step (less than one fp32 ulp off; a
+                // quotient of two 11-bit significands stays more than 2^-23 away from every fp16 tie), then
+                // clamped to +-(2^(BITS-1) - 0.01), in fp16 the neighbour of that with the same code
+                const half2_t v = pack_clamp<BITS>(pack_quotients(src[p], sf, rs));
+                float f0, f1;  // v - 0.5, exact
+                asm("v_fma_mix_f32 %0, %1, 1.0, -0.5 op_sel_hi:[1,0,0]" : "=v"(f0) : "v"(v));
+                asm("v_fma_mix_f32 %0, %1, 1.0, -0.5 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(f1) : "v"(v));
+                const uint32_t lo = __float_as_uint(f0 + magic), hi = __float_as_uint(f1 + magic);
+                // the sum's low 22 bits are 0..2^BITS - 1: four codes leave its exponent above 22 - 3 * 4 unmasked
+                uint32_t &w2 = half[p >> 1];
+                w2 = (p & 1) ? (lo << (2 * BITS)) | w2 : lo;
+                w2 = (hi << (BITS * (2 * (p & 1) + 1))) | w2;
             }
+            word[r] = (half[1] << (4 * BITS)) | (half[0] & ((1u << (4 * BITS)) - 1u));
         }
         uint8_t *o = qweight + (size_t)(k0 / 8 + j) * BITS * N + n0 + 4 * rq;
 #pragma unroll
@@ -323,9 +348,9 @@ hipError_t launch_pack(int bits, const __half *w, const int16_t *idx, uint8_t *q
     if (Kn > 0 && G % 8 == 0 && G <= 128 && N % 4 == 0 && C <= kPackMaxCherries && aligned(w, 16) && aligned(qweight, 4)) {
         const dim3 grid(ceil_div(Kn, G), ceil_div(N, kPackRows));
         if (bits == 4)
-            hipLaunchKernelGGL(pack_group_kernel<4>, grid, dim3(256), 0, stream, w, idx, qweight, scales, cherry_weight, K, N, C, G);
+            hipLaunchKernelGGL(pack_group_kernel<4>, grid, dim3(kPackThreads), 0, stream, w, idx, qweight, scales, cherry_weight, K, N, C, G);
         else
-            hipLaunchKernelGGL(pack_group_kernel<3>, grid, dim3(256), 0, stream, w, idx, qweight, scales, cherry_weight, K, N, C, G);
+            hipLaunchKernelGGL(pack_group_kernel<3>, grid, dim3(kPackThreads), 0, stream, w, idx, qweight, scales, cherry_weight, K, N, C, G);
         return hipGetLastError();
     }
     if (Kn > 0) {

@@ -111,7 +111,7 @@ __device__ inline void stream_header(const int16_t *__restrict__ cherry_indices,
 // wavefront writes the unit as one contiguous piece.  The last 8 blockIdx.y take the tiles' scales and
 // cherry rows; the first `heads` write the header, whose binary searches are a chain of loads that the rest hides (a
 // launch of its own was 4.9 us in front).  Bound by HBM: the packed bytes once in, once out.  MI355X, 5120 -> 13824 in
-// 3 bits: HDRUS us (3.5 TB/s read + written); one workgroup a tile gathering single bytes from 16-byte runs took 192.
+// 3 bits: 15 us (3.7 TB/s read + written); one workgroup a tile gathering single bytes from 16-byte runs took 192.
 constexpr int kPackTiles = 8;
 
 template <int BITS>
