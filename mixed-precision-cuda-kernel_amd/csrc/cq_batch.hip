@@ -1,4 +1,5 @@
-// Small-batch fused dequant + matmul (2 <= batch <= 16 rows per pass) on the gfx950 matrix cores.
+// Small-batch fused dequant + matmul (2 <= batch <= 16 rows per pass) on the gfx950 matrix cores.  From 5 rows on it takes the
+// calls that prompt_preferred leaves (cq_prompt.hip): layers of more than 64 MB and those it is as fast on.
 //
 // The weight stream is tiled exactly as in the batch-1 kernel (cq_matvec.hip): a wavefront owns
 // units of 128 compacted positions x 256 columns, four lane groups split the positions, a lane

@@ -7,7 +7,8 @@
 //
 // All of them are bound by latency at prompt lengths of a few hundred: what counts is the number of launches.  As
 // tensor operations they were some 35 launches a layer; now they are five (7B, 128 tokens, whole prompt: 11.5 -> 6.1 ms;
-// norm 3.9, keys and values 3.3, attention 5.3 us).
+// norm 3.9, keys and values 3.3, attention 5.3 us).  In the native pass over plain layers the norms and SiLU * up write the
+// next product's operands too (cq_prompt.hip).
 #include "cq_device.h"
 #include "cq_kernels.h"
 

@@ -1,4 +1,4 @@
-// Prompt-sized batches (17 rows and more) over the checkpoint layout: fused dequantise + matrix product.
+// Prompt-sized batches (17 rows and more, most layers from 5) over the checkpoint layout: fused dequantise + matrix product.
 //
 //   Y[M, N] (+)= Xn[M, Kn] * Wn[Kn, N] + Xc[M, C] * Wc[C, N]
 //
