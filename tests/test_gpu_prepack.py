@@ -444,6 +444,27 @@ def test_prepacked_rows_against_the_c_oracle(bits, k, n, b):
         np.testing.assert_array_equal(run(e), c_oracle.fused(e, p, bits, 128).astype(np.float16))
 
 
+@pytest.mark.parametrize("bits,k,c,first", [(4, 1160, 128, 0), (3, 1160, 128, 1032), (4, 1160, 64, 120), (3, 4104, 128, 1), (4, 4096, 8, 127),
+                                            (3, 136, 8, 128), (4, 256, 128, 64), (4, 9096, 104, 8992)])
+def test_prepacked_rows_every_cherry_channel_lands(qc, bits, k, c, first):
+    """A run of neighbouring cherries at either end of the row, across the border of two units of 128 positions, in a layer
+    of one unit and in one of more than 64: each channel alone, 16 at a time, bit for bit (products of one
+    nonzero activation are exact up to the one rounding of the result)."""
+    announce("every cherry", bits, k, c, first)
+    n = 40
+    p = orc.synthetic_packed_fast(k, n, bits, 128, seed=k + c, cherry_fraction=(c + 0.5) / k)
+    p["cherry_indices"] = np.arange(first, first + c).astype(np.int16)
+    stream = prepack(qc, bits, p, k)
+    out = torch.full((16, n), float("nan"), dtype=torch.float16, device="cuda")
+    for j in range(0, c, 16):
+        e = np.zeros((16, k), dtype=np.float16)
+        for r in range(16):
+            e[r, first + (j + r) % c] = np.float16(2.0 ** (r % 5 - 2))
+        qc.matvec_prepacked_cherryq(bits, torch.from_numpy(e).cuda(), stream, out, k, c)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out.cpu().numpy(), c_oracle.fused(e, p, bits, 128).astype(np.float16), err_msg=str(j))
+
+
 def test_prepacked_rows_on_random_small_layers(qc):
     """1 to 16 rows over randomly drawn small layers -- input widths that are no multiple of 512,
     0 to 128 cherry channels at random places (neighbours, the first and the last columns), widths
