@@ -472,6 +472,12 @@ size_t cherryq_prefill_matmul_group_scratch_bytes(int rows, int in_features, int
 int cherryq_prefill_matmul_group_f16(int w_bits, const void *vec, const cherryq_layer *layers, int n_layers, int rows, int in_features,
                                      int num_cherries, int group_size, int accumulate, void *workspace, size_t workspace_bytes,
                                      void *scratch, size_t scratch_bytes, void *stream);
+/*
+ * 1 where a product of `rows` rows and this shape, launched on `stream` now, goes to the prompt kernel; 0: another kernel, a call that
+ * is refused, or a stream under capture.  For callers that have a dense product as an alternative, which takes more (any
+ * group of whole bytes, buffers of any alignment) and shares no buffers between the replays of a graph and other calls.
+ */
+int cherryq_prompt_taken(int w_bits, int rows, int in_features, int out_features, int num_cherries, int group_size, void *stream);
 int cherryq_prefill_norm_f16(void *hidden, const void *delta /* may be NULL */, const void *weight, void *normed, int rows,
                              int hidden_size, float eps, void *stream);
 size_t cherryq_prefill_attention_bytes(int tokens, int n_kv_heads);

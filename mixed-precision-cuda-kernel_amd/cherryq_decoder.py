@@ -160,14 +160,16 @@ def matmul_group_supported(mods, rows) -> bool:
         if (m.w_bits, m.group_size, m.num_cherries, m.in_features) != (m0.w_bits, m0.group_size, m0.num_cherries, m0.in_features):
             return False
         k, n, c, b = m.in_features, m.out_features, m.num_cherries, m._buffers
-        if m.w_bits not in (3, 4) or m.group_size <= 0 or m.group_size % 32 or c >= k:
+        if m.w_bits not in (3, 4) or m.group_size <= 0 or m.group_size % 32 or (m.w_bits == 4 and m.group_size < 128) or c >= k:
+            return False
+        if rows >= m._dense_rows and not quant_cuda._lib.cherryq_prompt_taken(m.w_bits, rows, k, n, c, m.group_size, _stream()):
             return False
         for name, dt, shape in (("qweight", torch.uint8, ((k - c) // 8 * m.w_bits, n)), ("cherry_weight", torch.float16, (c, n)),
                                 ("scales", torch.float16, (-(-(k - c) // m.group_size), n)), ("cherry_indices", torch.int16, (c,))):
             t = b.get(name)
             if t is None or t.shape != shape or t.dtype != dt or not t.is_cuda or not t.is_contiguous():
                 return False
-            if t.get_device() != m0._buffers["qweight"].get_device():
+            if t.get_device() != m0._buffers["qweight"].get_device() or quant_cuda._misaligned(t, 4 if name == "cherry_indices" else 16):
                 return False
     return True
 
@@ -757,7 +759,8 @@ class CherryLlamaDecoder(nn.Module):
 
         def project(x, *mods):  # layers that read x: as one product where that is what their own calls compute
             outs = None
-            if T >= 17 and _plain(x, dev, T, hidden) and matmul_group_supported(mods, T):
+            if (T >= 17 and _plain(x, dev, T, hidden) and (T < QuantLinear._dense_rows or quant_cuda._host.ordinary(x))
+                    and matmul_group_supported(mods, T)):
                 outs = matmul_group(mods, x)
             return [m(x) for m in mods] if outs is None else outs
 
@@ -813,6 +816,8 @@ class CherryLlamaDecoder(nn.Module):
                 c.dtype == torch.float16 and c.is_contiguous() and c.shape == (n, cfg.num_key_value_heads, ml, 128) for c in caches):
             return None
         if torch.nn.modules.module._has_any_global_hook() or QuantLinear.forward is not _FORWARD:
+            return None
+        if T >= QuantLinear._dense_rows and not quant_cuda._host.ordinary(h):
             return None
         layers = (_PrefillLayer * n)()
         at, size = ctypes.addressof(layers), ctypes.sizeof(_PrefillLayer)

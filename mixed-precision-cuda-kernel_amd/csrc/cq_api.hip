@@ -803,6 +803,19 @@ int cherryq_decode_silu_mul_f16(const void *gate, const void *up, void *out, int
                                     reinterpret_cast<__half *>(out), n, reinterpret_cast<hipStream_t>(stream));
 }
 
+int cherryq_prompt_taken(int w_bits, int rows, int in_features, int out_features, int num_cherries, int group_size, void *stream) {
+    const int K = in_features, N = out_features, C = num_cherries, G = group_size;
+    if ((w_bits != 3 && w_bits != 4) || (w_bits == 4 && G < 128) || rows < cq::kPromptMinRows || K <= 0 || N <= 0 || C < 0 || C > K || K % 8 ||
+        N % 8 || C % 8 || G <= 0 || (C > 0 && K > 32768) || cq::force_generic() || !cq::prompt_supported(w_bits, rows, K, N, C, G))
+        return 0;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(reinterpret_cast<hipStream_t>(stream), &capture) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return capture == hipStreamCaptureStatusNone;
+}
+
 int cherryq_prefill_norm_f16(void *hidden, const void *delta, const void *weight, void *normed, int rows, int hidden_size,
                              float eps, void *stream) {
     if (!hidden || !weight || !normed) return CHERRYQ_E_NULL;

@@ -12,7 +12,10 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/TracerMode.h>
 #include <c10/core/InferenceMode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -41,6 +44,7 @@ using MatvecPrepackedFn = int (*)(int, const void *, const void *, size_t, void 
 using MatmulPrepackedFn = int (*)(int, const void *, const void *, size_t, void *, int, int, int, int, int, void *, size_t,
                                   void *);
 using ShapeFn = int (*)(int, int, int, int, int, int);
+using TakenFn = int (*)(int, int, int, int, int, int, void *);
 
 struct Api {
     VecquantFn vecquant4, vecquant3, vecquant3_f32;
@@ -50,6 +54,7 @@ struct Api {
     MatmulPrepackedFn matmul_prepacked;
     ShapeFn prepack_supported, rows_recommended;
 } api;
+TakenFn prompt_taken;  // cherryq_prompt_taken
 
 // ---- buffers kept per (device, stream) -----------------------------------------------------------
 // A zero-initialised workspace (the kernels leave it all zero after every call, so it is reusable as is)
@@ -96,6 +101,18 @@ inline const void *ptr(const Tensor &t) { return t.numel() ? t.const_data_ptr() 
 inline void *mut(const Tensor &t) { return t.numel() ? t.mutable_data_ptr() : nullptr; }
 
 inline void *current_stream(int device) { return c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream(); }
+
+// From so many rows QuantLinear has a dense product to go to (llama/qlinear.py); the prompt kernel is taken where it is sure to answer.
+constexpr int64_t kDenseRows = 512;
+
+// Whether a call is only that: nothing records, replaces or transforms the operations, which a launch of ours is not among.
+bool ordinary(const Tensor &x) {
+    using K = c10::DispatchKey;
+    return x.has_storage() && !at::tracer::impl::is_dispatch_enabled() && !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
+           !at::impl::torch_function_mode_enabled() &&
+           !c10::impl::tls_local_dispatch_key_set().included_.has_any(
+               c10::DispatchKeySet({K::FuncTorchDynamicLayerFrontMode, K::FuncTorchDynamicLayerBackMode, K::FuncTorchVmapMode}));
+}
 
 struct Packed {  // the checkpoint buffers of one layer
     const Tensor *qweight, *cherry_weight, *cherry_indices, *scales;
@@ -279,6 +296,9 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
         const int64_t most = limit.o && PyLong_Check(limit.o) ? PyLong_AsLongLong(limit.o) : -1;
         if (PyErr_Occurred()) PyErr_Clear();
         if (rows >= most) Py_RETURN_NONE;  // dequantise once and a dense product
+        if (rows >= kDenseRows && (!prompt_taken || !ordinary(*x) ||
+                                   !prompt_taken(bits, (int)std::min<int64_t>(rows, INT32_MAX), (int)k, (int)n, (int)c, (int)group, current_stream(device))))
+            Py_RETURN_NONE;
         auto buffer = [&](PyObject *name) {
             PyObject *o = PyDict_GetItemWithError(buffers, name);
             return o ? tensor(o) : nullptr;
@@ -356,6 +376,11 @@ PyObject *describe(PyObject *, PyObject *const *a, Py_ssize_t n) {
         } else if (product->w_bits != bits || product->in_features != k || product->num_cherries != c || product->group_size != group) {
             Py_RETURN_FALSE;
         }
+        // what the entry point takes; other layers' own calls may go to a dense product
+        auto misaligned = [](const Tensor &t, uintptr_t bytes) { return reinterpret_cast<uintptr_t>(ptr(t)) % bytes; };
+        if (group % 32 || (bits == 4 && group < 128) || misaligned(*t[0], 16) || misaligned(*t[1], 16) || misaligned(*t[2], 4) || misaligned(*t[3], 16) ||
+            (rows >= kDenseRows && (!prompt_taken || !prompt_taken((int)bits, (int)rows, (int)k, (int)columns, (int)c, (int)group, current_stream(device)))))
+            Py_RETURN_FALSE;
         for (int j = 0; j < 4; j++)
             if (PyList_Append(a[4], o[j])) return nullptr;
         product->layers[i - 5] = {static_cast<const uint8_t *>(ptr(*t[0])), ptr(*t[1]), static_cast<const int16_t *>(ptr(*t[2])), ptr(*t[3]),
@@ -415,8 +440,25 @@ PyObject *bind(PyObject *, PyObject *seq) {
     Py_RETURN_NONE;
 }
 
+// bind_prompt(address): cherryq_prompt_taken.  Without it no call of kDenseRows rows and more is taken.
+PyObject *bind_prompt(PyObject *, PyObject *address) {
+    prompt_taken = reinterpret_cast<TakenFn>(PyLong_AsVoidPtr(address));
+    if (PyErr_Occurred()) return nullptr;
+    Py_RETURN_NONE;
+}
+
+// ordinary(tensor)
+PyObject *is_ordinary(PyObject *, PyObject *x) {
+    HANDLE_TH_ERRORS
+    const Tensor *t = tensor(x);
+    return PyBool_FromLong(t && ordinary(*t));
+    END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
     {"bind", bind, METH_O, nullptr},
+    {"bind_prompt", bind_prompt, METH_O, nullptr},
+    {"ordinary", is_ordinary, METH_O, nullptr},
     {"vecquant", (PyCFunction)(void (*)())vecquant, METH_FASTCALL, nullptr},
     {"matvec_prepacked", (PyCFunction)(void (*)())matvec_prepacked, METH_FASTCALL, nullptr},
     {"linear", (PyCFunction)(void (*)())linear, METH_FASTCALL, nullptr},

@@ -66,10 +66,15 @@ class QuantLinear(nn.Module):
 
     _layerwise_dequantize = True
     # Rows at and above which the fused forward dequantises once and calls the library's dense GEMM
-    # instead of the fused dequantise + MFMA kernel.  MI355X, fused / dense in us with 2048 and 3072 rows: 4096 -> 11008
-    # 188 / 198 and 295 / 335, 4096 -> 4096 72 / 76 and 114 / 98, 8192 -> 28672 796 / 851 and 1225 / 1173, 5120 -> 13824 in
-    # 3 bits 279 / 278 and 413 / 376; below, the fused kernel is ahead by up to a third (512 rows of 8192 -> 28672: 230 / 340).
+    # instead of the fused dequantise + MFMA kernel.  MI355X, 42 layers of 2048 -> 1024 to 28672 -> 8192 in both widths of codes, the fused
+    # kernel's time over the dense path's: 0.79 on average with 1100 rows, 0.87 with 1536, 0.90 with 2048, 0.93 with 2303.  No line
+    # by shape holds: the library's product runs at 560 to 1250 TFLOP/s with neighbouring sizes (1700, 1900 and 2048 rows of 4 bits,
+    # fused / dense in us: 4096 -> 11008 166 / 261, 170 / 172, 173 / 188; 5120 -> 13824 216 / 234, 267 / 248, 273 / 248; 8192 -> 8192 212 / 202,
+    # 228 / 216, 236 / 218).  Above 2304 rows the library's better half decides (3072: 4096 -> 4096 107 / 94, 8192 -> 28672 1194 / 1160).
     prefill_rows = 2304
+    # From here on the dense product is also there for calls that the fused kernel refuses (groups, alignment, tensors on the host,
+    # operations that are recorded or transformed, a stream under capture).  kDenseRows in csrc/cq_host.cpp is the same line.
+    _dense_rows = 512
 
     @classmethod
     @contextmanager
@@ -248,7 +253,8 @@ class QuantLinear(nn.Module):
 
     # ---- forward ------------------------------------------------------------------------------
     def forward(self, x: torch.Tensor):
-        # one native call for the fused cases (the choice of path is that of _forward); None: not one of them
+        # one native call for the fused cases (the choice of path is that of _forward, which from _dense_rows rows has the
+        # dense product for what the native call does not take); None: not one of them
         out = quant_cuda._host.linear(self, x)
         return self._forward(x) if out is None else out
 
@@ -286,7 +292,7 @@ class QuantLinear(nn.Module):
                 for r0 in range(0, rows, 16):
                     quant_cuda.matvec_prepacked_cherryq(self.w_bits, x2[r0:r0 + 16], stream, out[r0:r0 + 16],
                                                         self.in_features, self.num_cherries)
-            elif x2.shape[0] >= self.prefill_rows:
+            elif x2.shape[0] >= min(self.prefill_rows, self._dense_rows):
                 # prompt-sized batches: one bit-exact dequantisation pass on the GPU into a transient
                 # dense weight, then a library fp16 GEMM -- the arithmetic of the dequantised branch
                 # below (llama/qlinear.py:183-195) without keeping the dense weight

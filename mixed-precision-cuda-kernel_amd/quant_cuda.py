@@ -110,6 +110,9 @@ _host.bind(tuple(ctypes.cast(getattr(_lib, f"cherryq_{n}"), _vp).value for n in 
     "vecquant4matmul_f16", "vecquant3matmul_f16", "vecquant3matmul_f32", "workspace_bytes", "scratch_bytes",
     "scratch_bytes_f32", "prepacked_scratch_bytes", "matvec_prepacked_f16", "matmul_prepacked_f16", "prepack_supported",
     "prepack_rows_recommended")))
+_lib.cherryq_prompt_taken.argtypes = [_int, _int, _int, _int, _int, _int, _vp]
+_lib.cherryq_prompt_taken.restype = _int
+_host.bind_prompt(ctypes.cast(_lib.cherryq_prompt_taken, _vp).value)
 
 
 def _fail(status: int, what: str):
@@ -159,6 +162,10 @@ def _current_stream(device_index: int) -> int:
     if _raw_stream is not None:
         return _raw_stream(device_index)
     return torch.cuda.current_stream(device_index).cuda_stream
+
+
+def _misaligned(t: torch.Tensor, nbytes: int) -> bool:
+    return bool(t.numel()) and t.data_ptr() % nbytes != 0
 
 
 def _ptr(t: torch.Tensor):

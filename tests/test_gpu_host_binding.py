@@ -140,3 +140,64 @@ def test_function_transforms_raise_and_leave_the_binding_usable():
         got = q(x)
     torch.cuda.current_stream().wait_stream(side)
     assert torch.equal(got, q(x))
+
+
+def _shifted(t, nbytes):
+    """The same values `nbytes` behind an address that is aligned."""
+    flat = torch.empty(t.numel() + 16, dtype=t.dtype, device=t.device)[nbytes // t.element_size():][:t.numel()]
+    return flat.view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("rows", [512, 600, 2303])
+@pytest.mark.parametrize("bits,group,moved", [(4, 64, None), (4, 136, None), (3, 24, None), (3, 32, None), (4, 128, "qweight"), (3, 128, "scales"),
+                                              (4, 128, "cherry_weight"), (3, 128, "x"), (4, 128, "wide x")])
+def test_many_rows_of_layers_that_the_fused_kernel_refuses(rows, bits, group, moved):
+    """From 512 rows there is the dense product: groups that are no multiple of 32 (4 bits: below 128), buffers off 16 bytes.  Weights are
+    rounded to fp16 in either path; a result is rounded once (2^-11), the sum of a thousand products far less."""
+    print("[case] many rows", bits, group, moved, rows, flush=True)
+    from llama.qlinear import QuantLinear
+    from llama.quantizer import FullSymQuantizer
+    k, n = 1024, 264
+    gen = torch.Generator(device="cuda").manual_seed(rows + group)
+    q = QuantLinear(bits, group, FullSymQuantizer, 1 / 64, k, n, bias=False).cuda()
+    q.qweight = torch.randint(0, 256, q.qweight.shape, dtype=torch.uint8, device="cuda", generator=gen)
+    q.scales = (torch.rand(q.scales.shape, device="cuda", generator=gen) * 0.02 + 0.001).half()
+    q.cherry_weight = torch.randn(q.cherry_weight.shape, device="cuda", generator=gen).half()
+    q.cherry_indices = torch.randperm(k, device="cuda", generator=gen)[:q.num_cherries].sort().values.to(torch.int16)
+    x = torch.randn(rows, k, device="cuda", generator=gen).half()
+    want = x.double() @ q.unpack().double().t()
+    if moved == "x":
+        x = _shifted(x, 2)
+    elif moved == "wide x":
+        x = torch.cat([x, x], 1)[:, :k]
+    elif moved is not None:
+        t = getattr(q, moved)
+        setattr(q, moved, _shifted(t, {"qweight": 4, "scales": 8, "cherry_weight": 2}[moved]))
+    assert float((q(x).double() - want).norm() / want.norm()) <= 2.0 ** -11
+
+
+def test_many_rows_transformed_and_captured():
+    """Calls of 512 rows and more under vmap, and captured: a graph shares no kept buffer with the calls between its replays."""
+    print("[case] many rows transformed", flush=True)
+    import quant_cuda
+    from llama.qlinear import QuantLinear
+    q = _layer(4, 1024, 256)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    x, other = (torch.randn(600, 1024, device="cuda", generator=gen).half() for _ in range(2))
+    dense = torch.matmul(other, q.unpack().t()).double()
+    assert QuantLinear._dense_rows <= 600 < QuantLinear.prefill_rows
+    both = torch.func.vmap(q)(torch.stack([x, other]))
+    assert float((both[1].double() - dense).norm() / dense.norm()) <= 2.0 ** -10
+    static, graph = x.clone(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = q(static)
+        stream = torch.cuda.current_stream().cuda_stream
+    # nothing was kept for the stream under capture: asked for now, its first buffer is the smallest there is
+    assert quant_cuda._host.scratch(0, stream, 8).numel() == 8
+    for inputs in (other, x, other):
+        static.copy_(inputs)
+        eager = q(inputs)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float((out.double() - eager.double()).norm() / eager.double().norm()) <= 2.0 ** -10

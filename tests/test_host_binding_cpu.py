@@ -265,3 +265,100 @@ def test_descriptions_of_plain_modules_only(host):
         assert describe(q) is None
     with QuantLinear.dmode(False):
         assert describe(mods[0]) is None
+
+
+def dense_layer(bits=4, group=128, k=K, n=N, seed=0):
+    from llama.qlinear import QuantLinear
+    from llama.quantizer import FullSymQuantizer
+    gen = torch.Generator().manual_seed(seed)
+    q = QuantLinear(bits, group, FullSymQuantizer, 1 / 16, k, n, bias=False)
+    q.qweight = torch.randint(0, 256, q.qweight.shape, dtype=torch.uint8, generator=gen)
+    q.scales = (torch.rand(q.scales.shape, generator=gen) * 0.02 + 0.001).half()
+    q.cherry_weight = torch.randn(q.cherry_weight.shape, generator=gen).half()
+    q.cherry_indices = torch.randperm(k, generator=gen)[:q.num_cherries].sort().values.to(torch.int16)
+    return q
+
+
+@pytest.mark.parametrize("rows", [512, 600, 2303])
+@pytest.mark.parametrize("bits,group", [(4, 128), (4, 64), (3, 24)])
+def test_many_rows_on_the_host(rows, bits, group):
+    """From 512 rows there is a dense product for what the fused kernel refuses, tensors on the host among it."""
+    q, x = dense_layer(bits, group), torch.randn(rows, K, generator=torch.Generator().manual_seed(1)).half()
+    assert torch.equal(q(x), torch.matmul(x, q.unpack().t()))
+    with pytest.raises(RuntimeError):
+        q(x[:511])
+
+
+class _DispatchMode(torch.utils._python_dispatch.TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+class _FunctionMode(torch.overrides.TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+def test_many_rows_are_taken_where_a_launch_is_sure_to_do(host):
+    """From 512 rows the native call asks whether the prompt kernel takes the product, and leaves calls whose operations something
+    records, replaces or transforms to torch's."""
+    module, calls, _ = host
+    answers, asked = [1], []
+    stub = ctypes.CFUNCTYPE(ctypes.c_int, *[ctypes.c_int] * 6, ctypes.c_void_p)(lambda *a: asked.append(a[:6]) or answers[0])
+    q, x = layer(), torch.ones(600, K, dtype=torch.float16)
+    want = torch.full((600, N), FILL, dtype=torch.float16)
+    assert module.linear(q, x) is None  # no one to ask
+    try:
+        module.bind_prompt(ctypes.cast(stub, ctypes.c_void_p).value)
+        assert torch.equal(module.linear(q, x), want) and asked == [(4, 600, K, N, q.num_cherries, 128)]
+        with _DispatchMode():
+            assert module.linear(q, x) is None
+        with _FunctionMode():
+            assert module.linear(q, x) is None
+        left = []
+        torch.func.vmap(lambda t: left.append(module.linear(q, t)) or t)(x.expand(2, 600, K))
+        torch.jit.trace(lambda t: left.append(module.linear(q, t)) or t * 1, x, check_trace=False)
+        assert left == [None, None]
+        assert torch.equal(module.linear(q, x), want)
+        answers[0] = 0
+        assert module.linear(q, x) is None
+        assert torch.equal(module.linear(q, x[:511]), want[:511])
+    finally:
+        module.bind_prompt(0)
+
+
+def test_traces_of_many_rows_hold_the_product():
+    q, gen = dense_layer(), torch.Generator().manual_seed(1)
+    x, other = (torch.randn(600, K, generator=gen).half() for _ in range(2))
+    traced = torch.jit.trace(q, x)
+    assert torch.equal(traced(other), q(other))
+
+
+def test_descriptions_of_layers_that_the_entry_point_takes(host):
+    """... only: the others' own calls may go to a dense product."""
+    import cherryq_decoder as dec
+    from llama.qlinear import QuantLinear
+    from llama.quantizer import FullSymQuantizer
+    module = host[0]
+    answers, product = [1], dec._PrefillProduct()
+    stub = ctypes.CFUNCTYPE(ctypes.c_int, *[ctypes.c_int] * 6, ctypes.c_void_p)(lambda *a: answers[0])
+
+    def described(q, rows=40):
+        return module.describe(ctypes.addressof(product), rows, -1, QuantLinear, [], q)
+
+    assert described(layer()) and not described(layer(), 600)
+    try:
+        module.bind_prompt(ctypes.cast(stub, ctypes.c_void_p).value)
+        assert described(layer(), 600)
+        answers[0] = 0
+        assert not described(layer(), 600)
+    finally:
+        module.bind_prompt(0)
+    for bits, group in ((4, 64), (3, 24)):
+        assert not described(QuantLinear(bits, group, FullSymQuantizer, 1 / 16, K, N, bias=False))
+    for name, nbytes in (("qweight", 4), ("scales", 8), ("cherry_weight", 2), ("cherry_indices", 2)):
+        q = layer()
+        t = getattr(q, name)
+        flat = torch.zeros(t.numel() + 8, dtype=t.dtype)[nbytes // t.element_size():][:t.numel()]
+        setattr(q, name, flat.view(t.shape))
+        assert not described(q), name
