@@ -428,6 +428,7 @@ class DecoderLayer(nn.Module):
 
 class CherryLlamaDecoder(nn.Module):
     """Random-init decoder; `generate()` does greedy decoding with a captured token step."""
+    _rope = None  # what _rope_tables has at hand: the tables of all positions, made with the model
 
     def __init__(self, cfg: DecoderConfig, seed: int = 0, device="cuda"):
         super().__init__()
@@ -466,7 +467,7 @@ class CherryLlamaDecoder(nn.Module):
         self.logits16 = torch.zeros(1, cfg.vocab_size, **f16)
         self.history = torch.zeros(ml, dtype=torch.int64, device=self.device_)  # history[p]: token predicted at position p
         self._graph = None
-        self._rope = None  # _rope_tables
+        self._rope = self._rope_key(), *self._rope_angles(ml)
         self.fuse_norm = True
         self.fuse_head = True  # final RMSNorm inside the head launch (False: a launch of its own in front)
         # Attention dealt to ATTN_SLICES workgroups per head, combined by a repacked o_proj's staging: None =
@@ -794,16 +795,22 @@ class CherryLlamaDecoder(nn.Module):
         self._head(self.normed, None)  # logits of the last prompt position; greedy tail: history[T-1], next embedding, pos = T
         return self.logits
 
+    def _rope_key(self):
+        return self.device_, self.cfg.rope_theta, self.cfg.head_dim, self.cfg.max_position_embeddings
+
+    def _rope_angles(self, T):
+        """cos and sin of the rotary angles of positions 0..T-1, (T, head_dim / 2) fp16 each."""
+        hd = self.cfg.head_dim
+        pos = torch.arange(T, device=self.device_, dtype=torch.float32)
+        inv = 1.0 / (self.cfg.rope_theta ** (torch.arange(0, hd, 2, device=self.device_, dtype=torch.float32) / hd))
+        fr = torch.outer(pos, inv)
+        return fr.cos().half(), fr.sin().half()
+
     def _rope_tables(self, T):
-        """cos and sin of the rotary angles of positions 0..T-1, (T, head_dim / 2) fp16 each: made once for all positions
-        (llama/modeling_llama_quant.py:95-210 keeps them too)."""
-        cfg, hd = self.cfg, self.cfg.head_dim
-        made_for = self.device_, cfg.rope_theta, hd, cfg.max_position_embeddings
-        if self._rope is None or self._rope[0] != made_for:
-            pos = torch.arange(cfg.max_position_embeddings, device=self.device_, dtype=torch.float32)
-            inv = 1.0 / (cfg.rope_theta ** (torch.arange(0, hd, 2, device=self.device_, dtype=torch.float32) / hd))
-            fr = torch.outer(pos, inv)
-            self._rope = made_for, fr.cos().half(), fr.sin().half()
+        """The same from the tables made with the model (llama/modeling_llama_quant.py:95-210 keeps them too).  Nothing made during a
+        pass is kept: under capture its values come with the replay.  A config changed since gets tables of the pass's own."""
+        if self._rope is None or self._rope[0] != self._rope_key():
+            return self._rope_angles(T)
         return self._rope[1][:T], self._rope[2][:T]
 
     def _prefill_layers(self, h, cos, sin):

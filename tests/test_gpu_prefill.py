@@ -320,3 +320,28 @@ def test_layers_in_one_call_against_single_calls(dec, bits, heads, kv, inter, to
         # 14 products' results and two norms' rounded to fp16, any of them to the neighbouring value
         assert rel(a, b.double().cpu()) < 16 * 2 ** -11
     assert model.pos.item() == tokens
+
+
+def test_first_pass_under_capture(dec):
+    """A model whose first prompt pass is captured: an eager pass before the replay, and the replays, give what another model of the
+    same seed gives."""
+    print("[case] prefill captured", flush=True)
+    cfg = dec.DecoderConfig(hidden_size=256, intermediate_size=512, num_hidden_layers=2, num_attention_heads=2,
+                            num_key_value_heads=1, vocab_size=512, max_position_embeddings=64)
+    ids = torch.arange(40, device="cuda") * 7 % 512
+    plain = dec.CherryLlamaDecoder(cfg, seed=1)
+    want = plain.prefill(ids).clone(), plain.k_cache.clone(), plain.v_cache.clone()
+    model, stream, graph = dec.CherryLlamaDecoder(cfg, seed=1), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        plain.prefill(ids)  # the stream's kept buffers exist before the capture
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        model.prefill(ids)
+    torch.cuda.synchronize()
+    for replay in (False, True, True):
+        model.k_cache.fill_(1.0)
+        graph.replay() if replay else model.prefill(ids)
+        torch.cuda.synchronize()
+        for got, w in zip((model.logits, model.k_cache, model.v_cache), want):
+            assert torch.equal(got, w)
