@@ -533,7 +533,9 @@ struct PromptColumn {
 };
 
 // (written out: the accumulator stays where it is.  The compiler's own form may name another destination and then
-// spills accumulators.)  Its result is next read 16 products later at the earliest, or behind mfma_drain().
+// spills accumulators.)  The compiler keeps no distances around these: products into the same accumulator need none; before other
+// instructions read a result there are eight more or mfma_drain(); and no vector instruction writes an operand less
+// than two in front, accumulators being zeroed long before.  tests/test_mfma_distances.py reads the built code.
 __device__ __forceinline__ void prompt_mfma(float4_t &acc, const u32x4 &a, const u32x4 &b) {
     asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
 }
@@ -591,15 +593,28 @@ __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(Pro
     constexpr int RED = MT * NC * 64 * 4;                          // four wavefronts' results
     __shared__ u32x4 s_b[2 * STAGE > RED ? 2 * STAGE : RED];
     __shared__ u32x2 s_sc[SUMS ? 2 : 1][WK][16];  // a stage's scales: SUMS
+    // Every 64-byte line of the arguments is asked for at once, not where its first word is used: one wait instead of four, each in front of
+    // the first load.  (With that, the order of the first loads and the cherries' buffer given back early, calls of few units of K
+    // are 0.3 to 0.6 us shorter: 102 rows of 1248 -> 2784 9.95 -> 9.4, 18 of 1360 -> 12520 in 3 bits 10.0 -> 9.3.)
+    asm volatile("" ::"s"(members.qweight[0]), "s"(members.scales[2]), "s"(members.first[2]), "s"(K), "s"(plan.steps), "s"(plan.partial_bytes));
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kq = lane >> 4, nl = lane & 15;
-    const int tiles = plan.mtiles * plan.ntiles, piece = ((int)blockIdx.x & 7) * ((int)gridDim.x >> 3) + ((int)blockIdx.x >> 3);
+    const int tiles = plan.mtiles * plan.ntiles, per_die = (tiles * plan.splits + 7) >> 3;  // the grid is 8 times that
+    const int piece = ((int)blockIdx.x & 7) * per_die + ((int)blockIdx.x >> 3);
     if (piece >= tiles * plan.splits) return;
-    const int split = piece / tiles, tile = piece % tiles;
+    // (each division is 0.1 us in front of the first load: small calls go without)
+    int split = 0, tile = piece;
+    if (plan.splits > 1) split = (unsigned)piece / (unsigned)tiles, tile = piece - split * tiles;
     // blocks of up to 8 row tiles, column tiles within: the 32 workgroups of a die at a time share rows and columns four and
     // more ways (8192 rows of 4096 -> 11008: 877 -> 697 us)
-    const int mblock = tile / (8 * plan.ntiles), mrows = min(8, plan.mtiles - 8 * mblock), in_block = tile - mblock * 8 * plan.ntiles;
-    const int mtile = 8 * mblock + in_block % mrows;
-    int ntile = in_block / mrows;
+    int mtile = 0, ntile = tile, mrows = plan.mtiles;
+    if (mrows > 8) {
+        mtile = (unsigned)tile / (unsigned)(8 * plan.ntiles) * 8;
+        ntile -= mtile * plan.ntiles, mrows = min(8, mrows - mtile);
+    }
+    if (mrows > 1) {
+        const int in_block = ntile;
+        ntile = (unsigned)in_block / (unsigned)mrows, mtile += in_block - ntile * mrows;
+    }
     // selected, not indexed: the arguments arrive with one scalar load
     const int layer = (ntile >= members.first[1] ? 1 : 0) + (ntile >= members.first[2] ? 1 : 0);
     auto of = [&](auto &what) { return layer == 0 ? what[0] : layer == 1 ? what[1] : what[2]; };
@@ -629,35 +644,48 @@ __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(Pro
 #pragma unroll
         for (int m = 0; m < MT; m++)
 #pragma unroll
-            for (int c = 0; c < NC; c++) acc[m][c] = (float4_t){0.f, 0.f, 0.f, 0.f};
+            for (int c = 0; c < NC; c++) {
+                acc[m][c] = (float4_t){0.f, 0.f, 0.f, 0.f};
+                asm volatile("" : "+v"(acc[m][c]));  // written here, not right in front of the first product (prompt_mfma)
+            }
         // the cherry step `cs`; past the last one: step AS - 1 of the units, which is next
         auto load_cherry = [&](int m, int cs) {
             const int u = u0 + (AS - 1) / 4 * WK + wk;
             const bool cherry = cs < csteps + wk, ok = cherry ? cs < csteps : u < u_end;
             return load_a(m, !ok ? 0 : cherry ? 4 * plan.units + cs : 4 * u + (AS - 1) % 4, ok);
         };
+        // (the cherry step's first: it is needed first, and loads return in order)
+#pragma unroll
+        for (int m = 0; m < MT; m++) a[AS - 1][m] = load_cherry(m, wk);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < AS - 1; j++)
 #pragma unroll
             for (int m = 0; m < MT; m++) a[j][m] = load_step(m, j);
-#pragma unroll
-        for (int m = 0; m < MT; m++) a[AS - 1][m] = load_cherry(m, wk);
         __builtin_amdgcn_s_setprio(1);
-        for (int c0 = 0; c0 < csteps; c0 += S * WK) {
+        // The weights' wavefronts wait for the cherries' buffer: it is theirs again when the chunk's last step is in registers, not when its
+        // activations have come and its products are done.
+        auto cherry_step = [&](int s, int next) {
+#pragma unroll
+            for (int c = 0; c < NC; c++) b[c] = frag[STAGE + (s * NC + c) * 64];
+            if (s == S - 1 || next >= csteps) stage_barrier();
+#pragma unroll
+            for (int c = 0; c < NC; c++)
+#pragma unroll
+                for (int m = 0; m < MT; m++) prompt_mfma(acc[m][c], a[AS - 1][m], b[c]);
+#pragma unroll
+            for (int m = 0; m < MT; m++) a[AS - 1][m] = load_cherry(m, next + wk);
+        };
+        if (csteps > 0) {
             stage_barrier();
+            cherry_step(0, WK);  // (not in the loop, whose activations may be those asked for last)
+            for (int c0 = 0, s = 1;; s = 0) {
 #pragma nounroll
-            for (int s = 0; s < S && c0 + s * WK < csteps; s++) {
-                const int next = c0 + (s + 1) * WK;
-#pragma unroll
-                for (int c = 0; c < NC; c++) {
-                    const u32x4 bc = frag[STAGE + (s * NC + c) * 64];
-#pragma unroll
-                    for (int m = 0; m < MT; m++) prompt_mfma(acc[m][c], a[AS - 1][m], bc);
-                }
-#pragma unroll
-                for (int m = 0; m < MT; m++) a[AS - 1][m] = load_cherry(m, next + wk);
+                for (; s < S && c0 + s * WK < csteps; s++) cherry_step(s, c0 + (s + 1) * WK);
+                c0 += S * WK;
+                if (c0 >= csteps) break;
+                stage_barrier();
             }
-            stage_barrier();
         }
         if (csteps == 0) stage_barrier();
 #pragma unroll
@@ -771,38 +799,39 @@ __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(Pro
                     frag[(st & 1) * STAGE + ((sub + NP / WK * i) * NC + c) * 64] = o;
                 }
         };
-        auto fill_cherries = [&](int c0) {
+        // A step's cherry rows.  The first ones are asked for in front of the weights and waited for behind them: one round trip to
+        // memory, not two.
+        s_t cw[8];
+        auto load_cherries = [&](int cs) {
+            const uint32_t off = col_ok ? (uint32_t)((32 * cs + 8 * kq) * N + n0) * 2u : kOobP;
 #pragma unroll
-            for (int i = 0; i < PS; i++) {
-                const int s = sub + NP / WK * i, cs = c0 + s * WK + wk;
-                if (c0 + s * WK >= csteps) break;
-                s_t cw[8];
-                const uint32_t off = col_ok ? (uint32_t)((32 * cs + 8 * kq) * N + n0) * 2u : kOobP;
+            for (int r = 0; r < 8; r++) cw[r] = PromptPiece<NC>::halves(rc, off + (uint32_t)(r * N * 2));
+        };
+        auto fill_cherries = [&](int s) {
 #pragma unroll
-                for (int r = 0; r < 8; r++) cw[r] = PromptPiece<NC>::halves(rc, off + (uint32_t)(r * N * 2));
+            for (int c = 0; c < NC; c++) {
+                u32x4 o;
 #pragma unroll
-                for (int c = 0; c < NC; c++) {
-                    u32x4 o;
-#pragma unroll
-                    for (int d = 0; d < 4; d++)
-                        o[d] = __builtin_amdgcn_perm(cw[2 * d + 1][c >> 1], cw[2 * d][c >> 1], (c & 1) ? 0x07060302u : 0x05040100u);
-                    frag[STAGE + (s * NC + c) * 64] = o;
-                }
+                for (int d = 0; d < 4; d++)
+                    o[d] = __builtin_amdgcn_perm(cw[2 * d + 1][c >> 1], cw[2 * d][c >> 1], (c & 1) ? 0x07060302u : 0x05040100u);
+                frag[STAGE + (s * NC + c) * 64] = o;
             }
         };
+        if (sub * WK < csteps) load_cherries(sub * WK + wk);
+#pragma unroll
+        for (int d = 0; d < D; d++) load(d, d);
         for (int c0 = 0; c0 < csteps; c0 += S * WK) {
             if (c0 > 0) stage_barrier();
-            fill_cherries(c0);
-            if (c0 == 0) {
 #pragma unroll
-                for (int d = 0; d < D; d++) load(d, d);
+            for (int i = 0; i < PS; i++) {
+                const int s = sub + NP / WK * i;
+                if (c0 + s * WK >= csteps) break;
+                if (i > 0) load_cherries(c0 + s * WK + wk);
+                fill_cherries(s);
             }
             if (c0 + S * WK >= csteps) break;
+            if (c0 + (S + sub) * WK < csteps) load_cherries(c0 + (S + sub) * WK + wk);
             stage_barrier();
-        }
-        if (csteps == 0) {
-#pragma unroll
-            for (int d = 0; d < D; d++) load(d, d);
         }
         fill(0, 0);
         load(0, D);
