@@ -743,8 +743,6 @@ class CherryLlamaDecoder(nn.Module):
         cos, sin = self._rope_tables(T)
         self.reset()
         h = self.embed_tokens[ids]
-        attend = self._prefill_attention(T, cos, sin) if hd == 128 else self._prefill_attention_torch(T, cos, sin)
-
         # The launches read raw memory.  What a hook, a replaced module or a cast of the decoder makes of a tensor goes
         # through the torch operations they stand for, which take it or say what does not fit.
         def add_norm(h, delta, weight, n=T, y=None):  # h + delta (in h's place where the launch forms it), its RMSNorm (in y)
@@ -782,6 +780,8 @@ class CherryLlamaDecoder(nn.Module):
             return act
 
         delta = self._prefill_layers(h, cos, sin) if hd == 128 and T >= 17 else None
+        if delta is None:
+            attend = (self._prefill_attention if hd == 128 else self._prefill_attention_torch)(T, cos, sin)
         # What a module reads or returns is written once: a hook or a replaced module may keep it.
         for li, layer in enumerate(self.layers if delta is None else ()):
             h, x = add_norm(h, delta, layer.input_layernorm)
@@ -847,7 +847,8 @@ class CherryLlamaDecoder(nn.Module):
         if not nbytes:
             return None
         ws = quant_cuda._workspace(h.device, stream, _lib.cherryq_prefill_layers_workspace_bytes(layers, n, T))
-        sc, delta = quant_cuda._scratch(h.device, stream, nbytes), torch.empty_like(h)
+        # of the pass: for a long prompt hundreds of MB, which the buffers kept for a stream would not give back
+        sc, delta = torch.empty(nbytes, dtype=torch.uint8, device=h.device), torch.empty_like(h)
         rc = _lib.cherryq_prefill_layers_f16(layers, n, h.data_ptr(), delta.data_ptr(), cos.data_ptr(), sin.data_ptr(), T, hidden,
                                              cfg.num_attention_heads, cfg.num_key_value_heads, ml, cfg.rms_norm_eps, ws.data_ptr(),
                                              ws.numel(), sc.data_ptr(), sc.numel(), stream)

@@ -345,3 +345,22 @@ def test_first_pass_under_capture(dec):
         torch.cuda.synchronize()
         for got, w in zip((model.logits, model.k_cache, model.v_cache), want):
             assert torch.equal(got, w)
+
+
+def test_a_pass_gives_its_memory_back(dec):
+    """The native pass leaves nothing in the scratch buffer kept for its stream, and none of its tensors allocated."""
+    print("[case] prefill memory", flush=True)
+    import quant_cuda
+    cfg = dec.DecoderConfig(hidden_size=512, intermediate_size=1408, num_hidden_layers=2, num_attention_heads=4,
+                            num_key_value_heads=2, vocab_size=512, max_position_embeddings=512)
+    model, stream = dec.CherryLlamaDecoder(cfg, seed=1), torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        model.prefill(torch.arange(40, device="cuda"))  # the stream's workspace
+        ids = torch.arange(400, device="cuda")
+        kept = quant_cuda._host.scratch(0, stream.cuda_stream, 8).numel()  # 8 where there was none
+        before = torch.cuda.memory_allocated()
+        model.prefill(ids)
+        assert torch.cuda.memory_allocated() == before
+        assert quant_cuda._host.scratch(0, stream.cuda_stream, 8).numel() == kept
+    torch.cuda.synchronize()
