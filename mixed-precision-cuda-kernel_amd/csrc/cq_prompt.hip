@@ -12,16 +12,17 @@
 //     MFMAs hardly overlaps them, and one weight is decoded once for all of a tile's rows;
 //   * loads of a wavefront return in order.  Activations (L2) that wait behind weights (HBM) in the same wavefront take HBM's
 //     latency in every step; here neither waits for the other.
-// Measured, 4 bits, preparation included (us), against the kernel that this replaces (every wavefront decoded its own operands
-// between its MFMAs and shared K with the others):
-//     rows              17      64     128     256     512    1024    2048
-//     4096 -> 11008   16.9    20.3    27.1    37.0    54.8     107     174
-//             before  17.4    20.9    28.5    38.9    63.6     109     186
-//     4096 -> 4096    12.3    14.4    17.9    22.3    30.5    44.3    69.1
-//             before  11.9    14.9    17.7    22.0    31.4    44.9    73.2
-//     11008 -> 4096   17.0    21.3    28.6    43.9    65.3     102     168
-//             before  17.6    21.9    31.1    45.6    68.3    96.7     173
-// (sizes that tiles or dies divide badly gain more: 60 drawn calls together 13 %, 75 rows of 22272 -> 4592 82 -> 42 us)
+// Tiles of few rows over 64 columns are another kernel's, without LDS in the loop (prompt_shared_k_kernel); it was the only one, with
+// larger tiles too.  Measured since there are both, 4 bits, the same call repeated, preparation included (us):
+//     rows                  17      64     128     256     512    1024    2048
+//     4096 -> 11008       15.1    18.3    24.7    36.3    54.0     105     172
+//     shared K alone      15.5    18.8    26.6    38.9    63.3     109     187
+//     4096 -> 4096        11.1    12.4    14.2    18.3    29.5    42.2    66.6
+//     shared K alone      11.4    14.0    14.8    19.1    31.8    43.9    71.7
+//     11008 -> 4096       15.0    20.6    27.4    39.9    63.7    95.1     162
+//     shared K alone      15.5    20.9    31.3    46.6    68.8    92.7     169
+// 110 drawn calls together take 16 % less than with shared K alone.  Slower are few large ones: 1827 rows of 24808 -> 4120 382 -> 408, whose
+// tiles of 128 x 256 were one round of 255 workgroups where 128 x 128 are two, and 1024 of 11008 -> 4096.
 // A lone wavefront's dependent vector instructions issue every 8 clocks, beside MFMAs every 12, and an operand of 512
 // weights takes 17: with 128 rows a tile the decode is the longer half, with 256 it is hidden.  At 2048 rows the clock falls to 1.95 GHz
 // (of 2.4) under the MFMAs' power: 32 accumulators of random numbers alone reach 1.5 PFLOP/s on this card for longer than 100 us.
@@ -76,53 +77,55 @@ static_assert(prompt_ord<4>(1) == 2 && prompt_ord<4>(2) == 1 && prompt_ord<4>(5)
 // sharing K, and NP wavefronts of weights.  They meet after every S steps of 32 positions a K share; activations are asked
 // for AS steps ahead, weights D meetings.
 //   Tiles of 64 columns have four K shares: small tiles want every one of the few workgroups to itself.  Eight wavefronts of
-// weights where registers allow three a SIMD and there are few products to hide the decode behind (32 and 48 rows: 17.5 -> 16.7
-// us at 4096 -> 11008).  128 columns are eight operands of weights to four of activations, half the bytes a
-// product from the L2; 256 rows decode a weight once for them all.
-// Two small workgroups a compute unit help where there are more tiles than compute units (23 rows of 7456 -> 8832 in 3 bits
-// 24.3 -> 20.3 us).
+// weights where registers allow three a SIMD and there are few products to hide the decode behind.  128 columns are eight operands of
+// weights to four of activations, half the bytes a product from the L2; 256 rows decode a weight once for them all.
+// Two small workgroups a compute unit help where there are more tiles than compute units.
 //        id MT NC WM WK S AS NP D
 #define CQ_PROMPT_SHAPES(X)      \
-    X(0, 2, 4, 1, 4, 2, 4, 8, 3) \
-    X(1, 3, 4, 1, 4, 2, 4, 8, 2) \
-    X(2, 4, 4, 1, 4, 2, 4, 4, 3) \
-    X(3, 5, 4, 1, 4, 4, 4, 4, 2) \
-    X(4, 7, 4, 1, 4, 4, 4, 4, 2) \
-    X(5, 4, 4, 2, 2, 4, 4, 4, 2) \
-    X(6, 3, 8, 2, 2, 4, 4, 4, 2) \
-    X(7, 4, 8, 2, 2, 4, 4, 4, 2) \
-    X(8, 3, 8, 4, 1, 4, 4, 4, 2) \
-    X(9, 4, 8, 4, 1, 4, 4, 4, 2) \
-    X(10, 2, 4, 1, 4, 2, 4, 4, 3) \
-    X(11, 3, 4, 1, 4, 2, 4, 4, 2) \
-    X(12, 1, 4, 1, 4, 2, 4, 8, 3) \
-    X(13, 1, 4, 1, 4, 2, 4, 4, 3)
+    X(0, 3, 4, 1, 4, 2, 4, 8, 2) \
+    X(1, 5, 4, 1, 4, 4, 4, 4, 2) \
+    X(2, 7, 4, 1, 4, 4, 4, 4, 2) \
+    X(3, 4, 4, 2, 2, 4, 4, 4, 2) \
+    X(4, 3, 8, 2, 2, 4, 4, 4, 2) \
+    X(5, 4, 8, 2, 2, 4, 4, 4, 2) \
+    X(6, 3, 8, 4, 1, 4, 4, 4, 2) \
+    X(7, 4, 8, 4, 1, 4, 4, 4, 2) \
+    X(8, 3, 4, 1, 4, 2, 4, 4, 2) \
+    X(9, 1, 4, 1, 4, 2, 4, 8, 3) \
+    X(10, 1, 4, 1, 4, 2, 4, 4, 3)
+// ... and of the kernel whose eight wavefronts share K and decode their own operands: 16 MT rows x 64 columns.
+//        id MT
+#define CQ_SHARED_K_SHAPES(X) \
+    X(11, 2)                  \
+    X(12, 4)
 
-// What a call takes with a tile shape, in microseconds, preparation included: a fit to 43000 measured calls (3 and 4 bits, K 1024
-// to 28672, N 512 to 28672, M 4 to 2048, 1 to 16 K splits).  `first`: a launch with one round of workgroups and no unit; `round`:
-// each further round; `unit`: 128 positions a K share, 1 + crowd times as long when all compute units are at it; `split`,
-// `mbyte`, `tile`: a split call, each megabyte of its partial tiles, and each 32 KB that its last workgroup reads; `rows`:
-// 1e6 M K.  Its choices are 0.3 % slower than the best measured ones on average, 5 % at the 99th percentile.
+// What a call takes with a tile shape, in microseconds, preparation included.  `first`: a launch with one round of workgroups and no unit;
+// `round`: each further round; `share`: a round's 128 positions of a K share, `unit`: of the workgroup; `crowd`: what a share's take longer
+// when all compute units are at it; `split`, `mbyte`, `tile`: a split call, each megabyte of its partial tiles, and each 32 KB that
+// its last workgroup reads; `rows`: 1e6 M K.
 // 1 << `per`: workgroups that a die of 32 compute units takes at a time; `crowd` of the pairs counts once there is a second one.
+//   The numbers are a fit, and stale once a kernel changes: 3100 calls drawn over the logarithm of their sizes (3 and 4 bits, K 1024 to
+// 28672, N 512 to 28672, M 5 to 2048, groups of 128, K / 256 cherries), each timed in a graph of 20 with every shape and 1 to 16 K
+// splits (100000 times), least squares of the relative error per shape, those within 15 % of their call's best four times as heavy.
+// The choices are 0.5 % slower than the best measured on average, 8 % at the 99th percentile, 13 % at worst.
 struct PromptCost {
     int per;
-    float first, round, unit, crowd, split, mbyte, rows, tile;
+    float first, round, share, unit, crowd, split, mbyte, rows, tile;
 };
 constexpr PromptCost kPromptCosts[] = {
-    {5, 6.27f, 1.87f, 1.23f, 0.002f, 0.560f, 0.738f, 1.87f, 1.10f},  // 32 x 64
-    {5, 6.37f, 2.07f, 1.41f, 0.007f, 0.600f, 0.688f, 1.88f, 0.736f},  // 48 x 64
-    {5, 6.76f, 2.19f, 1.50f, 0.024f, 0.753f, 0.631f, 1.73f, 0.720f},  // 64 x 64
-    {5, 7.31f, 2.56f, 1.66f, 0.000f, 0.894f, 0.575f, 1.52f, 0.718f},  // 80 x 64
-    {5, 7.55f, 2.76f, 2.03f, 0.000f, 1.59f, 0.501f, 1.19f, 0.648f},  // 112 x 64
-    {5, 6.91f, 1.97f, 1.18f, 0.000f, 1.31f, 0.502f, 1.23f, 0.647f},  // 128 x 64
-    {5, 8.63f, 4.92f, 1.25f, 0.148f, 2.68f, 0.350f, 1.19f, 0.564f},  // 96 x 128
-    {5, 10.04f, 6.30f, 1.35f, 0.272f, 2.76f, 0.297f, 0.960f, 0.574f},  // 128 x 128
-    {5, 9.64f, 6.38f, 0.896f, 0.288f, 2.38f, 0.366f, 0.892f, 0.565f},  // 192 x 128
-    {5, 10.76f, 7.50f, 1.12f, 0.276f, 2.16f, 0.379f, 0.839f, 0.563f},  // 256 x 128
-    {6, 6.19f, 0.538f, 1.27f, 0.835f, 1.14f, 0.324f, 1.92f, 0.942f},  // 32 x 64, two a compute unit
-    {6, 6.54f, 0.366f, 1.40f, 0.911f, 0.909f, 0.465f, 2.11f, 0.985f},  // 48 x 64, two a compute unit
-    {5, 6.15f, 1.94f, 0.996f, 0.076f, 0.703f, 0.955f, 1.59f, 2.11f},  // 16 x 64
-    {6, 5.86f, 0.945f, 1.10f, 0.843f, 0.995f, 0.555f, 2.19f, 2.14f},  // 16 x 64, two a compute unit
+    {5, 6.46f, 2.62f, 0.597f, 0.108f, 0.3f, 0.981f, 0.455f, 1.7f, 0.622f},  // 48 x 64
+    {5, 8.12f, 3.55f, 0.773f, 0.126f, 0.337f, 0.868f, 0.459f, 1.29f, 0.626f},  // 80 x 64
+    {5, 8.87f, 4.21f, 0.867f, 0.187f, 0.348f, 1.35f, 0.405f, 1.14f, 0.533f},  // 112 x 64
+    {5, 7.07f, 2.9f, 0.426f, 0.249f, 0.236f, 1.6f, 0.396f, 1.16f, 0.58f},  // 128 x 64
+    {5, 9.16f, 5.39f, 0.668f, 0.217f, 0.372f, 1.93f, 0.342f, 0.941f, 0.596f},  // 96 x 128
+    {5, 10.1f, 6.93f, 0.776f, 0.195f, 0.535f, 2.53f, 0.28f, 0.909f, 0.617f},  // 128 x 128
+    {5, 9.83f, 6.52f, 0.392f, 0.392f, 0.392f, 1.84f, 0.33f, 0.901f, 0.599f},  // 192 x 128
+    {5, 11.3f, 7.91f, 0.462f, 0.462f, 0.522f, 1.38f, 0.343f, 0.925f, 0.583f},  // 256 x 128
+    {6, 6.75f, 1.49f, 0.896f, 0.115f, 1.09f, 0.566f, 0.446f, 1.52f, 0.972f},  // 48 x 64, two a compute unit
+    {5, 6.31f, 2.47f, 0.478f, 0.082f, 0.236f, 0.653f, 0.353f, 0.219f, 2.11f},  // 16 x 64
+    {6, 6.04f, 0.1f, 0.745f, 0.088f, 0.727f, 0.666f, 0.535f, 0.312f, 2.11f},  // 16 x 64, two a compute unit
+    {6, 5.45f, 0.0612f, 0.0f, 0.285f, 1.68f, 0.991f, 0.513f, 1.76f, 0.776f},  // 32 x 64, shared K, two a compute unit
+    {5, 5.77f, 2.25f, 0.0f, 0.304f, 0.664f, 1.25f, 0.419f, 1.75f, 0.622f},  // 64 x 64, shared K
 };
 struct PromptShape {
     int mt, nc, wm, wk;
@@ -130,6 +133,9 @@ struct PromptShape {
 constexpr PromptShape kPromptShapes[] = {
 #define CQ_SHAPE_ROW(ID, MT, NC, WM, WK, S, AS, NP, D) {MT, NC, WM, WK},
     CQ_PROMPT_SHAPES(CQ_SHAPE_ROW)
+#undef CQ_SHAPE_ROW
+#define CQ_SHAPE_ROW(ID, MT) {MT, 4, 1, 8},
+    CQ_SHARED_K_SHAPES(CQ_SHAPE_ROW)
 #undef CQ_SHAPE_ROW
 };
 constexpr int kPromptShapeCount = sizeof(kPromptShapes) / sizeof(kPromptShapes[0]);
@@ -183,9 +189,10 @@ static PromptPlan find_prompt_plan(int M, int K, const int *N, int count, int C)
             if (p.splits < splits) continue;  // the same plan as with fewer
             // workgroups are dealt to eight dies of 32 compute units: the fullest die counts
             const unsigned load = (unsigned)((tiles * splits + 7) / 8), full = load >> f.per, rest = load & ((1u << f.per) - 1u);
-            const float crowd = f.crowd * (f.per == 5 ? (float)rest / 32.f : rest > 32 ? 1.f : 0.f);
-            float cost = f.first + f.round * (float)(full + (rest > 0) - 1) + f.rows * 1e-6f * (float)M * (float)K +
-                         f.unit * (float)ceil_div(p.units_per_split, s.wk) * ((float)full * (1.f + f.crowd) + (rest > 0 ? 1.f + crowd : 0.f));
+            const float rounds = (float)(full + (rest > 0)), crowd = (float)full + (f.per == 5 ? (float)rest / 32.f : rest > 32 ? 1.f : 0.f);
+            const float shares = (float)ceil_div(p.units_per_split, s.wk);
+            float cost = f.first + f.round * (rounds - 1.f) + f.rows * 1e-6f * (float)M * (float)K +
+                         (f.share * shares + f.unit * (float)p.units_per_split) * rounds + f.crowd * shares * crowd;
             if (splits > 1) cost += f.split + f.mbyte * (float)(tiles * splits) * kbytes * 1.024e-3f + f.tile * splits * kbytes / 32.f;
             p.cost = cost;
             if (cost < best_cost) best_cost = cost, best = p;
@@ -546,6 +553,12 @@ __device__ __forceinline__ void prompt_mfma(float4_t &acc, const u32x4 &a, const
 __device__ __forceinline__ void prompt_mfma_first(float4_t &acc, const u32x4 &a, const u32x4 &b) {
     asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
 }
+// In front of products whose operands vector instructions have just written.
+__device__ __forceinline__ void operands_written() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 1");
+    __builtin_amdgcn_sched_barrier(0);
+}
 __device__ __forceinline__ void mfma_drain() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
 
 // The wavefront's LDS accesses are done before it arrives; loads from memory stay in flight.
@@ -581,6 +594,110 @@ struct PromptPiece {
     }
 };
 
+// Where a workgroup is: its K split, its tile among all, and the tile's layer, row tile and column tile.
+struct PromptPlace {
+    int split, tile, layer, mtile, ntile;
+};
+__device__ __forceinline__ bool prompt_place(const PromptMembers &members, const PromptPlan &plan, PromptPlace &p) {
+    const int tiles = plan.mtiles * plan.ntiles, per_die = (tiles * plan.splits + 7) >> 3;  // the grid is 8 times that
+    const int piece = ((int)blockIdx.x & 7) * per_die + ((int)blockIdx.x >> 3);
+    if (piece >= tiles * plan.splits) return false;
+    // (each division is 0.1 us in front of the first load: small calls go without)
+    p.split = 0, p.tile = piece;
+    if (plan.splits > 1) p.split = (unsigned)piece / (unsigned)tiles, p.tile = piece - p.split * tiles;
+    // blocks of up to 8 row tiles, column tiles within: the 32 workgroups of a die at a time share rows and columns four and
+    // more ways (8192 rows of 4096 -> 11008: 877 -> 697 us)
+    p.mtile = 0, p.ntile = p.tile;
+    int mrows = plan.mtiles;
+    if (mrows > 8) {
+        p.mtile = (unsigned)p.tile / (unsigned)(8 * plan.ntiles) * 8;
+        p.ntile -= p.mtile * plan.ntiles, mrows = min(8, mrows - p.mtile);
+    }
+    if (mrows > 1) {
+        const int in_block = p.ntile;
+        p.ntile = (unsigned)in_block / (unsigned)mrows, p.mtile += in_block - p.ntile * mrows;
+    }
+    p.layer = (p.ntile >= members.first[1] ? 1 : 0) + (p.ntile >= members.first[2] ? 1 : 0);
+    p.ntile -= p.layer == 0 ? 0 : p.layer == 1 ? members.first[1] : members.first[2];
+    return true;
+}
+// A member's value, selected, not indexed: the arguments arrive with one scalar load
+template <typename T>
+__device__ __forceinline__ T prompt_of(const T (&what)[kPromptMaxGroup], int layer) {
+    return layer == 0 ? what[0] : layer == 1 ? what[1] : what[2];
+}
+
+// A tile's results, QUADS x 4 columns a thread (quad q T + tid of the tile): across workgroups where K is split, then to the output.
+template <int ROWS, int COLS, int T, int QUADS>
+__device__ __forceinline__ void prompt_finish(float4 (&sum)[QUADS], void *shared, const PromptPlace &at, const PromptPlan &plan,
+                                              float *__restrict__ partial, unsigned *__restrict__ tickets, __half *__restrict__ out, int M,
+                                              int N, int accumulate) {
+    const int tid = threadIdx.x;
+    // ---- across workgroups: tiles in scratch in the order [quad][thread]
+    if (plan.splits > 1) {
+        constexpr size_t TILE = (size_t)ROWS * COLS;
+        float *base = partial + (size_t)at.tile * TILE + tid * 4;
+        const size_t per_split = (size_t)(plan.mtiles * plan.ntiles) * TILE;
+        auto has = [&](int q) { return ROWS * COLS / 4 % T == 0 || tid + q * T < ROWS * COLS / 4; };
+        auto word = [&](int s, int q, int h) { return reinterpret_cast<unsigned long long *>(base + s * per_split + (size_t)q * (4 * T)) + h; };
+#pragma unroll
+        for (int q = 0; q < QUADS; q++) {
+            if (!has(q)) break;
+            const float2 lo = make_float2(sum[q].x, sum[q].y), hi = make_float2(sum[q].z, sum[q].w);
+            __hip_atomic_store(word(at.split, q, 0), __builtin_bit_cast(unsigned long long, lo), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(word(at.split, q, 1), __builtin_bit_cast(unsigned long long, hi), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();  // the sums are read
+        int *s_last = reinterpret_cast<int *>(shared);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (tid == 0) {
+            const unsigned old = __hip_atomic_fetch_add(&tickets[at.tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            *s_last = old == (unsigned)(plan.splits - 1);
+        }
+        __syncthreads();
+        if (!*s_last) return;
+        if (tid == 0) __hip_atomic_store(&tickets[at.tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int q = 0; q < QUADS; q++) sum[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 2
+        for (int s = 0; s < plan.splits; s++) {
+            float2 v[QUADS][2];
+#pragma unroll
+            for (int q = 0; q < QUADS; q++)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    v[q][h] = has(q) ? __builtin_bit_cast(float2, __hip_atomic_load(word(s, q, h), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                                     : make_float2(0.f, 0.f);
+#pragma unroll
+            for (int q = 0; q < QUADS; q++) {
+                sum[q].x += v[q][0].x, sum[q].y += v[q][0].y;
+                sum[q].z += v[q][1].x, sum[q].w += v[q][1].y;
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < QUADS; q++) {
+        const int e = tid + q * T, row = e / (COLS / 4), m = at.mtile * ROWS + row, n = at.ntile * COLS + e % (COLS / 4) * 4;
+        if (row < ROWS && m < M && n < N) {
+            uint2 *o = reinterpret_cast<uint2 *>(out + (size_t)m * N + n);
+            float v[4] = {sum[q].x, sum[q].y, sum[q].z, sum[q].w};
+            if (accumulate) {
+                const uint2 was = *o;
+                v[0] += __half2float(__ushort_as_half((unsigned short)was.x));
+                v[1] += __half2float(__ushort_as_half((unsigned short)(was.x >> 16)));
+                v[2] += __half2float(__ushort_as_half((unsigned short)was.y));
+                v[3] += __half2float(__ushort_as_half((unsigned short)(was.y >> 16)));
+            }
+            uint32_t h[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) h[c] = __half_as_ushort(__float2half_rn(v[c]));
+            *o = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+        }
+    }
+}
+
 // WHOLE: groups are whole units.  Then a tile of 16 rows takes codes u - c_b as operands and scales a stage's sums, in fp32: 16
 // multiplications for 64 in the decode, and no rounding of the weights.
 template <int BITS, int MT, int NC, int WM, int WK, int S, int AS, int NP, int D, bool WHOLE>
@@ -602,29 +719,10 @@ __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(Pro
     // are 0.3 to 0.6 us shorter: 102 rows of 1248 -> 2784 9.95 -> 9.4, 18 of 1360 -> 12520 in 3 bits 10.0 -> 9.3.)
     asm volatile("" ::"s"(members.qweight[0]), "s"(members.scales[2]), "s"(members.first[2]), "s"(K), "s"(plan.steps), "s"(plan.partial_bytes));
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kq = lane >> 4, nl = lane & 15;
-    const int tiles = plan.mtiles * plan.ntiles, per_die = (tiles * plan.splits + 7) >> 3;  // the grid is 8 times that
-    const int piece = ((int)blockIdx.x & 7) * per_die + ((int)blockIdx.x >> 3);
-    if (piece >= tiles * plan.splits) return;
-    // (each division is 0.1 us in front of the first load: small calls go without)
-    int split = 0, tile = piece;
-    if (plan.splits > 1) split = (unsigned)piece / (unsigned)tiles, tile = piece - split * tiles;
-    // blocks of up to 8 row tiles, column tiles within: the 32 workgroups of a die at a time share rows and columns four and
-    // more ways (8192 rows of 4096 -> 11008: 877 -> 697 us)
-    int mtile = 0, ntile = tile, mrows = plan.mtiles;
-    if (mrows > 8) {
-        mtile = (unsigned)tile / (unsigned)(8 * plan.ntiles) * 8;
-        ntile -= mtile * plan.ntiles, mrows = min(8, mrows - mtile);
-    }
-    if (mrows > 1) {
-        const int in_block = ntile;
-        ntile = (unsigned)in_block / (unsigned)mrows, mtile += in_block - ntile * mrows;
-    }
-    // selected, not indexed: the arguments arrive with one scalar load
-    const int layer = (ntile >= members.first[1] ? 1 : 0) + (ntile >= members.first[2] ? 1 : 0);
-    auto of = [&](auto &what) { return layer == 0 ? what[0] : layer == 1 ? what[1] : what[2]; };
-    __half *__restrict__ const out = of(members.out);
-    const int N = of(members.N);
-    ntile -= of(members.first);
+    PromptPlace at;
+    if (!prompt_place(members, plan, at)) return;
+    const int split = at.split, mtile = at.mtile, ntile = at.ntile, layer = at.layer, N = prompt_of(members.N, layer);
+    __half *__restrict__ const out = prompt_of(members.out, layer);
     const int u0 = split * plan.units_per_split, u_end = min(u0 + plan.units_per_split, plan.units);
     const int stages = ceil_div(u_end - u0, WK) * (4 / S);
     // cherry steps: the last split's, a chunk of S a K share at a time
@@ -757,9 +855,9 @@ __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(Pro
         __builtin_amdgcn_sched_barrier(0);
     } else {
         // ---- weights
-        const uint8_t *__restrict__ const qweight = of(members.qweight);
-        const __half *__restrict__ const cherry_weight = of(members.cherry_weight);
-        const __half *__restrict__ const scales = of(members.scales);
+        const uint8_t *__restrict__ const qweight = prompt_of(members.qweight, layer);
+        const __half *__restrict__ const cherry_weight = prompt_of(members.cherry_weight, layer);
+        const __half *__restrict__ const scales = prompt_of(members.scales, layer);
         const int Kn = K - C, wk = (wave - 4) / (NP / WK), sub = (wave - 4) % (NP / WK);
         const int n0 = ntile * COLS + NC * nl;
         const bool col_ok = n0 < N;
@@ -894,69 +992,173 @@ __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(Pro
             sum[q].x += o.x, sum[q].y += o.y, sum[q].z += o.z, sum[q].w += o.w;
         }
     }
-    // ---- across workgroups: tiles in scratch in the order [quad][thread]
-    if (plan.splits > 1) {
-        constexpr size_t TILE = (size_t)ROWS * COLS;
-        float *base = partial + (size_t)tile * TILE + tid * 4;
-        const size_t per_split = (size_t)tiles * TILE;
-        auto has = [&](int q) { return ROWS * COLS / 4 % T == 0 || tid + q * T < ROWS * COLS / 4; };
-        auto word = [&](int s, int q, int h) { return reinterpret_cast<unsigned long long *>(base + s * per_split + (size_t)q * (4 * T)) + h; };
+    prompt_finish<ROWS, COLS, T, QUADS>(sum, s_b, at, plan, partial, tickets, out, M, N, accumulate);
+}
+
+// ---- few units of K, few rows --------------------------------------------------------------------------
+// Tiles of 32 and 64 rows x 64 columns: the eight wavefronts share K, unit by unit, and each decodes its own operands in registers between
+// its products, a few instructions behind each (the scheduling barriers keep the order), so that nothing passes through LDS and nobody
+// waits at a barrier before the results meet at the end.  With two and four products an operand the kernel above is bound by LDS (32 KB
+// written and read a stage of 950 clocks) and, where K is short, by its start, a chain of load, decode, LDS and barrier; beyond 64 rows
+// a decode a wavefront costs more.  Best of all shapes for 36 % of 3100 drawn calls (us, the kernel above -> this one: 102 rows of
+// 1248 -> 2784 9.4 -> 8.6, 18 of 1360 -> 12520 in 3 bits 9.3 -> 8.7, 17 of 4096 -> 4096 12.6 -> 11.1, 64 13.2 -> 12.4).
+// Bound by the decode's vector instructions, and by one round trip to memory at the start.
+// A step's packed bytes are reloaded for the wavefront's next unit as soon as they are decoded, the activations as soon as their last
+// product is issued.
+template <int BITS, int MT, bool WHOLE>
+__global__ __launch_bounds__(512, MT == 2 ? 4 : 2) void prompt_shared_k_kernel(PromptMembers members, const u32x4 *__restrict__ a_all,
+                                                                        float *__restrict__ partial, unsigned *__restrict__ tickets, int M,
+                                                                        int K, int C, int G, unsigned group_magic, int accumulate,
+                                                                        PromptPlan plan) {
+    constexpr int KW = 8, NC = 4, COLS = 64, ROWS = 16 * MT, T = 64 * KW;
+    typedef typename PromptPiece<NC>::s_t s_t;
+    __shared__ __attribute__((aligned(16))) float s_red[KW][ROWS][COLS];
+    asm volatile("" ::"s"(members.qweight[0]), "s"(members.scales[2]), "s"(members.first[2]), "s"(K), "s"(plan.steps), "s"(plan.partial_bytes));
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kq = lane >> 4, nl = lane & 15;
+    PromptPlace at;
+    if (!prompt_place(members, plan, at)) return;
+    const uint8_t *__restrict__ const qweight = prompt_of(members.qweight, at.layer);
+    const __half *__restrict__ const cherry_weight = prompt_of(members.cherry_weight, at.layer);
+    const __half *__restrict__ const scales = prompt_of(members.scales, at.layer);
+    __half *__restrict__ const out = prompt_of(members.out, at.layer);
+    const u32x4 *const a_frag = a_all + at.layer * (plan.a_bytes / sizeof(u32x4));
+    const int N = prompt_of(members.N, at.layer), n0 = at.ntile * COLS + NC * nl, m16 = plan.mtiles * MT, Kn = K - C;
+    const bool col_ok = n0 < N;
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)qweight, 0, Kn / 8 * BITS * N, kRsrcFlagsP);
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)scales, 0, ceil_div(Kn, G) * N * 2, kRsrcFlagsP);
+    const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc((void *)cherry_weight, 0, C * N * 2, kRsrcFlagsP);
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)a_frag, 0, plan.steps * m16 * 1024, kRsrcFlagsP);
+
+    uint32_t w[4][BITS];
+    s_t sc[WHOLE ? 2 : 4];
+    u32x4 a[MT], b[2][NC];
+    // Units past the wavefront's last one are asked for as unit `plan.units`, which lies past the end of the packed bytes:
+    // the bounds of the buffer answer with zeros.
+    const uint32_t w_lane = col_ok ? (uint32_t)(kq * BITS * N + n0) : kOobP, sc_lane = col_ok ? (uint32_t)n0 * 2u : kOobP;
+    auto load_w = [&](int s, int u) {
+        const uint32_t off = w_lane + (uint32_t)((u * 4 + s) * 4 * BITS * N);
 #pragma unroll
-        for (int q = 0; q < QUADS; q++) {
-            if (!has(q)) break;
-            const float2 lo = make_float2(sum[q].x, sum[q].y), hi = make_float2(sum[q].z, sum[q].w);
-            __hip_atomic_store(word(split, q, 0), __builtin_bit_cast(unsigned long long, lo), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(word(split, q, 1), __builtin_bit_cast(unsigned long long, hi), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int r = 0; r < BITS; r++) w[s][r] = PromptPiece<NC>::codes(rw, off + (uint32_t)(r * N))[0];
+    };
+    auto load_sc = [&](int s, int u) {
+        return PromptPiece<NC>::halves(rs, sc_lane + __umulhi(2u * (unsigned)(4 * u + s), group_magic) * (uint32_t)N * 2u);
+    };
+    auto load_a = [&](int m, int step) {
+        return __builtin_amdgcn_raw_buffer_load_b128(ra, lane * 16, (step * m16 + at.mtile * MT + m) * 1024, 0);
+    };
+    const PromptDecode<BITS> decoder;
+    PromptColumn<BITS> column;
+    auto decode = [&](int s, const s_t &scale, int c, int g, u32x4 &o) {
+        column.template group<true>(decoder, g, w[s], c, scale[c >> 1], o);
+    };
+
+    float4_t acc[MT][NC];
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            acc[m][c] = (float4_t){0.f, 0.f, 0.f, 0.f};
+            asm volatile("" : "+v"(acc[m][c]));  // written here, not right in front of the first product (prompt_mfma)
         }
-        __syncthreads();  // the sums are read
-        int *s_last = reinterpret_cast<int *>(s_b);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        if (tid == 0) {
-            const unsigned old = __hip_atomic_fetch_add(&tickets[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            *s_last = old == (unsigned)(plan.splits - 1);
+
+    const int u0 = at.split * plan.units_per_split + wave, u_end = min((at.split + 1) * plan.units_per_split, plan.units);
+    auto unit_after = [&](int u) { return u + KW < u_end ? u + KW : plan.units; };
+    if (u0 < u_end) {
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            load_w(s, u0);
+            if (!WHOLE || s == 0) sc[s] = load_sc(s, u0);
         }
-        __syncthreads();
-        if (!*s_last) return;
-        if (tid == 0) __hip_atomic_store(&tickets[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (WHOLE) sc[1] = load_sc(0, unit_after(u0));
+    }
+    // Cherry steps (32 dense fp16 rows, 8 per lane group) while the packed bytes are on their way: behind the loop their own
+    // round trip to memory would be one more.
+    if (at.split == plan.splits - 1) {
+        for (int cs = KW - 1 - wave; cs < plan.csteps; cs += KW) {
+            s_t cw[8];
+            const uint32_t off = col_ok ? (uint32_t)((32 * cs + 8 * kq) * N + n0) * 2u : kOobP;
 #pragma unroll
-        for (int q = 0; q < QUADS; q++) sum[q] = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll 2
-        for (int s = 0; s < plan.splits; s++) {
-            float2 v[QUADS][2];
+            for (int r = 0; r < 8; r++) cw[r] = PromptPiece<NC>::halves(rc, off + (uint32_t)(r * N * 2));
 #pragma unroll
-            for (int q = 0; q < QUADS; q++)
+            for (int m = 0; m < MT; m++) a[m] = load_a(m, plan.units * 4 + cs);
 #pragma unroll
-                for (int h = 0; h < 2; h++)
-                    v[q][h] = has(q) ? __builtin_bit_cast(float2, __hip_atomic_load(word(s, q, h), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                                     : make_float2(0.f, 0.f);
+            for (int c = 0; c < NC; c++) {
 #pragma unroll
-            for (int q = 0; q < QUADS; q++) {
-                sum[q].x += v[q][0].x, sum[q].y += v[q][0].y;
-                sum[q].z += v[q][1].x, sum[q].w += v[q][1].y;
+                for (int d = 0; d < 4; d++)
+                    b[0][c][d] = __builtin_amdgcn_perm(cw[2 * d + 1][c >> 1], cw[2 * d][c >> 1], (c & 1) ? 0x07060302u : 0x05040100u);
             }
+            operands_written();
+#pragma unroll
+            for (int c = 0; c < NC; c++)
+#pragma unroll
+                for (int m = 0; m < MT; m++) prompt_mfma(acc[m][c], a[m], b[0][c]);
         }
     }
+    if (u0 < u_end) {
+#pragma unroll
+        for (int m = 0; m < MT; m++) a[m] = load_a(m, u0 * 4);
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+#pragma unroll
+            for (int g = 0; g < 8; g++) decode(0, sc[0], c, g, b[0][c]);
+        load_w(0, unit_after(u0));
+        if (!WHOLE) sc[0] = load_sc(0, unit_after(u0));
+    }
+#pragma nounroll
+    for (int u = u0; u < u_end;) {
+        const int un = unit_after(u), unn = unit_after(un);
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const int t = (s + 1) & 3;
+            const int next = s < 3 ? u * 4 + s + 1 : un < plan.units ? un * 4 : u * 4;  // the last step's own again
+            operands_written();
+#pragma unroll
+            for (int m = 0; m < MT; m++) {
+#pragma unroll
+                for (int c = 0; c < NC; c++) {
+                    prompt_mfma(acc[m][c], a[m], b[s & 1][c]);
+                    // MT * NC products take turns with NC columns' 8 groups
+                    const int slot = m * NC + c;
+#pragma unroll
+                    for (int k = slot * 8 / MT; k < (slot + 1) * 8 / MT; k++)
+                        decode(t, WHOLE ? sc[s < 3 ? 0 : 1] : sc[t], k / 8, k % 8, b[(s + 1) & 1][k / 8]);
+                    if (c == NC - 1) a[m] = load_a(m, next);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            load_w(t, s < 3 ? un : unn);
+            if (!WHOLE) sc[t] = load_sc(t, s < 3 ? un : unn);
+        }
+        if (WHOLE) {
+            sc[0] = sc[1];
+            sc[1] = load_sc(0, unn);
+        }
+        u = un < plan.units ? un : u_end;
+    }
+    mfma_drain();
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- across the wavefronts; a thread finishes QUADS x 4 columns
+    constexpr int QUADS = ROWS * COLS / 4 / T;
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            *reinterpret_cast<float4 *>(&s_red[wave][16 * m + 4 * kq + e][4 * nl]) =
+                make_float4(acc[m][0][e], acc[m][1][e], acc[m][2][e], acc[m][3][e]);
+    __syncthreads();
+    float4 sum[QUADS];
 #pragma unroll
     for (int q = 0; q < QUADS; q++) {
-        const int e = tid + q * T, row = e / (COLS / 4), m = mtile * ROWS + row, n = ntile * COLS + e % (COLS / 4) * 4;
-        if (row < ROWS && m < M && n < N) {
-            uint2 *o = reinterpret_cast<uint2 *>(out + (size_t)m * N + n);
-            float v[4] = {sum[q].x, sum[q].y, sum[q].z, sum[q].w};
-            if (accumulate) {
-                const uint2 was = *o;
-                v[0] += __half2float(__ushort_as_half((unsigned short)was.x));
-                v[1] += __half2float(__ushort_as_half((unsigned short)(was.x >> 16)));
-                v[2] += __half2float(__ushort_as_half((unsigned short)was.y));
-                v[3] += __half2float(__ushort_as_half((unsigned short)(was.y >> 16)));
-            }
-            uint32_t h[4];
+        const int e = tid + q * T, row = e / (COLS / 4), quad = e % (COLS / 4);
+        sum[q] = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-            for (int c = 0; c < 4; c++) h[c] = __half_as_ushort(__float2half_rn(v[c]));
-            *o = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+        for (int k = 0; k < KW; k++) {
+            const float4 o = *reinterpret_cast<const float4 *>(&s_red[k][row][4 * quad]);
+            sum[q].x += o.x, sum[q].y += o.y, sum[q].z += o.z, sum[q].w += o.w;
         }
     }
+    prompt_finish<ROWS, COLS, T, QUADS>(sum, s_red, at, plan, partial, tickets, out, M, N, accumulate);
 }
 
 bool prompt_supported(int bits, int M, int K, int N, int C, int G) {
@@ -967,9 +1169,10 @@ bool prompt_supported(int bits, int M, int K, int N, int C, int G) {
     return wbytes < 0x7fff0000ll && cbytes < 0x7fff0000ll && sbytes < 0x7fff0000ll && prompt_max_rows(K, C) > 0;
 }
 
-template <int BITS, int MT, int NC, int WM, int WK, int S, int AS, int NP, int D>
-static hipError_t launch_product(const PromptMember *layers, int count, int M, int K, int C, int G, int accumulate, const PromptPlan &plan,
-                                 void *workspace, void *scratch, hipStream_t stream) {
+using PromptKernel = void (*)(PromptMembers, const u32x4 *, float *, unsigned *, int, int, int, int, unsigned, int, PromptPlan);
+
+static hipError_t launch_product(PromptKernel kernel, int threads, const PromptMember *layers, int count, int M, int K, int C, int G,
+                                 int accumulate, const PromptPlan &plan, void *workspace, void *scratch, hipStream_t stream) {
     const u32x4 *a = reinterpret_cast<const u32x4 *>(scratch);
     float *partial = reinterpret_cast<float *>(reinterpret_cast<char *>(scratch) + count * plan.a_bytes);
     unsigned *tickets = reinterpret_cast<unsigned *>(workspace);
@@ -979,32 +1182,38 @@ static hipError_t launch_product(const PromptMember *layers, int count, int M, i
         const PromptMember &l = layers[i < count ? i : 0];
         members.qweight[i] = l.qweight, members.cherry_weight[i] = l.cherry_weight, members.scales[i] = l.scales, members.out[i] = l.out;
         members.N[i] = l.N, members.first[i] = first;
-        if (i < count) first += ceil_div(l.N, 16 * NC);
+        if (i < count) first += ceil_div(l.N, 16 * plan.nc);
     }
     const dim3 grid(8 * ceil_div(plan.mtiles * plan.ntiles * plan.splits, 8));
-    auto *const kernel =
-        G % kUnitK == 0 ? prompt_kernel<BITS, MT, NC, WM, WK, S, AS, NP, D, true> : prompt_kernel<BITS, MT, NC, WM, WK, S, AS, NP, D, false>;
     // ceil(2^31 / steps of a group): 2 s times it, shifted right by 32, is s / steps for every s below 2^31 / steps
     const unsigned group_magic = (unsigned)((0x80000000u + (unsigned)(G / 32) - 1u) / (unsigned)(G / 32));
-    hipLaunchKernelGGL(kernel, grid, dim3(256 + 64 * NP), 0, stream, members, a, partial, tickets, M, K, C, G, group_magic, accumulate, plan);
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, stream, members, a, partial, tickets, M, K, C, G, group_magic, accumulate, plan);
     return hipGetLastError();
 }
 
-template <int BITS>
+template <int BITS, bool WHOLE>
 static hipError_t launch_product_bits(const PromptMember *layers, int count, int M, int K, int C, int G, int accumulate,
                                       const PromptPlan &plan, void *workspace, void *scratch, hipStream_t stream) {
-#define CQ_PROMPT(ID, MT, NC, WM, WK, S, AS, NP, D) \
-    case ID:                                        \
-        return launch_product<BITS, MT, NC, WM, WK, S, AS, NP, D>(layers, count, M, K, C, G, accumulate, plan, workspace, scratch, stream);
-    switch (plan.shape) { CQ_PROMPT_SHAPES(CQ_PROMPT) }
+#define CQ_PROMPT(ID, MT, NC, WM, WK, S, AS, NP, D)                                                                                   \
+    case ID:                                                                                                                          \
+        return launch_product(prompt_kernel<BITS, MT, NC, WM, WK, S, AS, NP, D, WHOLE>, 256 + 64 * NP, layers, count, M, K, C, G,     \
+                              accumulate, plan, workspace, scratch, stream);
+#define CQ_SHARED_K(ID, MT)                                                                                                           \
+    case ID:                                                                                                                          \
+        return launch_product(prompt_shared_k_kernel<BITS, MT, WHOLE>, 512, layers, count, M, K, C, G, accumulate, plan, workspace,   \
+                              scratch, stream);
+    switch (plan.shape) { CQ_PROMPT_SHAPES(CQ_PROMPT) CQ_SHARED_K_SHAPES(CQ_SHARED_K) }
 #undef CQ_PROMPT
+#undef CQ_SHARED_K
     return hipErrorInvalidConfiguration;
 }
 
 hipError_t launch_prompt_product(int bits, const PromptMember *layers, int count, int M, int K, int C, int G, int accumulate,
                                  const PromptPlan &plan, void *workspace, void *scratch, hipStream_t stream) {
-    return bits == 4 ? launch_product_bits<4>(layers, count, M, K, C, G, accumulate, plan, workspace, scratch, stream)
-                     : launch_product_bits<3>(layers, count, M, K, C, G, accumulate, plan, workspace, scratch, stream);
+    const bool whole = G % kUnitK == 0;
+    auto *const launch = bits == 4 ? whole ? launch_product_bits<4, true> : launch_product_bits<4, false>
+                                   : whole ? launch_product_bits<3, true> : launch_product_bits<3, false>;
+    return launch(layers, count, M, K, C, G, accumulate, plan, workspace, scratch, stream);
 }
 
 // Small batches that the 16-row kernel (cq_batch.hip) takes as well.  What that takes, in us, as fitted to 4000 measured calls of 5 to

@@ -322,6 +322,46 @@ def test_layers_in_one_call_against_single_calls(dec, bits, heads, kv, inter, to
     assert model.pos.item() == tokens
 
 
+@pytest.mark.parametrize("hidden,inter,cherries", [(8192, 1032, 248), (1024, 28672, 248)])
+@pytest.mark.parametrize("adjacent", [False, True])
+def test_layers_in_one_call_at_their_limits(dec, hidden, inter, cherries, adjacent):
+    """The widest rows, RMSNorm's and SiLU's, and the most cherries that the native call takes, over more than eight row tiles, against the
+    same layer module by module."""
+    print("[case] prefill limits", hidden, inter, adjacent, flush=True)
+    cfg = dec.DecoderConfig(hidden_size=hidden, intermediate_size=inter, num_hidden_layers=1, num_attention_heads=hidden // 128,
+                            num_key_value_heads=2, vocab_size=512, max_position_embeddings=160, cherry_fraction=cherries / max(hidden, inter))
+    model = dec.CherryLlamaDecoder(cfg, seed=5)
+    most = [m for m in model.modules() if getattr(m, "num_cherries", 0) == cherries]
+    assert most
+    if adjacent:
+        for m in most:
+            m.cherry_indices.copy_(torch.arange(m.in_features - 37 - cherries, m.in_features - 37))
+    ids = torch.randint(0, 512, (150,), device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    cos, sin = model._rope_tables(150)
+    assert model._prefill_layers(model.embed_tokens[ids], cos, sin) is not None
+    got = model.prefill(ids).clone(), model.k_cache.clone(), model.v_cache.clone()
+    hook = model.layers[0].q_proj.register_forward_hook(lambda *a: None)
+    want = model.prefill(ids).clone(), model.k_cache.clone(), model.v_cache.clone()
+    hook.remove()
+    for a, b in zip(got, want):  # 7 products' results and two norms' rounded to fp16, any of them to the neighbouring value
+        assert rel(a, b.double().cpu()) < 9 * 2 ** -11
+
+
+def test_layers_beyond_the_limits_are_left_to_their_modules(dec):
+    print("[case] prefill beyond limits", flush=True)
+    cfg = dec.DecoderConfig(hidden_size=1024, intermediate_size=1032, num_hidden_layers=1, num_attention_heads=8, num_key_value_heads=2,
+                            vocab_size=512, max_position_embeddings=64, cherry_fraction=256 / 1024)
+    model = dec.CherryLlamaDecoder(cfg, seed=5)
+    ids = torch.arange(40, device="cuda") * 7 % 512
+    h = model.embed_tokens[ids]
+    model.k_cache.fill_(1.0), model.v_cache.fill_(2.0)
+    assert model._prefill_layers(h, *model._rope_tables(40)) is None
+    assert torch.equal(h, model.embed_tokens[ids]) and bool((model.k_cache == 1).all()) and bool((model.v_cache == 2).all())
+    got = model.prefill(ids).clone()
+    model.layers[0].q_proj.register_forward_hook(lambda *a: None)
+    assert rel(got, model.prefill(ids).double().cpu()) < 9 * 2 ** -11
+
+
 def test_first_pass_under_capture(dec):
     """A model whose first prompt pass is captured: an eager pass before the replay, and the replays, give what another model of the
     same seed gives."""

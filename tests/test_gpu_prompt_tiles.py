@@ -2,6 +2,8 @@
 import pytest
 import torch
 
+from prompt_cases import SHAPE_CASES
+
 pytestmark = pytest.mark.gpu
 
 
@@ -11,13 +13,7 @@ def qc():
     return quant_cuda
 
 
-# rows around every tile height; columns off the tiles' 64 and 128; one unit of 128 positions, fewer than K shares, a ragged last
-# one; no cherries, a partial step of 32, several chunks of steps; groups of whole units, and not
-@pytest.mark.parametrize("rows", [5, 16, 17, 33, 48, 64, 81, 112, 113, 129, 193, 257, 520])
-@pytest.mark.parametrize("bits,k,n,c,group", [(4, 128, 72, 0, 128), (3, 136, 64, 8, 32), (4, 520, 1032, 40, 160), (3, 1024, 264, 24, 96),
-                                              (4, 1800, 2056, 520, 192), (3, 2560, 520, 296, 256), (4, 4096, 11008, 16, 128)])
-def test_rows_around_the_tiles(qc, bits, k, n, c, group, rows):
-    print("[case] prompt tiles", bits, k, n, c, group, rows, flush=True)
+def against_64_bits(qc, bits, k, n, c, group, rows):
     gen = torch.Generator(device="cuda").manual_seed(rows * 7 + k)
     kn = k - c
     q = torch.randint(0, 256, (kn // 8 * bits, n), device="cuda", generator=gen, dtype=torch.uint8)
@@ -37,3 +33,21 @@ def test_rows_around_the_tiles(qc, bits, k, n, c, group, rows):
         qc.matmul_cherryq(bits, x, q, cw, idx, scales, out, group, accumulate=accumulate)
         want = ref + before.double() if accumulate else ref
         assert bool(((out.double() - want).abs() <= want.abs() * 2.0 ** -11 + slack * (1 + 2.0 ** -11)).all())
+
+
+# rows around every tile height; columns off the tiles' 64 and 128; one unit of 128 positions, fewer than K shares, a ragged last
+# one; no cherries, a partial step of 32, several chunks of steps; groups of whole units, and not
+@pytest.mark.parametrize("rows", [5, 16, 17, 33, 48, 64, 81, 112, 113, 129, 193, 257, 520])
+@pytest.mark.parametrize("bits,k,n,c,group", [(4, 128, 72, 0, 128), (3, 136, 64, 8, 32), (4, 520, 1032, 40, 160), (3, 1024, 264, 24, 96),
+                                              (4, 1800, 2056, 520, 192), (3, 2560, 520, 296, 256), (4, 4096, 11008, 16, 128)])
+def test_rows_around_the_tiles(qc, bits, k, n, c, group, rows):
+    print("[case] prompt tiles", bits, k, n, c, group, rows, flush=True)
+    against_64_bits(qc, bits, k, n, c, group, rows)
+
+
+# groups of whole units of 128 positions are another instance than others, which may straddle units
+@pytest.mark.parametrize("rows,k,n,c", SHAPE_CASES)
+@pytest.mark.parametrize("bits,group", [(4, 128), (4, 160), (3, 128), (3, 96)])
+def test_every_tile_shape(qc, bits, group, rows, k, n, c):
+    print("[case] prompt shapes", bits, k, n, c, group, rows, flush=True)
+    against_64_bits(qc, bits, k, n, c, group, rows)
