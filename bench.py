@@ -349,7 +349,7 @@ def main():
     ap.add_argument("--warmup", type=int, default=200)
     ap.add_argument("--workload", default="llama7b_gate_up_w4", choices=sorted(WORKLOADS))
     ap.add_argument("--group", type=int, default=128)
-    ap.add_argument("--batch", type=int, default=1, help="activation rows per call (2..4: streaming kernel with several rows or, the small-batch matrix-core kernel; from 5: that or the prompt kernel; above 16: prompt kernel)")
+    ap.add_argument("--batch", type=int, default=1, help="activation rows per call (2..4: streaming kernel with several rows or the small-batch matrix-core kernel; 5..16: the latter or the prompt kernels; more: these)")
     ap.add_argument("--all", action="store_true", help="also print a table of every workload to stderr")
     ap.add_argument("--unpack-only", action="store_true",
                     help="print the dense-dequantisation table to stderr and exit (for profiling that kernel)")

@@ -88,8 +88,8 @@ constexpr int kPromptMinRows = 17;  // fewer rows may go through the 16-row kern
 constexpr int kPromptMaxSplits = 16;
 struct PromptPlan {
     int shape;                        // the tile shape, by its place in the kernel's table
-    int mt, nc, ns;                   // 16-row and 16-column pieces of a workgroup's tile: mt x nc ns
-    int mtiles, ntiles;               // output tiles of 16 mt rows x 16 nc ns columns
+    int mt, nc;                       // 16-row and 16-column pieces of a workgroup's tile
+    int mtiles, ntiles;               // output tiles of 16 mt rows x 16 nc columns
     int units, csteps, steps;         // units of 128 positions, steps of 32 cherries, steps of 32 in all
     int splits, units_per_split;      // K splits
     size_t workspace_bytes;           // zero-kept: one ticket per output tile

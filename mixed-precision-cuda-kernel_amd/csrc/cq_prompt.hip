@@ -173,7 +173,7 @@ static PromptPlan find_prompt_plan(int M, int K, const int *N, int count, int C)
         const PromptShape &s = kPromptShapes[id];
         const PromptCost &f = kPromptCosts[id];
         PromptPlan p = {};
-        p.shape = id, p.mt = s.mt * s.wm, p.nc = s.nc, p.ns = 1;
+        p.shape = id, p.mt = s.mt * s.wm, p.nc = s.nc;
         if (p.mt > 1 ? M <= 8 * p.mt : M > 16) continue;  // half of every tile would be padding; 16 rows: up to one tile
         p.mtiles = ceil_div(M, 16 * p.mt);
         if (p.mt != 2 && (p.mtiles * p.mt > 65535 || steps * p.mtiles * p.mt > 0x7fff0000ll / 1024)) continue;
@@ -229,10 +229,10 @@ PromptBytes prompt_bytes(int M, int K, const int *N, int count, int C) {
     return bytes;
 }
 
-// #{m : at(m) <= p} for non-decreasing at(0 .. C - 1); p is first + STEP lane (others: any answer).  A whole wavefront: it compares 64 values at a time
-// with the range of its positions, and only the few inside lane by lane (a search takes a round trip to LDS per halving: 3.6 us of
-// 10 in prompt_norm_kernel).
-template <int STEP, typename At>
+// #{m : at(m) <= p} for non-decreasing at(0 .. C - 1); p is first + lane (others: any answer).  A whole wavefront: it compares 64 values at a
+// time with the range of its positions, and only the few inside lane by lane (a search takes a round trip to memory or LDS per
+// halving; in row_operands, which counts in the same way, that was 3.6 us of 10).
+template <typename At>
 __device__ __forceinline__ int count_upto(At at, int C, int first, int p) {
     const int lane = threadIdx.x & 63;
     int n = 0;
@@ -240,7 +240,7 @@ __device__ __forceinline__ int count_upto(At at, int C, int first, int p) {
     for (int k = 0; k < C; k += 64) {
         const int v = k + lane < C ? at(k + lane) : 0x7fffffff;
         n += __popcll(__ballot(v <= first));
-        for (unsigned long long in = __ballot(v > first && v <= first + 63 * STEP); in; in &= in - 1)
+        for (unsigned long long in = __ballot(v > first && v <= first + 63); in; in &= in - 1)
             n += __builtin_amdgcn_readlane(v, __builtin_ctzll(in)) <= p ? 1 : 0;
     }
     return n;
@@ -296,7 +296,7 @@ __global__ __launch_bounds__(256) void prompt_prep_kernel(const __half *__restri
         if (chunk && sr < M) v0 = *reinterpret_cast<const u32x4 *>(x + (size_t)sr * K + k0 + 8 * sch);
         if (chunk && sr + 8 < M) v1 = *reinterpret_cast<const u32x4 *>(x + (size_t)(sr + 8) * K + k0 + 8 * sch);
         // the offsets of the unit's positions, once for all rows, by two wavefronts (past Kn: not used)
-        if (t < kUnitK) s_off[t] = (uint16_t)count_upto<1>([&](int m) { return cherry_indices[m] - m; }, C, k0 + (t & ~63), k0 + t);
+        if (t < kUnitK) s_off[t] = (uint16_t)count_upto([&](int m) { return cherry_indices[m] - m; }, C, k0 + (t & ~63), k0 + t);
         if (chunk) {
             *reinterpret_cast<u32x4 *>(&s_x[t >> 5][8 * sch]) = v0;
             *reinterpret_cast<u32x4 *>(&s_x[(t >> 5) + 8][8 * sch]) = v1;
@@ -487,8 +487,8 @@ struct PromptDecode {
     }
 };
 
-// One column's 8 operands on their way from packed codes, as 8 small groups of independent instructions: the caller puts an
-// MFMA between any two.
+// One column's 8 operands on their way from packed codes, as 8 small groups of independent instructions: products can go between
+// any two (prompt_shared_k_kernel).
 template <int BITS>
 struct PromptColumn {
     uint32_t p[2], t[2], s2, f[4], y[4];
@@ -584,13 +584,11 @@ struct PromptPiece {
     typedef uint32_t s_t __attribute__((ext_vector_type(NC / 2)));
     static __device__ __forceinline__ w_t codes(const __amdgpu_buffer_rsrc_t r, uint32_t off) {
         if constexpr (NC == 8) return __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 2);
-        else if constexpr (NC == 4) return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 2);
-        else return (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 2);
+        else return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 2);
     }
     static __device__ __forceinline__ s_t halves(const __amdgpu_buffer_rsrc_t r, uint32_t off) {
         if constexpr (NC == 8) return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
-        else if constexpr (NC == 4) return __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
-        else return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
+        else return __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
     }
 };
 
@@ -704,7 +702,7 @@ template <int BITS, int MT, int NC, int WM, int WK, int S, int AS, int NP, int D
 __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(PromptMembers members, const u32x4 *__restrict__ a_all,
                                                               float *__restrict__ partial, unsigned *__restrict__ tickets, int M,
                                                               int K, int C, int G, unsigned group_magic, int accumulate, PromptPlan plan) {
-    static_assert(WM * WK == 4 && S * WK % NP == 0 && NP % WK == 0 && (AS % S == 0 || S % AS == 0) && (AS <= S || AS / S * S == 4), "");
+    static_assert((NC == 4 || NC == 8) && WM * WK == 4 && S * WK % NP == 0 && NP % WK == 0 && (AS % S == 0 || S % AS == 0) && (AS <= S || AS / S * S == 4), "");
     typedef typename PromptPiece<NC>::w_t w_t;
     typedef typename PromptPiece<NC>::s_t s_t;
     constexpr bool SUMS = WHOLE && MT == 1;
@@ -809,7 +807,7 @@ __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(Pro
         if constexpr (SUMS) sc[0] = s_sc[0][wk][nl];
         // Every operand is asked for again as soon as its products are issued: activations AS steps ahead, weights one.  A
         // stage's last step meets the producers once its own weights have arrived, and goes on with the next stage's.
-        constexpr int MEET = NC > 2 ? 1 : 0, U = AS > S ? AS / S : 1;
+        constexpr int MEET = 1, U = AS > S ? AS / S : 1;
 #pragma nounroll
         for (int st = 0; st < stages; st += U) {
 #pragma unroll
@@ -969,14 +967,10 @@ __global__ __launch_bounds__(256 + 64 * NP, (4 + NP) / 4) void prompt_kernel(Pro
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 float *const row = s_red + ((wave * MT + m) * 16 + 4 * kq + e) * COLS;
-                if constexpr (NC == 2) {
-                    *reinterpret_cast<float2 *>(row + 2 * nl) = make_float2(acc[m][0][e], acc[m][1][e]);
-                } else {
 #pragma unroll
-                    for (int d = 0; d < NC / 4; d++)
-                        *reinterpret_cast<float4 *>(row + 4 * swizzled(NC / 4 * nl + d)) =
-                            make_float4(acc[m][4 * d][e], acc[m][4 * d + 1][e], acc[m][4 * d + 2][e], acc[m][4 * d + 3][e]);
-                }
+                for (int d = 0; d < NC / 4; d++)
+                    *reinterpret_cast<float4 *>(row + 4 * swizzled(NC / 4 * nl + d)) =
+                        make_float4(acc[m][4 * d][e], acc[m][4 * d + 1][e], acc[m][4 * d + 2][e], acc[m][4 * d + 3][e]);
             }
     }
     __syncthreads();
