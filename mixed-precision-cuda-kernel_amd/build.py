@@ -19,7 +19,7 @@ CSRC = HERE / "csrc"
 OBJ = HERE / "build"
 LIB = HERE / "libcherryq.so"
 PROBE_LIB = HERE / "libcherryq_probe.so"  # bench-only roofline reference kernels, not part of the product library
-SOURCES = ["cq_api.hip", "cq_generic.hip", "cq_matvec.hip", "cq_stream.hip", "cq_stream_cu.hip", "cq_batch.hip", "cq_prompt.hip", "cq_f32.hip", "cq_decode.hip", "cq_prefill.hip", "cq_pack.hip", "cq_fakequant.hip"]
+SOURCES = ["cq_api.hip", "cq_generic.hip", "cq_matvec.hip", "cq_stream.hip", "cq_stream_cu.hip", "cq_batch.hip", "cq_prompt.hip", "cq_f32.hip", "cq_decode.hip", "cq_prefill.hip", "cq_pack.hip", "cq_fakequant.hip", "cq_gemm.hip"]
 HOST_LIB = HERE / "cherryq_host.so"  # host side of the Python binding (g++, linked against torch)
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

@@ -296,6 +296,24 @@ static int fake_quant_entry(cq::FqDtype dtype, int w_bits, const void *weight, c
                                       reinterpret_cast<hipStream_t>(stream));
 }
 
+size_t cherryq_gemm_workspace_bytes(int M, int N, int K) { return M > 0 && N > 0 && K > 0 ? cq::gemm_plan(M, N, K).workspace_bytes : 0; }
+
+size_t cherryq_gemm_scratch_bytes(int M, int N, int K) { return M > 0 && N > 0 && K > 0 ? cq::gemm_plan(M, N, K).scratch_bytes : 0; }
+
+int cherryq_gemm_preferred(int a_by_k, int b_by_k, int M, int N, int K) { return cq::gemm_preferred(a_by_k, b_by_k, M, N, K) ? 1 : 0; }
+
+int cherryq_gemm_16(int bf16, int a_by_k, int b_by_k, const void *a, const void *b, void *out, int M, int N, int K, void *workspace,
+                    size_t workspace_size, void *scratch, size_t scratch_size, void *stream) {
+    if (M <= 0 || N <= 0 || K <= 0) return CHERRYQ_E_SHAPE;
+    if (!a || !b || !out) return CHERRYQ_E_NULL;
+    if (!cq::aligned(a, 16) || !cq::aligned(b, 16) || !cq::aligned(out, 16)) return CHERRYQ_E_ALIGN;
+    if (!cq::gemm_supported(a_by_k, b_by_k, M, N, K)) return CHERRYQ_E_UNSUPPORTED;
+    const cq::GemmPlan plan = cq::gemm_plan(M, N, K);
+    if (plan.workspace_bytes && (!workspace || !cq::aligned(workspace, 8) || workspace_size < plan.workspace_bytes)) return CHERRYQ_E_WORKSPACE;
+    if (plan.scratch_bytes && (!scratch || !cq::aligned(scratch, 16) || scratch_size < plan.scratch_bytes)) return CHERRYQ_E_WORKSPACE;
+    return (int)cq::launch_gemm(bf16, a_by_k, b_by_k, a, b, out, M, N, K, plan, workspace, scratch, reinterpret_cast<hipStream_t>(stream));
+}
+
 int cherryq_fake_quant_f16(int w_bits, const void *weight, const int32_t *cherry_indices, void *out, int in_features,
                            int out_features, int num_cherries, int group_size, int ste, void *stream) {
     return fake_quant_entry(cq::FqDtype::f16, w_bits, weight, cherry_indices, out, in_features, out_features, num_cherries,

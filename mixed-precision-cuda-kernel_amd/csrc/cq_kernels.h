@@ -216,6 +216,19 @@ bool fake_quant_supported(int K, int C, int G);
 hipError_t launch_fake_quant(int bits, FqDtype dtype, const void *w, const int32_t *idx, void *out, int K, int N, int C,
                              int G, int ste, hipStream_t stream);
 
+// cq_gemm.hip: dense 16-bit products D[M, N] = sum_k A(m, k) B(n, k); by_k: the operand lies as [K][free], not [free][K]
+struct GemmPlan {
+    int mtiles, ntiles, steps;          // tiles of 256 x 256, steps of 64 positions of K
+    int full, rest, splits, per_split;  // tiles of whole rounds of 256; the others, the workgroups that share one, their steps
+    float cost;                         // microseconds, estimated
+    size_t scratch_bytes, workspace_bytes;
+};
+GemmPlan gemm_plan(int M, int N, int K);
+bool gemm_supported(bool a_by_k, bool b_by_k, int M, int N, int K);
+bool gemm_preferred(bool a_by_k, bool b_by_k, int M, int N, int K);  // faster than the library's product
+hipError_t launch_gemm(bool bf16, bool a_by_k, bool b_by_k, const void *a, const void *b, void *out, int M, int N, int K, const GemmPlan &plan,
+                       void *workspace, void *scratch, hipStream_t stream);
+
 // cq_decode.hip: batch-1 decode-step glue kernels.
 hipError_t launch_add_rmsnorm(__half *h, const __half *delta, const __half *weight, __half *y, int H, float eps,
                               hipStream_t stream);

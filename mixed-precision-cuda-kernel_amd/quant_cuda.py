@@ -61,6 +61,13 @@ _FAKE_QUANT = {torch.float16: "cherryq_fake_quant_f16", torch.bfloat16: "cherryq
 for _name in _FAKE_QUANT.values():
     getattr(_lib, _name).argtypes = [_int, _vp, _vp, _vp, _int, _int, _int, _int, _int, _vp]
     getattr(_lib, _name).restype = _int
+for _name in ("cherryq_gemm_workspace_bytes", "cherryq_gemm_scratch_bytes"):
+    getattr(_lib, _name).argtypes = [_int, _int, _int]
+    getattr(_lib, _name).restype = _sz
+_lib.cherryq_gemm_preferred.argtypes = [_int, _int, _int, _int, _int]
+_lib.cherryq_gemm_preferred.restype = _int
+_lib.cherryq_gemm_16.argtypes = [_int, _int, _int, _vp, _vp, _vp, _int, _int, _int, _vp, _sz, _vp, _sz, _vp]
+_lib.cherryq_gemm_16.restype = _int
 _lib.cherryq_vecquant_matmul_f16_static.argtypes = [_int, _vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _int, _int, _vp]
 _lib.cherryq_vecquant_matmul_f16_static.restype = _int
 _lib.cherryq_set_force_generic.argtypes = [_int]
@@ -583,4 +590,33 @@ def fake_quant_cherryq(w_bits, weight, cherry_indices, group_size, ste=False, ou
                 _current_stream(dev.index))
     if rc != 0:
         _fail(rc, "fake_quant_cherryq")
+    return out
+
+
+def gemm_preferred(a_by_k, b_by_k, m, n, k) -> bool:
+    """Whether gemm() supports these sizes and is expected to be faster than torch's product."""
+    return bool(_lib.cherryq_gemm_preferred(a_by_k, b_by_k, m, n, k))
+
+
+def gemm(a, b, a_by_k=False, b_by_k=False, shape=None):
+    """a @ b.T for 16-bit matrices, fp32 sums; `a_by_k` / `b_by_k`: the operand is given transposed (contraction first);
+    `shape`: the result's, of as many elements.  No counterpart in the reference extension."""
+    _check(a, "a", a.dtype, 2)
+    _check(b, "b", a.dtype, 2, a.device)
+    m, k = a.shape[::-1] if a_by_k else a.shape
+    n, kb = b.shape[::-1] if b_by_k else b.shape
+    if k != kb or a.dtype not in (torch.float16, torch.bfloat16):
+        raise RuntimeError(f"gemm: {tuple(a.shape)} and {tuple(b.shape)} of {a.dtype} do not multiply")
+    dev = a.device
+    with torch.cuda.device(dev):
+        out = torch.empty((m, n) if shape is None else shape, dtype=a.dtype, device=dev)
+        if out.numel() != m * n:
+            raise RuntimeError(f"gemm: {m} x {n} results do not fit shape {tuple(shape)}")
+        stream = _current_stream(dev.index)
+        ws = _workspace(dev, stream, _lib.cherryq_gemm_workspace_bytes(m, n, k))
+        scratch = torch.empty(_lib.cherryq_gemm_scratch_bytes(m, n, k), dtype=torch.uint8, device=dev)  # the call's own
+        rc = _lib.cherryq_gemm_16(a.dtype == torch.bfloat16, a_by_k, b_by_k, a.data_ptr(), b.data_ptr(), out.data_ptr(), m, n, k,
+                                  ws.data_ptr(), ws.numel(), _ptr(scratch), scratch.numel(), stream)
+    if rc != 0:
+        _fail(rc, "gemm")
     return out
