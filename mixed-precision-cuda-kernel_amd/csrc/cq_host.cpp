@@ -14,11 +14,13 @@
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/TracerMode.h>
+#include <ATen/autocast_mode.h>
 #include <c10/core/InferenceMode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
@@ -55,6 +57,17 @@ struct Api {
     ShapeFn prepack_supported, rows_recommended;
 } api;
 TakenFn prompt_taken;  // cherryq_prompt_taken
+
+using FakeQuantFn = int (*)(int, const void *, const void *, void *, int, int, int, int, int, void *);
+using GemmSizeFn = size_t (*)(int, int, int);
+using GemmPreferredFn = int (*)(int, int, int, int, int);
+using GemmFn = int (*)(int, int, int, const void *, const void *, void *, int, int, int, void *, size_t, void *, size_t, void *);
+struct TrainApi {
+    FakeQuantFn fake_quant_f16, fake_quant_bf16, fake_quant_f32;
+    GemmSizeFn gemm_workspace, gemm_scratch;
+    GemmPreferredFn gemm_preferred;
+    GemmFn gemm;
+} train;
 
 // ---- buffers kept per (device, stream) -----------------------------------------------------------
 // A zero-initialised workspace (the kernels leave it all zero after every call, so it is reusable as is)
@@ -447,6 +460,136 @@ PyObject *bind_prompt(PyObject *, PyObject *address) {
     Py_RETURN_NONE;
 }
 
+// ---- the training layer ----------------------------------------------------------------------------
+// A pass over a small layer is bound by the host: the fake quantisation's and the product's autograd nodes in Python, their checks, and
+// torch's own linear took 180 us for a forward and a backward whose kernels take 30.
+
+inline bool whole(const Tensor &t) { return t.is_contiguous() && reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0; }
+
+// out[m, n] = sum_k a(m, k) b(n, k) of 16-bit matrices (an operand by_k lies as [k, n]) where the kernel takes it and is faster than
+// torch's product; undefined elsewhere.  The result is laid out as `shape`.
+Tensor product(const Tensor &a, bool a_by_k, const Tensor &b, bool b_by_k, int64_t m, int64_t n, int64_t k, at::IntArrayRef shape) {
+    constexpr int64_t most = INT32_MAX;
+    if ((a.scalar_type() != at::kHalf && a.scalar_type() != at::kBFloat16) || a.scalar_type() != b.scalar_type() || !whole(a) || !whole(b) || m > most ||
+        n > most || k > most || !train.gemm_preferred(a_by_k, b_by_k, (int)m, (int)n, (int)k))
+        return {};
+    const int device = a.get_device();
+    void *const stream = current_stream(device);
+    const Tensor out = at::empty(shape, a.options());
+    const int64_t zero_bytes = (int64_t)train.gemm_workspace((int)m, (int)n, (int)k), bytes = (int64_t)train.gemm_scratch((int)m, (int)n, (int)k);
+    // the call's own, given back behind it in the stream's order: two streams never share it
+    const Tensor scratch = bytes ? at::empty({bytes}, a.options().dtype(at::kByte)) : Tensor();
+    const Tensor zero = zero_bytes ? workspaces.get(device, stream, zero_bytes) : Tensor();
+    const int rc = train.gemm(a.scalar_type() == at::kBFloat16, a_by_k, b_by_k, a.const_data_ptr(), b.const_data_ptr(), out.mutable_data_ptr(), (int)m, (int)n,
+                              (int)k, bytes ? zero.mutable_data_ptr() : nullptr, bytes ? (size_t)zero.numel() : 0,
+                              bytes ? scratch.mutable_data_ptr() : nullptr, (size_t)bytes, stream);
+    TORCH_CHECK(rc == 0, "training product: status ", rc);
+    return out;
+}
+
+// `value` with `weight`'s gradient, for second derivatives
+struct StraightThrough : torch::autograd::Function<StraightThrough> {
+    static Tensor forward(torch::autograd::AutogradContext *, const Tensor &, const Tensor &value) { return value.clone(); }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *, torch::autograd::variable_list grads) {
+        return {grads[0], Tensor()};
+    }
+};
+
+// linear(x, quantised) with the straight-through gradient for the weight that was quantised (llama/cherry_linear.py:97-98)
+struct TrainLinear : torch::autograd::Function<TrainLinear> {
+    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &x, const Tensor &weight, const Tensor &quantised) {
+        // what a gradient reads and no more: the other may be changed in place or given back
+        ctx->save_for_backward({weight.requires_grad() ? x : Tensor(), x.requires_grad() ? quantised : Tensor()});
+        ctx->saved_data["weight"] = weight;  // for second derivatives only, so the optimiser may have stepped
+        const int64_t n = weight.size(0), k = weight.size(1), rows = x.numel() / k;
+        std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
+        shape.back() = n;
+        Tensor out = product(x, false, quantised, false, rows, n, k, shape);
+        return out.defined() ? out : at::linear(x, quantised);
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &g = grads[0], &x = saved[0];
+        Tensor quantised = saved[1], dx, dw;
+        const bool twice = at::GradMode::is_enabled();  // a graph of the gradients is asked for
+        const int64_t n = g.size(-1);
+        if (quantised.defined()) {
+            const int64_t k = quantised.size(1);
+            std::vector<int64_t> shape(g.sizes().begin(), g.sizes().end());
+            shape.back() = k;
+            if (twice) {
+                quantised = StraightThrough::apply(ctx->saved_data["weight"].toTensor(), quantised);
+            } else if (n) {
+                dx = product(g, false, quantised, true, g.numel() / n, k, n, shape);
+            }
+            if (!dx.defined()) dx = g.matmul(quantised);
+        }
+        if (x.defined()) {
+            const int64_t k = x.size(-1), rows = g.numel() / std::max<int64_t>(n, 1);
+            const Tensor g2 = g.reshape({rows, n}), x2 = x.reshape({rows, k});
+            if (!twice && n) dw = product(g2, true, x2, true, n, k, rows, {n, k});
+            if (!dw.defined()) dw = g2.t().matmul(x2);
+        }
+        return {dx, dw, Tensor()};
+    }
+};
+
+// bind_train(addresses): as listed in TrainApi
+PyObject *bind_train(PyObject *, PyObject *seq) {
+    constexpr Py_ssize_t count = sizeof(train) / sizeof(void *);
+    if (!PyTuple_Check(seq) || PyTuple_GET_SIZE(seq) != count) {
+        PyErr_Format(PyExc_TypeError, "bind_train() takes a tuple of %zd addresses", count);
+        return nullptr;
+    }
+    void *at[count];
+    for (Py_ssize_t i = 0; i < count; i++) {
+        at[i] = PyLong_AsVoidPtr(PyTuple_GET_ITEM(seq, i));
+        if (!at[i]) {
+            if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "null address");
+            return nullptr;
+        }
+    }
+    memcpy(&train, at, sizeof(train));
+    Py_RETURN_NONE;
+}
+
+// train_linear(x, weight, cherry_indices, w_bits, group_size): linear with the straight-through fake-quantised weight; None where a tensor or
+// the moment is not ordinary, and nothing launched
+PyObject *train_linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (nargs != 5) {
+        PyErr_SetString(PyExc_TypeError, "train_linear() takes 5 arguments");
+        return nullptr;
+    }
+    const Tensor *x = tensor(args[0]), *weight = tensor(args[1]), *t = weight, *indices = tensor(args[2]);
+    if (!x || !weight || !indices || !PyLong_CheckExact(args[3]) || !PyLong_CheckExact(args[4]) || !train.gemm) Py_RETURN_NONE;
+    const long bits = PyLong_AsLong(args[3]), group = PyLong_AsLong(args[4]);
+    if (PyErr_Occurred()) return nullptr;
+    if (!t->is_cuda() || t->dim() != 2 || !t->is_contiguous() || !ordinary(*x) || !ordinary(*t)) Py_RETURN_NONE;
+    const int device = t->get_device();
+    const auto type = t->scalar_type();
+    const FakeQuantFn quantise = type == at::kHalf ? train.fake_quant_f16 : type == at::kBFloat16 ? train.fake_quant_bf16 : type == at::kFloat ? train.fake_quant_f32 : nullptr;
+    const int64_t n = t->size(0), k = t->size(1);
+    if (!quantise || x->scalar_type() != type || x->device() != t->device() || x->dim() < 2 || x->size(-1) != k || !x->numel() || n <= 0 || n > INT32_MAX ||
+        k > INT32_MAX || group > INT32_MAX || !is(indices, at::kInt, 1, device) || indices->numel() > INT32_MAX || !indices->has_storage() ||
+        c10::hip::current_device() != device || at::autocast::is_autocast_enabled(t->device().type()) || x->_fw_grad(0).defined() || t->_fw_grad(0).defined())
+        Py_RETURN_NONE;
+    Tensor quantised, out;
+    {
+        at::NoGradGuard plain;
+        quantised = at::empty({n, k}, t->options());
+    }
+    const int rc = quantise((int)bits, t->const_data_ptr(), ptr(*indices), quantised.mutable_data_ptr(), (int)k, (int)n, (int)indices->numel(),
+                            group > 0 ? (int)group : (int)k, 1, current_stream(device));
+    if (rc != 0) Py_RETURN_NONE;  // refused before the launch: the general route words it
+    {
+        Unlocked<Tensor, Tensor, Tensor> free(*x, *weight, quantised);
+        out = TrainLinear::apply(free.held[0], free.held[1], free.held[2]);
+    }
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
 // ordinary(tensor)
 PyObject *is_ordinary(PyObject *, PyObject *x) {
     HANDLE_TH_ERRORS
@@ -458,6 +601,8 @@ PyObject *is_ordinary(PyObject *, PyObject *x) {
 PyMethodDef methods[] = {
     {"bind", bind, METH_O, nullptr},
     {"bind_prompt", bind_prompt, METH_O, nullptr},
+    {"bind_train", bind_train, METH_O, nullptr},
+    {"train_linear", (PyCFunction)(void (*)())train_linear, METH_FASTCALL, nullptr},
     {"ordinary", is_ordinary, METH_O, nullptr},
     {"vecquant", (PyCFunction)(void (*)())vecquant, METH_FASTCALL, nullptr},
     {"matvec_prepacked", (PyCFunction)(void (*)())matvec_prepacked, METH_FASTCALL, nullptr},

@@ -153,6 +153,18 @@ class QuantLinear(nn.Linear):
             real_weight = real_weight - weight.detach() + weight
         return real_weight
 
+    def _native_linear(self, x, weight):
+        """The whole branch of the training forward in one native call, with one autograd node; None where it is not the
+        plain case (the caller's route then takes it or raises)."""
+        own = self.__dict__
+        if (torch.compiler.is_compiling() or self.quantizer is not FullSymQuantizer or self.weight_layerwise
+                or not own.get("cherry_indices_registered") or "_adjust_weight" in own or "_fused_fake_quant" in own
+                or type(self)._adjust_weight is not QuantLinear._adjust_weight
+                or type(self)._fused_fake_quant is not QuantLinear._fused_fake_quant or not weight.is_cuda):
+            return None
+        import quant_cuda
+        return quant_cuda.train_linear(x, weight, self.cherry_indices, self.w_bits, self.group_size)
+
     @torch.inference_mode()
     def prepare_weight_for_inference(self, weight):
         """Replace `self.weight` by its fake-quantised value once (llama/cherry_linear.py:48-61)."""
@@ -171,13 +183,16 @@ class QuantLinear(nn.Linear):
     # ---- forward ------------------------------------------------------------------------------
     def quant_forward(self, input_):
         assert self.weight.ndimension() == 2
+        out = None
         if self.w_bits >= 16:
             weight = self.weight
         elif self.w_bits > 1:
             weight = self.weight
             if self.cherryq:
                 if self.training:
-                    weight = self._adjust_weight(weight)
+                    out = self._native_linear(input_, weight)
+                    if out is None:
+                        weight = self._adjust_weight(weight)
                 elif not self.dequantized:
                     weight = self.prepare_weight_for_inference(weight)
             elif self.training and self._fused_plain(weight):
@@ -191,7 +206,8 @@ class QuantLinear(nn.Linear):
                 weight = self.prepare_weight_for_inference(weight)
         else:
             raise NotImplementedError(f"Quantization for {self.w_bits}bit is not implemented yet.")
-        out = nn.functional.linear(input_, weight)
+        if out is None:
+            out = nn.functional.linear(input_, weight)
         if self.bias is not None:
             out += self.bias
         return out

@@ -117,6 +117,9 @@ _host.bind(tuple(ctypes.cast(getattr(_lib, f"cherryq_{n}"), _vp).value for n in 
     "vecquant4matmul_f16", "vecquant3matmul_f16", "vecquant3matmul_f32", "workspace_bytes", "scratch_bytes",
     "scratch_bytes_f32", "prepacked_scratch_bytes", "matvec_prepacked_f16", "matmul_prepacked_f16", "prepack_supported",
     "prepack_rows_recommended")))
+_host.bind_train(tuple(ctypes.cast(getattr(_lib, f"cherryq_{n}"), _vp).value for n in (
+    "fake_quant_f16", "fake_quant_bf16", "fake_quant_f32", "gemm_workspace_bytes", "gemm_scratch_bytes", "gemm_preferred", "gemm_16")))
+train_linear = _host.train_linear  # (x, weight, cherry_indices, w_bits, group_size) -> linear with the fake-quantised weight, or None
 _lib.cherryq_prompt_taken.argtypes = [_int, _int, _int, _int, _int, _int, _vp]
 _lib.cherryq_prompt_taken.restype = _int
 _host.bind_prompt(ctypes.cast(_lib.cherryq_prompt_taken, _vp).value)

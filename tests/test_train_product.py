@@ -1,12 +1,147 @@
-"""The training layer's matrix products (csrc/cq_gemm.hip).
+"""The training layer in one native call (csrc/cq_host.cpp: train_linear) and its matrix products (csrc/cq_gemm.hip).
 
 Bound of the kernel: fp32 sums of exact 16-bit products, rounded once.  The rounding is half an ulp of the result's type, at most
 2^-11 (fp16) or 2^-8 (bf16) of an element, its 2-norm about 0.6 of that; a sum of K terms of random signs adds about sqrt(K) 2^-24 of
 the result, 2^-17 at the largest K here.  So 2^-11 / 2^-8 of the 2-norm holds with room."""
+import ctypes
+import shutil
+from pathlib import Path
+
 import pytest
 import torch
 
+import llama.cherry_linear as cl
+
 LIMIT = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+
+
+# ---- the native call, built for CPU tensors, with stand-ins for the kernels -----------------------------------
+@pytest.fixture(scope="module")
+def native(tmp_path_factory):
+    """(train_linear, calls): the stand-in for the fake quantisation halves the weight; products come from torch."""
+    import test_host_binding_cpu as t
+    if shutil.which("g++") is None or not Path("/opt/rocm/include").is_dir():
+        pytest.skip("needs g++ and the HIP headers")
+    directory = tmp_path_factory.mktemp("train")
+    t.build_cpu_host(directory)
+    host, _, stubs = t.load_cpu_host(directory)
+    vp, i, sz, calls = ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t, []
+
+    def at(address, rows, cols, dtype):
+        return torch.frombuffer((ctypes.c_uint8 * (rows * cols * dtype.itemsize)).from_address(address), dtype=dtype).view(rows, cols)
+
+    def quantise(dtype):
+        def f(bits, w, idx, out, k, n, c, g, ste, stream):
+            if bits > 4:
+                return -1
+            calls.append("quantise")
+            at(out, n, k, dtype).copy_(at(w, n, k, dtype) / 2)
+            return 0
+        return ctypes.CFUNCTYPE(i, i, vp, vp, vp, i, i, i, i, i, vp)(f)
+
+    def gemm(bf16, a_by_k, b_by_k, a, b, out, m, n, k, ws, wsz, sc, scz, stream):
+        calls.append((a_by_k, b_by_k))
+        dtype = torch.bfloat16 if bf16 else torch.float16
+        x, y = at(a, k if a_by_k else m, m if a_by_k else k, dtype), at(b, k if b_by_k else n, n if b_by_k else k, dtype)
+        assert wsz >= 16 and scz == 64
+        at(out, m, n, dtype).copy_((x.t() if a_by_k else x).float() @ (y if b_by_k else y.t()).float())
+        return 0
+
+    size = ctypes.CFUNCTYPE(sz, i, i, i)
+    mine = [quantise(d) for d in (torch.float16, torch.bfloat16, torch.float32)]
+    mine += [size(lambda *_: 16), size(lambda *_: 64), ctypes.CFUNCTYPE(i, i, i, i, i, i)(lambda *a: 1),
+             ctypes.CFUNCTYPE(i, i, i, i, vp, vp, vp, i, i, i, vp, sz, vp, sz, vp)(gemm)]
+    host.bind_train(tuple(ctypes.cast(f, vp).value for f in mine))
+    yield lambda x, w, bits=4: host.train_linear(x, w, torch.arange(8, dtype=torch.int32), bits, 8), calls
+    del stubs, mine
+
+
+def through_torch(x, w):
+    return torch.nn.functional.linear(x, (w.detach() / 2 - w).detach() + w)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape", [(8, 16), (2, 3, 16)])
+@pytest.mark.parametrize("needs", [(True, True), (True, False), (False, True)])
+def test_native_call_and_gradients_equal_torch(native, dtype, shape, needs):
+    torch.manual_seed(0)
+    x, w, g = torch.randn(shape).to(dtype), torch.randn(24, 16).to(dtype), torch.randn(*shape[:-1], 24).to(dtype)
+    results = []
+    for f in (native[0], through_torch):
+        native[1].clear()
+        xs, ws = x.clone().requires_grad_(needs[0]), w.clone().requires_grad_(needs[1])
+        y = f(xs, ws)
+        y += 1  # a bias, in place
+        y.backward(g)
+        results.append((y.detach(), xs.grad, ws.grad))
+        if f is native[0]:
+            own = [] if dtype == torch.float32 else [(0, 0)] + [(0, 1)] * needs[0] + [(1, 1)] * needs[1]
+            assert native[1] == ["quantise"] + own
+    for a, b in zip(*results):
+        assert (a is None) == (b is None)
+        if a is not None:  # another order of the sums, rounded once more
+            torch.testing.assert_close(a, b, rtol=2 * torch.finfo(dtype).eps, atol=8 * torch.finfo(dtype).eps)
+
+
+def test_native_call_keeps_what_a_gradient_reads(native):
+    x, w = torch.randn(6, 16, requires_grad=True), torch.randn(24, 16)
+    h = x * 1
+    y = native[0](h, w)
+    h.add_(1)  # torch's linear with a frozen weight does not keep its input
+    y.sum().backward()
+    torch.testing.assert_close(x.grad, w.sum(0).expand_as(x) / 2)
+    w.requires_grad_()
+    y = native[0](x.detach(), w)
+    with torch.no_grad():
+        w.add_(1)  # an optimiser's step in front of the gradients: the quantised weight is what was multiplied
+    y.sum().backward()
+    torch.testing.assert_close(w.grad, x.detach().sum(0).expand_as(w))
+    kept = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: kept.append(t) or len(kept) - 1, lambda i: kept[i] * 2):
+        y = native[0](x, w)
+    dx, dw = torch.autograd.grad(y, (x, w), torch.ones_like(y))
+    assert len(kept) == 2
+    torch.testing.assert_close((dx, dw), ((w.sum(0).expand_as(x)).detach(), 2 * x.sum(0).expand_as(w).detach()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_second_derivatives_equal_torch(native, dtype):
+    torch.manual_seed(1)
+    x, w, v = torch.randn(4, 16).to(dtype), torch.randn(8, 16).to(dtype), torch.randn(4, 16).to(dtype)
+    results = []
+    for f in (native[0], through_torch):
+        xs, ws = x.clone().requires_grad_(), w.clone().requires_grad_()
+        (dx, dw) = torch.autograd.grad((f(xs, ws).float() ** 2).sum(), (xs, ws), create_graph=True)
+        results.append(torch.autograd.grad((dx * v).float().sum() + (dw.float() ** 2).mean(), (xs, ws)))
+    torch.testing.assert_close(*results, rtol=40 * torch.finfo(dtype).eps, atol=100 * torch.finfo(dtype).eps)
+
+
+def test_calls_that_are_not_plain_are_left_to_the_general_route(native):
+    f, calls = native
+    x, w = torch.randn(6, 16), torch.randn(24, 16)
+    assert f(x, w) is not None and f(x[:, ::2].repeat(1, 2), w) is not None
+    calls.clear()
+
+    class Sub(torch.Tensor):
+        pass
+
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    assert all(r is None for r in (f(x.double(), w.double()), f(x.half(), w), f(x[:, :8], w), f(x[0], w), f(x, w.t().contiguous().t()), f(x, w, 8),
+                                   f(x[:0], w), f(x.as_subclass(Sub), w), f(x.to("meta"), w)))
+    with torch.autograd.forward_ad.dual_level():
+        assert f(torch.autograd.forward_ad.make_dual(x, x), w) is None
+        assert f(x, torch.autograd.forward_ad.make_dual(w, w)) is None
+    with Mode():
+        assert f(x, w) is None
+    with torch.autocast("cpu", torch.bfloat16):
+        assert f(x, w) is None
+    torch.func.vmap(lambda x: [x, [None for r in [f(x, w)] if r is not None][:1]][0])(x[None])
+    assert calls == []
 
 
 def test_sizes_the_kernel_is_not_for():
@@ -107,3 +242,27 @@ def test_gemm_in_a_graph_and_on_two_streams():
             results.append(quant_cuda.gemm(a, b, False, True))
     torch.cuda.synchronize()
     assert all(torch.equal(r, want) for r in results)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,k,n", [((3, 683), 4096, 4104), ((5, 7), 264, 72)])  # the kernel's products, and torch's
+def test_training_pass_equals_the_general_route(dtype, rows, k, n):
+    import quant_cuda
+    with torch.device("cuda"):
+        lin = cl.QuantLinear(k, n, bias=True, w_bits=4, group_size=128, cherryq=True, cherry_fraction=1 / 16).to(dtype).train()
+    lin.register_cherry_indices(torch.arange(lin.num_cherries) * 7)
+    x = torch.randn(*rows, k, device="cuda").to(dtype).requires_grad_()
+    g = torch.randn(*rows, n, device="cuda").to(dtype)
+    assert quant_cuda.gemm_preferred(True, True, n, k, rows[0] * rows[1]) == (k == 4096)
+    results = []
+    for native in (True, False):
+        if not native:
+            lin._native_linear = lambda *_: None
+        x.grad = lin.weight.grad = lin.bias.grad = None
+        y = lin(x)
+        assert ("TrainLinear" in type(y.grad_fn.next_functions[0][0]).__name__ + y.grad_fn.next_functions[0][0].name()) == native
+        y.backward(g)
+        results.append([y.detach(), x.grad, lin.weight.grad, lin.bias.grad])
+    for a, b in zip(*results):
+        assert a.shape == b.shape and ((a.double() - b.double()).norm() / b.double().norm()).item() < 2 * LIMIT.get(dtype, 2.0 ** -18)
