@@ -633,18 +633,19 @@ __device__ __forceinline__ void prompt_finish(float4 (&sum)[QUADS], void *shared
     const int tid = threadIdx.x;
     // ---- across workgroups: tiles in scratch in the order [quad][thread]
     if (plan.splits > 1) {
-        constexpr size_t TILE = (size_t)ROWS * COLS;
-        float *base = partial + (size_t)at.tile * TILE + tid * 4;
-        const size_t per_split = (size_t)(plan.mtiles * plan.ntiles) * TILE;
+        constexpr uint32_t TILE = ROWS * COLS * sizeof(float);
+        const uint32_t per_split = (uint32_t)(plan.mtiles * plan.ntiles) * TILE;  // the plan keeps all of them below 2 GiB
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(partial, 0, plan.splits * per_split, kRsrcFlagsP);
+        const uint32_t base = (uint32_t)at.tile * TILE + tid * 16;
         auto has = [&](int q) { return ROWS * COLS / 4 % T == 0 || tid + q * T < ROWS * COLS / 4; };
-        auto word = [&](int s, int q, int h) { return reinterpret_cast<unsigned long long *>(base + s * per_split + (size_t)q * (4 * T)) + h; };
+        constexpr int kDevice = 16;  // past the die's L2
+        // (whole 16 bytes a lane: as 8-byte stores at a stride of 16 every line went to memory in two halves, 357 rows of 26848 -> 1792 69.4 us
+        // instead of 65.6.  Reading them in 16 bytes gains nothing there and costs small tiles 1.4 us.
+        // The whole offset in one vector register: behind a store with a scalar one the compiler writes the data's registers at once, which
+        // this card still reads.)
 #pragma unroll
-        for (int q = 0; q < QUADS; q++) {
-            if (!has(q)) break;
-            const float2 lo = make_float2(sum[q].x, sum[q].y), hi = make_float2(sum[q].z, sum[q].w);
-            __hip_atomic_store(word(at.split, q, 0), __builtin_bit_cast(unsigned long long, lo), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(word(at.split, q, 1), __builtin_bit_cast(unsigned long long, hi), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        for (int q = 0; q < QUADS; q++)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sum[q]), r, has(q) ? at.split * per_split + base + q * (16 * T) : kOobP, 0, kDevice);
         __syncthreads();  // the sums are read
         int *s_last = reinterpret_cast<int *>(shared);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -659,6 +660,7 @@ __device__ __forceinline__ void prompt_finish(float4 (&sum)[QUADS], void *shared
         if (tid == 0) __hip_atomic_store(&tickets[at.tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
         for (int q = 0; q < QUADS; q++) sum[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+        const unsigned long long *const words = reinterpret_cast<const unsigned long long *>(partial) + base / 8;
 #pragma unroll 2
         for (int s = 0; s < plan.splits; s++) {
             float2 v[QUADS][2];
@@ -666,7 +668,8 @@ __device__ __forceinline__ void prompt_finish(float4 (&sum)[QUADS], void *shared
             for (int q = 0; q < QUADS; q++)
 #pragma unroll
                 for (int h = 0; h < 2; h++)
-                    v[q][h] = has(q) ? __builtin_bit_cast(float2, __hip_atomic_load(word(s, q, h), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                    v[q][h] = has(q) ? __builtin_bit_cast(float2, __hip_atomic_load(words + (s * per_split + q * (16 * T)) / 8 + h, __ATOMIC_RELAXED,
+                                                                                    __HIP_MEMORY_SCOPE_AGENT))
                                      : make_float2(0.f, 0.f);
 #pragma unroll
             for (int q = 0; q < QUADS; q++) {
