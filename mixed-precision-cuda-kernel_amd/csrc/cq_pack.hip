@@ -106,7 +106,7 @@ __global__ __launch_bounds__(256) void pack_cherry_kernel(const __half *__restri
 // general form spent its time on).  A row of 65 dwords makes both the scatter (16 chunks x 4 rows) and
 // the later reads free of bank conflicts; bytes of four neighbouring rows leave as one dword, 128 bytes a line.
 // Bound by vector ALU first (about 14 operations an element, twice as many wavefronts a CU change nothing) and by one
-// read of the weight.  MI355X, 13824 x 5120 to 3 bits: 51 us (3.4 TB/s read + written; 28672 x 8192 to 4 bits 160),
+// read of the weight.  MI355X, 13824 x 5120 to 3 bits: 49 us (3.5 TB/s read + written),
 // with an address formed for each half and row, comparisons around loads and stores, cherry columns stored half by
 // half in the scatter and quotients of six operations 59 (188); the general form's three launches took 549.
 constexpr int kPackRows = 128, kPackStride = 65;  // dwords of LDS a row; halves 128 and 129 take what belongs nowhere
@@ -206,6 +206,12 @@ __global__ __launch_bounds__(kPackThreads) void pack_group_kernel(const __half *
 #pragma unroll
         for (int e = 0; e < 8; e++) at[e] = reinterpret_cast<unsigned short *>(s_w + row * kPackStride) + m.off[e];
     };
+    // The chunk or two that cherries and alignment push the range beyond 16, one a thread, and the first cherry columns, one value a
+    // thread, are asked for with the rest: behind it their round trip was one more (13824 x 5120 to 3 bits 51.2 -> 49.2 us).
+    const int more_row = t % kPackRows, more = 16 + t / kPackRows, cherry0 = col0 - k0, cherries = col1 - k1 - cherry0, cherry = t / kPackRows;
+    const __half *const more_at = w + (size_t)min(n0 + more_row, N - 1) * K;
+    uint4 mq = make_uint4(0, 0, 0, 0);
+    __half first_cherry = __half(0.f);
     {
         // A thread without a chunk or a row of its own repeats the last one: the same bytes to the same place (rows past N are
         // not read again), and neither loads nor stores wait for a comparison.
@@ -214,6 +220,8 @@ __global__ __launch_bounds__(kPackThreads) void pack_group_kernel(const __half *
 #pragma unroll
         for (int i = 0; i < kPackLoads; i++)
             q[i] = *reinterpret_cast<const uint4 *>(w + (size_t)min(n0 + r0 + kPackThreads / 16 * i, N - 1) * K + 8 * (c0 + ci));
+        if (more < nch) mq = *reinterpret_cast<const uint4 *>(more_at + 8 * (c0 + more));
+        if (cherry < cherries) first_cherry = more_at[s_idx[cherry0 + cherry]];
         const PackChunk m = pack_chunk(s_idx, C, 8 * (c0 + ci), k0, k1);
         unsigned short *at[8];
         columns(m, r0, at);
@@ -224,19 +232,18 @@ __global__ __launch_bounds__(kPackThreads) void pack_group_kernel(const __half *
             if ((t & 15) == 0) atomicMax(&s_max[r0 + kPackThreads / 16 * i], mx);
         }
     }
-    // the chunk or two that cherries and alignment push the range beyond 16
     for (int e = t; e < (nch - 16) * kPackRows; e += kPackThreads) {
-        const int row = e & (kPackRows - 1), c = c0 + 16 + e / kPackRows;
+        const int row = e % kPackRows, c = c0 + 16 + e / kPackRows;
+        if (e != t) mq = *reinterpret_cast<const uint4 *>(more_at + 8 * c);
         const PackChunk m = pack_chunk(s_idx, C, 8 * c, k0, k1);
         unsigned short *at[8];
         columns(m, row, at);
-        atomicMax(&s_max[row], place(m, at, *reinterpret_cast<const uint4 *>(w + (size_t)min(n0 + row, N - 1) * K + 8 * c), 0));
+        atomicMax(&s_max[row], place(m, at, mq, 0));
     }
-    // the cherry columns among them, from the lines just read: 128 neighbouring halves of an output row leave together
-    const int cherry0 = col0 - k0, cherries = col1 - k1 - cherry0;
+    // the cherry columns: 128 neighbouring halves of an output row leave together
     for (int e = t; e < cherries * kPackRows; e += kPackThreads) {
-        const int row = e & (kPackRows - 1), c = cherry0 + e / kPackRows;
-        if (n0 + row < N) cherry_weight[(size_t)c * N + n0 + row] = w[(size_t)(n0 + row) * K + s_idx[c]];
+        const int c = cherry0 + e / kPackRows;
+        if (n0 + more_row < N) cherry_weight[(size_t)c * N + n0 + more_row] = e == t ? first_cherry : more_at[s_idx[c]];
     }
     __syncthreads();
     if (t < kPackRows) {
