@@ -5,7 +5,7 @@
 // draw: 4096 x 4096 x 8192 runs at 1.35 PFLOP/s with the clock at 1.91 GHz (of 2.4) and the matrix cores busy 68 % of the time.
 //   * A workgroup of eight wavefronts owns a tile of 256 x 256, a wavefront 128 x 64 of it: 128 accumulators, two wavefronts a
 //     SIMD, so that one's waits lie behind the other's products (four wavefronts of 128 x 128: 5 to 10 % slower at every size).
-//   * K in steps of 64 through two LDS buffers of 64 KB, filled by loads that go straight to LDS (through registers: 5 us a tile
+//   * K in steps of 64 through two LDS buffers of 64 KB, filled by loads that go straight to LDS (through registers: 3 us a tile
 //     more at its ends).  A buffer is asked for again while its other half of products is still running, a load every three
 //     products (all at once, in front or behind: 3 to 5 % slower).
 //   * LDS holds the operands as they come, 128 bytes of a row of [free][K], 512 of a row of [K][free], in 16- or 32-byte pieces
