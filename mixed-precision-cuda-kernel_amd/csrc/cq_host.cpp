@@ -464,16 +464,27 @@ PyObject *bind_prompt(PyObject *, PyObject *address) {
 // A pass over a small layer is bound by the host: the fake quantisation's and the product's autograd nodes in Python, their checks, and
 // torch's own linear took 180 us for a forward and a backward whose kernels take 30.
 
+// Whether a launch may take the tensor's memory for its values, now: a gradient, or what a saved-tensor hook hands back, may be batched, a
+// wrapper, sparse, lazily negated, zeros without memory or carry a tangent, and modes may have been entered since the forward pass.  Asked
+// before the tensor's address, which some of these do not have.
+bool plain_memory(const Tensor &t) {
+    using K = c10::DispatchKey;
+    return t.layout() == at::kStrided && ordinary(t) && !t.is_nested() &&
+           !t.key_set().has_any(c10::DispatchKeySet({K::Negative, K::Conjugate, K::ZeroTensor, K::Python, K::Functionalize})) && !t._fw_grad(0).defined() &&
+           !at::autocast::is_autocast_enabled(t.device().type());
+}
+
 inline bool whole(const Tensor &t) { return t.is_contiguous() && reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0; }
 
 // out[m, n] = sum_k a(m, k) b(n, k) of 16-bit matrices (an operand by_k lies as [k, n]) where the kernel takes it and is faster than
 // torch's product; undefined elsewhere.  The result is laid out as `shape`.
 Tensor product(const Tensor &a, bool a_by_k, const Tensor &b, bool b_by_k, int64_t m, int64_t n, int64_t k, at::IntArrayRef shape) {
     constexpr int64_t most = INT32_MAX;
-    if ((a.scalar_type() != at::kHalf && a.scalar_type() != at::kBFloat16) || a.scalar_type() != b.scalar_type() || !whole(a) || !whole(b) || m > most ||
-        n > most || k > most || !train.gemm_preferred(a_by_k, b_by_k, (int)m, (int)n, (int)k))
+    if ((a.scalar_type() != at::kHalf && a.scalar_type() != at::kBFloat16) || a.scalar_type() != b.scalar_type() || a.device() != b.device() ||
+        !plain_memory(a) || !plain_memory(b) || m > most || n > most || k > most || a.numel() != m * k || b.numel() != n * k || !whole(a) || !whole(b))
         return {};
     const int device = a.get_device();
+    if (c10::hip::current_device() != device || !train.gemm_preferred(a_by_k, b_by_k, (int)m, (int)n, (int)k)) return {};
     void *const stream = current_stream(device);
     const Tensor out = at::empty(shape, a.options());
     const int64_t zero_bytes = (int64_t)train.gemm_workspace((int)m, (int)n, (int)k), bytes = (int64_t)train.gemm_scratch((int)m, (int)n, (int)k);

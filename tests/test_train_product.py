@@ -144,6 +144,104 @@ def test_calls_that_are_not_plain_are_left_to_the_general_route(native):
     assert calls == []
 
 
+def other_dual(g):
+    return torch.autograd.forward_ad.make_dual(g, torch.full_like(g, 0.5))
+
+
+class Counted(torch.utils._python_dispatch.TorchDispatchMode):
+    """The products that a dispatch mode sees."""
+    products = 0
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.products += func.overloadpacket in (torch.ops.aten.mm, torch.ops.aten.bmm, torch.ops.aten.addmm)
+        return func(*args, **(kwargs or {}))
+
+
+def gradients_with_a_tangent(f, x, w, g):
+    with torch.autograd.forward_ad.dual_level():
+        out = torch.autograd.grad(f(x, w), (x, w), other_dual(g))
+        return [torch.autograd.forward_ad.unpack_dual(t).tangent for t in out]
+
+
+def a_later_layer_with_a_tangent(f, x, w, g):
+    with torch.autograd.forward_ad.dual_level():
+        y = torch.nn.functional.linear(f(x, w), other_dual(w[:, :8].repeat(1, 3).detach()))
+        out = torch.autograd.grad((y * y).mean(), (x, w))
+        return [torch.autograd.forward_ad.unpack_dual(t).tangent for t in out]
+
+
+def under_a_mode(f, x, w, g):
+    y = f(x, w)
+    with Counted() as mode:
+        out = torch.autograd.grad(y, (x, w), g)
+    return [*out, torch.tensor(float(mode.products))]
+
+
+def under_autocast(f, x, w, g):
+    y, other = f(x, w), torch.float16 if x.dtype == torch.bfloat16 else torch.bfloat16
+    with torch.autocast("cpu", other):
+        return torch.autograd.grad(y, (x, w), g)
+
+
+def of_a_wrapper(f, x, w, g):
+    from torch.testing._internal.two_tensor import TwoTensor
+    out = torch.autograd.grad(f(x, w), (x, w), TwoTensor(g, g * 2))
+    return [t for two in out for t in (two.a, two.b)]
+
+
+def kept(change):
+    def call(f, x, w, g):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t.detach(), change):
+            y = f(x, w)
+        return torch.autograd.grad(y, (x, w), g)
+    return call
+
+
+# what arrives at the backward of a forward pass that was plain
+ARRIVES = {
+    "tangent": gradients_with_a_tangent,
+    "later tangent": a_later_layer_with_a_tangent,
+    "batched": lambda f, x, w, g: torch.autograd.grad(f(x, w), (x, w), torch.stack([g, 2 * g, g * g]), is_grads_batched=True),
+    "vmap": lambda f, x, w, g: (lambda y: torch.func.vmap(lambda v: torch.autograd.grad(y, (x, w), v, retain_graph=True))(torch.stack([g, 2 * g])))(f(x, w)),
+    "jacobian": lambda f, x, w, g: torch.autograd.functional.jacobian(f, (x, w), vectorize=True),
+    "negated": lambda f, x, w, g: torch.autograd.grad(f(x, w), (x, w), torch._neg_view(g)),
+    "zeros": lambda f, x, w, g: torch.autograd.grad(f(x, w), (x, w), torch._efficientzerotensor(g.shape, dtype=g.dtype, device=g.device)),
+    "mode": under_a_mode,
+    "autocast": under_autocast,
+    "wrapper": of_a_wrapper,
+    "kept negated": kept(torch._neg_view),
+    "kept elsewhere": kept(lambda t: t.to("meta")),
+}
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", ARRIVES)
+def test_gradients_of_what_is_not_plain_are_left_to_torch(native, case, dtype):
+    """A launch sees addresses: what arrives at the backward has to be asked there, whatever the forward's arguments were."""
+    torch.manual_seed(2)
+    x, w, g = (torch.randn(shape).to(dtype) for shape in ((6, 16), (24, 16), (6, 24)))
+    results = []
+    for f in (native[0], through_torch):
+        native[1].clear()
+        results.append(ARRIVES[case](f, x.clone().requires_grad_(), w.clone().requires_grad_(), g))
+        assert not {(0, 1), (1, 1)} & set(native[1]), native[1]
+    for a, b in zip(*results):
+        assert a is not None and a.shape == b.shape and a.device == b.device
+        if case != "kept elsewhere":
+            torch.testing.assert_close(a, b, rtol=4 * torch.finfo(dtype).eps, atol=32 * torch.finfo(dtype).eps)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_a_saved_weight_of_another_shape_raises(native, dtype):
+    x, w = torch.randn(6, 16).to(dtype).requires_grad_(), torch.randn(24, 16).to(dtype)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t[:2].clone()):
+        y = native[0](x, w)
+    native[1].clear()
+    with pytest.raises(RuntimeError):
+        y.backward(torch.ones_like(y))
+    assert native[1] == []
+
+
 def test_sizes_the_kernel_is_not_for():
     import quant_cuda
     for by_k in ((False, False), (False, True), (True, True)):
