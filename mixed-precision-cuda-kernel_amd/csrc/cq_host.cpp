@@ -470,8 +470,7 @@ PyObject *bind_prompt(PyObject *, PyObject *address) {
 bool plain_memory(const Tensor &t) {
     using K = c10::DispatchKey;
     return t.layout() == at::kStrided && ordinary(t) && !t.is_nested() &&
-           !t.key_set().has_any(c10::DispatchKeySet({K::Negative, K::Conjugate, K::ZeroTensor, K::Python, K::Functionalize})) && !t._fw_grad(0).defined() &&
-           !at::autocast::is_autocast_enabled(t.device().type());
+           !t.key_set().has_any(c10::DispatchKeySet({K::Negative, K::Conjugate, K::ZeroTensor, K::Python, K::Functionalize})) && !t._fw_grad(0).defined();
 }
 
 inline bool whole(const Tensor &t) { return t.is_contiguous() && reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0; }
@@ -484,7 +483,9 @@ Tensor product(const Tensor &a, bool a_by_k, const Tensor &b, bool b_by_k, int64
         !plain_memory(a) || !plain_memory(b) || m > most || n > most || k > most || a.numel() != m * k || b.numel() != n * k || !whole(a) || !whole(b))
         return {};
     const int device = a.get_device();
-    if (c10::hip::current_device() != device || !train.gemm_preferred(a_by_k, b_by_k, (int)m, (int)n, (int)k)) return {};
+    if (c10::hip::current_device() != device || at::autocast::is_autocast_enabled(a.device().type()) ||
+        !train.gemm_preferred(a_by_k, b_by_k, (int)m, (int)n, (int)k))
+        return {};
     void *const stream = current_stream(device);
     const Tensor out = at::empty(shape, a.options());
     const int64_t zero_bytes = (int64_t)train.gemm_workspace((int)m, (int)n, (int)k), bytes = (int64_t)train.gemm_scratch((int)m, (int)n, (int)k);
@@ -576,14 +577,15 @@ PyObject *train_linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     if (!x || !weight || !indices || !PyLong_CheckExact(args[3]) || !PyLong_CheckExact(args[4]) || !train.gemm) Py_RETURN_NONE;
     const long bits = PyLong_AsLong(args[3]), group = PyLong_AsLong(args[4]);
     if (PyErr_Occurred()) return nullptr;
-    if (!t->is_cuda() || t->dim() != 2 || !t->is_contiguous() || !ordinary(*x) || !ordinary(*t)) Py_RETURN_NONE;
+    if (!t->is_cuda() || !plain_memory(*x) || !plain_memory(*t) || !plain_memory(*indices) || t->dim() != 2 || !t->is_contiguous())
+        Py_RETURN_NONE;
     const int device = t->get_device();
     const auto type = t->scalar_type();
     const FakeQuantFn quantise = type == at::kHalf ? train.fake_quant_f16 : type == at::kBFloat16 ? train.fake_quant_bf16 : type == at::kFloat ? train.fake_quant_f32 : nullptr;
     const int64_t n = t->size(0), k = t->size(1);
     if (!quantise || x->scalar_type() != type || x->device() != t->device() || x->dim() < 2 || x->size(-1) != k || !x->numel() || n <= 0 || n > INT32_MAX ||
-        k > INT32_MAX || group > INT32_MAX || !is(indices, at::kInt, 1, device) || indices->numel() > INT32_MAX || !indices->has_storage() ||
-        c10::hip::current_device() != device || at::autocast::is_autocast_enabled(t->device().type()) || x->_fw_grad(0).defined() || t->_fw_grad(0).defined())
+        k > INT32_MAX || group > INT32_MAX || !is(indices, at::kInt, 1, device) || indices->numel() > INT32_MAX ||
+        c10::hip::current_device() != device || at::autocast::is_autocast_enabled(t->device().type()))
         Py_RETURN_NONE;
     Tensor quantised, out;
     {

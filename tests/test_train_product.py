@@ -231,6 +231,17 @@ def test_gradients_of_what_is_not_plain_are_left_to_torch(native, case, dtype):
             torch.testing.assert_close(a, b, rtol=4 * torch.finfo(dtype).eps, atol=32 * torch.finfo(dtype).eps)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_inputs_without_sizes_and_negated_weights_are_left_to_the_general_route(native, dtype):
+    """A nested tensor has rows of its own for every sequence, which torch's linear takes and a launch does not."""
+    x, w = torch.randn(6, 16).to(dtype), torch.randn(24, 16).to(dtype)
+    nested = torch.nested.nested_tensor([torch.randn(2, 16), torch.randn(3, 16)], dtype=dtype)
+    native[1].clear()
+    for args in ((nested, w), (x, torch._neg_view(w)), (x, torch._efficientzerotensor(w.shape, dtype=dtype, device="cpu")), (x.to_sparse(), w), (torch._neg_view(x), w)):
+        assert native[0](*args) is None
+    assert native[1] == []
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_a_saved_weight_of_another_shape_raises(native, dtype):
     x, w = torch.randn(6, 16).to(dtype).requires_grad_(), torch.randn(24, 16).to(dtype)
