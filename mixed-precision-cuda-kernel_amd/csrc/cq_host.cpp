@@ -538,7 +538,8 @@ struct TrainLinear : torch::autograd::Function<TrainLinear> {
         }
         if (x.defined()) {
             const int64_t k = x.size(-1), rows = g.numel() / std::max<int64_t>(n, 1);
-            const Tensor g2 = g.reshape({rows, n}), x2 = x.reshape({rows, k});
+            // (matrices as they are: a sparse one multiplies, but does not reshape)
+            const Tensor g2 = g.dim() == 2 ? g : g.reshape({rows, n}), x2 = x.dim() == 2 ? x : x.reshape({rows, k});
             if (!twice && n) dw = product(g2, true, x2, true, n, k, rows, {n, k});
             if (!dw.defined()) dw = g2.t().matmul(x2);
         }

@@ -210,6 +210,8 @@ ARRIVES = {
     "autocast": under_autocast,
     "wrapper": of_a_wrapper,
     "kept negated": kept(torch._neg_view),
+    "sparse": lambda f, x, w, g: torch.autograd.grad(f(x, w), (x, w), g.to_sparse()),
+    "kept sparse": kept(lambda t: t.to_sparse()),
     "kept elsewhere": kept(lambda t: t.to("meta")),
 }
 
