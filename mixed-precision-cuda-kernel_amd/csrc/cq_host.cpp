@@ -525,7 +525,8 @@ struct TrainLinear : torch::autograd::Function<TrainLinear> {
         Tensor quantised = saved[1], dx, dw;
         const bool twice = at::GradMode::is_enabled();  // a graph of the gradients is asked for
         const int64_t n = g.size(-1);
-        if (quantised.defined()) {
+        // (a call may ask for one of them: autograd.grad of the input alone, backward(inputs=...))
+        if (quantised.defined() && ctx->needs_input_grad(0)) {
             const int64_t k = quantised.size(1);
             std::vector<int64_t> shape(g.sizes().begin(), g.sizes().end());
             shape.back() = k;
@@ -536,7 +537,7 @@ struct TrainLinear : torch::autograd::Function<TrainLinear> {
             }
             if (!dx.defined()) dx = g.matmul(quantised);
         }
-        if (x.defined()) {
+        if (x.defined() && ctx->needs_input_grad(1)) {
             const int64_t k = x.size(-1), rows = g.numel() / std::max<int64_t>(n, 1);
             // (matrices as they are: a sparse one multiplies, but does not reshape)
             const Tensor g2 = g.dim() == 2 ? g : g.reshape({rows, n}), x2 = x.dim() == 2 ? x : x.reshape({rows, k});

@@ -3,6 +3,7 @@
 Bound of the kernel: fp32 sums of exact 16-bit products, rounded once.  The rounding is half an ulp of the result's type, at most
 2^-11 (fp16) or 2^-8 (bf16) of an element, its 2-norm about 0.6 of that; a sum of K terms of random signs adds about sqrt(K) 2^-24 of
 the result, 2^-17 at the largest K here.  So 2^-11 / 2^-8 of the 2-norm holds with room."""
+import contextlib
 import ctypes
 import shutil
 from pathlib import Path
@@ -102,6 +103,23 @@ def test_native_call_keeps_what_a_gradient_reads(native):
     dx, dw = torch.autograd.grad(y, (x, w), torch.ones_like(y))
     assert len(kept) == 2
     torch.testing.assert_close((dx, dw), ((w.sum(0).expand_as(x)).detach(), 2 * x.sum(0).expand_as(w).detach()))
+
+
+@pytest.mark.parametrize("twice", [False, True])
+def test_gradients_that_nobody_asks_for_are_not_computed(native, twice):
+    f, calls = native
+    x, w, g = torch.randn(6, 16).half().requires_grad_(), torch.randn(24, 16).half().requires_grad_(), torch.randn(6, 24).half()
+    want = torch.autograd.grad(f(x, w), (x, w), g)
+    for i, asked in enumerate((x, w)):
+        y = f(x, w)
+        calls.clear()
+        with Counted() if twice else contextlib.nullcontext() as mode:
+            dt, = torch.autograd.grad(y, asked, g, create_graph=twice)
+        assert (calls == [] and mode.products == 1) if twice else calls == [(i, 1)]
+        torch.testing.assert_close(dt.detach(), want[i], rtol=2 ** -9, atol=2 ** -7)
+    y = f(x, w)
+    y.backward(g, inputs=[x])
+    assert calls[-1] == (0, 1) and w.grad is None
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
