@@ -82,20 +82,31 @@ struct Pool {
     int64_t floor;
 
     Tensor get(int device, void *stream, int64_t bytes) {
-        std::lock_guard<std::mutex> hold(lock);
-        Tensor &t = live[{device, reinterpret_cast<uintptr_t>(stream)}];
-        if (!t.defined() || t.numel() < bytes) {
-            if (t.defined()) {
-                outgrown.push_back(t);
-                bytes = std::max(bytes, 2 * t.numel());
-            }
+        const std::pair<int, uintptr_t> key{device, reinterpret_cast<uintptr_t>(stream)};
+        int64_t size = std::max(bytes, floor);
+        {
+            std::lock_guard<std::mutex> hold(lock);
+            const Tensor &t = live[key];
+            if (t.defined() && t.numel() >= bytes) return t;
+            if (t.defined()) size = std::max(size, 2 * t.numel());
+        }
+        // Without the lock: callers come with and without the interpreter's, and an allocation may ask for that one (a record of
+        // allocations with Python's stacks).  Who comes second drops what they made.
+        Tensor made;
+        {
             // plain tensors, whatever mode or function transform the first caller is in
             using K = c10::DispatchKey;
             c10::InferenceMode normal(false);
             c10::impl::ExcludeDispatchKeyGuard untouched(c10::DispatchKeySet({K::FuncTorchDynamicLayerFrontMode, K::FuncTorchDynamicLayerBackMode,
                                                                               K::FuncTorchVmapMode, K::Python, K::PythonTLSSnapshot}));
             const auto opts = at::TensorOptions().dtype(at::kByte).device(at::kCUDA, device);
-            t = zeroed ? at::zeros({std::max(bytes, floor)}, opts) : at::empty({std::max(bytes, floor)}, opts);
+            made = zeroed ? at::zeros({size}, opts) : at::empty({size}, opts);
+        }
+        std::lock_guard<std::mutex> hold(lock);
+        Tensor &t = live[key];
+        if (!t.defined() || t.numel() < bytes) {
+            if (t.defined()) outgrown.push_back(t);
+            t = made;
         }
         return t;
     }

@@ -205,6 +205,47 @@ def test_tensors_without_memory_raise(host):
     assert run.returncode == 0 and "done" in run.stdout, (run.returncode, run.stdout[-500:], run.stderr[-2000:])
 
 
+def test_kept_buffers_are_made_without_the_pools_lock(tmp_path, monkeypatch):
+    """Autograd's threads ask for a kept buffer without the interpreter's lock, other callers with it; an allocation that asks for
+    the interpreter (a record of allocations with Python's stacks) does not meet a caller that holds it and waits for the pool."""
+    if shutil.which("g++") is None or not Path("/opt/rocm/include").is_dir():
+        pytest.skip("needs g++ and the HIP headers")
+    asks = """#include <Python.h>
+#include <ATen/ATen.h>
+static at::Tensor asking_zeros(at::IntArrayRef sizes, const at::TensorOptions &options) {
+    const PyGILState_STATE state = PyGILState_Ensure();
+    PyRun_SimpleString("allocating()");
+    PyGILState_Release(state);
+    return at::zeros(sizes, options);
+}
+namespace {
+
+using at::Tensor;"""
+    monkeypatch.setattr(sys.modules[__name__], "_CPU", [*_CPU, ("at::zeros(", "asking_zeros("), ("namespace {\n\nusing at::Tensor;", asks)])
+    build_cpu_host(tmp_path)
+    script = f"""
+import importlib.util, threading, torch
+spec = importlib.util.spec_from_file_location("cherryq_host_cpu", {str(tmp_path / "cherryq_host_cpu.so")!r})
+host = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(host)
+threads, results = [], []
+
+def allocating():
+    if not threads:
+        threads.append(threading.Thread(target=lambda: results.append(host.workspace(-1, 7, 64))))
+        threads[0].start()
+        threads[0].join()
+
+results.append(host.workspace(-1, 7, 64))
+assert len(threads) == 1 and len(results) == 2 and results[0].data_ptr() == results[1].data_ptr() == host.workspace(-1, 7, 64).data_ptr()
+grown = host.workspace(-1, 7, results[0].numel() + 1)
+assert grown.numel() == 2 * results[0].numel() and not grown.any() and host.workspace(-1, 7, 64).data_ptr() == grown.data_ptr()
+print("done")
+"""
+    r = subprocess.run([sys.executable, "-c", script], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout == "done\n", r.stderr
+
+
 def test_the_library_beside_the_module_is_loaded(tmp_path):
     """... whatever lies on sys.path in front of it or was imported under its name."""
     (tmp_path / "cherryq_host.py").write_text("built_for = linear = None\n")
