@@ -213,6 +213,11 @@ size_t cherryq_gemm_scratch_bytes(int M, int N, int K);
 int cherryq_gemm_preferred(int a_by_k, int b_by_k, int M, int N, int K);
 int cherryq_gemm_16(int bf16, int a_by_k, int b_by_k, const void *a, const void *b, void *out, int M, int N, int K, void *workspace,
                     size_t workspace_bytes, void *scratch, size_t scratch_bytes, void *stream);
+/*
+ * 1 while `stream` records a graph (or does not say).  A buffer kept for the stream is shared with other graphs and other calls then, and
+ * zeros that a graph writes are not there before its first replay: a recorded call takes a zeroed workspace of its own.
+ */
+int cherryq_stream_capturing(void *stream);
 
 /*
  * cherryq_vecquant{3,4}matmul_f16 for callers that cannot allocate device memory or carry a

@@ -296,6 +296,15 @@ static int fake_quant_entry(cq::FqDtype dtype, int w_bits, const void *weight, c
                                       reinterpret_cast<hipStream_t>(stream));
 }
 
+int cherryq_stream_capturing(void *stream) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(reinterpret_cast<hipStream_t>(stream), &capture) != hipSuccess) {
+        (void)hipGetLastError();
+        return 1;
+    }
+    return capture != hipStreamCaptureStatusNone;
+}
+
 size_t cherryq_gemm_workspace_bytes(int M, int N, int K) { return M > 0 && N > 0 && K > 0 ? cq::gemm_plan(M, N, K).workspace_bytes : 0; }
 
 size_t cherryq_gemm_scratch_bytes(int M, int N, int K) { return M > 0 && N > 0 && K > 0 ? cq::gemm_plan(M, N, K).scratch_bytes : 0; }
@@ -826,12 +835,7 @@ int cherryq_prompt_taken(int w_bits, int rows, int in_features, int out_features
     if ((w_bits != 3 && w_bits != 4) || (w_bits == 4 && G < 128) || rows < cq::kPromptMinRows || K <= 0 || N <= 0 || C < 0 || C > K || K % 8 ||
         N % 8 || C % 8 || G <= 0 || (C > 0 && K > 32768) || cq::force_generic() || !cq::prompt_supported(w_bits, rows, K, N, C, G))
         return 0;
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(reinterpret_cast<hipStream_t>(stream), &capture) != hipSuccess) {
-        (void)hipGetLastError();
-        return 0;
-    }
-    return capture == hipStreamCaptureStatusNone;
+    return !cherryq_stream_capturing(stream);
 }
 
 int cherryq_prefill_norm_f16(void *hidden, const void *delta, const void *weight, void *normed, int rows, int hidden_size,

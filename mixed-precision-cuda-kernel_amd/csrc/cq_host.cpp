@@ -57,6 +57,8 @@ struct Api {
     ShapeFn prepack_supported, rows_recommended;
 } api;
 TakenFn prompt_taken;  // cherryq_prompt_taken
+using CapturingFn = int (*)(void *);
+CapturingFn capturing;  // cherryq_stream_capturing
 
 using FakeQuantFn = int (*)(int, const void *, const void *, void *, int, int, int, int, int, void *);
 using GemmSizeFn = size_t (*)(int, int, int);
@@ -471,6 +473,13 @@ PyObject *bind_prompt(PyObject *, PyObject *address) {
     Py_RETURN_NONE;
 }
 
+// bind_capturing(address): cherryq_stream_capturing.  Without it no stream is taken to record a graph.
+PyObject *bind_capturing(PyObject *, PyObject *address) {
+    capturing = reinterpret_cast<CapturingFn>(PyLong_AsVoidPtr(address));
+    if (PyErr_Occurred()) return nullptr;
+    Py_RETURN_NONE;
+}
+
 // ---- the training layer ----------------------------------------------------------------------------
 // A pass over a small layer is bound by the host: the fake quantisation's and the product's autograd nodes in Python, their checks, and
 // torch's own linear took 180 us for a forward and a backward whose kernels take 30.
@@ -502,7 +511,11 @@ Tensor product(const Tensor &a, bool a_by_k, const Tensor &b, bool b_by_k, int64
     const int64_t zero_bytes = (int64_t)train.gemm_workspace((int)m, (int)n, (int)k), bytes = (int64_t)train.gemm_scratch((int)m, (int)n, (int)k);
     // the call's own, given back behind it in the stream's order: two streams never share it
     const Tensor scratch = bytes ? at::empty({bytes}, a.options().dtype(at::kByte)) : Tensor();
-    const Tensor zero = zero_bytes ? workspaces.get(device, stream, zero_bytes) : Tensor();
+    // (so are a recorded call's tickets, zeroed in the graph: the stream's kept ones are other graphs' and other calls', too, and zeros that
+    // were only recorded are not there yet when another graph is replayed first)
+    const Tensor zero = !zero_bytes                       ? Tensor()
+                        : capturing && capturing(stream) ? at::zeros({zero_bytes}, a.options().dtype(at::kByte))
+                                                         : workspaces.get(device, stream, zero_bytes);
     const int rc = train.gemm(a.scalar_type() == at::kBFloat16, a_by_k, b_by_k, a.const_data_ptr(), b.const_data_ptr(), out.mutable_data_ptr(), (int)m, (int)n,
                               (int)k, bytes ? zero.mutable_data_ptr() : nullptr, bytes ? (size_t)zero.numel() : 0,
                               bytes ? scratch.mutable_data_ptr() : nullptr, (size_t)bytes, stream);
@@ -627,6 +640,7 @@ PyObject *is_ordinary(PyObject *, PyObject *x) {
 PyMethodDef methods[] = {
     {"bind", bind, METH_O, nullptr},
     {"bind_prompt", bind_prompt, METH_O, nullptr},
+    {"bind_capturing", bind_capturing, METH_O, nullptr},
     {"bind_train", bind_train, METH_O, nullptr},
     {"train_linear", (PyCFunction)(void (*)())train_linear, METH_FASTCALL, nullptr},
     {"ordinary", is_ordinary, METH_O, nullptr},

@@ -123,6 +123,9 @@ train_linear = _host.train_linear  # (x, weight, cherry_indices, w_bits, group_s
 _lib.cherryq_prompt_taken.argtypes = [_int, _int, _int, _int, _int, _int, _vp]
 _lib.cherryq_prompt_taken.restype = _int
 _host.bind_prompt(ctypes.cast(_lib.cherryq_prompt_taken, _vp).value)
+_lib.cherryq_stream_capturing.argtypes = [_vp]
+_lib.cherryq_stream_capturing.restype = _int
+_host.bind_capturing(ctypes.cast(_lib.cherryq_stream_capturing, _vp).value)
 
 
 def _fail(status: int, what: str):
@@ -616,7 +619,10 @@ def gemm(a, b, a_by_k=False, b_by_k=False, shape=None):
         if out.numel() != m * n:
             raise RuntimeError(f"gemm: {m} x {n} results do not fit shape {tuple(shape)}")
         stream = _current_stream(dev.index)
-        ws = _workspace(dev, stream, _lib.cherryq_gemm_workspace_bytes(m, n, k))
+        nbytes = _lib.cherryq_gemm_workspace_bytes(m, n, k)
+        # a recorded call's tickets are its own: other graphs and other calls use the stream's kept ones
+        ws = (torch.zeros(nbytes, dtype=torch.uint8, device=dev) if nbytes and _lib.cherryq_stream_capturing(stream)
+              else _workspace(dev, stream, nbytes))
         scratch = torch.empty(_lib.cherryq_gemm_scratch_bytes(m, n, k), dtype=torch.uint8, device=dev)  # the call's own
         rc = _lib.cherryq_gemm_16(a.dtype == torch.bfloat16, a_by_k, b_by_k, a.data_ptr(), b.data_ptr(), out.data_ptr(), m, n, k,
                                   ws.data_ptr(), ws.numel(), _ptr(scratch), scratch.numel(), stream)

@@ -26,7 +26,7 @@ def native(tmp_path_factory):
     directory = tmp_path_factory.mktemp("train")
     t.build_cpu_host(directory)
     host, _, stubs = t.load_cpu_host(directory)
-    vp, i, sz, calls = ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t, []
+    vp, i, sz, calls, workspaces = ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t, [], []
 
     def at(address, rows, cols, dtype):
         return torch.frombuffer((ctypes.c_uint8 * (rows * cols * dtype.itemsize)).from_address(address), dtype=dtype).view(rows, cols)
@@ -45,6 +45,7 @@ def native(tmp_path_factory):
         dtype = torch.bfloat16 if bf16 else torch.float16
         x, y = at(a, k if a_by_k else m, m if a_by_k else k, dtype), at(b, k if b_by_k else n, n if b_by_k else k, dtype)
         assert wsz >= 16 and scz == 64
+        workspaces.append((ctypes.string_at(ws, 16), wsz))
         at(out, m, n, dtype).copy_((x.t() if a_by_k else x).float() @ (y if b_by_k else y.t()).float())
         return 0
 
@@ -53,7 +54,12 @@ def native(tmp_path_factory):
     mine += [size(lambda *_: 16), size(lambda *_: 64), ctypes.CFUNCTYPE(i, i, i, i, i, i)(lambda *a: 1),
              ctypes.CFUNCTYPE(i, i, i, i, vp, vp, vp, i, i, i, vp, sz, vp, sz, vp)(gemm)]
     host.bind_train(tuple(ctypes.cast(f, vp).value for f in mine))
-    yield lambda x, w, bits=4: host.train_linear(x, w, torch.arange(8, dtype=torch.int32), bits, 8), calls
+
+    def call(x, w, bits=4):
+        return host.train_linear(x, w, torch.arange(8, dtype=torch.int32), bits, 8)
+
+    call.host, call.workspaces = host, workspaces
+    yield call, calls
     del stubs, mine
 
 
@@ -262,6 +268,20 @@ def test_inputs_without_sizes_and_negated_weights_are_left_to_the_general_route(
     assert native[1] == []
 
 
+def test_recorded_products_take_tickets_of_their_own(native):
+    """A stream under capture: nothing kept is used, the sizes are exactly what the call asks for, and the tickets are zeros."""
+    f, _ = native
+    stub = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p)(lambda stream: recording)
+    f.host.bind_capturing(ctypes.cast(stub, ctypes.c_void_p).value)
+    try:
+        for recording in (0, 1, 0):
+            f.workspaces.clear()
+            f(torch.randn(6, 16).half().requires_grad_(), torch.randn(24, 16).half().requires_grad_()).backward(torch.ones(6, 24).half())
+            assert len(f.workspaces) == 3 and all(zeros == bytes(16) and (size == 16) == recording for zeros, size in f.workspaces)
+    finally:
+        f.host.bind_capturing(0)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_a_saved_weight_of_another_shape_raises(native, dtype):
     x, w = torch.randn(6, 16).to(dtype).requires_grad_(), torch.randn(24, 16).to(dtype)
@@ -395,3 +415,46 @@ def test_training_pass_equals_the_general_route(dtype, rows, k, n):
         results.append([y.detach(), x.grad, lin.weight.grad, lin.bias.grad])
     for a, b in zip(*results):
         assert a.shape == b.shape and ((a.double() - b.double()).norm() / b.double().norm()).item() < 2 * LIMIT.get(dtype, 2.0 ** -18)
+
+
+@pytest.mark.gpu
+def test_training_passes_in_two_graphs():
+    """Forward and backward captured twice on one stream, replayed the other way round, with eager passes between and what is kept for
+    that stream full of other calls' counts: a graph's tickets are its own."""
+    import quant_cuda
+    rows, k, n = 2048, 3584, 10752
+    print("training passes in two graphs", rows, k, n, flush=True)
+    for form in ((False, False, rows, n, k), (False, True, rows, k, n), (True, True, n, k, rows)):
+        assert quant_cuda.gemm_preferred(*form) and quant_cuda._lib.cherryq_gemm_workspace_bytes(*form[2:]) > 0
+    with torch.device("cuda"):
+        lin = cl.QuantLinear(k, n, bias=False, w_bits=4, group_size=128, cherryq=True, cherry_fraction=1 / 16).bfloat16().train()
+    lin.register_cherry_indices(torch.arange(lin.num_cherries) * 7)
+    inputs = [(torch.randn(rows, k, device="cuda").bfloat16().requires_grad_(), torch.randn(rows, n, device="cuda").bfloat16()) for _ in range(2)]
+
+    def step(x, g):
+        y = lin(x)
+        return [y.detach(), *torch.autograd.grad(y, (x, lin.weight), g)]
+
+    want, stream = [step(*i) for i in inputs], torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        step(*inputs[0])
+    torch.cuda.synchronize()
+    graphs, outs = [torch.cuda.CUDAGraph() for _ in inputs], []
+    for graph, i in zip(graphs, inputs):
+        with torch.cuda.graph(graph, stream=stream):
+            outs.append(step(*i))
+    kept = quant_cuda._host.workspace(0, stream.cuda_stream, 8)
+    torch.cuda.synchronize()
+    kept.fill_(0x7f)
+    for which in (1, 0, 0, 1, 0):
+        for t in outs[which]:
+            t.zero_()
+        graphs[which].replay()
+        eager = step(*inputs[which])
+        torch.cuda.synchronize()
+        for got, again, w in zip(outs[which], eager, want[which]):
+            assert torch.equal(got, w) and torch.equal(again, w)
+    assert (kept == 0x7f).all()
+    kept.zero_()
+    torch.cuda.synchronize()
