@@ -48,6 +48,7 @@ constexpr int kLoads = 2 * kChunks;
 constexpr uint32_t kTileSums = kTile * kTile * sizeof(float);
 constexpr uint32_t kRsrcFlagsG = 0x00020000u, kOobG = 0x80000000u;
 constexpr int kDeviceScope = 16;  // of a buffer access: past the die's L2
+constexpr int kPolls = 1 << 18;   // a microsecond or so each
 
 // (The compiler's own form may name another destination and then copies accumulators.  Distances: products into the same accumulator
 // need none, fragments come from LDS behind a wait, and the results are read behind the s_nop at the loop's end, which names the last
@@ -273,7 +274,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(const void *__restric
         }
     };
     // ---- across workgroups where K is split.  All but the last to arrive leave their sums and end (more than two: the last one too); the
-    // last one waits only for workgroups that have arrived, which wait for nobody
+    // last one waits only for workgroups that have arrived, which wait for nobody.  It waits for some 10 us at most; counts that another
+    // call has changed (a workspace that is shared against the rule) end the wait all the same, and the tile is NaN
     if (rest >= 0 && plan.splits > 1) {
         unsigned *const arrived = tickets + 2 * rest, *const written = arrived + 1;
         char *const all = scratch + (size_t)rest * plan.splits * kTileSums;
@@ -297,11 +299,20 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(const void *__restric
             }
         }
         if (tid == 0) {
-            while (__hip_atomic_load(written, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (unsigned)(plan.splits - 1)) __builtin_amdgcn_s_sleep(2);
+            int polls = kPolls;
+            while (__hip_atomic_load(written, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (unsigned)(plan.splits - 1) && --polls) __builtin_amdgcn_s_sleep(2);
+            s_order[1] = polls;
             __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(written, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         __syncthreads();
+        if (__builtin_amdgcn_readfirstlane(s_order[1]) == 0) {  // counts that are not this call's: say so, and end
+            const u32x4 nan = {0x7fff7fffu, 0x7fff7fffu, 0x7fff7fffu, 0x7fff7fffu};  // in fp16 and in bfloat16
+            const int col = nt * kTile + 8 * (tid & 31);
+            for (int row = mt * kTile + (tid >> 5); row < min(M, (mt + 1) * kTile) && col < N; row += kThreads / 32)
+                *reinterpret_cast<u32x4 *>(out + (size_t)row * N + col) = nan;
+            return;
+        }
         const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(all, 0, plan.splits * kTileSums, kRsrcFlagsG);
         auto part = [&](int s, int m, int n) {
             return __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(r, at + (m * kColFrags + n) * 1024, s * kTileSums, kDeviceScope));

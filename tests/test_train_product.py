@@ -458,3 +458,28 @@ def test_training_passes_in_two_graphs():
     assert (kept == 0x7f).all()
     kept.zero_()
     torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_a_wait_for_counts_that_never_come_ends(dtype):
+    """A workspace that is not zero, against the interface: the last workgroup of each split tile gives its wait up (a quarter of a second
+    or so) and its tile is NaN; tiles that are not split are as ever."""
+    import quant_cuda
+    m, n, k = 4096, 4352, 2056
+    lib, lead = quant_cuda._lib, 256
+    tiles, nbytes = lib.cherryq_gemm_workspace_bytes(m, n, k) // 8, lib.cherryq_gemm_scratch_bytes(m, n, k)
+    print("a wait that ends", m, n, k, tiles, flush=True)
+    assert 0 < tiles < m // lead * (n // lead)
+    a, b = operands(m, n, k, False, False, dtype)
+    want, out = quant_cuda.gemm(a, b), torch.empty(m, n, device="cuda", dtype=dtype)
+    counts, scratch = torch.zeros(2 * tiles, dtype=torch.int32, device="cuda"), torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    for planted in (1 << 30, 0):
+        counts[1::2] = planted
+        assert lib.cherryq_gemm_16(dtype == torch.bfloat16, 0, 0, a.data_ptr(), b.data_ptr(), out.data_ptr(), m, n, k, counts.data_ptr(),
+                                   4 * counts.numel(), scratch.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        nan = out.isnan().view(m // lead, lead, n // lead, lead).transpose(1, 2).flatten(2)
+        assert torch.equal(nan.any(-1), nan.all(-1)) and int(nan.all(-1).sum()) == (tiles if planted else 0)
+        assert torch.equal(out[~out.isnan()], want[~out.isnan()])
+        counts.zero_()
