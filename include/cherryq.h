@@ -203,10 +203,11 @@ int cherryq_fake_quant_f32(int w_bits, const void *weight, const int32_t *cherry
  * The training layer's products in 16 bits (fp16, or bfloat16 where bf16 != 0) with fp32 sums and one rounding:
  * out[M][N] = sum over K of A(m, k) * B(n, k), all row-major and contiguous, `a` as [M][K], or [K][M] where a_by_k != 0, `b` as
  * [N][K], or [K][N] where b_by_k != 0.  Pointers aligned to 16 bytes; N, the length of every other row (M where a_by_k, K for an
- * operand that is not by_k) multiples of 8; operands below 2 GiB: CHERRYQ_E_UNSUPPORTED otherwise.  `workspace` is zero and left
- * zero, `scratch` uninitialised, both may be null where their size is 0; calls that share them must not overlap (counts that
- * another call has changed can give wrong tiles or tiles of NaN, and no call that does not end).  The same inputs give the same bits.  cherryq_gemm_preferred: whether this is faster than the library's product (estimated; 0 also where a
- * call is not supported).
+ * operand that is not by_k) multiples of 8; operands below 2 GiB, rows of an operand by_k no longer than 34087038:
+ * CHERRYQ_E_UNSUPPORTED otherwise (the sizes of buffers are 0 where no form is supported).  `workspace` is zero and left zero, `scratch`
+ * uninitialised, both may be null where their size is 0; calls that share them must not overlap (counts that another call has
+ * changed can give wrong tiles or tiles of NaN; every call ends).  The same inputs give the same bits.  cherryq_gemm_preferred:
+ * whether this is faster than the library's product (estimated; 0 also where a call is not supported).
  */
 size_t cherryq_gemm_workspace_bytes(int M, int N, int K);
 size_t cherryq_gemm_scratch_bytes(int M, int N, int K);

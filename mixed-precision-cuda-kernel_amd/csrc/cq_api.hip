@@ -305,9 +305,9 @@ int cherryq_stream_capturing(void *stream) {
     return capture != hipStreamCaptureStatusNone;
 }
 
-size_t cherryq_gemm_workspace_bytes(int M, int N, int K) { return M > 0 && N > 0 && K > 0 ? cq::gemm_plan(M, N, K).workspace_bytes : 0; }
+size_t cherryq_gemm_workspace_bytes(int M, int N, int K) { return cq::gemm_sizes(M, N, K) ? cq::gemm_plan(M, N, K).workspace_bytes : 0; }
 
-size_t cherryq_gemm_scratch_bytes(int M, int N, int K) { return M > 0 && N > 0 && K > 0 ? cq::gemm_plan(M, N, K).scratch_bytes : 0; }
+size_t cherryq_gemm_scratch_bytes(int M, int N, int K) { return cq::gemm_sizes(M, N, K) ? cq::gemm_plan(M, N, K).scratch_bytes : 0; }
 
 int cherryq_gemm_preferred(int a_by_k, int b_by_k, int M, int N, int K) { return cq::gemm_preferred(a_by_k, b_by_k, M, N, K) ? 1 : 0; }
 

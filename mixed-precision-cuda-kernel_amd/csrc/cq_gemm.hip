@@ -376,11 +376,19 @@ bool gemm_preferred(bool a_by_k, bool b_by_k, int M, int N, int K) {
     return gemm_plan(M, N, K).cost < 0.95f * library;
 }
 
-// Whole 16-byte pieces along every row, and one buffer descriptor an operand
+// One buffer descriptor an operand, and numbers of tiles that fit the plan's
+bool gemm_sizes(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0) return false;
+    const long long most = 0x7fff0000ll, mtiles = (M - 1ll) / kTile + 1, ntiles = (N - 1ll) / kTile + 1;
+    return 2ll * M * K < most && 2ll * N * K < most && 2ll * M * N < (1ll << 40) && mtiles * ntiles < (1 << 24);
+}
+
+// Besides, whole 16-byte pieces along every row.  A step's last row of [K][free] starts 63 rows on: that has to fit 32 bits, or rows past K come
+// round to the array's start instead of reading zeros (only rows of 64 MB and more, of which there are few).
 bool gemm_supported(bool a_by_k, bool b_by_k, int M, int N, int K) {
-    if (M <= 0 || N <= 0 || K <= 0 || N % 8 || (a_by_k && M % 8) || (!(a_by_k && b_by_k) && K % 8)) return false;
-    const long long most = 0x7fff0000ll;
-    return 2ll * M * K < most && 2ll * N * K < most && 2ll * M * N < (1ll << 40) && (long long)ceil_div(M, kTile) * ceil_div(N, kTile) < (1 << 24);
+    constexpr int longest = ((1ll << 32) - 512) / (2 * 63);
+    return gemm_sizes(M, N, K) && N % 8 == 0 && (!a_by_k || (M % 8 == 0 && M <= longest)) && (!b_by_k || N <= longest) &&
+           ((a_by_k && b_by_k) || K % 8 == 0);
 }
 
 template <bool BF16>

@@ -224,6 +224,7 @@ struct GemmPlan {
     size_t scratch_bytes, workspace_bytes;
 };
 GemmPlan gemm_plan(int M, int N, int K);
+bool gemm_sizes(int M, int N, int K);  // what a plan is made for, whatever the form
 bool gemm_supported(bool a_by_k, bool b_by_k, int M, int N, int K);
 bool gemm_preferred(bool a_by_k, bool b_by_k, int M, int N, int K);  // faster than the library's product
 hipError_t launch_gemm(bool bf16, bool a_by_k, bool b_by_k, const void *a, const void *b, void *out, int M, int N, int K, const GemmPlan &plan,

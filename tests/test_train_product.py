@@ -301,6 +301,26 @@ def test_sizes_the_kernel_is_not_for():
     assert not quant_cuda.gemm_preferred(True, True, 4096, 1 << 20, 2048)  # past 2 GiB
 
 
+def test_limits_of_the_sizes():
+    """Offsets are 32 bits: rows of an operand by_k that 63 rows of which do not fit them are refused (in front of anything that reads the
+    pointers); sizes that no form takes have no plan, so nothing is computed from numbers of tiles that do not fit 32 bits."""
+    import quant_cuda
+    lib, fake, unsupported = quant_cuda._lib, 4096, -7
+    if torch.cuda.is_available():
+        pytest.skip("calls the entry point with addresses that are none: without a GPU only")
+
+    def refused(a_by_k, b_by_k, m, n, k):
+        return lib.cherryq_gemm_16(0, a_by_k, b_by_k, fake, fake, fake, m, n, k, None, 0, None, 0, None) == unsupported
+
+    wide = 34087040
+    for k in (8, 16, 24):
+        assert 2 * wide * k < 0x7FFF0000 and 63 * 2 * wide + 512 >= 1 << 32 > 63 * 2 * (wide - 8) + 512
+        assert refused(True, True, wide, 8, k) and refused(True, False, wide, 8, k) and refused(True, True, 8, wide, k) and refused(False, True, 8, wide, k)
+        assert not quant_cuda.gemm_preferred(True, True, wide, 8, k)
+    for m, n, k in ((2 ** 31 - 1, 2 ** 31 - 8, 8), (2 ** 31 - 1, 8, 8), (1 << 20, 1 << 20, 8), (1 << 21, 1 << 15, 1 << 11), (0, 8, 8), (8, 8, -8)):
+        assert lib.cherryq_gemm_workspace_bytes(m, n, k) == lib.cherryq_gemm_scratch_bytes(m, n, k) == 0
+
+
 def test_kernels_keep_their_distances(tmp_path):
     """The products are written out as inline assembly, around which the compiler keeps no distances (tests/test_mfma_distances.py)."""
     import os
