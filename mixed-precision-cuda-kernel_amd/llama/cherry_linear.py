@@ -155,12 +155,13 @@ class QuantLinear(nn.Linear):
 
     def _native_linear(self, x, weight):
         """The whole branch of the training forward in one native call, with one autograd node; None where it is not the
-        plain case (the caller's route then takes it or raises)."""
+        plain case (the caller's route then takes it or raises), and where a function that it stands for has been replaced
+        (torch's linear by a profiler or a sharding wrapper, the fake quantisation by a subclass, an instance or a patch)."""
         own = self.__dict__
         if (torch.compiler.is_compiling() or self.quantizer is not FullSymQuantizer or self.weight_layerwise
                 or not own.get("cherry_indices_registered") or "_adjust_weight" in own or "_fused_fake_quant" in own
-                or type(self)._adjust_weight is not QuantLinear._adjust_weight
-                or type(self)._fused_fake_quant is not QuantLinear._fused_fake_quant or not weight.is_cuda):
+                or (type(self)._adjust_weight, type(self)._fused_fake_quant) != _FAKE_QUANT_METHODS
+                or nn.functional.linear is not torch._C._nn.linear or not weight.is_cuda):
             return None
         import quant_cuda
         return quant_cuda.train_linear(x, weight, self.cherry_indices, self.w_bits, self.group_size)
@@ -214,3 +215,6 @@ class QuantLinear(nn.Linear):
 
     def forward(self, x: torch.Tensor, **kwargs) -> torch.Tensor:
         return self.quant_forward(x, **kwargs)
+
+
+_FAKE_QUANT_METHODS = (QuantLinear._adjust_weight, QuantLinear._fused_fake_quant)  # what the native call stands for

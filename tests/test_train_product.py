@@ -293,6 +293,24 @@ def test_a_saved_weight_of_another_shape_raises(native, dtype):
     assert native[1] == []
 
 
+def test_replaced_functions_are_called(monkeypatch):
+    """What the native call stands for may have been replaced: torch's linear, the class's fake quantisation, an instance's."""
+    from types import SimpleNamespace
+
+    import quant_cuda
+    lin = cl.QuantLinear(16, 24, w_bits=4, group_size=8, cherryq=True, cherry_fraction=1 / 2).train()
+    lin.register_cherry_indices(torch.arange(8))
+    on_gpu, taken = SimpleNamespace(is_cuda=True), object()
+    monkeypatch.setattr(quant_cuda, "train_linear", lambda *_: taken)
+    assert lin._native_linear(None, on_gpu) is taken
+    for where, name in ((vars(torch.nn.functional), "linear"), (cl.QuantLinear, "_adjust_weight"), (cl.QuantLinear, "_fused_fake_quant"),
+                        (vars(lin), "_adjust_weight"), (vars(lin), "_fused_fake_quant")):
+        with monkeypatch.context() as patch:
+            (patch.setitem if isinstance(where, dict) else patch.setattr)(where, name, lambda *a, **b: None)
+            assert lin._native_linear(None, on_gpu) is None, name
+        assert lin._native_linear(None, on_gpu) is taken
+
+
 def test_sizes_the_kernel_is_not_for():
     import quant_cuda
     for by_k in ((False, False), (False, True), (True, True)):
