@@ -92,6 +92,10 @@ struct Pool {
             if (t.defined() && t.numel() >= bytes) return t;
             if (t.defined()) size = std::max(size, 2 * t.numel());
         }
+        // Zeros that a graph writes are there only from its first replay on, so a call of another graph or outside would count from
+        // whatever lies there: while the stream records, what is missing is made for the call alone (a warm stream has it).
+        const bool own = zeroed && capturing && capturing(stream);
+        if (own) size = std::max<int64_t>(bytes, 1);
         // Without the lock: callers come with and without the interpreter's, and an allocation may ask for that one (a record of
         // allocations with Python's stacks).  Who comes second drops what they made.
         Tensor made;
@@ -104,6 +108,7 @@ struct Pool {
             const auto opts = at::TensorOptions().dtype(at::kByte).device(at::kCUDA, device);
             made = zeroed ? at::zeros({size}, opts) : at::empty({size}, opts);
         }
+        if (own) return made;
         std::lock_guard<std::mutex> hold(lock);
         Tensor &t = live[key];
         if (!t.defined() || t.numel() < bytes) {

@@ -621,11 +621,11 @@ def gemm(a, b, a_by_k=False, b_by_k=False, shape=None):
         stream = _current_stream(dev.index)
         nbytes = _lib.cherryq_gemm_workspace_bytes(m, n, k)
         # a recorded call's tickets are its own: other graphs and other calls use the stream's kept ones
-        ws = (torch.zeros(nbytes, dtype=torch.uint8, device=dev) if nbytes and _lib.cherryq_stream_capturing(stream)
+        ws = (None if not nbytes else torch.zeros(nbytes, dtype=torch.uint8, device=dev) if _lib.cherryq_stream_capturing(stream)
               else _workspace(dev, stream, nbytes))
         scratch = torch.empty(_lib.cherryq_gemm_scratch_bytes(m, n, k), dtype=torch.uint8, device=dev)  # the call's own
         rc = _lib.cherryq_gemm_16(a.dtype == torch.bfloat16, a_by_k, b_by_k, a.data_ptr(), b.data_ptr(), out.data_ptr(), m, n, k,
-                                  ws.data_ptr(), ws.numel(), _ptr(scratch), scratch.numel(), stream)
+                                  None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _ptr(scratch), scratch.numel(), stream)
     if rc != 0:
         _fail(rc, "gemm")
     return out

@@ -95,6 +95,36 @@ def test_replaced_buffers_and_workspace_growth():
     assert grown.numel() == 1 << 19 and int(grown.sum()) == 0
 
 
+def test_graphs_on_a_stream_without_a_workspace():
+    """The first calls on a stream are recorded, in two graphs, and the second one is replayed first: no graph counts from what only
+    the other one sets to zero, and nothing that a graph sets to zero is kept for calls outside."""
+    print("[case] host graphs on a new stream", flush=True)
+    import quant_cuda as qc
+    q, stream = _layer(4, 11008, 512), torch.cuda.Stream()
+    inputs = [torch.randn(rows, 11008, device="cuda").half() for rows in (1, 16)]
+    a = torch.randn(256, 64, device="cuda").half()
+    outs = [torch.empty(x.shape[0], 512, device="cuda", dtype=torch.float16) for x in inputs]
+    want = []
+    for x, out in zip(inputs, outs):
+        qc.vecquant4matmul_cherryq(x, q.qweight, q.cherry_weight, q.cherry_indices, q.scales, out.zero_(), 128)
+        want.append(out.clone())
+    graphs, made = [torch.cuda.CUDAGraph() for _ in inputs], []
+    for graph, x, out in zip(graphs, inputs, outs):
+        with torch.cuda.graph(graph, stream=stream):
+            qc.gemm(a, a)
+            out.zero_()
+            qc.vecquant4matmul_cherryq(x, q.qweight, q.cherry_weight, q.cherry_indices, q.scales, out, 128)
+            made.append(qc._host.workspace(0, stream.cuda_stream, 8))
+    kept = qc._host.workspace(0, stream.cuda_stream, 8)
+    assert len({t.data_ptr() for t in (*made, kept)}) == 3
+    for which in (1, 0, 0, 1):
+        outs[which].fill_(7)
+        graphs[which].replay()
+        torch.cuda.synchronize()
+        assert torch.equal(outs[which], want[which])
+    assert not kept.any()
+
+
 @pytest.mark.parametrize("stream", [False, True])
 def test_every_form_of_a_bias_is_added(stream):
     print("[case] host bias forms", stream, flush=True)

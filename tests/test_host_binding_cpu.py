@@ -246,6 +246,27 @@ print("done")
     assert r.returncode == 0 and r.stdout == "done\n", r.stderr
 
 
+def test_a_workspace_made_while_a_stream_records_is_not_kept(host):
+    """Its zeros are only recorded: another graph, or a call outside, would count from whatever lies there before the first replay."""
+    module, recording = host[0], 1
+    asks = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p)(lambda stream: recording if stream == 9 else 0)
+    module.bind_capturing(ctypes.cast(asks, ctypes.c_void_p).value)
+    try:
+        one, two = module.workspace(-1, 9, 64), module.workspace(-1, 9, 64)
+        assert one.data_ptr() != two.data_ptr() and one.numel() == two.numel() == 64 and not one.any()
+        recording = 0
+        kept = module.workspace(-1, 9, 64)
+        assert kept.data_ptr() not in (one.data_ptr(), two.data_ptr()) and kept.numel() > 64
+        recording = 1
+        assert module.workspace(-1, 9, 64).data_ptr() == kept.data_ptr()  # a warm stream's is there
+        larger = module.workspace(-1, 9, kept.numel() + 1)
+        assert larger.numel() == kept.numel() + 1 and module.workspace(-1, 9, 64).data_ptr() == kept.data_ptr()
+        scratch = module.scratch(-1, 9, 64)  # holds nothing from call to call
+        assert module.scratch(-1, 9, 64).data_ptr() == scratch.data_ptr()
+    finally:
+        module.bind_capturing(0)
+
+
 def test_the_library_beside_the_module_is_loaded(tmp_path):
     """... whatever lies on sys.path in front of it or was imported under its name."""
     (tmp_path / "cherryq_host.py").write_text("built_for = linear = None\n")
