@@ -207,7 +207,8 @@ int cherryq_fake_quant_f32(int w_bits, const void *weight, const int32_t *cherry
  * CHERRYQ_E_UNSUPPORTED otherwise (the sizes of buffers are 0 where no form is supported).  `workspace` is zero and left zero, `scratch`
  * uninitialised, both may be null where their size is 0; calls that share them must not overlap (counts that another call has
  * changed can give wrong tiles or tiles of NaN; every call ends).  The same inputs give the same bits.  cherryq_gemm_preferred:
- * whether this is faster than the library's product (estimated; 0 also where a call is not supported).
+ * whether this is faster than the library's product (estimated from the layer's three forms; 0 also for a_by_k without b_by_k,
+ * which was not compared, and where a call is not supported).
  */
 size_t cherryq_gemm_workspace_bytes(int M, int N, int K);
 size_t cherryq_gemm_scratch_bytes(int M, int N, int K);

@@ -367,9 +367,10 @@ GemmPlan gemm_plan(int M, int N, int K) {
 
 // Where the library's product takes longer: its time on the same 180 products (11 % off on average), by operations, bytes, depth, and for
 // two [K][free] operands the results' size, where it is slowest.  Chosen so, all of them take 8.1 ms, the library alone 9.8, the faster of
-// both each time 7.9; none is more than 6 % slower than the library.
+// both each time 7.9; none is more than 6 % slower than the library.  The fourth form, `a` as [K][M] and `b` as [N][K], is no product of the
+// layer and none of these: nothing is said of it.
 bool gemm_preferred(bool a_by_k, bool b_by_k, int M, int N, int K) {
-    if (!gemm_supported(a_by_k, b_by_k, M, N, K)) return false;
+    if ((a_by_k && !b_by_k) || !gemm_supported(a_by_k, b_by_k, M, N, K)) return false;
     const float m = (float)M, n = (float)N, k = (float)K, mbytes = 2e-6f * (m * k + n * k + m * n);
     float library = 7.1f + 1.69e-9f * m * n * k + 0.23f * mbytes + 1.9e-3f * k;
     if (a_by_k && b_by_k) library += 0.16f * mbytes + 0.55e-6f * m * n;

@@ -604,9 +604,9 @@ def gemm_preferred(a_by_k, b_by_k, m, n, k) -> bool:
     return bool(_lib.cherryq_gemm_preferred(a_by_k, b_by_k, m, n, k))
 
 
-def gemm(a, b, a_by_k=False, b_by_k=False, shape=None):
-    """a @ b.T for 16-bit matrices, fp32 sums; `a_by_k` / `b_by_k`: the operand is given transposed (contraction first);
-    `shape`: the result's, of as many elements.  No counterpart in the reference extension."""
+def gemm(a, b, a_by_k=False, b_by_k=False):
+    """a @ b.T for 16-bit matrices, fp32 sums; `a_by_k` / `b_by_k`: the operand is given transposed (contraction first).
+    No counterpart in the reference extension."""
     _check(a, "a", a.dtype, 2)
     _check(b, "b", a.dtype, 2, a.device)
     m, k = a.shape[::-1] if a_by_k else a.shape
@@ -615,9 +615,7 @@ def gemm(a, b, a_by_k=False, b_by_k=False, shape=None):
         raise RuntimeError(f"gemm: {tuple(a.shape)} and {tuple(b.shape)} of {a.dtype} do not multiply")
     dev = a.device
     with torch.cuda.device(dev):
-        out = torch.empty((m, n) if shape is None else shape, dtype=a.dtype, device=dev)
-        if out.numel() != m * n:
-            raise RuntimeError(f"gemm: {m} x {n} results do not fit shape {tuple(shape)}")
+        out = torch.empty((m, n), dtype=a.dtype, device=dev)
         stream = _current_stream(dev.index)
         nbytes = _lib.cherryq_gemm_workspace_bytes(m, n, k)
         # a recorded call's tickets are its own: other graphs and other calls use the stream's kept ones

@@ -319,6 +319,14 @@ def test_sizes_the_kernel_is_not_for():
     assert not quant_cuda.gemm_preferred(True, True, 4096, 1 << 20, 2048)  # past 2 GiB
 
 
+@pytest.mark.parametrize("m,n,k", [(2048, 11008, 4096), (4096, 11008, 2048), (11008, 4096, 2048), (8, 8, 8)])
+def test_the_form_that_was_not_compared_is_not_preferred(m, n, k):
+    import quant_cuda
+    assert not quant_cuda.gemm_preferred(True, False, m, n, k)
+    for by_k in ((False, False), (False, True), (True, True)):
+        assert quant_cuda.gemm_preferred(*by_k, m, n, k) == (k > 8)
+
+
 def test_limits_of_the_sizes():
     """Offsets are 32 bits: rows of an operand by_k that 63 rows of which do not fit them are refused (in front of anything that reads the
     pointers); sizes that no form takes have no plan, so nothing is computed from numbers of tiles that do not fit 32 bits."""
