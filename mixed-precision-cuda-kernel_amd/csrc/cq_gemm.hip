@@ -1,8 +1,10 @@
 // Dense 16-bit matrix products of quantisation-aware training,  D[M, N] = sum_k A(m, k) B(n, k)  with fp32 sums and one rounding:
 // the training layer's output  x W'^T  and its gradients  g W'  and  g^T x  (llama/cherry_linear.py:101-126 and autograd).
 //
-// Either operand may lie as [free][K] or as [K][free], so no transposed copy is made.  Bound by the power that the matrix cores
-// draw: 4096 x 4096 x 8192 runs at 1.35 PFLOP/s with the clock at 1.91 GHz (of 2.4) and the matrix cores busy 68 % of the time.
+// Either operand may lie as [free][K] or as [K][free], so no transposed copy is made.  One whole round of tiles is bound by the power
+// that the matrix cores draw: 4096 x 4096 x 8192 runs at 1.35 PFLOP/s with the clock at 1.91 GHz (of 2.4) and the matrix cores busy
+// 68 % of the time.  2048 rows of 4096 -> 11008 are not: 53 to 59 % at 2.05 to 2.14 GHz.  Their tiles leave an uneven last round (96, 86
+// and 96 steps where a compute unit's share is 86); the rest are a tile's two ends (7 us), sums through scratch (8 us) and the barrier a step.
 //   * A workgroup of eight wavefronts owns a tile of 256 x 256, a wavefront 128 x 64 of it: 128 accumulators, two wavefronts a
 //     SIMD, so that one's waits lie behind the other's products (four wavefronts of 128 x 128: 5 to 10 % slower at every size).
 //   * K in steps of 64 through two LDS buffers of 64 KB, filled by loads that go straight to LDS (through registers: 3 us a tile

@@ -103,10 +103,11 @@ __global__ __launch_bounds__(256) void pack_cherry_kernel(const __half *__restri
 // a contiguous range; 16 threads take a row of it in 16-byte chunks and scatter the halves to their
 // compacted positions in LDS.  Where a chunk's halves go does not depend on the row, so a thread
 // finds it once for the 8 rows it loads (two searches of the index list per chunk and row were what the
-// general form spent its time on).  A row of 65 dwords makes both the scatter (16 chunks x 4 rows) and
-// the later reads free of bank conflicts; bytes of four neighbouring rows leave as one dword, 128 bytes a line.
-// Bound by vector ALU first (about 14 operations an element, twice as many wavefronts a CU change nothing) and by one
-// read of the weight.  MI355X, 13824 x 5120 to 3 bits: 49 us (3.5 TB/s read + written),
+// general form spent its time on).  A row of 65 dwords spreads the scatter (16 chunks x 4 rows) and
+// the later reads over the banks; bytes of four neighbouring rows leave as one dword, 128 bytes a line.
+// No one unit bounds it: of 130 k cycles the vector ALU is busy 68 k (16 operations an element) and a compute unit's LDS 48 k, 29 k of
+// these in bank conflicts; the weight's lines are fetched 1.4 times, since neighbouring groups share them.  Twice as many
+// wavefronts a CU change nothing.  MI355X, 13824 x 5120 to 3 bits: 49 us (3.5 TB/s read + written),
 // with an address formed for each half and row, comparisons around loads and stores, cherry columns stored half by
 // half in the scatter and quotients of six operations 59 (188); the general form's three launches took 549.
 constexpr int kPackRows = 128, kPackStride = 65;  // dwords of LDS a row; halves 128 and 129 take what belongs nowhere
