@@ -528,20 +528,31 @@ Tensor product(const Tensor &a, bool a_by_k, const Tensor &b, bool b_by_k, int64
     return out;
 }
 
-// `value` with `weight`'s gradient, for second derivatives
-struct StraightThrough : torch::autograd::Function<StraightThrough> {
-    static Tensor forward(torch::autograd::AutogradContext *, const Tensor &, const Tensor &value) { return value.clone(); }
-    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *, torch::autograd::variable_list grads) {
-        return {grads[0], Tensor()};
-    }
+// A gradient handed on as it is
+struct StraightThrough : torch::autograd::Node {
+    torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override { return {grads[0]}; }
 };
+
+// `quantised` with the gradient of the weight that it was made from, for second derivatives.  The node that runs holds where that leads since
+// the forward pass; the weight itself may have been changed, replaced or given back.
+Tensor of_the_weight(const Tensor &quantised) {
+    const auto node = torch::autograd::get_current_node();
+    TORCH_CHECK(node, "second derivatives of the training layer are taken by autograd's engine");
+    const Tensor value = quantised.detach();
+    const auto &edge = node->next_edge(1);
+    if (edge.is_valid()) {
+        const std::shared_ptr<StraightThrough> on(new StraightThrough(), torch::autograd::deleteNode);
+        on->add_next_edge(edge);
+        torch::autograd::impl::set_gradient_edge(value, {on, on->add_input_metadata(value)});
+    }
+    return value;
+}
 
 // linear(x, quantised) with the straight-through gradient for the weight that was quantised (llama/cherry_linear.py:97-98)
 struct TrainLinear : torch::autograd::Function<TrainLinear> {
     static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &x, const Tensor &weight, const Tensor &quantised) {
         // what a gradient reads and no more: the other may be changed in place or given back
         ctx->save_for_backward({weight.requires_grad() ? x : Tensor(), x.requires_grad() ? quantised : Tensor()});
-        ctx->saved_data["weight"] = weight;  // for second derivatives only, so the optimiser may have stepped
         const int64_t n = weight.size(0), k = weight.size(1), rows = x.numel() / k;
         std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
         shape.back() = n;
@@ -560,7 +571,7 @@ struct TrainLinear : torch::autograd::Function<TrainLinear> {
             std::vector<int64_t> shape(g.sizes().begin(), g.sizes().end());
             shape.back() = k;
             if (twice) {
-                quantised = StraightThrough::apply(ctx->saved_data["weight"].toTensor(), quantised);
+                quantised = of_the_weight(quantised);
             } else if (n) {
                 dx = product(g, false, quantised, true, g.numel() / n, k, n, shape);
             }

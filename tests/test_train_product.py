@@ -5,7 +5,9 @@ Bound of the kernel: fp32 sums of exact 16-bit products, rounded once.  The roun
 the result, 2^-17 at the largest K here.  So 2^-11 / 2^-8 of the 2-norm holds with room."""
 import contextlib
 import ctypes
+import gc
 import shutil
+import weakref
 from pathlib import Path
 
 import pytest
@@ -138,6 +140,28 @@ def test_second_derivatives_equal_torch(native, dtype):
         (dx, dw) = torch.autograd.grad((f(xs, ws).float() ** 2).sum(), (xs, ws), create_graph=True)
         results.append(torch.autograd.grad((dx * v).float().sum() + (dw.float() ** 2).mean(), (xs, ws)))
     torch.testing.assert_close(*results, rtol=40 * torch.finfo(dtype).eps, atol=100 * torch.finfo(dtype).eps)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_second_derivatives_reach_the_weight_as_it_was(native, dtype):
+    """A computed weight that is changed in place behind the forward pass: the gradient goes where it came from then.  The node keeps
+    what its gradients multiply, not the weight."""
+    torch.manual_seed(3)
+    x, w = torch.randn(4, 16).to(dtype), torch.randn(8, 16).to(dtype)
+    results = []
+    for f in (native[0], through_torch):
+        xs, ws = x.clone().requires_grad_(), w.clone().requires_grad_()
+        h = ws * 1
+        y = f(xs, h)
+        h.mul_(3)
+        dx, = torch.autograd.grad((y.float() ** 2).sum(), xs, create_graph=True)
+        results.append(torch.autograd.grad(dx.float().sum(), (xs, ws)))
+    torch.testing.assert_close(*results, rtol=40 * torch.finfo(dtype).eps, atol=100 * torch.finfo(dtype).eps)
+    h = w.clone().requires_grad_() * 1
+    y, gone = native[0](x.clone().requires_grad_(), h), weakref.ref(h)
+    del h
+    gc.collect()
+    assert gone() is None and y.grad_fn is not None
 
 
 def test_calls_that_are_not_plain_are_left_to_the_general_route(native):
