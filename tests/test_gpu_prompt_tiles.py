@@ -58,3 +58,43 @@ def test_every_tile_shape(qc, bits, group, rows, k, n, c):
 def test_more_tiles_than_compute_units(qc, bits, group, rows, k, n, c):
     print("[case] prompt rounds", bits, k, n, c, group, rows, flush=True)
     against_64_bits(qc, bits, k, n, c, group, rows)
+
+
+# pieces of four columns, of eight and of 96 columns, 16 rows, shared K
+SCALE_CASES = [(66, 912, 11320, 112), (306, 320, 8456, 40), (423, 344, 4176, 0), (5, 264, 656, 8), (20, 272, 104, 8), (36, 264, 8304, 8)]
+
+
+@pytest.mark.parametrize("rows,k,n,c", SCALE_CASES)
+@pytest.mark.parametrize("bits,group", [(4, 128), (4, 160), (3, 128), (3, 96)])
+def test_weights_are_the_dense_ones_at_any_scale(qc, bits, group, rows, k, n, c):
+    """Rows that are ones of the identity: the product is the dense weight's value, whose one rounding from code times scale it has, bit for bit.
+    Half of the scales lie below 2^-12, where a half of them need not have an fp16 value."""
+    print("[case] prompt scales", bits, k, n, c, group, rows, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    kn, shape = k - c, (-(-(k - c) // group), n)
+    small, any_ = (torch.randint(1, end, shape, device="cuda", generator=gen, dtype=torch.int16) for end in (0x0c00, 0x6c00))
+    scales = torch.where(torch.rand(shape, device="cuda", generator=gen) < 0.5, small, any_).view(torch.float16)
+    q = torch.randint(0, 256, (kn // 8 * bits, n), device="cuda", generator=gen, dtype=torch.uint8)
+    cw = torch.randn((c, n), device="cuda", generator=gen).half()
+    idx = torch.randperm(k, device="cuda", generator=gen)[:c].sort().values.to(torch.int16)
+    at = torch.randint(0, k, (rows,), device="cuda", generator=gen)
+    x = torch.nn.functional.one_hot(at, k).half()
+    out = torch.zeros((rows, n), dtype=torch.float16, device="cuda")
+    qc.matmul_cherryq(bits, x, q, cw, idx, scales, out, group)
+    assert torch.equal(out, qc.unpack_cherryq(bits, q, cw, idx, scales, k, group).t()[at])
+
+
+@pytest.mark.parametrize("bits,group", [(4, 128), (4, 160), (3, 128), (3, 96)])
+@pytest.mark.parametrize("rows", [24, 100, 300])
+def test_an_infinite_scale_is_no_nan(qc, bits, group, rows):
+    print("[case] prompt infinite scale", bits, group, rows, flush=True)
+    k, n = 1280, 1032
+    q = torch.zeros((k // 8 * bits, n), device="cuda", dtype=torch.uint8)  # the lowest code: weights of -c_b s
+    scales = torch.ones((-(-k // group), n), device="cuda", dtype=torch.float16)
+    scales[1, 3::5] = float("inf")
+    cw, idx = torch.zeros((0, n), dtype=torch.float16, device="cuda"), torch.zeros(0, dtype=torch.int16, device="cuda")
+    out = torch.zeros((rows, n), dtype=torch.float16, device="cuda")
+    qc.matmul_cherryq(bits, torch.ones((rows, k), dtype=torch.float16, device="cuda"), q, cw, idx, scales, out, group)
+    want = torch.full((rows, n), -k * (2 ** bits - 1) / 2, device="cuda")
+    want[:, 3::5] = float("-inf")
+    assert torch.equal(out.float(), want.half().float())
