@@ -212,7 +212,8 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(const __half *__
         }
         const unsigned long long cherries = __ballot(cherry >= 0);
         const int behind = 64 * wave + lane - (before - front) - __popcll(cherries & ((1ull << lane) - 1ull));  // normal ones of the head in front
-        // (channels that are not in order or not distinct are nobody's: what becomes of them stays within the arrays)
+        // (channels that are not in order or not distinct are nobody's: what becomes of them stays within the arrays, by the masks here and
+        // where the bytes are read, of which some are then never written, and by the bound on `cherries`)
         if (cherry >= 0) s_cherry[(cherry - front) & 127] = (uint8_t)(64 * wave + lane);
         else s_normal[behind & 127] = (uint8_t)(64 * wave + lane);
         if (wave == 1 && lane == 0) s_first[0] = front, s_first[1] = before + __popcll(cherries);
@@ -251,7 +252,7 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(const __half *__
         } else {
             *reinterpret_cast<half8_t *>(&s_row[row][8 * c]) = res;
             __syncthreads();
-            const int front = s_first[0], cherries = s_first[1] - front, p0 = max(128 * head - front, 0), p1 = p0 + 128 - cherries;
+            const int front = s_first[0], cherries = min(s_first[1] - front, 128), p0 = max(128 * head - front, 0), p1 = p0 + 128 - cherries;
             const int last = head == n_heads - 1 ? to.units * 16 : ceil_div(p1, 8);  // the last head's: zeros up to the unit's end
             _Float16 *const a = reinterpret_cast<_Float16 *>(to.a + (size_t)(q0 / 16) * 64 + (t & 15));
             auto place = [&](int eight) { return a + ((size_t)(eight >> 2) * to.m16 * 64 + (eight & 3) * 16) * 8; };
@@ -260,7 +261,7 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(const __half *__
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
                     const int p = 8 * eight + prompt_ord<BITS>(e);
-                    v[e] = p >= p0 && p < p1 ? s_row[t & 15][s_normal[p - p0]] : (_Float16)0.f;
+                    v[e] = p >= p0 && p < p1 ? s_row[t & 15][s_normal[p - p0] & 127] : (_Float16)0.f;
                 }
                 if (8 * eight >= p0 && (8 * eight + 8 <= p1 || head == n_heads - 1)) {
                     *reinterpret_cast<half8_t *>(place(eight)) = v;
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(const __half *__
                     }
                 }
             }
-            for (int j = t >> 4; j < cherries; j += 16) place(to.units * 16 + (front + j) / 8)[(front + j) & 7] = s_row[t & 15][s_cherry[j]];
+            for (int j = t >> 4; j < cherries; j += 16) place(to.units * 16 + (front + j) / 8)[(front + j) & 7] = s_row[t & 15][s_cherry[j] & 127];
             if (head == n_heads - 1) {
                 const half8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
                 for (int eight = to.C / 8 + (t >> 4); eight < to.csteps * 4; eight += 16)
