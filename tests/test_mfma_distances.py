@@ -78,6 +78,8 @@ def test_prompt_kernels_keep_their_distances(tmp_path):
             code = [line.split("//")[0].split(None, 1) for line in body.splitlines() if line.strip() and not line.rstrip().endswith(":")]
             kernels[symbol] = [(x[0], [o.strip() for o in x[1].split(",")] if len(x) > 1 else []) for x in code if x]
     products = {symbol: code for symbol, code in kernels.items() if any(op.startswith("v_mfma") for op, _ in code)}
-    assert len(products) >= 52
+    source = open(os.path.join(os.path.dirname(LIB), "csrc", "cq_prompt.hip")).read()
+    shapes = len(re.findall(r"^    X\(\d+,", source, re.M))  # each in both widths of codes, for groups of whole units and others
+    assert shapes >= 15 and len(products) == 4 * shapes
     for symbol, code in products.items():
         assert not too_close(code), (symbol, too_close(code)[:4])
