@@ -26,3 +26,7 @@ SHAPE_CASES = [
 # more tiles of 192 or 256 rows than there are compute units, so that a workgroup goes on to further ones: one unit of 128 positions, an even and an
 # odd number of them, a ragged last one; no cherries, some, several chunks of steps
 ROUND_CASES = [(2000, 128, 8200, 0), (2000, 264, 8200, 8), (1990, 392, 8264, 8), (1700, 1000, 12296, 40), (1500, 904, 13000, 520)]
+# the same with K split: a workgroup goes on from one split's tile to another's, so that its units, cherry steps (the last split's only: none, one, two
+# chunks and more) and tickets change; ragged last splits
+SPLIT_ROUND_CASES = [(950, 9808, 4136, 0), (516, 11128, 7048, 136), (306, 25216, 5520, 520), (207, 23344, 12640, 40), (398, 16944, 9088, 264),
+                     (395, 16424, 8304, 520)]

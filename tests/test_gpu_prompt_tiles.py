@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from prompt_cases import ROUND_CASES, SHAPE_CASES
+from prompt_cases import ROUND_CASES, SHAPE_CASES, SPLIT_ROUND_CASES
 
 pytestmark = pytest.mark.gpu
 
@@ -53,7 +53,7 @@ def test_every_tile_shape(qc, bits, group, rows, k, n, c):
     against_64_bits(qc, bits, k, n, c, group, rows)
 
 
-@pytest.mark.parametrize("rows,k,n,c", ROUND_CASES)
+@pytest.mark.parametrize("rows,k,n,c", ROUND_CASES + SPLIT_ROUND_CASES)
 @pytest.mark.parametrize("bits,group", [(4, 128), (3, 96)])
 def test_more_tiles_than_compute_units(qc, bits, group, rows, k, n, c):
     print("[case] prompt rounds", bits, k, n, c, group, rows, flush=True)
