@@ -78,8 +78,25 @@ def test_prompt_kernels_keep_their_distances(tmp_path):
             code = [line.split("//")[0].split(None, 1) for line in body.splitlines() if line.strip() and not line.rstrip().endswith(":")]
             kernels[symbol] = [(x[0], [o.strip() for o in x[1].split(",")] if len(x) > 1 else []) for x in code if x]
     products = {symbol: code for symbol, code in kernels.items() if any(op.startswith("v_mfma") for op, _ in code)}
-    source = open(os.path.join(os.path.dirname(LIB), "csrc", "cq_prompt.hip")).read()
-    shapes = len(re.findall(r"^    X\(\d+,", source, re.M))  # each in both widths of codes, for groups of whole units and others
-    assert shapes >= 15 and len(products) == 4 * shapes
+    assert len(products) >= 52
     for symbol, code in products.items():
         assert not too_close(code), (symbol, too_close(code)[:4])
+
+
+@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="needs ROCm's llvm-objdump")
+def test_every_prompt_kernel_is_among_those_checked(tmp_path):
+    """One kernel a line of the shape tables, both widths of codes, groups of whole units and others: all of them by the names that the test
+    above looks for, with matrix instructions inside."""
+    lib = shutil.copy(LIB, tmp_path)
+    subprocess.run([OBJDUMP, "--offloading", lib], check=True, capture_output=True, cwd=tmp_path)
+    products = 0
+    for name in sorted(os.listdir(tmp_path)):
+        path = str(tmp_path / name)
+        if name.endswith("gfx950") and b"prompt_shared_k_kernel" in open(path, "rb").read():
+            text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--no-leading-addr", path], check=True, capture_output=True,
+                                  text=True).stdout
+            bodies = re.findall(r"^<\S*prompt_\w*kernel\S*>:\n(.*?)(?=^<|\Z)", text, re.S | re.M)
+            products += sum("v_mfma" in body for body in bodies)
+    source = open(os.path.join(os.path.dirname(LIB), "csrc", "cq_prompt.hip")).read()
+    shapes = len(re.findall(r"^    X\(\d+,", source, re.M))
+    assert shapes >= 15 and products == 4 * shapes
