@@ -730,8 +730,7 @@ class CherryLlamaDecoder(nn.Module):
         """The whole prompt in one batched pass, as the reference's model processes it
         (llama/modeling_llama_quant.py:1009-1100): every linear sees all T rows at once (the prompt
         kernels from 17 rows, mostly also below); residual + RMSNorm, rotary + cache write, causal
-        attention and SiLU * up are launches with the reference's rounding points (_prefill_layers: all of them in one call, whose
-        RMSNorms read the residual's sum before it is rounded).  Fills the KV
+        attention and SiLU * up are launches with the reference's rounding points (_prefill_layers: all of them in one call).  Fills the KV
         caches for positions 0..T-1, leaves the decoder exactly where T token steps would (position T, the
         first generated token predicted and embedded) and returns the last position's logits."""
         cfg, dev = self.cfg, self.k_cache.get_device()
