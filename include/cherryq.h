@@ -510,8 +510,8 @@ int cherryq_prefill_attention_f16(const void *q, const void *k, const void *v, c
 /*
  * The decoder layers of a prompt of `tokens` (17 and more) positions from 0, in one call: residual + RMSNorm, q/k/v, attention with
  * cache writes, o_proj, residual + RMSNorm, gate/up, SiLU * up, down_proj (llama/modeling_llama_quant.py:754-775), with
- * the roundings of the single calls above.  RMSNorm and SiLU hand their rows to the products in the order these
- * read.  hidden (tokens, hidden_size) is updated in place; delta (tokens, hidden_size) receives the last layer's
+ * the roundings of the single calls above.  RMSNorm, SiLU and, for up to 512 tiles of 16 positions x heads, the attention hand
+ * their rows to the products in the order these read.  hidden (tokens, hidden_size) is updated in place; delta (tokens, hidden_size) receives the last layer's
  * down_proj, which is still to be added.  `mul` of the products' layers is not used.  hidden_size at most 8192, intermediate sizes
  * at most 28672, at most 248 cherries a layer, head_dim 128; o_proj reads n_heads * 128 features.
  * workspace (all zero before and after) and scratch (uninitialised) of the sizes that the two functions answer, 256-byte aligned.
