@@ -53,10 +53,17 @@ def test_every_tile_shape(qc, bits, group, rows, k, n, c):
     against_64_bits(qc, bits, k, n, c, group, rows)
 
 
-@pytest.mark.parametrize("rows,k,n,c", ROUND_CASES + SPLIT_ROUND_CASES)
+@pytest.mark.parametrize("rows,k,n,c", ROUND_CASES)
 @pytest.mark.parametrize("bits,group", [(4, 128), (3, 96)])
 def test_more_tiles_than_compute_units(qc, bits, group, rows, k, n, c):
     print("[case] prompt rounds", bits, k, n, c, group, rows, flush=True)
+    against_64_bits(qc, bits, k, n, c, group, rows)
+
+
+@pytest.mark.parametrize("rows,k,n,c", SPLIT_ROUND_CASES)
+@pytest.mark.parametrize("bits,group", [(4, 128), (3, 96)])
+def test_more_pieces_of_split_tiles_than_compute_units(qc, bits, group, rows, k, n, c):
+    print("[case] prompt split rounds", bits, k, n, c, group, rows, flush=True)
     against_64_bits(qc, bits, k, n, c, group, rows)
 
 
